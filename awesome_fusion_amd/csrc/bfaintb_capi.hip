@@ -23,6 +23,8 @@ hipError_t launch_probe_read(const void* src, size_t bytes, void* sink, hipStrea
 hipError_t launch_pack_colmajor(uint8_t* dst, const uint8_t* src, uint32_t n, uint32_t k, uint32_t ldb_bytes, int bits, hipStream_t stream);
 hipError_t launch_pack(uint8_t* dst, const uint8_t* src, uint32_t n, uint32_t k, uint32_t ldb_bytes, int bits, bool unpack,
                        hipStream_t stream);
+hipError_t launch_quantize(uint8_t* b, uint16_t* scale, const void* w, int type, uint32_t n, uint32_t k, uint32_t ldw, uint32_t ldb_bytes,
+                           int bits, uint32_t group_size, hipStream_t stream);
 hipError_t launch_decode_packed(const GemmParams& p, int bits, hipStream_t stream);
 hipError_t launch_prefill_packed(const GemmParams& p, int bits, hipStream_t stream, bool wreg);
 hipError_t launch_prefill128(const GemmParams& p, int bits, bool packed, hipStream_t stream);
@@ -1061,6 +1063,23 @@ static int repack(void* dst, const void* src, uint32_t n, uint32_t k, uint32_t l
     if (misaligned16(dst) || misaligned16(src)) return BFAINTB_ERR_ALIGNMENT;
     return (int)bfaintb::launch_pack(static_cast<uint8_t*>(dst), static_cast<const uint8_t*>(src), n, k,
                                      weight_bits == 8 ? ldb : ldb / 2u, weight_bits, unpack, static_cast<hipStream_t>(stream));
+}
+
+int bfaintb_quantize(void* b, void* scale, const void* w, int weight_type, uint32_t n, uint32_t k, uint32_t ldw, int weight_bits,
+                     uint32_t group_size, void* stream)
+{
+    int e = check_format(k, weight_bits, group_size);
+    if (e) return e;
+    if (weight_type != BFAINTB_WEIGHT_BF16 && weight_type != BFAINTB_WEIGHT_F16 && weight_type != BFAINTB_WEIGHT_F32) return BFAINTB_ERR_UNSUPPORTED;
+    e = check_shape(1, n, k, weight_bits);
+    if (e) return e;
+    if (k > (1u << 21)) return BFAINTB_ERR_BAD_SHAPE;  // (tiles and groups along k are the grid's y)
+    if (ldw < k || ldw % 8u != 0) return BFAINTB_ERR_BAD_LD;
+    if (n == 0) return BFAINTB_OK;
+    if (b == nullptr || scale == nullptr || w == nullptr) return BFAINTB_ERR_NULL_POINTER;
+    if (misaligned16(b) || misaligned16(scale) || misaligned16(w)) return BFAINTB_ERR_ALIGNMENT;
+    return (int)bfaintb::launch_quantize(static_cast<uint8_t*>(b), static_cast<uint16_t*>(scale), w, weight_type, n, k, ldw, n * (uint32_t)weight_bits / 8u,
+                                         weight_bits, group_size, static_cast<hipStream_t>(stream));
 }
 
 int bfaintb_prepack(void* packed, const void* b, uint32_t n, uint32_t k, uint32_t ldb, int weight_bits, void* stream)

@@ -47,33 +47,68 @@ __device__ __forceinline__ size_t packed_offset(uint32_t row, uint32_t col, uint
     }
 }
 
-// one thread per packed byte: gathers its 1 or 2 codes from the row-major matrix
-template <int BITS>
-__global__ void __launch_bounds__(256) pack_kernel(uint8_t* __restrict__ dst, const uint8_t* __restrict__ src, uint32_t n, uint32_t k,
-                                                   uint32_t ldb_bytes)
+// Four bytes of four dwords, transposed: byte j of row i -> byte i of row j.
+__device__ __forceinline__ void transpose_bytes4(uint32_t (&x)[4])
 {
-    const size_t total = (size_t)n * k * BITS / 8;
-    const uint32_t chunks = k / PackedFormat<BITS>::kChunkRows;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
-        const size_t lane_slot = i >> 4;
-        const uint32_t within = (uint32_t)(i & 15u);
-        const uint32_t lane = (uint32_t)(lane_slot & 63u);
-        const size_t chunk = lane_slot >> 6;
-        const uint32_t kc = (uint32_t)(chunk % chunks), nb = (uint32_t)(chunk / chunks);
-        const uint32_t nl = lane & 15u, kg = lane >> 4;
-        const uint32_t col = 16u * nb + nl;
-        if constexpr (BITS == 8) {
-            const uint32_t h = within >> 3, r = within & 7u;
-            const uint32_t row = 64u * kc + 32u * h + 8u * kg + r;
-            dst[i] = src[(size_t)row * ldb_bytes + col];
-        } else {
-            const uint32_t h = within >> 2, r0 = (within & 3u) * 2u;
-            const uint32_t row = 128u * kc + 32u * h + 8u * kg + r0;
-            const uint32_t shift = (col & 1u) * 4u;
-            const uint32_t lo = (src[(size_t)row * ldb_bytes + (col >> 1)] >> shift) & 15u;
-            const uint32_t hi = (src[(size_t)(row + 1u) * ldb_bytes + (col >> 1)] >> shift) & 15u;
-            dst[i] = (uint8_t)(lo | (hi << 4));
+    const uint32_t a = __builtin_amdgcn_perm(x[1], x[0], 0x05010400u), b = __builtin_amdgcn_perm(x[1], x[0], 0x07030602u);
+    const uint32_t c = __builtin_amdgcn_perm(x[3], x[2], 0x05010400u), d = __builtin_amdgcn_perm(x[3], x[2], 0x07030602u);
+    x[0] = __builtin_amdgcn_perm(c, a, 0x05040100u);
+    x[1] = __builtin_amdgcn_perm(c, a, 0x07060302u);
+    x[2] = __builtin_amdgcn_perm(d, b, 0x05040100u);
+    x[3] = __builtin_amdgcn_perm(d, b, 0x07060302u);
+}
+
+// Eight nibbles of eight dwords, transposed: nibble j of row i -> nibble i of row j.
+__device__ __forceinline__ void transpose_nibbles8(uint32_t (&x)[8])
+{
+    // nibbles within bytes, between rows one apart; then the bytes of the even and of the odd rows are two 4 x 4 transposes
+    uint32_t even[4], odd[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        even[i] = (x[2 * i] & 0x0f0f0f0fu) | ((x[2 * i + 1] & 0x0f0f0f0fu) << 4);
+        odd[i] = ((x[2 * i] >> 4) & 0x0f0f0f0fu) | (x[2 * i + 1] & 0xf0f0f0f0u);
+    }
+    transpose_bytes4(even);
+    transpose_bytes4(odd);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[2 * j] = even[j], x[2 * j + 1] = odd[j];
+}
+
+// Row-major -> packed.  A thread owns a dword's worth of columns (8 of 4-bit, 4 of 8-bit codes) and the rows one k-group of
+// lanes (kg) holds of a chunk: it loads those dwords — the 64 lanes of a wave side by side, 256 bytes of a row — turns each
+// run of 8 rows in registers and stores the 16 bytes of each of its columns; a thread's stores are 128 (64) bytes in a row.
+// Bound by memory: 11008 x 4096 4-bit, 22 MB in and 22 MB out (a thread per packed byte, gathering its codes one by one,
+// took 81 us).
+template <int BITS>
+__global__ void __launch_bounds__(256) pack_kernel(uint8_t* __restrict__ dst, const uint8_t* __restrict__ src, uint32_t n, uint32_t chunks,
+                                                   uint32_t ldb_bytes, uint32_t col_blocks)
+{
+    constexpr uint32_t kCols = 32u / BITS, kBlocks = PackedFormat<BITS>::kBlocks;
+    const uint32_t col = (blockIdx.x % col_blocks * 64u + (threadIdx.x & 63u)) * kCols, kg = threadIdx.x >> 6, kc = blockIdx.x / col_blocks;
+    if (col >= n) return;
+    const uint8_t* from = src + (size_t)(kc * PackedFormat<BITS>::kChunkRows + 8u * kg) * ldb_bytes + col * BITS / 8u;
+    uint32_t x[kBlocks][8];
+#pragma unroll
+    for (uint32_t h = 0; h < kBlocks; ++h)
+#pragma unroll
+        for (uint32_t r = 0; r < 8; ++r) x[h][r] = *reinterpret_cast<const uint32_t*>(from + (size_t)(32u * h + r) * ldb_bytes);
+    uint4* to = reinterpret_cast<uint4*>(dst) + ((size_t)(col >> 4) * chunks + kc) * 64u + 16u * kg + (col & 15u);
+    if constexpr (BITS == 8) {
+        uint32_t lo[2][4], hi[2][4];  // rows 0 .. 3 and 4 .. 7 of each K-block
+#pragma unroll
+        for (uint32_t h = 0; h < 2; ++h) {
+#pragma unroll
+            for (uint32_t r = 0; r < 4; ++r) lo[h][r] = x[h][r], hi[h][r] = x[h][4 + r];
+            transpose_bytes4(lo[h]);
+            transpose_bytes4(hi[h]);
         }
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) to[j] = make_uint4(lo[0][j], hi[0][j], lo[1][j], hi[1][j]);
+    } else {
+#pragma unroll
+        for (uint32_t h = 0; h < 4; ++h) transpose_nibbles8(x[h]);
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) to[j] = make_uint4(x[0][j], x[1][j], x[2][j], x[3][j]);
     }
 }
 
@@ -142,11 +177,14 @@ hipError_t launch_pack_colmajor(uint8_t* dst, const uint8_t* src, uint32_t n, ui
 hipError_t launch_pack(uint8_t* dst, const uint8_t* src, uint32_t n, uint32_t k, uint32_t ldb_bytes, int bits, bool unpack,
                        hipStream_t stream)
 {
+    if (!unpack) {
+        const uint32_t col_blocks = (n / (32u / (uint32_t)bits) + 63u) / 64u, chunks = k / (bits == 8 ? PackedFormat<8>::kChunkRows : PackedFormat<4>::kChunkRows);
+        return launch_kernel(bits == 8 ? pack_kernel<8> : pack_kernel<4>, dim3(col_blocks * chunks, 1, 1), dim3(256, 1, 1), 0, stream, dst, src, n,
+                             chunks, ldb_bytes, col_blocks);
+    }
     const size_t total = (size_t)n * k * (uint32_t)bits / 8;
     const uint32_t grid = (uint32_t)((total + 255) / 256 < 65536 ? (total + 255) / 256 : 65536);
-    void (*kernel)(uint8_t*, const uint8_t*, uint32_t, uint32_t, uint32_t) =
-        bits == 8 ? (unpack ? unpack_kernel<8> : pack_kernel<8>) : (unpack ? unpack_kernel<4> : pack_kernel<4>);
-    return launch_kernel(kernel, dim3(grid, 1, 1), dim3(256, 1, 1), 0, stream, dst, src, n, k, ldb_bytes);
+    return launch_kernel(bits == 8 ? unpack_kernel<8> : unpack_kernel<4>, dim3(grid, 1, 1), dim3(256, 1, 1), 0, stream, dst, src, n, k, ldb_bytes);
 }
 
 // ---------------------------------------------------------------------------------------------------------------

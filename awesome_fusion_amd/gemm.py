@@ -108,6 +108,8 @@ def lib():
         L.bfaintb_prepack.argtypes = [_vp, _vp, _u32, _u32, _u32, C.c_int, _vp]
         L.bfaintb_prepack_colmajor.restype = C.c_int
         L.bfaintb_prepack_colmajor.argtypes = [_vp, _vp, _u32, _u32, _u32, C.c_int, _vp]
+        L.bfaintb_quantize.restype = C.c_int
+        L.bfaintb_quantize.argtypes = [_vp, _vp, _vp, C.c_int, _u32, _u32, _u32, C.c_int, _u32, _vp]
         L.bfaintb_unpack.restype = C.c_int
         L.bfaintb_unpack.argtypes = [_vp, _vp, _u32, _u32, _u32, C.c_int, _vp]
         L.bfaintb_gemm_prepacked.restype = C.c_int
@@ -353,6 +355,17 @@ def prepack_colmajor(packed, b, n, k, ldb=None, weight_bits=8, stream=None, chec
     rc = lib().bfaintb_prepack_colmajor(_ptr(packed), _ptr(b), n, k, k if ldb is None else ldb, weight_bits, _stream_handle(stream))
     if rc and check:
         raise BfaintbError(rc, "bfaintb_prepack_colmajor")
+    return rc
+
+
+WEIGHT_BF16, WEIGHT_F16, WEIGHT_F32 = 0, 1, 2
+
+
+def quantize(b, scale, w, n, k, ldw=None, weight_type=WEIGHT_BF16, weight_bits=8, group_size=0, stream=None, check=True):
+    """Float weight [n, ldw] (k contiguous) -> row-major codes [k, n * bits / 8] and bf16 scales [groups, n] (bfaintb_quantize)."""
+    rc = lib().bfaintb_quantize(_ptr(b), _ptr(scale), _ptr(w), weight_type, n, k, k if ldw is None else ldw, weight_bits, group_size, _stream_handle(stream))
+    if rc and check:
+        raise BfaintbError(rc, "bfaintb_quantize")
     return rc
 
 

@@ -25,7 +25,7 @@ import torch
 from .gemm import (gemm as _gemm, gemm_prepacked as _gemm_prepacked, prepack as _prepack, prepack_bytes as _prepack_bytes,
                    prepack_colmajor as _prepack_colmajor,
                    prepacked_workspace_bytes as _prepacked_workspace_bytes,
-                   workspace_bytes as _workspace_bytes, workspace_init as _workspace_init)
+                   quantize as _quantize, workspace_bytes as _workspace_bytes, workspace_init as _workspace_init)
 
 _LIB_NAME = "awesome_fusion"
 _workspaces = {}
@@ -181,11 +181,35 @@ def prepack_weight(b, weight_bits=8, column_major=False):
     return packed
 
 
+_WEIGHT_TYPES = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
+
+
+def _quantizes_on_device(weight, weight_bits, group_size):
+    """Whether bfaintb_quantize serves this weight: on the GPU, of a type and shape the GEMM kernels can go on to read
+    (anything else, and the CPU, takes the torch form, which gives the same codes)."""
+    n, k = weight.shape
+    return (weight.is_cuda and weight.dtype in _WEIGHT_TYPES and weight_bits in (8, 4) and n % 16 == 0 and k % 8 == 0 and 0 < n and 0 < k <= 1 << 21
+            and (group_size == 0 or (group_size % 32 == 0 and k % group_size == 0)))
+
+
+def _quantize_on_device(w, weight_bits, group_size):
+    n, k = w.shape
+    if w.stride(1) != 1 or w.stride(0) < k or w.stride(0) % 8 or w.data_ptr() % 16:
+        w = w.contiguous()
+    b = torch.empty((k, n * weight_bits // 8), dtype=torch.uint8, device=w.device)
+    scale = torch.empty((k // group_size if group_size else 1, n), dtype=torch.bfloat16, device=w.device)
+    with torch.cuda.device(w.device):
+        _quantize(b, scale, w, n, k, ldw=w.stride(0), weight_type=_WEIGHT_TYPES[w.dtype], weight_bits=weight_bits, group_size=group_size)
+    return b, scale
+
+
 def quantize_weight(weight, weight_bits=8, group_size=0):
     """float weight [n_out, k_in] (a torch Linear's layout) -> (b uint8 [k, n*bits/8], scale bf16 [groups, n]).
 
     Symmetric: scale = max|w| over the group / qmax, rounded to bf16 first, q = round(w / scale) clamped to the
     code range, stored in the library's wire format (excess-128 bytes; excess-8 nibbles, even column low)."""
+    if _quantizes_on_device(weight, weight_bits, group_size):
+        return _quantize_on_device(weight.detach(), weight_bits, group_size)
     w = weight.detach().float().t().contiguous()  # [k, n]
     k, n = w.shape
     g = group_size if group_size else k
@@ -203,25 +227,42 @@ def quantize_weight(weight, weight_bits=8, group_size=0):
     return b, scale
 
 
+def _check_features(in_features, out_features):
+    if out_features % 16 or in_features % 8:
+        raise ValueError("QuantLinear: the kernels need out_features % 16 == 0 (rows of B stay 16-byte aligned) and in_features % 8 == 0")
+
+
 class QuantLinear(torch.nn.Module):
     """y = x @ dequant(B, scale) (+ bias): a Linear whose weight lives as int8/int4 codes and bf16 scales.
 
     The bias, if any, is added inside the kernel, to the fp32 sums."""
 
     def __init__(self, in_features, out_features, weight_bits=8, group_size=0, bias=False, device=None):
-        super().__init__()
-        if out_features % 16 or in_features % 8:
-            raise ValueError("QuantLinear: the kernels need out_features % 16 == 0 (rows of B stay 16-byte aligned) and in_features % 8 == 0")
+        _check_features(in_features, out_features)
         groups = in_features // group_size if group_size else 1
+        self._set_up(in_features, out_features, weight_bits, group_size,
+                     torch.zeros((in_features, out_features * weight_bits // 8), dtype=torch.uint8, device=device),
+                     torch.zeros((groups, out_features), dtype=torch.bfloat16, device=device),
+                     torch.zeros(out_features, dtype=torch.bfloat16, device=device) if bias else None)
+
+    def _set_up(self, in_features, out_features, weight_bits, group_size, qweight, scales, bias):
+        super().__init__()
         self.in_features, self.out_features = in_features, out_features
         self.weight_bits, self.group_size = weight_bits, group_size
         self.prepacked = False
-        self.register_buffer("qweight", torch.zeros((in_features, out_features * weight_bits // 8), dtype=torch.uint8, device=device))
-        self.register_buffer("scales", torch.zeros((groups, out_features), dtype=torch.bfloat16, device=device))
-        self.bias = torch.nn.Parameter(torch.zeros(out_features, dtype=torch.bfloat16, device=device)) if bias else None
+        self.register_buffer("qweight", qweight)
+        self.register_buffer("scales", scales)
+        self.bias = None if bias is None else torch.nn.Parameter(bias)
 
     @classmethod
     def from_float(cls, linear, weight_bits=8, group_size=0):
+        if cls is QuantLinear:  # the quantiser's own tensors become the buffers: nothing is zeroed first and copied over
+            _check_features(linear.in_features, linear.out_features)
+            b, s = quantize_weight(linear.weight, weight_bits, group_size)
+            q = cls.__new__(cls)
+            q._set_up(linear.in_features, linear.out_features, weight_bits, group_size, b, s,
+                      None if linear.bias is None else linear.bias.detach().to(torch.bfloat16, copy=True))
+            return q
         q = cls(linear.in_features, linear.out_features, weight_bits, group_size, linear.bias is not None, linear.weight.device)
         b, s = quantize_weight(linear.weight, weight_bits, group_size)
         q.qweight.copy_(b)

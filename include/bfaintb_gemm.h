@@ -257,6 +257,19 @@ BFAINTB_API int bfaintb_static_scratch_reset(void* stream);
 BFAINTB_API int bfaintb_debug_control(uint32_t what, uint32_t value);
 
 /*
+ * Quantises a float weight on the device: w [n, ldw] (row i = output column i, k contiguous; ldw >= k, a multiple of 8), of
+ * type weight_type, -> row-major codes b [k, n] in the stored form bfaintb_gemm reads (tightly packed, ldb = n) and bf16
+ * scales [k / group_size or 1, n].  Per column and group: scale = bf16(max(max|w| / qmax, 1e-12)), qmax = 127 or 7, code =
+ * round-to-even(w / scale) clamped to [-qmax - 1, qmax].  n and k as for bfaintb_gemm (k up to 2^21); all pointers 16-byte aligned.
+ * Asynchronous on `stream`, allocates nothing.  No counterpart in the reference, whose codes are generated on the host.
+ */
+#define BFAINTB_WEIGHT_BF16 0
+#define BFAINTB_WEIGHT_F16 1
+#define BFAINTB_WEIGHT_F32 2
+BFAINTB_API int bfaintb_quantize(void* b, void* scale, const void* w, int weight_type, uint32_t n, uint32_t k, uint32_t ldw, int weight_bits,
+                                 uint32_t group_size, void* stream);
+
+/*
  * Pre-packed weights.  bfaintb_prepack reorders a row-major B (the layout above) once, offline, into the operand
  * order of the matrix instruction ("mfma16": column blocks of 16, K-chunks of 64 rows, a lane's two 8-row operands
  * adjacent; bfaintb_packed.hip states it byte by byte); bfaintb_gemm_prepacked multiplies by the packed copy.  A
