@@ -9,7 +9,7 @@ import os
 import subprocess
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
-_LIB = os.path.join(_HERE, "libbfaintb_gemm.so")
+_LIB = _PACKAGE_LIB = os.path.join(_HERE, "libbfaintb_gemm.so")
 
 AUTO, DECODE, PREFILL = 0, 1, 2
 PREFILL_256, PREFILL_128 = 3, 4  # the tiled variant with its tile size forced (tests, tuning)
@@ -157,6 +157,31 @@ def lib():
     return _lib
 
 
+_binding = None
+
+
+def binding():
+    """The native PyTorch binding (_torch_binding.so): the calls below go through it where torch is installed.  None without
+    torch, and while a library other than the package's own is loaded (an instrumented build)."""
+    global _binding
+    if _LIB != _PACKAGE_LIB:
+        return None
+    if _binding is None:
+        lib()  # (raises if it is not built; loads torch first)
+        try:
+            import torch  # noqa: F401
+        except ImportError:
+            return None
+        try:
+            from . import _torch_binding
+        except ImportError as e:
+            raise RuntimeError("awesome_fusion_amd/_torch_binding.so does not load: build it with `make -C awesome_fusion_amd/csrc` "
+                               f"(or __graft_entry__.build()), against the torch that is imported here: {e}") from e
+        _torch_binding.set_error_class(BfaintbError)
+        _binding = _torch_binding
+    return _binding
+
+
 def error_string(code):
     return lib().bfaintb_error_string(int(code)).decode()
 
@@ -283,11 +308,15 @@ def static_scratch_reset(stream=None):
         raise BfaintbError(rc, "bfaintb_static_scratch_reset")
 
 
+def _ldr(ldr, n, activation):
+    return (n // 2 if activation == ACT_SILU_GATE else n) if ldr is None else ldr
+
+
 def _epilogue(bias, residual, ldr, n, activation=ACT_NONE):
     ep = Epilogue()
     ep.bias = _ptr(bias)
     ep.residual = _ptr(residual)
-    ep.ldr = (n // 2 if activation == ACT_SILU_GATE else n) if ldr is None else ldr
+    ep.ldr = _ldr(ldr, n, activation)
     ep.activation = activation
     return ep
 
@@ -300,17 +329,24 @@ def gemm(c, a, b, scale, m, n, k, lda=None, ldb=None, ldc=None, weight_bits=8, g
     lda = k if lda is None else lda
     ldb = n if ldb is None else ldb
     ldc = (n // 2 if activation == ACT_SILU_GATE else n) if ldc is None else ldc
+    if (which != AUTO or force_split_k) and (residual is not None or activation != ACT_NONE):
+        raise ValueError("bfaintb_gemm_fused takes no forced variant or split factor")
+    if (which != AUTO or force_split_k) and bias is not None:
+        raise ValueError("bfaintb_gemm_bias takes no forced variant or split factor")
+    native = _binding or binding()
+    if native is not None and _LIB is _PACKAGE_LIB:
+        rc = native.gemm_call(False, c, a, b, scale, bias, residual, _ldr(ldr, n, activation), activation, m, n, k, lda, ldb, ldc, weight_bits, group_size,
+                              workspace, workspace_nbytes, stream if stream is None or isinstance(stream, int) else stream.cuda_stream, which, force_split_k)
+        if rc and check:
+            raise BfaintbError(rc, "bfaintb_gemm")
+        return rc
     if workspace_nbytes is None:
         workspace_nbytes = 0 if workspace is None or isinstance(workspace, int) else workspace.numel() * workspace.element_size()
     if residual is not None or activation != ACT_NONE:
-        if which != AUTO or force_split_k:
-            raise ValueError("bfaintb_gemm_fused takes no forced variant or split factor")
         ep = _epilogue(bias, residual, ldr, n, activation)
         rc = lib().bfaintb_gemm_fused(_ptr(c), _ptr(a), _ptr(b), _ptr(scale), C.byref(ep), m, n, k, lda, ldb, ldc, weight_bits, group_size,
                                       _ptr(workspace), workspace_nbytes, _stream_handle(stream))
     elif bias is not None:
-        if which != AUTO or force_split_k:
-            raise ValueError("bfaintb_gemm_bias takes no forced variant or split factor")
         rc = lib().bfaintb_gemm_bias(_ptr(c), _ptr(a), _ptr(b), _ptr(scale), _ptr(bias), m, n, k, lda, ldb, ldc, weight_bits,
                                      group_size, _ptr(workspace), workspace_nbytes, _stream_handle(stream))
     else:
@@ -388,11 +424,21 @@ def gemm_prepacked(c, a, packed_b, scale, m, n, k, lda=None, ldc=None, weight_bi
                    workspace_nbytes=None, stream=None, which=AUTO, check=True, residual=None, ldr=None, activation=ACT_NONE):
     """C = A x dequant(B, scale) (+ bias) with B in the packed order, through bfaintb_gemm_prepacked_ex; with a residual
     (AUTO variant only) through bfaintb_gemm_prepacked_fused."""
+    fused = residual is not None or activation != ACT_NONE
+    if fused and which != AUTO:
+        raise ValueError("bfaintb_gemm_prepacked_fused takes no forced variant")
+    native = _binding or binding()
+    if native is not None and _LIB is _PACKAGE_LIB:
+        lda = k if lda is None else lda
+        ldc = (n // 2 if activation == ACT_SILU_GATE else n) if ldc is None else ldc
+        rc = native.gemm_call(True, c, a, packed_b, scale, bias, residual, _ldr(ldr, n, activation), activation, m, n, k, lda, n, ldc, weight_bits, group_size,
+                              workspace, workspace_nbytes, stream if stream is None or isinstance(stream, int) else stream.cuda_stream, which, 0)
+        if rc and check:
+            raise BfaintbError(rc, "bfaintb_gemm_prepacked_fused" if fused else "bfaintb_gemm_prepacked")
+        return rc
     if workspace_nbytes is None:
         workspace_nbytes = 0 if workspace is None or isinstance(workspace, int) else workspace.numel() * workspace.element_size()
-    if residual is not None or activation != ACT_NONE:
-        if which != AUTO:
-            raise ValueError("bfaintb_gemm_prepacked_fused takes no forced variant")
+    if fused:
         ep = _epilogue(bias, residual, ldr, n, activation)
         out_n = n // 2 if activation == ACT_SILU_GATE else n
         rc = lib().bfaintb_gemm_prepacked_fused(_ptr(c), _ptr(a), _ptr(packed_b), _ptr(scale), C.byref(ep), m, n, k,

@@ -1,0 +1,100 @@
+"""The native side of the PyTorch binding (awesome_fusion_amd/csrc/torch_binding.cpp): the linear layer's short way against
+the operator it calls, what it hands on to the long way, its errors, and the operators' workspaces."""
+import pytest
+import torch
+
+import awesome_fusion_amd as af
+import awesome_fusion_amd.torch_op as top
+
+
+def test_layers_and_tensors_the_short_way_does_not_know_take_the_long_one():
+    class Other(torch.Tensor):
+        pass
+
+    layer = top.QuantLinear(64, 32)
+    short = top._native.linear_forward
+    x = torch.zeros((2, 64), dtype=torch.bfloat16)
+    assert short(layer.__dict__, x.as_subclass(Other), None) is NotImplemented
+    assert short(layer.__dict__, None, None) is NotImplemented
+    assert short({}, x, None) is NotImplemented
+    with pytest.raises(RuntimeError, match="GPU only"):
+        layer(x)
+    with pytest.raises(ValueError, match="activation"):
+        torch.ops.awesome_fusion.bfaintb_gemm(x, layer.qweight, layer.scales, 8, 0, None, None, 2)
+    with pytest.raises(TypeError):
+        torch.ops.awesome_fusion.bfaintb_gemm(x.float(), layer.qweight, layer.scales, 8, 0)
+
+
+def _layer(n, k, bits, bias):
+    lin = torch.nn.Linear(k, n, bias=bias).cuda()
+    return top.QuantLinear.from_float(lin, bits, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("lead", [(512,), (1, 512), (3, 512), (0, 512), (2, 3, 512)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_short_and_long_way_agree(lead, dtype):
+    torch.manual_seed(4)
+    layer = _layer(272, 512, 8, True)
+    x = torch.randn(lead, device="cuda", dtype=dtype)
+    r = torch.randn(lead[:-1] + (272,), device="cuda", dtype=dtype)
+    y = layer(x, residual=r)
+    assert y.shape == r.shape and y.dtype == torch.bfloat16
+    want = torch.ops.awesome_fusion.bfaintb_gemm(x.reshape(-1, 512).to(torch.bfloat16), layer.qweight, layer.scales, 8, 0, layer.bias,
+                                                 r.reshape(-1, 272).to(torch.bfloat16))
+    assert torch.equal(y.reshape(-1, 272), want)
+
+
+@pytest.mark.gpu
+def test_gradients_are_refused_and_library_errors_keep_their_code():
+    layer = _layer(64, 128, 8, True)
+    x = torch.randn((2, 128), device="cuda", dtype=torch.bfloat16)
+    y = layer(x)
+    assert y.requires_grad  # the bias is a parameter
+    with pytest.raises(RuntimeError, match="autograd"):
+        y.sum().backward()
+    with torch.no_grad():
+        assert not layer(x).requires_grad
+    with pytest.raises(af.BfaintbError) as e:
+        torch.ops.awesome_fusion.bfaintb_gemm(x, layer.qweight, layer.scales.repeat(3, 1)[:2].contiguous(), 8, 48 + 16 - 1)
+    assert e.value.code == -5
+
+
+@pytest.mark.gpu
+def test_workspaces_by_stream_growth_and_capture():
+    """Calls that split k: on several streams at once, growing, given back in between, and captured (the graph's workspace
+    is not the one later calls outgrow or give back)."""
+    torch.manual_seed(5)
+    small, large = _layer(1024, 4096, 8, False), _layer(4096, 8192, 8, False)
+    xs, xl = torch.randn((4, 4096), device="cuda", dtype=torch.bfloat16), torch.randn((32, 8192), device="cuda", dtype=torch.bfloat16)
+    assert af.split_k(4, 1024, 4096) > 1 and af.split_k(32, 4096, 8192) > 1
+    want_s, want_l = small(xs), large(xl)
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    outs = []
+    for i in range(6):
+        with torch.cuda.stream(streams[i % 3]):
+            outs.append((small(xs), large(xl)))
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, want_s) and torch.equal(b, want_l) for a, b in outs)
+    for warm in (True, False):  # with and without a workspace made before the capture
+        top.release_workspaces()
+        stream = torch.cuda.Stream()
+        if warm:
+            with torch.cuda.stream(stream):
+                small(xs)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            c = small(xs)
+        for _ in range(3):
+            c.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(c, want_s)
+            with torch.cuda.stream(stream):
+                big = large(xl)
+            top.release_workspaces()
+            torch.full((64 << 20,), 7, dtype=torch.uint8, device="cuda")
+            torch.cuda.synchronize()
+            assert torch.equal(big, want_l)
