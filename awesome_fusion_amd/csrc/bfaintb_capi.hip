@@ -253,9 +253,11 @@ static bool use_small_tiles(int v, uint32_t m, uint32_t n, int bits)
 // family).  Worth it while tiles x splits still fit one workgroup per CU.
 struct TilePlan {
     uint32_t k_per_wg, splits;
+    uint32_t finish_launch;  // 1: every split's sums go to the workspace and a second launch adds them
     double us;
 };
 constexpr uint32_t kMaxTileSplits = 16;
+constexpr uint32_t kFinishLaunchSplits = 6;  // from here on a second launch adds the sums (unless the split factor is the caller's)
 
 static size_t split_workspace_bytes(uint32_t splits, uint32_t m, uint32_t n)
 {
@@ -263,6 +265,9 @@ static size_t split_workspace_bytes(uint32_t splits, uint32_t m, uint32_t n)
     // the header, then one fp32 word per (split but the last, row, column), rounded up to 256 bytes
     return bfaintb::kWorkspaceHeaderBytes + ((((size_t)(splits - 1u) * m * n * sizeof(float)) + 255u) & ~(size_t)255u);
 }
+
+// (with a second launch the last split's sums lie there as well)
+static size_t tile_workspace_bytes(const TilePlan& t, uint32_t m, uint32_t n) { return split_workspace_bytes(t.splits + t.finish_launch, m, n); }
 
 static TilePlan tile128_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint32_t forced_splits)
 {
@@ -272,6 +277,7 @@ static TilePlan tile128_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint3
     const double fill = (double)m / (double)((m + 127u) / 128u * 128u);  // the share of the tiles' rows that exist
     auto shape = [&](uint32_t want) {
         TilePlan t;
+        t.finish_launch = 0u;
         if (want > kMaxTileSplits) want = kMaxTileSplits;
         if (want < 1u) want = 1u;
         const uint32_t per = (ksteps + want - 1u) / want;
@@ -302,12 +308,30 @@ static TilePlan tile128_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint3
         return t;
     };
     if (forced_splits) return shape(forced_splits);
+    // with the second launch: the steps as above, 6.75 us for the two launches' beginnings and ends (one more where a
+    // thread fetches twice, beyond eight splits), and the words' way through
+    // memory (fitted on 70 shapes, m = 33 .. 352, n = 1040 .. 5300, k = 2048 .. 15500, both code widths and weight orders: within
+    // 5 % rms; 8-bit, us, measured / this: 220 x 2464 x 4480, 6 splits 18.2 / 17.5; 64 x 2832 x 14976, 8 splits 22.1 / 21.1)
+    auto finish_us = [&](const TilePlan& t) {
+        const double load = tiles * t.splits / cus;
+        const double step = ((bits == 4 ? 0.41 : 0.40) + 0.15 * load * load * load) * (0.8 + 0.2 * fill);
+        return (t.splits > 8u ? 7.75 : 6.75) + t.k_per_wg / 64u * step + t.splits * (double)m * n * 4.0 / 2.36e6;
+    };
     TilePlan best = shape(1);
-    static const uint32_t kCandidates[] = {2, 3, 4, 6, 8};
+    static const uint32_t kCandidates[] = {2, 3, 4, 6, 7, 8, 10, 12, 14, 16};
     for (uint32_t s : kCandidates) {
         if (tiles * s > cus) break;
-        const TilePlan t = shape(s);
+        TilePlan t = shape(s);
         if (t.splits != s) continue;  // k does not divide that way
+        // from six splits on their sums are added by a second launch, if all of them fit the scratch of the entry point that
+        // brings its own
+        // (not for 4-bit codes beyond 256 rows: there the family's rule above keeps the shapes that would split so far)
+        if (s >= kFinishLaunchSplits) {
+            if (bits == 4 && m > 256u) break;
+            t.finish_launch = 1u;
+            if (tile_workspace_bytes(t, m, n) > BFAINTB_STATIC_SCRATCH_BYTES) break;
+            t.us = finish_us(t);
+        }
         // (at most 256 tiles' worth of sums in all, 14 MiB: within the 32-bit offsets of the kernel and within the scratch of
         // the entry point that brings its own)
         if (t.us < best.us) best = t;
@@ -344,6 +368,23 @@ static double prefill_estimate_us(uint32_t m, uint32_t n, uint32_t k, int bits)
     const double tiles = (double)((m + 255u) / 256u) * (double)((n + 255u) / 256u);
     const double rounds = (double)(uint64_t)((tiles + cus - 1.0) / cus);
     return 4.0 + rounds * (k / 64.0) * 1.5;
+}
+
+// Whether the row-blocked family, at its estimated time, is the one to run.  Tiles whose sums a second launch adds are estimated
+// within 5 %; the family's estimate is not that good where it meets them, which one factor per kind of weights makes up
+// for (the ratio of the two estimates above which the tiles were the faster form, over 180 measured shapes).  Rows of B that are
+// not whole cache lines slow the family's reads by 30 % (8-bit; 127 x 1072 x 6016 18.1 us, tiles 13.6) and the tiles' copies by
+// little; in whole lines the family holds small weights (4-bit 64 x 4096 x 4096 11.7 against 13.6, 128 x 2048 x 8192 16.4
+// against 18.1) and loses long ones (8-bit 96 x 4096 x 11008 35.0 / 23.4, 64 rows 24.0 / 19.7; packed 29.6 / 22.6 and 21.5 / 19.5).
+static bool family_leads_tiles(double family_us, uint32_t m, uint32_t n, uint32_t k, int bits, bool packed)
+{
+    double us = prefill_estimate_us(m, n, k, bits);
+    if (prefill_small_tiles(m, n, bits) && tile128_plan(m, n, k, bits, 0).finish_launch) {
+        const bool lines = n % (packed ? 128u : 1024u / (uint32_t)bits) == 0;  // (packed: whole workgroups of columns)
+        if (packed) us *= bits == 8 ? 0.95 : lines ? 1.06 : 0.95;
+        else us *= bits == 8 ? (lines ? 1.06 : 0.84) : (lines ? 1.2 : 1.0);
+    }
+    return family_us < us;
 }
 
 // The decode family in row blocks: grid z walks blocks of 16*mb rows.  128 columns x 64 rows (mb = 4, 4 waves: one
@@ -622,7 +663,7 @@ int resolve_variant(uint32_t m, uint32_t n, uint32_t k, int bits, int variant)
         if (m <= kDecodeAutoMaxM) return BFAINTB_VARIANT_DECODE;
         if (m > kDecodeFamilyAutoMaxM) return BFAINTB_VARIANT_PREFILL;
         const DecodePlan pl = decode_plan(m, n, k, bits, 0);
-        return decode_family_time_us(m, n, k, bits, pl) < prefill_estimate_us(m, n, k, bits) ? BFAINTB_VARIANT_DECODE : BFAINTB_VARIANT_PREFILL;
+        return family_leads_tiles(decode_family_time_us(m, n, k, bits, pl), m, n, k, bits, false) ? BFAINTB_VARIANT_DECODE : BFAINTB_VARIANT_PREFILL;
     }
     if (variant == BFAINTB_VARIANT_DECODE) return m <= kDecodeMaxM ? variant : BFAINTB_ERR_BAD_VARIANT;
     if (is_prefill(variant)) return variant;
@@ -636,7 +677,7 @@ size_t workspace_need(uint32_t m, uint32_t n, uint32_t k, int bits, int variant,
 {
     if (m == 0 || n == 0) return 0;
     if (variant == BFAINTB_VARIANT_DECODE) return split_workspace_bytes(decode_plan(m, n, k, bits, forced_split).splits, m, n);
-    if (is_prefill(variant) && tiled_may_split(variant, m, n, bits)) return split_workspace_bytes(tile128_plan(m, n, k, bits, forced_split).splits, m, n);
+    if (is_prefill(variant) && tiled_may_split(variant, m, n, bits)) return tile_workspace_bytes(tile128_plan(m, n, k, bits, forced_split), m, n);
     return 0;
 }
 
@@ -963,6 +1004,7 @@ static int gemm_impl(void* c, const void* a, const void* b, const void* scale, c
             const TilePlan tp = tile128_plan(m, n, k, weight_bits, split_k);
             p.k_per_wg = tp.k_per_wg;
             p.splits = tp.splits;
+            p.finish_launch = tp.finish_launch;
         }
     } else {
         const DecodePlan pl = decode_plan(m, n, k, weight_bits, split_k);
@@ -973,7 +1015,7 @@ static int gemm_impl(void* c, const void* a, const void* b, const void* scale, c
         p.decode_mb = pl.mb;
     }
     // (every argument check comes before the first runtime call)
-    const size_t need = split_workspace_bytes(p.splits, m, n);
+    const size_t need = split_workspace_bytes(p.splits + p.finish_launch, m, n);
     if (p.splits > 1 && !use_static_scratch) {
         e = attach_workspace(p, workspace, workspace_bytes, need);
         if (e) return e;
@@ -1252,7 +1294,7 @@ static int packed_variant(uint32_t m, uint32_t n, uint32_t k, int bits, int vari
     if (packed_uses_slab(m, n, k, bits) || m <= kDecodeAutoMaxM) return BFAINTB_VARIANT_DECODE;
     if (m > kDecodeFamilyAutoMaxM) return BFAINTB_VARIANT_PREFILL;
     const DecodePlan pl = packed_family_plan(m, n, k, bits);
-    return packed_family_time_us(m, n, k, bits, pl) < prefill_estimate_us(m, n, k, bits) ? BFAINTB_VARIANT_DECODE : BFAINTB_VARIANT_PREFILL;
+    return family_leads_tiles(packed_family_time_us(m, n, k, bits, pl), m, n, k, bits, true) ? BFAINTB_VARIANT_DECODE : BFAINTB_VARIANT_PREFILL;
 }
 
 int bfaintb_gemm_prepacked_variant(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint32_t group_size)
@@ -1270,7 +1312,7 @@ int bfaintb_gemm_prepacked_variant(uint32_t m, uint32_t n, uint32_t k, int weigh
 static size_t packed_workspace_need(uint32_t m, uint32_t n, uint32_t k, int bits, int v)
 {
     if (m == 0 || n == 0) return 0;
-    if (is_prefill(v)) return tiled_may_split(v, m, n, bits) ? split_workspace_bytes(tile128_plan(m, n, k, bits, 0).splits, m, n) : 0;
+    if (is_prefill(v)) return tiled_may_split(v, m, n, bits) ? tile_workspace_bytes(tile128_plan(m, n, k, bits, 0), m, n) : 0;
     if (v != BFAINTB_VARIANT_DECODE || packed_uses_slab(m, n, k, bits)) return 0;
     const DecodePlan pl = packed_family_plan(m, n, k, bits);
     if (pl.splits <= 1) return 0;
@@ -1335,6 +1377,7 @@ static int gemm_prepacked_impl(void* c, const void* a, const void* packed_b, con
             const TilePlan tp = tile128_plan(m, n, k, weight_bits, 0);
             p.k_per_wg = tp.k_per_wg;
             p.splits = tp.splits;
+            p.finish_launch = tp.finish_launch;
             if (p.splits > 1) {
                 e = attach_workspace(p, workspace, workspace_bytes, packed_workspace_need(m, n, k, weight_bits, v));
                 if (e) return e;
@@ -1538,10 +1581,11 @@ int bfaintb_gemm_plan(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint3
         if (wreg) {
             const TilePlan tp = tile128_plan(m, n, k, weight_bits, packed ? 0u : split_k);
             out->splits = tp.splits;
+            out->launches = 1u + tp.finish_launch;
+            out->workspace_bytes = tile_workspace_bytes(tp, m, n);
             out->k_per_workgroup = tp.k_per_wg;
         }
         out->workgroups = ((m + 127u) / 128u) * ((n + 127u) / 128u) * out->splits;
-        out->workspace_bytes = split_workspace_bytes(out->splits, m, n);
         return BFAINTB_OK;
     }
     if (v == BFAINTB_VARIANT_PREFILL_256X128 || (v == BFAINTB_VARIANT_PREFILL && prefill_tall_tiles(m, n, weight_bits))) {

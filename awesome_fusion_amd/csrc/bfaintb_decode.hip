@@ -252,41 +252,6 @@ __host__ __device__ inline uint32_t decode_red_floats(uint32_t waves, uint32_t r
     return waves * rows * (cols + 4u);
 }
 
-// Finishes four neighbouring columns of one row: t += bias[col .. col+3]; then either += residual[row][col .. col+3] and
-// four bf16 outputs at C[row][col ..], or (gated) the two outputs silu(t.x) * t.y and silu(t.z) * t.w, += residual[row]
-// [col/2 ..], at C[row][col/2 ..].  All additions in fp32, one rounding (a truncation with the reference's arithmetic).
-__device__ __forceinline__ void finish_row4(const GemmParams& p, float4 t, uint32_t row, uint32_t col)
-{
-    if (p.bias != nullptr) {
-        const uint2 raw = *reinterpret_cast<const uint2*>(p.bias + col);
-        t.x += bf16_bits_to_f32(raw.x & 0xffffu);
-        t.y += bf16_bits_to_f32(raw.x >> 16);
-        t.z += bf16_bits_to_f32(raw.y & 0xffffu);
-        t.w += bf16_bits_to_f32(raw.y >> 16);
-    }
-    if (p.activation == kActSiluGate) {
-        float o0 = silu_gate(t.x, t.y), o1 = silu_gate(t.z, t.w);
-        if (p.residual != nullptr) {
-            const uint32_t raw = *reinterpret_cast<const uint32_t*>(p.residual + (size_t)row * p.ldr + col / 2u);
-            o0 += bf16_bits_to_f32(raw & 0xffffu);
-            o1 += bf16_bits_to_f32(raw >> 16);
-        }
-        *reinterpret_cast<uint32_t*>(p.c + (size_t)row * p.ldc + col / 2u) = p.reference_arith ? pack_bf16_rtz(o0, o1) : pack_bf16_rne(o0, o1);
-        return;
-    }
-    if (p.residual != nullptr) {
-        const uint2 raw = *reinterpret_cast<const uint2*>(p.residual + (size_t)row * p.ldr + col);
-        t.x += bf16_bits_to_f32(raw.x & 0xffffu);
-        t.y += bf16_bits_to_f32(raw.x >> 16);
-        t.z += bf16_bits_to_f32(raw.y & 0xffffu);
-        t.w += bf16_bits_to_f32(raw.y >> 16);
-    }
-    uint2 o;
-    o.x = p.reference_arith ? pack_bf16_rtz(t.x, t.y) : pack_bf16_rne(t.x, t.y);
-    o.y = p.reference_arith ? pack_bf16_rtz(t.z, t.w) : pack_bf16_rne(t.z, t.w);
-    *reinterpret_cast<uint2*>(p.c + (size_t)row * p.ldc + col) = o;
-}
-
 // Split-K, the reducing workgroup's part for one thread: R rows (first_row + rs, + nrs, ...; `rows` of
 // them exist from first_row on) of 4 columns.  Fetches the other splits' partial sums, adds them in
 // split order with the thread's own sums last, writes bf16 C and leaves the workspace words empty

@@ -102,6 +102,7 @@ struct GemmParams {
     uint32_t decode_mb;    // blocks of 16 rows of A per workgroup of the decode variant (1, 2 or 4)
     uint32_t decode_scale_lds;  // byte offset, in dynamic LDS, of the waves' scale tables (packed weights, grouped scales)
     uint32_t splits;     // workgroups along k
+    uint32_t finish_launch;  // small tiles: every split leaves its sums in `partials` (then [splits][m][n]) for a second launch to finish
     unsigned long long* partials;  // [splits - 1][m][n] fp32 partial sums; kEmptyWord wherever none is waiting
     uint32_t partial_bytes;        // size of that area (below 2^31)
     uint32_t* ws_header;           // the workspace's header (see kWorkspaceHeaderBytes), or null without split-K
@@ -184,6 +185,41 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi)
 {
     if constexpr (RTZ) return pack_bf16_rtz(lo, hi);
     else return pack_bf16_rne(lo, hi);
+}
+
+// Finishes four neighbouring columns of one row: t += bias[col .. col+3]; then either += residual[row][col .. col+3] and
+// four bf16 outputs at C[row][col ..], or (gated) the two outputs silu(t.x) * t.y and silu(t.z) * t.w, += residual[row]
+// [col/2 ..], at C[row][col/2 ..].  All additions in fp32, one rounding (a truncation with the reference's arithmetic).
+__device__ __forceinline__ void finish_row4(const GemmParams& p, float4 t, uint32_t row, uint32_t col)
+{
+    if (p.bias != nullptr) {
+        const uint2 raw = *reinterpret_cast<const uint2*>(p.bias + col);
+        t.x += bf16_bits_to_f32(raw.x & 0xffffu);
+        t.y += bf16_bits_to_f32(raw.x >> 16);
+        t.z += bf16_bits_to_f32(raw.y & 0xffffu);
+        t.w += bf16_bits_to_f32(raw.y >> 16);
+    }
+    if (p.activation == kActSiluGate) {
+        float o0 = silu_gate(t.x, t.y), o1 = silu_gate(t.z, t.w);
+        if (p.residual != nullptr) {
+            const uint32_t raw = *reinterpret_cast<const uint32_t*>(p.residual + (size_t)row * p.ldr + col / 2u);
+            o0 += bf16_bits_to_f32(raw & 0xffffu);
+            o1 += bf16_bits_to_f32(raw >> 16);
+        }
+        *reinterpret_cast<uint32_t*>(p.c + (size_t)row * p.ldc + col / 2u) = p.reference_arith ? pack_bf16_rtz(o0, o1) : pack_bf16_rne(o0, o1);
+        return;
+    }
+    if (p.residual != nullptr) {
+        const uint2 raw = *reinterpret_cast<const uint2*>(p.residual + (size_t)row * p.ldr + col);
+        t.x += bf16_bits_to_f32(raw.x & 0xffffu);
+        t.y += bf16_bits_to_f32(raw.x >> 16);
+        t.z += bf16_bits_to_f32(raw.y & 0xffffu);
+        t.w += bf16_bits_to_f32(raw.y >> 16);
+    }
+    uint2 o;
+    o.x = p.reference_arith ? pack_bf16_rtz(t.x, t.y) : pack_bf16_rne(t.x, t.y);
+    o.y = p.reference_arith ? pack_bf16_rtz(t.z, t.w) : pack_bf16_rne(t.z, t.w);
+    *reinterpret_cast<uint2*>(p.c + (size_t)row * p.ldc + col) = o;
 }
 
 // Signed byte `I` of a dword as fp32: one v_cvt_f32_i32 with an SDWA sign-extending byte select.

@@ -107,9 +107,18 @@ bfaintb_prefill128_wreg_kernel(const GemmParams p)
     //      logical ids, which walk groups of 8 tile-rows column by column)
     const uint32_t tiles_m = (p.m + kTw - 1) / kTw, tiles_n = (p.n + kTw - 1) / kTw;
     const uint32_t wgs = tiles_m * tiles_n;
-    const uint32_t per_xcd = (wgs + 7u) / 8u;
-    const uint32_t logical = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
-    if (logical >= wgs) return;
+    // (with a second launch no workgroup waits for another, so tiles x splits are dealt out as one run: 42 tiles x 6 splits
+    // dealt split by split are 36 workgroups on each of seven XCDs of 32 CUs and none on the eighth; 139 x 1072
+    // x 15488, 18 tiles x 14 splits: 32.0 us so, 19.8 as one run; 82 x 5296 x 10240 4-bit, 42 x 6: 37.4 and 23.9)
+    const uint32_t items = p.finish_launch ? wgs * p.splits : wgs;
+    const uint32_t per_xcd = (items + 7u) / 8u;
+    uint32_t logical = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
+    if (logical >= items) return;
+    uint32_t ks = blockIdx.y;
+    if (p.finish_launch) {
+        ks = logical / wgs;
+        logical -= ks * wgs;
+    }
     const uint32_t group = logical / (8u * tiles_n);
     const uint32_t first_m = group * 8u;
     const uint32_t group_rows = tiles_m - first_m < 8u ? tiles_m - first_m : 8u;
@@ -132,10 +141,9 @@ bfaintb_prefill128_wreg_kernel(const GemmParams p)
                : __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.b + (BITS == 8 ? n0 : n0 / 2u)), 0,
                                                    (int)((p.k - 1u) * p.ldb_bytes + (BITS == 8 ? cols_valid : cols_valid / 2u)), kBufferFlags);
 
-    // K-steps of this workgroup: all of them, or the share of split blockIdx.y (p.k_per_wg rows each; the host makes sure
+    // K-steps of this workgroup: all of them, or the share of split ks (p.k_per_wg rows each; the host makes sure
     // every split has at least one).  kt below counts within the share; kbase + kt is the step of the whole matrix.
     const uint32_t ksteps_all = (p.k + kTwK - 1u) / kTwK;
-    const uint32_t ks = blockIdx.y;
     const uint32_t kbase = ks * (p.k_per_wg / kTwK);
     const uint32_t ksteps = p.k_per_wg / kTwK < ksteps_all - kbase ? p.k_per_wg / kTwK : ksteps_all - kbase;
     const uint32_t last_chunks = (p.k - (ksteps_all - 1u) * kTwK) / 8u;  // valid 16-byte chunks per row of A in the last step
@@ -682,7 +690,7 @@ bfaintb_prefill128_wreg_kernel(const GemmParams p)
         const uint32_t row = hrow + kHStride * i;
         return reinterpret_cast<float4*>(c_rows(row >> 5) + (row & 31u) * kTw + hcol);
     };
-    if (ks != p.splits - 1u) {
+    if (ks != p.splits - 1u || p.finish_launch) {
         if (p.debug_flags & kDebugWithholdPartials) return;  // test hook: lets the reducer's wait run out
 #pragma unroll
         for (uint32_t i = 0; i < kHeld; ++i) {
@@ -774,16 +782,60 @@ bfaintb_prefill128_wreg_kernel(const GemmParams p)
     }
 }
 
+// The second launch of a product whose k is split many ways (p.finish_launch): adds the splits' sums of four columns of a row in
+// split order, finishes the outputs and leaves the words empty, as every launch that uses the workspace expects them.  A
+// word that is still empty was never produced: its sum stays the NaN it is and the header remembers it.
+//
+// Bound by the latency of one fetch past the L2s and by splits x m x n words read and written.  Within the one launch, the
+// workgroup of a tile's last split draws all of it through its CU, two splits per round trip (15 - 20 GB/s); a launch of its
+// own spreads it over the machine: 8-bit, 64 x 4096 x 11008, k split 8 ways: 19.7 us (4 ways in one launch: 29.0), 96 rows,
+// 7 ways: 24.8 (32.9).  Device-scope accesses on both sides, as in the one launch: 64 x 4096 x 4096 14.1 us; with ordinary
+// ones here 16.2 (every emptied word is still in an L2 when the kernel ends), with ordinary stores by the producers 16.9.
+constexpr uint32_t kFinishBatch = 8;  // splits whose words a thread fetches together
+__global__ void __launch_bounds__(256) bfaintb_split_finish_kernel(const GemmParams p)
+{
+    const uint32_t quads = p.n / 4u;
+    const uint32_t id = blockIdx.x * 256u + threadIdx.x;
+    if (id >= p.m * quads) return;
+    const uint32_t row = id / quads, col = 4u * (id - row * quads);
+    // (the sums of all splits fit 16 MiB: 32-bit offsets)
+    const __amdgpu_buffer_rsrc_t ws = __builtin_amdgcn_make_buffer_rsrc(p.partials, 0, (int)p.partial_bytes, kBufferFlags);
+    const uint32_t off = (row * p.n + col) * 4u, split_bytes = p.m * p.n * 4u;
+    const u32x4_t empty4 = {kEmptyWord, kEmptyWord, kEmptyWord, kEmptyWord};
+    float4 total = make_float4(0.f, 0.f, 0.f, 0.f);
+    bool complete = true;
+    for (uint32_t sp0 = 0; sp0 < p.splits; sp0 += kFinishBatch) {
+        u32x4_t w[kFinishBatch];
+#pragma unroll
+        for (uint32_t j = 0; j < kFinishBatch; ++j)  // (the bound is the same for every thread)
+            if (sp0 + j < p.splits) w[j] = __builtin_amdgcn_raw_buffer_load_b128(ws, (int)off, (int)((sp0 + j) * split_bytes), kAuxDeviceScope);
+#pragma unroll
+        for (uint32_t j = 0; j < kFinishBatch; ++j) {
+            if (sp0 + j >= p.splits) continue;
+            __builtin_amdgcn_raw_buffer_store_b128(empty4, ws, (int)off, (int)((sp0 + j) * split_bytes), kAuxDeviceScope);
+            complete = complete && w[j][0] != kEmptyWord && w[j][1] != kEmptyWord && w[j][2] != kEmptyWord && w[j][3] != kEmptyWord;
+            total.x += __uint_as_float(w[j][0]);
+            total.y += __uint_as_float(w[j][1]);
+            total.z += __uint_as_float(w[j][2]);
+            total.w += __uint_as_float(w[j][3]);
+        }
+    }
+    if (!complete) __hip_atomic_store(p.ws_header, kWorkspaceGaveUp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    finish_row4(p, total, row, col);
+}
+
 template <int BITS, bool GROUPED, bool PACKED>
 static hipError_t launch_prefill128_wreg_t(const GemmParams& p, hipStream_t stream)
 {
     const uint32_t tiles = ((p.m + kTw - 1) / kTw) * ((p.n + kTw - 1) / kTw);
-    const uint32_t grid = (tiles + 7u) / 8u * 8u;  // a whole number of workgroups per XCD; ids past the last tile exit at once
+    const uint32_t grid = (p.finish_launch ? tiles * p.splits + 7u : tiles + 7u) / 8u * 8u;  // a whole number of workgroups per XCD; ids past the last tile exit at once
     // two waves per column group; with grouped scales, the copying wave on top
     // (at most 64 rows in all: the form that multiplies only the first four blocks of 16 rows)
     void (*kernel)(const GemmParams) = p.m <= 64u ? bfaintb_prefill128_wreg_kernel<BITS, GROUPED, PACKED, 2, GROUPED, 4>
                                                   : bfaintb_prefill128_wreg_kernel<BITS, GROUPED, PACKED, 2, GROUPED, 8>;
-    return launch_kernel(kernel, dim3(grid, p.splits, 1), dim3(512 + (GROUPED ? 64 : 0), 1, 1), 0, stream, p);
+    const hipError_t e = launch_kernel(kernel, dim3(grid, p.finish_launch ? 1u : p.splits, 1), dim3(512 + (GROUPED ? 64 : 0), 1, 1), 0, stream, p);
+    if (e != hipSuccess || !p.finish_launch) return e;
+    return launch_kernel(bfaintb_split_finish_kernel, dim3((p.m * (p.n / 4u) + 255u) / 256u, 1, 1), dim3(256, 1, 1), 0, stream, p);
 }
 
 // Whether this kernel can serve a launch: this library's own arithmetic (either order of the weights).
