@@ -766,6 +766,9 @@ int static_scratch(DeviceState& st, hipStream_t stream, void** out)
 
 extern "C" {
 
+static uint32_t row_split_head(uint32_t m, uint32_t n, uint32_t k, int bits, bool packed);
+static size_t row_split_workspace(uint32_t head, uint32_t rest, uint32_t n, uint32_t k, int bits, bool packed);
+
 int bfaintb_version(void) { return BFAINTB_VERSION; }
 
 const char* bfaintb_error_string(int code)
@@ -799,7 +802,14 @@ int bfaintb_gemm_variant(uint32_t m, uint32_t n, uint32_t k, int weight_bits, ui
 
 uint32_t bfaintb_gemm_split_k(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint32_t group_size)
 {
-    const int v = bfaintb_gemm_variant(m, n, k, weight_bits, group_size);
+    int v = bfaintb_gemm_variant(m, n, k, weight_bits, group_size);
+    if (v >= 0) {
+        const uint32_t head = row_split_head(m, n, k, weight_bits, false);
+        if (head != 0u) {
+            m = head;
+            v = resolve_variant(m, n, k, weight_bits, BFAINTB_VARIANT_AUTO);
+        }
+    }
     if (v == BFAINTB_VARIANT_DECODE) return decode_plan(m, n, k, weight_bits, 0).splits;
     if (v == BFAINTB_VARIANT_PREFILL && tiled_may_split(v, m, n, weight_bits)) return tile128_plan(m, n, k, weight_bits, 0).splits;
     return 1;
@@ -811,6 +821,10 @@ size_t bfaintb_gemm_workspace_bytes_ex(uint32_t m, uint32_t n, uint32_t k, int w
     if (check_format(k, weight_bits, group_size) || check_shape(m, n, k, weight_bits)) return 0;
     const int v = resolve_variant(m, n, k, weight_bits, variant);
     if (v < 0) return 0;
+    if (variant == BFAINTB_VARIANT_AUTO && split_k == 0) {
+        const uint32_t head = row_split_head(m, n, k, weight_bits, false);
+        if (head != 0u) return row_split_workspace(head, m - head, n, k, weight_bits, false);
+    }
     return workspace_need(m, n, k, weight_bits, v, split_k);
 }
 
@@ -919,6 +933,13 @@ struct Epilogue {
     bool reference_arith = false;
     // columns of C (and of the residual) for n columns of B
     uint32_t out_cols(uint32_t n) const { return activation == BFAINTB_ACT_SILU_GATE ? n / 2u : n; }
+    // the same for the rows of C from `row` on
+    Epilogue from_row(uint32_t row) const
+    {
+        Epilogue e = *this;
+        if (residual != nullptr) e.residual = static_cast<const uint16_t*>(residual) + (size_t)row * ldr;
+        return e;
+    }
 };
 
 static int read_epilogue(Epilogue& out, const bfaintb_epilogue* ep, uint32_t n)
@@ -948,9 +969,21 @@ static int attach_workspace(GemmParams& p, void* workspace, size_t workspace_byt
     return BFAINTB_OK;
 }
 
+// Whether two launches by rows can be made with what the caller brings: the scratch they need (a caller who brings less, or
+// none, gets the one launch over all rows, which may need none), and a device whose set-up is done or can be done now (one
+// launch of the tiled kernels needs none, so a capture before any other call keeps working).
+static bool row_split_served(const void* workspace, size_t workspace_bytes, size_t need, bool use_static_scratch, hipStream_t stream)
+{
+    DeviceState* dev = nullptr;
+    if (!use_static_scratch && need != 0 && (workspace == nullptr || workspace_bytes < need || misaligned16(workspace))) return false;
+    if (device_state(stream, &dev) != 0) return false;
+    void* scratch_ptr = nullptr;
+    return !use_static_scratch || need == 0 || static_scratch(*dev, stream, &scratch_ptr) == 0;
+}
+
 static int gemm_impl(void* c, const void* a, const void* b, const void* scale, const Epilogue& ep, uint32_t m, uint32_t n, uint32_t k,
                      uint32_t lda, uint32_t ldb, uint32_t ldc, int weight_bits, uint32_t group_size, void* workspace,
-                     size_t workspace_bytes, void* stream, int variant, uint32_t split_k, bool use_static_scratch = false)
+                     size_t workspace_bytes, void* stream, int variant, uint32_t split_k, bool use_static_scratch = false, bool whole = false)
 {
     const void* bias = ep.bias;
     int e = check_format(k, weight_bits, group_size);
@@ -966,6 +999,18 @@ static int gemm_impl(void* c, const void* a, const void* b, const void* scale, c
     if (c == nullptr || a == nullptr || b == nullptr || scale == nullptr) return BFAINTB_ERR_NULL_POINTER;
     if (misaligned16(c) || misaligned16(a) || misaligned16(b) || misaligned16(scale) || misaligned16(bias) || misaligned16(ep.residual))
         return BFAINTB_ERR_ALIGNMENT;
+    if (!whole && variant == BFAINTB_VARIANT_AUTO && split_k == 0 && !ep.reference_arith) {
+        const uint32_t head = row_split_head(m, n, k, weight_bits, false);
+        if (head != 0u && row_split_served(workspace, workspace_bytes, row_split_workspace(head, m - head, n, k, weight_bits, false), use_static_scratch,
+                                           static_cast<hipStream_t>(stream))) {
+            e = gemm_impl(c, a, b, scale, ep, head, n, k, lda, ldb, ldc, weight_bits, group_size, workspace, workspace_bytes, stream, variant, 0,
+                          use_static_scratch, true);
+            if (e) return e;
+            return gemm_impl(static_cast<uint16_t*>(c) + (size_t)head * ldc, static_cast<const uint16_t*>(a) + (size_t)head * lda, b, scale,
+                             ep.from_row(head), m - head, n, k, lda, ldb, ldc, weight_bits, group_size, workspace, workspace_bytes, stream, variant, 0,
+                             use_static_scratch, true);
+        }
+    }
 
     GemmParams p{};
     p.bias = static_cast<const uint16_t*>(bias);
@@ -1319,11 +1364,101 @@ static size_t packed_workspace_need(uint32_t m, uint32_t n, uint32_t k, int bits
     return bfaintb::kWorkspaceHeaderBytes + ((((size_t)(pl.splits - 1u) * m * n * sizeof(float)) + 255u) & ~(size_t)255u);
 }
 
+// ---- A product in two launches, by rows of A.  The tiled kernels take the time of whole rounds of tiles: a few rows more than
+//      fill one cost up to a round.  Where the times below say so, the rows that fill their tiles go first and the rest is a
+//      product of its own, by whatever kernel suits it (packed weights, us, one launch / two: 528 x 22016 x 4096 4-bit, 258 large
+//      tiles, 162 / 114; 577 rows 164 / 127; 1040 x 13824 x 5120 4-bit 203 / 141; 784 x 5120 x 13824 4-bit 186 / 126; 640 x 28672 x
+//      8192 4-bit 313 / 253; 1040 x 4096 x 4096 8-bit 57 / 44; 2176 x 8192 x 8192 8-bit 294 / 230).
+
+// What one launch of the library's own choice takes, in microseconds, for more rows than the estimates that choose between
+// kernels are asked about: the large tiles by their number (a round at a load below one CU each runs at a higher clock; us per
+// K-step at 162 / 216 / 256 tiles, 4-bit 1.39 / 1.49 / 1.55, 8-bit, at 172 / 256, 1.26 / 1.52), the thin last round as the half tiles
+// it runs as; up to 32 rows the stream of the weights.
+static double launch_time_us(uint32_t m, uint32_t n, uint32_t k, int bits, bool packed)
+{
+    const double cus = (double)machine_cus(), steps = k / 64.0;
+    if (m <= kDecodeAutoMaxM) return 6.0 + (double)n * k * bits / 8.0 / 3.3e6 * (m <= 16u ? 1.0 : 1.25);
+    const int v = packed ? packed_variant(m, n, k, bits, BFAINTB_VARIANT_AUTO) : resolve_variant(m, n, k, bits, BFAINTB_VARIANT_AUTO);
+    if (v == BFAINTB_VARIANT_DECODE)
+        return packed ? packed_family_time_us(m, n, k, bits, packed_family_plan(m, n, k, bits)) : decode_family_time_us(m, n, k, bits, decode_plan(m, n, k, bits, 0));
+    if (prefill_small_tiles(m, n, bits) || prefill_tall_tiles(m, n, bits)) return prefill_estimate_us(m, n, k, bits);
+    const uint32_t tiles = ((m + 255u) / 256u) * ((n + 255u) / 256u);
+    const uint32_t thin = bfaintb::thin_round_tiles(tiles, m, machine_cus()), full = tiles - thin;
+    auto round_us = [&](double load) { return steps * (bits == 8 ? 1.0 + 0.5 * load : 1.1 + 0.45 * load); };
+    const uint32_t whole = full / machine_cus(), rest = full - whole * machine_cus();
+    double us = 4.0 + whole * round_us(1.0) + (rest != 0u ? round_us(rest / cus) : 0.0);
+    if (thin != 0u) {
+        const double load = 2.0 * thin / cus;
+        us += 4.0 + steps * (0.83 + 0.17 * load * load * load);
+    }
+    return us;
+}
+
+static size_t row_split_workspace(uint32_t head, uint32_t rest, uint32_t n, uint32_t k, int bits, bool packed)
+{
+    size_t need = 0;
+    for (const uint32_t rows : {head, rest}) {
+        const size_t part = packed ? packed_workspace_need(rows, n, k, bits, packed_variant(rows, n, k, bits, BFAINTB_VARIANT_AUTO))
+                                   : workspace_need(rows, n, k, bits, resolve_variant(rows, n, k, bits, BFAINTB_VARIANT_AUTO), 0);
+        if (part > need) need = part;
+    }
+    return need;
+}
+
+// Rows of the first launch, or 0 for one launch over all of them.
+static uint32_t row_split_rule(uint32_t m, uint32_t n, uint32_t k, int bits, bool packed)
+{
+    if (m <= 256u || n < 16u || g_force_row_block.load(std::memory_order_relaxed) != 0u) return 0;
+    const uint64_t cus = machine_cus();
+    const uint32_t cols256 = (n + 255u) / 256u, cols128 = (n + 127u) / 128u;
+    // the rows that whole rounds of large tiles hold; one round of tall tiles; one of small ones; and all whole large tiles, or
+    // all but one row of them
+    const uint64_t rounds = (uint64_t)((m + 255u) / 256u) * cols256 / cus;
+    const uint64_t candidates[] = {rounds * cus / cols256 * 256u, cus / cols128 * 256u, cus / cols128 * 128u, (m - 1u) / 256u * 256u,
+                                   (m - 1u) / 256u * 256u - 256u};
+    const double one = launch_time_us(m, n, k, bits, packed);
+    // (0.94: the estimates' error.  Of 200 shapes, m = 257 .. 4096, 25 go in two launches so, 1.25 times
+    // as fast on average and none slower; at 0.97 three of 49 are, by 4 - 9 %)
+    double best = 0.94 * one;
+    uint32_t head = 0;
+    for (const uint64_t c : candidates) {
+        if (c == 0u || c >= m) continue;
+        const uint32_t rows = (uint32_t)c;
+        const double two = launch_time_us(rows, n, k, bits, packed) + launch_time_us(m - rows, n, k, bits, packed) + 1.0;
+        if (two >= best) continue;
+        if (row_split_workspace(rows, m - rows, n, k, bits, packed) > BFAINTB_STATIC_SCRATCH_BYTES) continue;
+        best = two;
+        head = rows;
+    }
+    return head;
+}
+
+// (a call asks two or three times, for its scratch and for its launch, and a model asks about the same few shapes: each
+// thread keeps the last answers, one per slot of a hash of the question)
+static uint32_t row_split_head(uint32_t m, uint32_t n, uint32_t k, int bits, bool packed)
+{
+    if (m <= 256u) return 0;
+    struct Answer {
+        uint32_t m, n, k, kind, cus, row_block, head;
+    };
+    static thread_local Answer answers[32] = {};
+    const uint32_t kind = (uint32_t)bits * 2u + (packed ? 1u : 0u), cus = machine_cus(), row_block = g_force_row_block.load(std::memory_order_relaxed);
+    Answer& a = answers[((m * 2654435761u) ^ (n * 2246822519u) ^ (k * 3266489917u) ^ kind) >> 27];
+    if (a.m != m || a.n != n || a.k != k || a.kind != kind || a.cus != cus || a.row_block != row_block)
+        a = Answer{m, n, k, kind, cus, row_block, row_split_rule(m, n, k, bits, packed)};
+    return a.head;
+}
+
 size_t bfaintb_gemm_prepacked_workspace_bytes_ex(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint32_t group_size, int variant)
 {
     if (check_format(k, weight_bits, group_size) || check_shape(m, n, k) || check_packed_shape(n, k, weight_bits)) return 0;
     const int v = packed_variant(m, n, k, weight_bits, variant);
-    return v < 0 ? 0 : packed_workspace_need(m, n, k, weight_bits, v);
+    if (v < 0) return 0;
+    if (variant == BFAINTB_VARIANT_AUTO) {
+        const uint32_t head = row_split_head(m, n, k, weight_bits, true);
+        if (head != 0u) return row_split_workspace(head, m - head, n, k, weight_bits, true);
+    }
+    return packed_workspace_need(m, n, k, weight_bits, v);
 }
 
 size_t bfaintb_gemm_prepacked_workspace_bytes(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint32_t group_size)
@@ -1333,7 +1468,7 @@ size_t bfaintb_gemm_prepacked_workspace_bytes(uint32_t m, uint32_t n, uint32_t k
 
 static int gemm_prepacked_impl(void* c, const void* a, const void* packed_b, const void* scale, const Epilogue& ep, uint32_t m,
                                uint32_t n, uint32_t k, uint32_t lda, uint32_t ldc, int weight_bits, uint32_t group_size,
-                               void* workspace, size_t workspace_bytes, void* stream, int variant)
+                               void* workspace, size_t workspace_bytes, void* stream, int variant, bool whole = false)
 {
     const void* bias = ep.bias;
     int e = check_format(k, weight_bits, group_size);
@@ -1350,6 +1485,18 @@ static int gemm_prepacked_impl(void* c, const void* a, const void* packed_b, con
     if (misaligned16(c) || misaligned16(a) || misaligned16(packed_b) || misaligned16(scale) || misaligned16(bias) ||
         misaligned16(ep.residual))
         return BFAINTB_ERR_ALIGNMENT;
+    if (!whole && variant == BFAINTB_VARIANT_AUTO) {
+        const uint32_t head = row_split_head(m, n, k, weight_bits, true);
+        if (head != 0u && row_split_served(workspace, workspace_bytes, row_split_workspace(head, m - head, n, k, weight_bits, true), false,
+                                           static_cast<hipStream_t>(stream))) {
+            e = gemm_prepacked_impl(c, a, packed_b, scale, ep, head, n, k, lda, ldc, weight_bits, group_size, workspace, workspace_bytes, stream, variant,
+                                    true);
+            if (e) return e;
+            return gemm_prepacked_impl(static_cast<uint16_t*>(c) + (size_t)head * ldc, static_cast<const uint16_t*>(a) + (size_t)head * lda, packed_b,
+                                       scale, ep.from_row(head), m - head, n, k, lda, ldc, weight_bits, group_size, workspace, workspace_bytes, stream,
+                                       variant, true);
+        }
+    }
     GemmParams p{};
     p.residual = static_cast<const uint16_t*>(ep.residual);
     p.ldr = ep.ldr;
@@ -1528,21 +1675,12 @@ int bfaintb_probe_read(const void* src, size_t bytes, void* sink, void* stream)
     return (int)bfaintb::launch_probe_read(src, bytes, sink, static_cast<hipStream_t>(stream));
 }
 
-// What a call would launch, without launching it: the queries above rolled into one description, for callers that want
-// to log or check the library's choice and for the scans that hold the choice against measurements.
-int bfaintb_gemm_plan(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint32_t group_size, int packed, int variant, uint32_t split_k,
+// One launch of a checked question's answer (two where a kernel's own last round or hand-over is one): see bfaintb_gemm_plan.
+static int plan_whole(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint32_t group_size, int packed, int variant, uint32_t split_k,
                       bfaintb_plan* out)
 {
-    if (out == nullptr) return BFAINTB_ERR_NULL_POINTER;
     memset(out, 0, sizeof(*out));
-    int e = check_format(k, weight_bits, group_size);
-    if (e) return e;
-    e = check_shape(m, n, k, packed ? 8 : weight_bits);
-    if (e) return e;
-    if (packed) {
-        e = check_packed_shape(n, k, weight_bits);
-        if (e) return e;
-    }
+    (void)group_size;
     const int v = packed ? packed_variant(m, n, k, weight_bits, variant) : resolve_variant(m, n, k, weight_bits, variant);
     if (v < 0) return v;
     out->compute_units = machine_cus();
@@ -1609,6 +1747,39 @@ int bfaintb_gemm_plan(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint3
         out->launches = (tiles - halves != 0u ? 1u : 0u) + (halves != 0u ? 1u : 0u);
     }
     return BFAINTB_OK;
+}
+
+// What a call would launch, without launching it: the queries above rolled into one description, for callers that want
+// to log or check the library's choice and for the scans that hold the choice against measurements.
+int bfaintb_gemm_plan(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint32_t group_size, int packed, int variant, uint32_t split_k,
+                      bfaintb_plan* out)
+{
+    if (out == nullptr) return BFAINTB_ERR_NULL_POINTER;
+    memset(out, 0, sizeof(*out));
+    int e = check_format(k, weight_bits, group_size);
+    if (e) return e;
+    e = check_shape(m, n, k, packed ? 8 : weight_bits);
+    if (e) return e;
+    if (packed) {
+        e = check_packed_shape(n, k, weight_bits);
+        if (e) return e;
+    }
+    const int v = packed ? packed_variant(m, n, k, weight_bits, variant) : resolve_variant(m, n, k, weight_bits, variant);
+    if (v < 0) return v;
+    if (variant == BFAINTB_VARIANT_AUTO && (packed || split_k == 0)) {
+        const uint32_t head = row_split_head(m, n, k, weight_bits, packed != 0);
+        if (head != 0u) {  // the first launch, described as such; of the second one its workgroups
+            bfaintb_plan rest;
+            e = plan_whole(head, n, k, weight_bits, group_size, packed, variant, 0, out);
+            if (e == 0) e = plan_whole(m - head, n, k, weight_bits, group_size, packed, variant, 0, &rest);
+            if (e) return e;
+            out->tail_workgroups += rest.workgroups + rest.tail_workgroups;
+            out->launches += rest.launches;
+            out->workspace_bytes = row_split_workspace(head, m - head, n, k, weight_bits, packed != 0);
+            return BFAINTB_OK;
+        }
+    }
+    return plan_whole(m, n, k, weight_bits, group_size, packed, variant, split_k, out);
 }
 
 uint32_t bfaintb_prefill_tile(uint32_t m, uint32_t n) { return prefill_small_tiles(m, n, 8) ? 128u : 256u; }

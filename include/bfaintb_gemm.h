@@ -364,8 +364,8 @@ typedef struct bfaintb_plan {
     uint32_t splits;           /* workgroups along k per tile */
     uint32_t k_per_workgroup;  /* rows of k one workgroup covers */
     uint32_t workgroups;       /* of the launch (the first one, if there are two) */
-    uint32_t tail_workgroups;  /* of a second launch over a last, thin round of tiles, or 0 */
-    uint32_t launches;         /* 1 or 2 */
+    uint32_t tail_workgroups;  /* of further launches over a last, thin round of tiles or over the last rows, or 0 */
+    uint32_t launches;         /* kernels launched: 1, or more with a tail or with split sums added by a launch of their own */
     uint32_t compute_units;    /* what the plan was made for */
     uint32_t reserved;
     uint64_t workspace_bytes;  /* what bfaintb_gemm[_prepacked]_workspace_bytes_ex reports for the same arguments */
