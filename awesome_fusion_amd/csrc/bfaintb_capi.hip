@@ -476,6 +476,23 @@ DecodePlan decode_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint32_t fo
     // 34.9, 42.8 / 37.3).  More weights stream better in whole lines per workgroup (14336 x 8192, m = 8 /
     // 16: 22.8 / 19.9, 25.1 / 21.2; 16384 x 8192, m = 1 .. 16: 12 - 15 % slower; 12288 x 12288, m = 8 .. 32: 10 - 44 %; 8192 x
     // 28672, m = 1 .. 32: 9 - 31 %; 28672 x 8192: 2 - 5 %).
+    // A short k and more than half a round of 128-column blocks: those, unsplit — a split's hand-over costs more than the k it
+    // saves (us, this / the plan below, m = 1 / 8 / 16 / 32: 24576 x 1536 8-bit 10.0 / 10.8 / 11.9 / 14.4 against 11.5 / 12.1 /
+    // 13.6 / 19.5, 4-bit 9.3 / 9.7 / 10.5 / 12.6 against 10.1 / 11.4 / 12.3 / 19.0; 24576 x 2048 4-bit, m = 8 / 16 / 32: 12.1 / 12.9 /
+    // 15.4 against 12.9 / 13.8 / 18.9; 16640 x 2048 8-bit, m = 32: 15.0 / 17.5).  At k = 2048 few rows are level or lose: 20480 x
+    // 2048 8-bit, m = 1 / 16: 13.0 / 14.8 against 11.7 / 14.2.  From three quarters of a round on 4 waves lead 8 by 1 - 5 %
+    // up to 16 rows (32768 x 1536 8-bit, m = 1: 10.8 / 11.6).
+    if (!packed && forced_splits == 0 && m <= 32u && (k <= 1536u || (k <= 2048u && (m > 16u || (bits == 4 && m >= 8u))))) {
+        const uint32_t blocks = (n + 127u) / 128u, cus = machine_cus();
+        if (blocks * 2u > cus && blocks <= cus) {
+            DecodePlan pl;
+            pl.cols = 128u;
+            pl.waves = m <= 16u && blocks * 4u >= cus * 3u ? 4u : 8u;
+            pl.mb = m <= 16u ? 1u : 2u;
+            set_splits(pl, k, bits, 1u);
+            return pl;
+        }
+    }
     if (bits == 4 && !packed) {
         const uint64_t code_bytes = (uint64_t)n * k / 2u;
         if (code_bytes <= (24ull << 20) || (m >= 16u && code_bytes <= (40ull << 20)) || (m > 16u && code_bytes <= (64ull << 20)))
@@ -513,6 +530,14 @@ DecodePlan decode_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint32_t fo
         // launch), for m >= 8 (partial sums weigh most), and elsewhere when its best split factor fills whole
         // rounds; otherwise large matrices stream better in 256-byte row segments.  4-bit codes: wide.
         const bool few = weight_bytes <= (32ull << 20);
+        // Up to 8 rows and 24 to 72 MiB of weights, the narrow form runs 4 waves instead of 8: each has twice the steps behind its
+        // first loads, the workgroup half the sums to add through LDS, and k divides into more split factors (us, 8 / 4 waves,
+        // m = 1 / 8: 4096 x 11008 13.2 / 12.0 and 13.9 / 13.1; 8192 x 4096 10.3 / 9.4 and 11.0 / 10.1; 3072 x 8192 9.8 / 9.2 and 10.8 /
+        // 9.9; 8192 x 8192 15.8 / 14.8 and 16.6 / 16.2; 3584 x 18944 15.8 / 15.3 and 17.1 / 16.2; level at 4096 x 14336 and
+        // 11008 x 4096).  Fewer bytes are over before the longer chain pays (4096 x 4096, m = 1: 7.4 / 8.3), more rows want the
+        // waves to hide their activations behind (m = 16: 3072 x 8192 11.7 / 12.0, 2560 x 10240 11.4 / 13.0).
+        // (rows of B that are not whole cache lines: 1 % on average and up to 8 % slower over 24 shapes, so whole lines only)
+        const bool four_waves = bits == 8 && !packed && !nibbles && m <= 8u && n % 128u == 0 && weight_bytes >= (24ull << 20) && weight_bytes <= (72ull << 20);
         // the split-K partial sums (written, read back and cleared as fp32) stay below a quarter of the weight bytes
         uint32_t cap = (uint32_t)(((uint64_t)k * (uint32_t)bits) / (256u * (m ? m : 1u)));
         if (cap < 1) cap = 1;
@@ -531,7 +556,7 @@ DecodePlan decode_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint32_t fo
             DecodePlan probe{};
             probe.unit_bits = nibbles ? 4u : 0u;
             probe.cols = 128u;
-            probe.waves = 8u;
+            probe.waves = four_waves ? 4u : 8u;
             probe.mb = m <= 16 ? 1u : 2u;
             set_splits(probe, k, bits, s, packed);
             if (probe.splits != s) continue;
@@ -553,6 +578,19 @@ DecodePlan decode_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint32_t fo
         // m = 1 / 8 / 16: 36864 x 4096, 6 splits x 288 blocks = 6.75 rounds, 39.8 / 43.3 / 47.9 us, its best factor, 2, 37.1 /
         // 39.4 / 42.7, wide 31.5 / 33.2 / 35.4; 24576 x 4096, 4 x 192 = 3 rounds, 23.6 / 25.7 / 28.2 against 20.5 / 21.8 / 23.5)
         const bool fills_rounds = narrow_wgs <= cus && narrow_wgs * 20u >= cus * 19u;
+        // 4-bit codes, 17 to 32 rows, up to 192 blocks of 128 columns, and too many of 256 for three splits in a round: that form
+        // makes one thin round of 4-wave workgroups, k split in two; the 128-column form with 4 waves and k split four ways puts two to three on every CU (us at m = 18 / 32:
+        // 22016 x 4096 20.6 / 23.9 against 25.6 / 26.7; 24576 x 4096 24.1 / 27.8 against 26.6 / 27.7; 22016 x 5120 24.2 / 28.3
+        // against 29.1 / 30.0; rows of B that are not whole lines lose 3 - 6 % by it: 24000 x 4608, m = 32: 30.5 / 29.5).
+        if (nibbles && !packed && forced_splits == 0 && m > 16u && (n + 255u) / 256u * 3u > cus && narrow_blocks * 4u <= cus * 3u && n % 256u == 0 &&
+            k <= 5120u) {
+            DecodePlan probe = pl;
+            probe.cols = 128u;
+            probe.waves = 4u;
+            probe.mb = 2u;
+            set_splits(probe, k, bits, 4u, packed);
+            if (probe.splits == 4u) return probe;
+        }
         // m >= 8 on a wide matrix: once 256-column blocks fill their one round with at most 3 splits (more than 64 of
         // them) their partial sums no longer outweigh the better stream (m = 8 / 16 / 32, wide against narrow:
         // 22016 x 4096 20.9 / 22.7 / 28.2 against 21.9 / 23.4 / 31.6 us; 28672 x 8192 46.2 / 48.3 / 54.2 against 49.8 / 53.1 /
@@ -575,7 +613,7 @@ DecodePlan decode_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint32_t fo
         // 8192 x 8192: 17.2 / 19.2, 28672 x 8192: 36.2 / 37.5; m = 8: 10.1 / 11.2, 10.2 / 12.7, 15.7 / 17.8, 35.1 / 35.3;
         // no difference at m = 1).  The kernels over packed 4-bit codes are built for 4 waves.
         const bool wide8 = bits == 4 && m >= 8u && !packed;
-        pl.waves = (narrow || wide8) ? 8u : 4u;
+        pl.waves = ((narrow && !four_waves) || wide8) ? 8u : 4u;
         pl.mb = m <= 16 ? 1u : 2u;
         uint32_t splits = forced_splits;
         if (splits == 0) {

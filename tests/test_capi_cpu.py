@@ -351,3 +351,17 @@ def test_product_does_not_reach_for_the_oracle():
             if f.endswith((".py", ".hip", ".hpp", ".h", ".cc", ".cpp", "Makefile")):
                 text = open(os.path.join(dirpath, f), errors="ignore").read()
                 assert "oracle" not in text.lower(), os.path.join(dirpath, f)
+
+
+@pytest.mark.parametrize("m,n,k,bits,group,want", [
+    # up to 8 rows and 24 to 72 MiB of whole lines: 4 waves; below, beyond and with rows of B that are not whole lines: 8
+    (1, 4096, 11008, 8, 0, (128, 4, 8)), (8, 8192, 4096, 8, 0, (128, 4, 4)), (9, 8192, 4096, 8, 0, (128, 8, 4)), (1, 4096, 4096, 8, 0, (128, 8, 8)),
+    (1, 8208, 4096, 8, 0, (256, 4, 7)),
+    # a short k and more than half a round of 128-column blocks: unsplit, 4 waves from three quarters of a round up to 16 rows
+    (1, 24576, 1536, 8, 0, (128, 4, 1)), (16, 20480, 1536, 8, 0, (128, 8, 1)), (32, 24576, 2048, 4, 128, (128, 8, 1)), (8, 24576, 2048, 4, 128, (128, 4, 1)),
+    # 4-bit codes, 17 to 32 rows: four splits of 4 waves; not where three splits of 256 columns fit a round
+    (32, 22016, 4096, 4, 128, (128, 4, 4)), (32, 21760, 4096, 4, 128, (256, 4, 3)), (32, 24576, 5248, 4, 128, (256, 4, 2))])
+def test_launch_shapes_of_the_decode_family(m, n, k, bits, group, want):
+    p = af.plan(m, n, k, bits, group)
+    if p.compute_units == 256:
+        assert (p.tile_cols, p.waves, p.splits) == want, p.as_dict()
