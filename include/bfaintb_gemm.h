@@ -179,8 +179,9 @@ BFAINTB_API int bfaintb_gemm_reference_ex(void* c, const void* a, const void* b,
                               int variant, uint32_t split_k);
 
 /* Scratch the GEMM needs for a shape: a 256-byte header, then one fp32 word per (split but the last, row,
- * column) of the split-K partial sums, rounded up to 256 bytes; 0 when the shape runs without split-K.  Depends only
- * on its arguments.  The reference kernel has no scratch (no split-K, bfAintBGemm.cc:107-109). */
+ * column) of the split-K partial sums — of every split where a launch of its own adds them — rounded up to 256 bytes; 0 when
+ * the shape runs without split-K.  A product made in two launches by rows needs the larger of the two parts' scratch, and
+ * falls back to one launch without it.  Depends only on its arguments.  The reference kernel has no scratch (no split-K, bfAintBGemm.cc:107-109). */
 BFAINTB_API size_t bfaintb_gemm_workspace_bytes(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint32_t group_size);
 BFAINTB_API size_t bfaintb_gemm_workspace_bytes_ex(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint32_t group_size,
                                        int variant, uint32_t split_k);
