@@ -766,12 +766,24 @@ int device_state(hipStream_t stream, DeviceState** out)
     return BFAINTB_OK;
 }
 
+// The launches of one call that meet in a workspace (the tiles of a product and the second launch that adds their sums; the two
+// fills of an initialisation) leave and expect it at rest as one: on a stream nothing else that uses the workspace may come
+// between them, also where two host threads share stream and workspace.  So every launch that uses a workspace is made under
+// a lock that belongs to the workspace's address (one of 64: threads with workspaces of their own hardly ever meet), held
+// over all of the call's launches and nothing else.
+std::mutex& workspace_order(const void* workspace)
+{
+    static std::mutex locks[64];
+    return locks[(reinterpret_cast<uintptr_t>(workspace) >> 8) * 0x9e3779b97f4a7c15ull >> 58];
+}
+
 int init_workspace_on(void* workspace, size_t workspace_bytes, hipStream_t stream)
 {
     if (workspace_bytes % 4 != 0 || workspace_bytes / 4 >= (1ull << 32) || workspace_bytes < bfaintb::kWorkspaceHeaderBytes)
         return BFAINTB_ERR_WORKSPACE;
     // every word becomes "no partial sum here" (and "no failure" in the header), then the header gets its mark; fill
     // kernels rather than hipMemsetAsync, so that the call may be recorded into a HIP graph
+    std::lock_guard<std::mutex> in_order(workspace_order(workspace));
     hipError_t e = bfaintb::launch_fill_u32(static_cast<uint32_t*>(workspace), (uint32_t)(workspace_bytes / 4), kEmptyWord, stream);
     if (e == hipSuccess) e = bfaintb::launch_fill_u32(static_cast<uint32_t*>(workspace) + 1, 1u, bfaintb::kWorkspaceMagic, stream);
     return (int)e;
@@ -1115,6 +1127,8 @@ static int gemm_impl(void* c, const void* a, const void* b, const void* scale, c
         e = attach_workspace(p, workspace, BFAINTB_STATIC_SCRATCH_BYTES, need);
         if (e) return e;
     }
+    std::unique_lock<std::mutex> in_order;
+    if (p.splits > 1) in_order = std::unique_lock<std::mutex>(workspace_order(p.ws_header));
     if (tiled) {
         if (small_wreg) return (int)bfaintb::launch_prefill128_wreg(p, weight_bits, false, st);
         if ((v == BFAINTB_VARIANT_PREFILL_256X128 || (v == BFAINTB_VARIANT_PREFILL && prefill_tall_tiles(m, n, weight_bits))) && !p.reference_arith)
@@ -1563,9 +1577,11 @@ static int gemm_prepacked_impl(void* c, const void* a, const void* packed_b, con
             p.k_per_wg = tp.k_per_wg;
             p.splits = tp.splits;
             p.finish_launch = tp.finish_launch;
+            std::unique_lock<std::mutex> in_order;
             if (p.splits > 1) {
                 e = attach_workspace(p, workspace, workspace_bytes, packed_workspace_need(m, n, k, weight_bits, v));
                 if (e) return e;
+                in_order = std::unique_lock<std::mutex>(workspace_order(p.ws_header));
             }
             return (int)bfaintb::launch_prefill128_wreg(p, weight_bits, true, st);
         }
@@ -1595,6 +1611,8 @@ static int gemm_prepacked_impl(void* c, const void* a, const void* packed_b, con
         DeviceState* dev = nullptr;
         e = device_state(st, &dev);
         if (e) return e;
+        std::unique_lock<std::mutex> in_order;
+        if (p.splits > 1) in_order = std::unique_lock<std::mutex>(workspace_order(p.ws_header));
         return (int)bfaintb::launch_decode_family_packed(p, weight_bits, st);
     }
     return (int)bfaintb::launch_decode_packed(p, weight_bits, st);
