@@ -307,14 +307,15 @@ PyObject* linear_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs)
     Tensor y;
     {
         pybind11::gil_scoped_release release;
-        Tensor x2 = x.dim() == 2 && x.size(1) == in ? x : x.reshape({-1, in});
+        const bool as_it_is = x.dim() == 2 && x.size(1) == in;
+        Tensor x2 = as_it_is ? x : x.reshape({-1, in});
         if (x2.scalar_type() != at::kBFloat16) x2 = x2.to(at::kBFloat16);
         if (r.has_value()) {
             if (r->dim() != 2 || r->size(1) != out) r = r->reshape({-1, out});
             if (r->scalar_type() != at::kBFloat16) r = r->to(at::kBFloat16);
         }
         y = (packed ? op_handle<true>() : op_handle<false>()).call(x2, w, s, bits, group, b, r, 0);
-        if (x.dim() != 2) {
+        if (!as_it_is) {  // (also of two dimensions but another width: refused here, by the number of elements)
             auto shape = x.sizes().vec();
             if (shape.empty()) shape.push_back(out);
             shape.back() = out;

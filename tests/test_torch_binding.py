@@ -25,6 +25,33 @@ def test_layers_and_tensors_the_short_way_does_not_know_take_the_long_one():
         torch.ops.awesome_fusion.bfaintb_gemm(x.float(), layer.qweight, layer.scales, 8, 0)
 
 
+@pytest.fixture
+def stand_in():
+    """The row-major operator on CPU tensors: every output is the sum of its row of ``a``."""
+    lib = torch.library.Library("awesome_fusion", "IMPL")
+    lib.impl("bfaintb_gemm", lambda a, b, scale, bits, group, bias=None, residual=None, activation=0:
+             a.float().sum(1, keepdim=True).expand(-1, scale.shape[1]).to(torch.bfloat16).contiguous(), "CPU", allow_override=True)
+    yield
+    lib._destroy()
+
+
+@pytest.mark.filterwarnings("ignore:Warning only once for all operators")
+@pytest.mark.parametrize("shape", [(2, 64), (64,), (0, 64), (0, 32), (2, 3, 64), (1, 1, 1, 64), (0, 2, 64),
+                                   (4, 32), (2, 128), (64, 1), (128,), (2, 3, 32), (4, 16, 4)])
+def test_inputs_of_another_width_are_refused(stand_in, shape):
+    """Both ways through the layer take the same inputs: [..., in_features] (and nothing of another width whose number of
+    elements happens to be a multiple of it)."""
+    layer = top.QuantLinear(64, 32)
+    x = torch.ones(shape, dtype=torch.bfloat16)
+    want = x.reshape(-1, 64).float().sum(1, keepdim=True).expand(-1, 32).to(torch.bfloat16)
+    if shape[-1] == 64 or x.numel() == 0:
+        y = layer(x)
+        assert y.shape == shape[:-1] + (32,) and torch.equal(y.reshape(-1, 32), want)
+    else:
+        with pytest.raises(RuntimeError, match="invalid for input of size"):
+            layer(x)
+
+
 def _layer(n, k, bits, bias):
     lin = torch.nn.Linear(k, n, bias=bias).cuda()
     return top.QuantLinear.from_float(lin, bits, 0)
