@@ -15,6 +15,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/library.h>
 
 #include <algorithm>
@@ -279,7 +280,9 @@ bool plain_tensor(PyObject* o) { return o != nullptr && THPVariable_CheckTypeExa
 PyObject* linear_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs)
 {
     HANDLE_TH_ERRORS
-    if (nargs != 3 || !PyDict_Check(args[0]) || !plain_tensor(args[1]) || at::impl::torch_function_mode_enabled()) Py_RETURN_NOTIMPLEMENTED;
+    // (torch.jit.trace writes sizes read here down as constants: the long way's stay those of the input)
+    if (nargs != 3 || !PyDict_Check(args[0]) || !plain_tensor(args[1]) || at::impl::torch_function_mode_enabled() || torch::jit::tracer::isTracing())
+        Py_RETURN_NOTIMPLEMENTED;
     PyObject* const d = args[0];
     PyObject* const buffers = PyDict_GetItem(d, g_names.buffers);
     PyObject* const parameters = PyDict_GetItem(d, g_names.parameters);

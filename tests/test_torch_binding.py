@@ -52,6 +52,19 @@ def test_inputs_of_another_width_are_refused(stand_in, shape):
             layer(x)
 
 
+@pytest.mark.filterwarnings("ignore:Warning only once for all operators", "ignore:.*torch.jit.trace:DeprecationWarning")
+@pytest.mark.parametrize("lead,others", [((2, 3), [(5, 3), (2, 7), (4, 1)]), ((2,), [(7,), (1,)]), ((), [()])])
+def test_traces_follow_the_leading_sizes(stand_in, lead, others):
+    """torch.jit.trace of the layer, with and without a residual in the call, at other leading sizes than the traced ones."""
+    layer = top.QuantLinear(64, 32)
+    ones = lambda sizes, width: torch.ones(sizes + (width,), dtype=torch.bfloat16)
+    for extra in (False, True):
+        inputs = lambda sizes: (ones(sizes, 64), ones(sizes, 32)) if extra else (ones(sizes, 64),)
+        traced = torch.jit.trace(layer, inputs(lead), check_trace=False)
+        for sizes in [lead] + others:
+            assert torch.equal(traced(*inputs(sizes)), layer(*inputs(sizes))), (lead, sizes, extra)
+
+
 def _layer(n, k, bits, bias):
     lin = torch.nn.Linear(k, n, bias=bias).cuda()
     return top.QuantLinear.from_float(lin, bits, 0)
