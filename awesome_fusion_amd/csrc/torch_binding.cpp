@@ -329,6 +329,9 @@ PyObject* linear_forward(PyObject*, PyObject* const* args, Py_ssize_t nargs)
     END_HANDLE_TH_ERRORS
 }
 
+// The device pointer of an argument.  WRITTEN: what the call writes to — a tensor that shares its memory with a lazy copy
+// gets memory of its own first.
+template <bool WRITTEN>
 bool pointer_of(PyObject* o, const void** out)
 {
     if (o == Py_None) {
@@ -340,7 +343,8 @@ bool pointer_of(PyObject* o, const void** out)
         return !PyErr_Occurred();
     }
     if (THPVariable_Check(o)) {
-        *out = THPVariable_Unpack(o).const_data_ptr();
+        const Tensor& t = THPVariable_Unpack(o);
+        *out = WRITTEN ? t.mutable_data_ptr() : t.const_data_ptr();
         return true;
     }
     PyObject* const address = PyObject_CallMethod(o, "data_ptr", nullptr);  // (whatever else carries a device pointer)
@@ -361,8 +365,8 @@ PyObject* gemm_call(PyObject*, PyObject* const* args, Py_ssize_t nargs)
         return nullptr;
     }
     const void *c, *a, *b, *scale, *bias, *residual, *workspace;
-    if (!pointer_of(args[1], &c) || !pointer_of(args[2], &a) || !pointer_of(args[3], &b) || !pointer_of(args[4], &scale) || !pointer_of(args[5], &bias) ||
-        !pointer_of(args[6], &residual) || !pointer_of(args[17], &workspace))
+    if (!pointer_of<true>(args[1], &c) || !pointer_of<false>(args[2], &a) || !pointer_of<false>(args[3], &b) || !pointer_of<false>(args[4], &scale) ||
+        !pointer_of<false>(args[5], &bias) || !pointer_of<false>(args[6], &residual) || !pointer_of<true>(args[17], &workspace))
         return nullptr;
     uint32_t v[22] = {};
     for (int i : {7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 20, 21}) {

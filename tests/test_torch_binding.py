@@ -65,6 +65,20 @@ def test_traces_follow_the_leading_sizes(stand_in, lead, others):
             assert torch.equal(traced(*inputs(sizes)), layer(*inputs(sizes))), (lead, sizes, extra)
 
 
+@pytest.mark.parametrize("packed", [False, True])
+def test_what_a_call_writes_is_no_lazy_copy(packed):
+    """The output and the workspace of a call have memory of their own before the call gets their addresses; what it only
+    reads stays shared.  (The call itself is one that the library refuses before any launch.)"""
+    call = af.gemm_prepacked if packed else af.gemm
+    shared = [torch.zeros(4096, dtype=torch.uint8) for _ in range(7)]
+    c, a, b, scale, bias, residual, workspace = copies = [torch._lazy_clone(t) for t in shared]
+    assert all(torch._C._is_cow_tensor(t) for t in copies)
+    rc = call(c, a, b, scale, 1, 16, 128, lda=8, bias=bias, residual=residual, workspace=workspace, stream=0, check=False)
+    assert rc == -3
+    assert [torch._C._is_cow_tensor(t) for t in copies] == [False, True, True, True, True, True, False]
+    assert c.data_ptr() != shared[0].data_ptr() and workspace.data_ptr() != shared[6].data_ptr()
+
+
 def _layer(n, k, bits, bias):
     lin = torch.nn.Linear(k, n, bias=bias).cuda()
     return top.QuantLinear.from_float(lin, bits, 0)
