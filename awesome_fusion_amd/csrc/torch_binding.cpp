@@ -355,8 +355,8 @@ bool pointer_of(PyObject* o, const void** out)
 }
 
 // gemm_call(packed, c, a, b, scale, bias, residual, ldr, activation, m, n, k, lda, ldb, ldc, weight_bits, group_size, workspace,
-//           workspace_nbytes, stream, which, force_split_k) -> return code.  workspace_nbytes None: all of the tensor;
-//           stream None: torch's current one on c's device.
+//           workspace_nbytes, stream, which, force_split_k) -> return code.  workspace_nbytes None: all of the workspace (0 for a
+//           bare address); stream None: torch's current one on the current device.
 PyObject* gemm_call(PyObject*, PyObject* const* args, Py_ssize_t nargs)
 {
     HANDLE_TH_ERRORS
@@ -379,6 +379,16 @@ PyObject* gemm_call(PyObject*, PyObject* const* args, Py_ssize_t nargs)
         if (ws_bytes == (size_t)-1 && PyErr_Occurred()) return nullptr;
     } else if (THPVariable_Check(args[17])) {
         ws_bytes = THPVariable_Unpack(args[17]).nbytes();
+    } else if (args[17] != Py_None && !PyLong_Check(args[17])) {  // (whatever else carries a device pointer, as above)
+        size_t factors[2];
+        for (int i = 0; i < 2; ++i) {
+            PyObject* const value = PyObject_CallMethod(args[17], i == 0 ? "numel" : "element_size", nullptr);
+            if (value == nullptr) return nullptr;
+            factors[i] = PyLong_AsSize_t(value);
+            Py_DECREF(value);
+            if (factors[i] == (size_t)-1 && PyErr_Occurred()) return nullptr;
+        }
+        ws_bytes = factors[0] * factors[1];
     }
     void* stream = nullptr;
     if (args[19] == Py_None) stream = c10::hip::getCurrentHIPStream().stream();

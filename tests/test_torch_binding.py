@@ -79,6 +79,30 @@ def test_what_a_call_writes_is_no_lazy_copy(packed):
     assert c.data_ptr() != shared[0].data_ptr() and workspace.data_ptr() != shared[6].data_ptr()
 
 
+def test_a_workspace_of_another_kind_brings_its_own_size():
+    """Whatever has data_ptr, numel and element_size serves as a workspace, as it does as an operand: large enough (refused for
+    its alignment, the check after the size's), too small, without a size."""
+    class Memory:
+        def __init__(self, words):
+            self.words = words
+
+        def data_ptr(self):
+            return 0x10008
+
+        def numel(self):
+            return self.words
+
+        def element_size(self):
+            return 4
+
+    call = lambda ws: af.gemm(*[0x10000] * 4, 1, 4096, 4096, workspace=ws, stream=0, check=False)
+    need = af.workspace_bytes(1, 4096, 4096)
+    assert need > 0 and call(Memory(need // 4)) == -4 and call(Memory(need // 4 - 1)) == -6 and call(Memory(0)) == -6
+    Memory.numel = None
+    with pytest.raises(TypeError):
+        call(Memory(need))
+
+
 def _layer(n, k, bits, bias):
     lin = torch.nn.Linear(k, n, bias=bias).cuda()
     return top.QuantLinear.from_float(lin, bits, 0)
