@@ -269,7 +269,9 @@ static size_t split_workspace_bytes(uint32_t splits, uint32_t m, uint32_t n)
 // (with a second launch the last split's sums lie there as well)
 static size_t tile_workspace_bytes(const TilePlan& t, uint32_t m, uint32_t n) { return split_workspace_bytes(t.splits + t.finish_launch, m, n); }
 
-static TilePlan tile128_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint32_t forced_splits)
+// second_launch: whether the plan may be one whose sums a second launch adds.  Here and below, false is for the caller who
+// brings less scratch than such a plan needs (all splits' sums) and gets what the library does without it.
+static TilePlan tile128_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint32_t forced_splits, bool second_launch = true)
 {
     const uint32_t ksteps = (k + 63u) / 64u;
     const double tiles = (double)((m + 127u) / 128u) * (double)((n + 127u) / 128u);
@@ -326,7 +328,8 @@ static TilePlan tile128_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint3
         // from six splits on their sums are added by a second launch, if all of them fit the scratch of the entry point that
         // brings its own
         // (not for 4-bit codes beyond 256 rows: there the family's rule above keeps the shapes that would split so far)
-        if (s >= kFinishLaunchSplits) {
+        if (!second_launch && (s == 7u || s > 8u)) continue;  // (measured with the second launch only)
+        if (second_launch && s >= kFinishLaunchSplits) {
             if (bits == 4 && m > 256u) break;
             t.finish_launch = 1u;
             if (tile_workspace_bytes(t, m, n) > BFAINTB_STATIC_SCRATCH_BYTES) break;
@@ -353,9 +356,9 @@ static TilePlan tile128_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint3
     return best;
 }
 
-static double prefill_estimate_us(uint32_t m, uint32_t n, uint32_t k, int bits)
+static double prefill_estimate_us(uint32_t m, uint32_t n, uint32_t k, int bits, bool second_launch = true)
 {
-    if (prefill_small_tiles(m, n, bits)) return tile128_plan(m, n, k, bits, 0).us;
+    if (prefill_small_tiles(m, n, bits)) return tile128_plan(m, n, k, bits, 0, second_launch).us;
     const double cus = (double)machine_cus();
     if (prefill_tall_tiles(m, n, bits)) {
         // one tile of 256 rows x 128 columns per CU at most (8-bit, us per K-step: 512 x 11008 x 4096, 172 tiles: 0.87;
@@ -376,10 +379,10 @@ static double prefill_estimate_us(uint32_t m, uint32_t n, uint32_t k, int bits)
 // not whole cache lines slow the family's reads by 30 % (8-bit; 127 x 1072 x 6016 18.1 us, tiles 13.6) and the tiles' copies by
 // little; in whole lines the family holds small weights (4-bit 64 x 4096 x 4096 11.7 against 13.6, 128 x 2048 x 8192 16.4
 // against 18.1) and loses long ones (8-bit 96 x 4096 x 11008 35.0 / 23.4, 64 rows 24.0 / 19.7; packed 29.6 / 22.6 and 21.5 / 19.5).
-static bool family_leads_tiles(double family_us, uint32_t m, uint32_t n, uint32_t k, int bits, bool packed)
+static bool family_leads_tiles(double family_us, uint32_t m, uint32_t n, uint32_t k, int bits, bool packed, bool second_launch)
 {
-    double us = prefill_estimate_us(m, n, k, bits);
-    if (prefill_small_tiles(m, n, bits) && tile128_plan(m, n, k, bits, 0).finish_launch) {
+    double us = prefill_estimate_us(m, n, k, bits, second_launch);
+    if (prefill_small_tiles(m, n, bits) && tile128_plan(m, n, k, bits, 0, second_launch).finish_launch) {
         const bool lines = n % (packed ? 128u : 1024u / (uint32_t)bits) == 0;  // (packed: whole workgroups of columns)
         if (packed) us *= bits == 8 ? 0.95 : lines ? 1.06 : 0.95;
         else us *= bits == 8 ? (lines ? 1.06 : 0.84) : (lines ? 1.2 : 1.0);
@@ -695,13 +698,13 @@ DecodePlan decode_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint32_t fo
 
 // The decode family up to 32 rows of A; beyond that whichever of the two the estimates favour (the prefill
 // kernel's 256x256 tiles leave most of the machine idle until m*n reaches a few hundred tiles).
-int resolve_variant(uint32_t m, uint32_t n, uint32_t k, int bits, int variant)
+int resolve_variant(uint32_t m, uint32_t n, uint32_t k, int bits, int variant, bool second_launch = true)
 {
     if (variant == BFAINTB_VARIANT_AUTO) {
         if (m <= kDecodeAutoMaxM) return BFAINTB_VARIANT_DECODE;
         if (m > kDecodeFamilyAutoMaxM) return BFAINTB_VARIANT_PREFILL;
         const DecodePlan pl = decode_plan(m, n, k, bits, 0);
-        return family_leads_tiles(decode_family_time_us(m, n, k, bits, pl), m, n, k, bits, false) ? BFAINTB_VARIANT_DECODE : BFAINTB_VARIANT_PREFILL;
+        return family_leads_tiles(decode_family_time_us(m, n, k, bits, pl), m, n, k, bits, false, second_launch) ? BFAINTB_VARIANT_DECODE : BFAINTB_VARIANT_PREFILL;
     }
     if (variant == BFAINTB_VARIANT_DECODE) return m <= kDecodeMaxM ? variant : BFAINTB_ERR_BAD_VARIANT;
     if (is_prefill(variant)) return variant;
@@ -1033,7 +1036,8 @@ static bool row_split_served(const void* workspace, size_t workspace_bytes, size
 
 static int gemm_impl(void* c, const void* a, const void* b, const void* scale, const Epilogue& ep, uint32_t m, uint32_t n, uint32_t k,
                      uint32_t lda, uint32_t ldb, uint32_t ldc, int weight_bits, uint32_t group_size, void* workspace,
-                     size_t workspace_bytes, void* stream, int variant, uint32_t split_k, bool use_static_scratch = false, bool whole = false)
+                     size_t workspace_bytes, void* stream, int variant, uint32_t split_k, bool use_static_scratch = false, bool whole = false,
+                     bool second_launch = true)
 {
     const void* bias = ep.bias;
     int e = check_format(k, weight_bits, group_size);
@@ -1043,7 +1047,7 @@ static int gemm_impl(void* c, const void* a, const void* b, const void* scale, c
     if (e) return e;
     if (lda < k || ldb < n || ldc < ep.out_cols(n) || lda % 8u != 0 || ldb % 16u != 0 || ldc % 8u != 0) return BFAINTB_ERR_BAD_LD;
     if (ldb >= (1u << 27)) return BFAINTB_ERR_BAD_LD;  // a lane's offset within 32 rows of B is kept in 32 bits
-    const int v = resolve_variant(m, n, k, weight_bits, variant);
+    const int v = resolve_variant(m, n, k, weight_bits, variant, second_launch);
     if (v < 0) return v;
     if (m == 0 || n == 0) return BFAINTB_OK;
     if (c == nullptr || a == nullptr || b == nullptr || scale == nullptr) return BFAINTB_ERR_NULL_POINTER;
@@ -1096,7 +1100,7 @@ static int gemm_impl(void* c, const void* a, const void* b, const void* scale, c
         // row-major weights on small tiles: that form, unless the other one is asked for by name
         small_wreg = tiled_may_split(v, m, n, weight_bits) && bfaintb::prefill128_wreg_serves(p);
         if (small_wreg) {
-            const TilePlan tp = tile128_plan(m, n, k, weight_bits, split_k);
+            const TilePlan tp = tile128_plan(m, n, k, weight_bits, split_k, second_launch);
             p.k_per_wg = tp.k_per_wg;
             p.splits = tp.splits;
             p.finish_launch = tp.finish_launch;
@@ -1113,6 +1117,9 @@ static int gemm_impl(void* c, const void* a, const void* b, const void* scale, c
     const size_t need = split_workspace_bytes(p.splits + p.finish_launch, m, n);
     if (p.splits > 1 && !use_static_scratch) {
         e = attach_workspace(p, workspace, workspace_bytes, need);
+        if (e && second_launch)  // less than this plan needs: what the library does without a second launch may need less, or none
+            return gemm_impl(c, a, b, scale, ep, m, n, k, lda, ldb, ldc, weight_bits, group_size, workspace, workspace_bytes, stream, variant, split_k, false,
+                             true, false);
         if (e) return e;
     }
     if (use_static_scratch && need > BFAINTB_STATIC_SCRATCH_BYTES) return BFAINTB_ERR_STATIC_SCRATCH;
@@ -1383,7 +1390,7 @@ static double packed_family_time_us(uint32_t m, uint32_t n, uint32_t k, int bits
 }
 // Which kernel multiplies by packed weights: the decode kernels (the slab-streaming one while packed_uses_slab, the
 // row-blocked family without a split along k beyond) or the tiled kernel, by the estimates that choose for row-major weights.
-static int packed_variant(uint32_t m, uint32_t n, uint32_t k, int bits, int variant)
+static int packed_variant(uint32_t m, uint32_t n, uint32_t k, int bits, int variant, bool second_launch = true)
 {
     if (variant == BFAINTB_VARIANT_DECODE) return m <= kDecodeMaxM ? variant : BFAINTB_ERR_BAD_VARIANT;
     if (is_prefill(variant)) return variant;
@@ -1391,7 +1398,7 @@ static int packed_variant(uint32_t m, uint32_t n, uint32_t k, int bits, int vari
     if (packed_uses_slab(m, n, k, bits) || m <= kDecodeAutoMaxM) return BFAINTB_VARIANT_DECODE;
     if (m > kDecodeFamilyAutoMaxM) return BFAINTB_VARIANT_PREFILL;
     const DecodePlan pl = packed_family_plan(m, n, k, bits);
-    return family_leads_tiles(packed_family_time_us(m, n, k, bits, pl), m, n, k, bits, true) ? BFAINTB_VARIANT_DECODE : BFAINTB_VARIANT_PREFILL;
+    return family_leads_tiles(packed_family_time_us(m, n, k, bits, pl), m, n, k, bits, true, second_launch) ? BFAINTB_VARIANT_DECODE : BFAINTB_VARIANT_PREFILL;
 }
 
 int bfaintb_gemm_prepacked_variant(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint32_t group_size)
@@ -1406,10 +1413,10 @@ int bfaintb_gemm_prepacked_variant(uint32_t m, uint32_t n, uint32_t k, int weigh
 }
 
 // Scratch of the packed path: the decode family (where the slab kernel is not used) and the small tiles split along k.
-static size_t packed_workspace_need(uint32_t m, uint32_t n, uint32_t k, int bits, int v)
+static size_t packed_workspace_need(uint32_t m, uint32_t n, uint32_t k, int bits, int v, bool second_launch = true)
 {
     if (m == 0 || n == 0) return 0;
-    if (is_prefill(v)) return tiled_may_split(v, m, n, bits) ? tile_workspace_bytes(tile128_plan(m, n, k, bits, 0), m, n) : 0;
+    if (is_prefill(v)) return tiled_may_split(v, m, n, bits) ? tile_workspace_bytes(tile128_plan(m, n, k, bits, 0, second_launch), m, n) : 0;
     if (v != BFAINTB_VARIANT_DECODE || packed_uses_slab(m, n, k, bits)) return 0;
     const DecodePlan pl = packed_family_plan(m, n, k, bits);
     if (pl.splits <= 1) return 0;
@@ -1520,7 +1527,7 @@ size_t bfaintb_gemm_prepacked_workspace_bytes(uint32_t m, uint32_t n, uint32_t k
 
 static int gemm_prepacked_impl(void* c, const void* a, const void* packed_b, const void* scale, const Epilogue& ep, uint32_t m,
                                uint32_t n, uint32_t k, uint32_t lda, uint32_t ldc, int weight_bits, uint32_t group_size,
-                               void* workspace, size_t workspace_bytes, void* stream, int variant, bool whole = false)
+                               void* workspace, size_t workspace_bytes, void* stream, int variant, bool whole = false, bool second_launch = true)
 {
     const void* bias = ep.bias;
     int e = check_format(k, weight_bits, group_size);
@@ -1530,7 +1537,7 @@ static int gemm_prepacked_impl(void* c, const void* a, const void* packed_b, con
     e = check_packed_shape(n, k, weight_bits);
     if (e) return e;
     if (lda < k || ldc < ep.out_cols(n) || lda % 8u != 0 || ldc % 8u != 0) return BFAINTB_ERR_BAD_LD;
-    const int v = packed_variant(m, n, k, weight_bits, variant);
+    const int v = packed_variant(m, n, k, weight_bits, variant, second_launch);
     if (v < 0) return v;
     if (m == 0 || n == 0) return BFAINTB_OK;
     if (c == nullptr || a == nullptr || packed_b == nullptr || scale == nullptr) return BFAINTB_ERR_NULL_POINTER;
@@ -1566,6 +1573,10 @@ static int gemm_prepacked_impl(void* c, const void* a, const void* packed_b, con
     bfaintb::set_group_division(p);
     p.cus = machine_cus();
     hipStream_t st = static_cast<hipStream_t>(stream);
+    auto attach = [&] { return attach_workspace(p, workspace, workspace_bytes, packed_workspace_need(m, n, k, weight_bits, v, second_launch)); };
+    auto without_second_launch = [&] {  // (as in gemm_impl)
+        return gemm_prepacked_impl(c, a, packed_b, scale, ep, m, n, k, lda, ldc, weight_bits, group_size, workspace, workspace_bytes, stream, variant, true, false);
+    };
     if (is_prefill(v)) {
         // a tile's 16 column blocks and a 256-row panel of A are addressed through 32-bit buffer extents
         if ((uint64_t)k * 256u * (uint32_t)weight_bits / 8u >= (1ull << 31) || (uint64_t)256 * lda * 2u >= (1ull << 31))
@@ -1573,14 +1584,14 @@ static int gemm_prepacked_impl(void* c, const void* a, const void* packed_b, con
         if (tiled_may_split(v, m, n, weight_bits) && bfaintb::prefill128_wreg_serves(p)) {
             // small tiles: the kernel that keeps the weights in registers, with the plan (split along k included) and the
             // workspace protocol of the row-major path
-            const TilePlan tp = tile128_plan(m, n, k, weight_bits, 0);
+            const TilePlan tp = tile128_plan(m, n, k, weight_bits, 0, second_launch);
             p.k_per_wg = tp.k_per_wg;
             p.splits = tp.splits;
             p.finish_launch = tp.finish_launch;
             std::unique_lock<std::mutex> in_order;
             if (p.splits > 1) {
-                e = attach_workspace(p, workspace, workspace_bytes, packed_workspace_need(m, n, k, weight_bits, v));
-                if (e) return e;
+                e = attach();
+                if (e) return second_launch ? without_second_launch() : e;
                 in_order = std::unique_lock<std::mutex>(workspace_order(p.ws_header));
             }
             return (int)bfaintb::launch_prefill128_wreg(p, weight_bits, true, st);
@@ -1605,8 +1616,8 @@ static int gemm_prepacked_impl(void* c, const void* a, const void* packed_b, con
         p.decode_cols = pl.cols;
         p.decode_mb = pl.mb;
         if (p.splits > 1) {
-            e = attach_workspace(p, workspace, workspace_bytes, packed_workspace_need(m, n, k, weight_bits, v));
-            if (e) return e;
+            e = attach();
+            if (e) return second_launch ? without_second_launch() : e;
         }
         DeviceState* dev = nullptr;
         e = device_state(st, &dev);

@@ -1,7 +1,7 @@
 // Calls from two host threads that share a stream and a workspace, on a stand-in for the HIP runtime that only writes down
 // who launches what: the launches of one call that meet in the workspace follow one another, with no other launch that uses
 // it in between.  (The executable's own definitions of the runtime's functions come before the runtime's.)
-#include <hip/hip_runtime.h>
+#include "stand_in_runtime.hpp"
 
 #include <chrono>
 #include <condition_variable>
@@ -17,7 +17,6 @@ static std::mutex g_mutex;
 static std::condition_variable g_cond;
 static std::vector<int> g_order;        // the thread of every launch
 static thread_local int t_thread = 0;   // 0: launches of the main thread pass unseen
-static alignas(256) unsigned char g_scratch[256];
 
 extern "C" {
 hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t)
@@ -31,13 +30,6 @@ hipError_t hipLaunchKernel(const void*, dim3, dim3, void**, size_t, hipStream_t)
     g_cond.wait_for(lock, std::chrono::milliseconds(100), [&] { return g_order.size() > seen && g_order.back() != t_thread; });
     return hipSuccess;
 }
-hipError_t hipGetDevice(int* device) { *device = 0; return hipSuccess; }
-hipError_t hipDeviceGetAttribute(int* value, hipDeviceAttribute_t, int) { *value = 256; return hipSuccess; }
-hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
-hipError_t hipGetLastError(void) { return hipSuccess; }
-hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* status) { *status = hipStreamCaptureStatusNone; return hipSuccess; }
-hipError_t hipGetSymbolAddress(void** address, const void*) { *address = g_scratch; return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 }
 
 static void* const kDev = reinterpret_cast<void*>(0x10000);        // never dereferenced

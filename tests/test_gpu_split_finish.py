@@ -33,6 +33,26 @@ def test_second_launch_matches_oracle_and_the_one_launch_form(m, n, k, bits, gro
     assert_close_gated(g, run_gemm(g, activation=af.ACT_SILU_GATE), "gated")
 
 
+@pytest.mark.parametrize("m,n,k,bits,packed", [(124, 2800, 1664, 8, False), (105, 4560, 3200, 8, True), (474, 1136, 1920, 8, False)])
+def test_without_scratch_no_second_launch_is_made(m, n, k, bits, packed):
+    """Calls that need scratch for the second launch only are served without any, by one launch."""
+    import torch
+    import awesome_fusion_amd as af
+    from helpers import from_dev_u16, to_dev
+    assert af.plan(m, n, k, bits, packed=packed).launches >= 2
+    p = Problem(m, n, k, bits, seed=m)
+    c = torch.zeros((m, n), dtype=torch.int16, device="cuda")
+    a, b, s = to_dev(p.a_bf), to_dev(p.b_bytes), to_dev(p.s_bf)
+    if packed:
+        w = torch.empty(af.prepack_bytes(n, k, bits), dtype=torch.uint8, device="cuda")
+        af.prepack(w, b, n, k, weight_bits=bits)
+        af.gemm_prepacked(c, a, w, s, m, n, k, weight_bits=bits)
+    else:
+        af.gemm(c, a, b, s, m, n, k, weight_bits=bits)
+    torch.cuda.synchronize()
+    assert_close_ulp(p, from_dev_u16(c), f"no scratch: {m}x{n}x{k} bits={bits} packed={packed}")
+
+
 def test_second_launch_reports_sums_that_never_came():
     """As in the one launch: NaNs, a poisoned header, and all well after initialisation."""
     import torch

@@ -1,0 +1,77 @@
+"""What calls launch, in what order and with how much scratch: the library on a stand-in for the HIP runtime (tests/cpp), and the
+same between two threads on the GPU."""
+import os
+import subprocess
+import threading
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def on_stand_in(tmp_path, name, lines=""):
+    import awesome_fusion_amd as af
+    lib, exe = os.path.dirname(af.library_path()), str(tmp_path / name)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-rdynamic", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(ROOT, "tests", "cpp", name + ".cc"), "-o", exe, "-L" + lib, "-l:libbfaintb_gemm.so",
+                    "-Wl,-rpath," + lib, "-L/opt/rocm/lib", "-lamdhip64", "-Wl,-rpath,/opt/rocm/lib", "-lpthread"], check=True)
+    return subprocess.run([exe], input=lines, capture_output=True, text=True, timeout=60)
+
+
+def test_launches_of_one_call_follow_one_another(tmp_path):
+    r = on_stand_in(tmp_path, "test_launch_order")
+    assert r.returncode == 0 and "all checks passed" in r.stdout, r.stdout[-3000:]
+
+
+# (shape, code width, packed, bytes without a second launch: what these calls needed before there was one)
+SCRATCH = [((124, 2800, 1664), 8, 0, 0), ((235, 1168, 1792), 8, 0, 0), ((105, 4560, 3200), 8, 1, 0), ((96, 4096, 11008), 8, 0, 4718848),
+           ((96, 4112, 7296), 4, 1, 3158272), ((33, 3200, 4608), 4, 0, 1689856), ((474, 1136, 1920), 8, 0, 0), ((991, 4832, 11392), 4, 0, 0),
+           ((1522, 2784, 8448), 8, 1, 0), ((314, 1120, 12672), 8, 1, 5627136), ((1, 4096, 4096), 8, 0, 114944)]
+
+
+def test_less_scratch_than_the_plan_needs(tmp_path):
+    """A caller who brings less than a second launch needs gets the product without one, if it fits, in one launch (or two
+    that share nothing); who brings less than that is refused."""
+    import awesome_fusion_amd as af
+    asked, wants = [], []
+    for (m, n, k), bits, packed, least in SCRATCH:
+        full = (af.prepacked_workspace_bytes if packed else af.workspace_bytes)(m, n, k, bits)
+        launches = af.plan(m, n, k, bits, packed=packed).launches
+        assert full > least or launches == 1
+        for nbytes, want in ((full, (0, launches)), (full - 256, (0, 1) if full > least else (-6, 0)), (least, (0, 1)), (least - 256, (-6, 0))):
+            if nbytes >= 0:
+                asked.append(f"{m} {n} {k} {bits} {packed} {nbytes}")
+                wants.append(want)
+    r = on_stand_in(tmp_path, "call_launches", "\n".join(asked))
+    got = [tuple(map(int, line.split())) for line in r.stdout.split("\n") if line]
+    assert got == wants, [x for x in zip(asked, got, wants) if x[1] != x[2]]
+
+
+@pytest.mark.gpu
+def test_two_threads_share_a_stream():
+    """The operators' workspace is one per stream: products in two launches and split decode calls from two threads."""
+    import torch
+    import awesome_fusion_amd as af
+    import awesome_fusion_amd.torch_op as top
+    torch.manual_seed(11)
+    shapes = [(96, 4096, 11008), (1, 4096, 4096)]
+    assert af.plan(*shapes[0]).launches == 2 and af.plan(*shapes[1]).splits > 1
+    layers = [top.QuantLinear.from_float(torch.nn.Linear(k, n, bias=False).cuda(), 8, 0) for _, n, k in shapes]
+    xs = [torch.randn((m, k), device="cuda", dtype=torch.bfloat16) for m, _, k in shapes]
+    want = [layer(x) for layer, x in zip(layers, xs)]
+    torch.cuda.synchronize()
+    outs = [[], []]
+
+    def work(i):
+        for rep in range(40):
+            j = (rep + i) % 2
+            outs[i].append((j, layers[j](xs[j])))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert all(len(o) == 40 for o in outs)
+    assert all(torch.equal(c, want[j]) for o in outs for j, c in o)
