@@ -1113,24 +1113,28 @@ static int gemm_impl(void* c, const void* a, const void* b, const void* scale, c
         p.decode_cols = pl.cols;
         p.decode_mb = pl.mb;
     }
+    // with less scratch than this plan needs: what the library does without a second launch may need less, or none
+    auto without_second_launch = [&] {
+        return gemm_impl(c, a, b, scale, ep, m, n, k, lda, ldb, ldc, weight_bits, group_size, workspace, workspace_bytes, stream, variant, split_k,
+                         use_static_scratch, true, false);
+    };
     // (every argument check comes before the first runtime call)
     const size_t need = split_workspace_bytes(p.splits + p.finish_launch, m, n);
     if (p.splits > 1 && !use_static_scratch) {
         e = attach_workspace(p, workspace, workspace_bytes, need);
-        if (e && second_launch)  // less than this plan needs: what the library does without a second launch may need less, or none
-            return gemm_impl(c, a, b, scale, ep, m, n, k, lda, ldb, ldc, weight_bits, group_size, workspace, workspace_bytes, stream, variant, split_k, false,
-                             true, false);
-        if (e) return e;
+        if (e) return second_launch ? without_second_launch() : e;
     }
     if (use_static_scratch && need > BFAINTB_STATIC_SCRATCH_BYTES) return BFAINTB_ERR_STATIC_SCRATCH;
     DeviceState* dev = nullptr;
     if (!tiled || (p.splits > 1 && use_static_scratch)) {
         e = device_state(st, &dev);
-        if (e) return e;
+        if (e) return p.finish_launch ? without_second_launch() : e;  // (a first call under capture)
     }
     if (p.splits > 1 && use_static_scratch) {
-        e = static_scratch(*dev, st, &workspace);
-        if (e) return e;
+        void* static_ptr = nullptr;
+        e = static_scratch(*dev, st, &static_ptr);
+        if (e) return p.finish_launch ? without_second_launch() : e;
+        workspace = static_ptr;
         e = attach_workspace(p, workspace, BFAINTB_STATIC_SCRATCH_BYTES, need);
         if (e) return e;
     }

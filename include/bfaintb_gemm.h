@@ -104,8 +104,10 @@ enum {
  *   workspace     device scratch of at least bfaintb_gemm_workspace_bytes(...) bytes that has been
  *                 passed through bfaintb_workspace_init once.
  *                 The call leaves it in that state again, ready for the next call of any shape.
- *                 Two calls that may run concurrently must not share a workspace.  May be NULL
- *                 when the required size is 0.
+ *                 Two calls that may run concurrently must not share a workspace (calls that two host
+ *                 threads make on one stream do not).  May be NULL when the required size is 0; with less
+ *                 than that size a shape whose sums a second launch adds is still served where the library
+ *                 can do without that launch, at the speed it has without.
  */
 BFAINTB_API int bfaintb_gemm(void* c, const void* a, const void* b, const void* scale, uint32_t m, uint32_t n, uint32_t k,
                  uint32_t lda, uint32_t ldb, uint32_t ldc, int weight_bits, uint32_t group_size, void* workspace,

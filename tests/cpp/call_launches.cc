@@ -1,5 +1,6 @@
-// Makes the calls it reads (m n k weight_bits packed workspace_bytes, one per line; 0 bytes: no workspace) on a stand-in for the
-// HIP runtime and prints what each returned and how many kernels it launched.
+// Makes the calls it reads (m n k weight_bits kind workspace_bytes, one per line; kind 0: bfaintb_gemm, 1: bfaintb_gemm_prepacked,
+// 2: bfaintb_gemm_static under capture; 0 bytes: no workspace) on a stand-in for the HIP runtime and prints what each returned
+// and how many kernels it launched.
 #include "stand_in_runtime.hpp"
 
 #include <cstdio>
@@ -18,13 +19,15 @@ int main()
 {
     void* const p = reinterpret_cast<void*>(0x10000);  // never dereferenced
     unsigned m, n, k;
-    int bits, packed;
+    int bits, kind;
     size_t bytes;
-    while (scanf("%u %u %u %d %d %zu", &m, &n, &k, &bits, &packed, &bytes) == 6) {
+    while (scanf("%u %u %u %d %d %zu", &m, &n, &k, &bits, &kind, &bytes) == 6) {
         void* const ws = bytes ? p : nullptr;
         g_launches = 0;
-        const int rc = packed ? bfaintb_gemm_prepacked(p, p, p, p, nullptr, m, n, k, k, n, bits, 0, ws, bytes, nullptr)
-                              : bfaintb_gemm(p, p, p, p, m, n, k, k, n, n, bits, 0, ws, bytes, nullptr);
+        g_capturing = kind == 2;
+        const int rc = kind == 2   ? bfaintb_gemm_static(p, p, p, p, m, n, k, k, n, n, bits, 0, nullptr)
+                       : kind == 1 ? bfaintb_gemm_prepacked(p, p, p, p, nullptr, m, n, k, k, n, bits, 0, ws, bytes, nullptr)
+                                   : bfaintb_gemm(p, p, p, p, m, n, k, k, n, n, bits, 0, ws, bytes, nullptr);
         printf("%d %d\n", rc, g_launches);
     }
     return 0;

@@ -47,6 +47,14 @@ def test_less_scratch_than_the_plan_needs(tmp_path):
     assert got == wants, [x for x in zip(asked, got, wants) if x[1] != x[2]]
 
 
+def test_a_first_call_under_capture_needs_no_second_launch(tmp_path):
+    """bfaintb_gemm_static before the device is set up, under capture: shapes that need its scratch for a second launch only are
+    served without one; a shape for the decode kernels, which need the set-up, is refused."""
+    shapes = [(63, 4784, 1368), (54, 4160, 1328), (96, 4096, 11008), (4096, 4096, 4096)]
+    r = on_stand_in(tmp_path, "call_launches", "\n".join("%d %d %d 8 2 0" % s for s in shapes))
+    assert r.stdout.split("\n")[:4] == ["0 1", "0 1", "-8 0", "0 1"]
+
+
 @pytest.mark.gpu
 def test_two_threads_share_a_stream():
     """The operators' workspace is one per stream: products in two launches and split decode calls from two threads."""
