@@ -18,6 +18,13 @@ def on_stand_in(tmp_path, name, lines=""):
     return subprocess.run([exe], input=lines, capture_output=True, text=True, timeout=60)
 
 
+def calls(tmp_path, lines):
+    """(return code, launches, workgroups of the first launch) of each call: "m n k weight_bits kind workspace_bytes"."""
+    r = on_stand_in(tmp_path, "call_launches", "\n".join(lines))
+    assert r.returncode == 0
+    return [tuple(map(int, line.split())) for line in r.stdout.split("\n") if line]
+
+
 def test_launches_of_one_call_follow_one_another(tmp_path):
     r = on_stand_in(tmp_path, "test_launch_order")
     assert r.returncode == 0 and "all checks passed" in r.stdout, r.stdout[-3000:]
@@ -42,8 +49,7 @@ def test_less_scratch_than_the_plan_needs(tmp_path):
             if nbytes >= 0:
                 asked.append(f"{m} {n} {k} {bits} {packed} {nbytes}")
                 wants.append(want)
-    r = on_stand_in(tmp_path, "call_launches", "\n".join(asked))
-    got = [tuple(map(int, line.split())) for line in r.stdout.split("\n") if line]
+    got = [x[:2] for x in calls(tmp_path, asked)]
     assert got == wants, [x for x in zip(asked, got, wants) if x[1] != x[2]]
 
 
@@ -51,8 +57,20 @@ def test_a_first_call_under_capture_needs_no_second_launch(tmp_path):
     """bfaintb_gemm_static before the device is set up, under capture: shapes that need its scratch for a second launch only are
     served without one; a shape for the decode kernels, which need the set-up, is refused."""
     shapes = [(63, 4784, 1368), (54, 4160, 1328), (96, 4096, 11008), (4096, 4096, 4096)]
-    r = on_stand_in(tmp_path, "call_launches", "\n".join("%d %d %d 8 2 0" % s for s in shapes))
-    assert r.stdout.split("\n")[:4] == ["0 1", "0 1", "-8 0", "0 1"]
+    assert [x[:2] for x in calls(tmp_path, ["%d %d %d 8 2 0" % s for s in shapes])] == [(0, 1), (0, 1), (-8, 0), (0, 1)]
+
+
+def test_reference_arithmetic_takes_the_kernel_it_has(tmp_path):
+    """The reference's arithmetic has no tiles with k split: where only those lead the decode family, it gets the family, with
+    the scratch that bfaintb_gemm_workspace_bytes asks for; without scratch it gets the tiles, unsplit."""
+    import awesome_fusion_amd as af
+    for shape in ((96, 4096, 11008), (64, 4096, 11008), (124, 2800, 1664), (300, 1040, 8192)):
+        assert af.variant(*shape) == af.PREFILL
+        family = af.plan(*shape, which=af.DECODE)
+        line = "%d %d %d 8 3 " % shape
+        (rc, launches, workgroups), bare = calls(tmp_path, [line + str(af.workspace_bytes(*shape)), line + "0"])
+        assert (rc, launches, workgroups) == (0, 1, family.workgroups), (shape, workgroups, family.workgroups)
+        assert bare[:2] == (0, 1) and (family.splits == 1 or bare[2] < workgroups)
 
 
 @pytest.mark.gpu
