@@ -19,6 +19,7 @@
 #include <torch/library.h>
 
 #include <algorithm>
+#include <atomic>
 #include <list>
 #include <mutex>
 #include <optional>
@@ -33,13 +34,16 @@ using OptTensor = std::optional<Tensor>;
 
 // ---- split-K workspaces: one per (device, stream).  Calls ordered on a stream may share one, calls on different streams
 //      may overlap and must not.  A workspace grows to at least twice its size, and the kMaxWorkspaces most recently used
-//      ones are kept.  What a captured graph may hold the address of is never given back (a replay does not come through here).
+//      ones are kept.  What a captured graph uses stays until the graph is gone, whatever becomes of it here (a replay does
+//      not come through here): the graph owns an object whose end says so.
 constexpr size_t kMaxWorkspaces = 64;
 constexpr int64_t kFirstWorkspaceBytes = 4 << 20;
 
-struct Workspace {
-    Tensor memory;
-    bool in_graph = false;
+// The workspaces of one capture, held until every graph made from it is gone.
+struct GraphHold {
+    unsigned long long capture;
+    std::vector<Tensor> held;
+    std::atomic<bool> gone{false};
 };
 struct WorkspaceKey {
     int device;
@@ -52,12 +56,40 @@ struct WorkspaceKeyHash {
 class WorkspacePool {
     std::mutex mutex_;
     std::list<WorkspaceKey> recent_;  // most recently made first
-    std::unordered_map<WorkspaceKey, Workspace, WorkspaceKeyHash> pool_;
-    std::vector<Tensor> in_graphs_;  // outgrown or dropped, and part of a captured graph
+    std::unordered_map<WorkspaceKey, Tensor, WorkspaceKeyHash> pool_;
+    std::vector<GraphHold*> graphs_;
 
-    void retire(Workspace& w)
+    // (called by the runtime, on a thread and under locks of its own, once the last graph is destroyed and has run: the rest is done
+    // by drop_gone)
+    static void graph_gone(void* hold) { static_cast<GraphHold*>(hold)->gone.store(true, std::memory_order_release); }
+
+    void drop_gone()
     {
-        if (w.in_graph) in_graphs_.push_back(std::move(w.memory));
+        const auto keep = std::partition(graphs_.begin(), graphs_.end(), [](const GraphHold* h) { return !h->gone.load(std::memory_order_acquire); });
+        std::for_each(keep, graphs_.end(), [](GraphHold* h) { delete h; });
+        graphs_.erase(keep, graphs_.end());
+    }
+
+    void hold_for_graph(const Tensor& memory, hipStream_t stream)
+    {
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        unsigned long long capture = 0;
+        hipGraph_t graph = nullptr;
+        const bool known = hipStreamGetCaptureInfo_v2(stream, &status, &capture, &graph, nullptr, nullptr) == hipSuccess && status == hipStreamCaptureStatusActive;
+        if (!known) capture = 0;
+        auto it = std::find_if(graphs_.begin(), graphs_.end(), [&](const GraphHold* h) { return h->capture == capture; });
+        if (it == graphs_.end()) {
+            drop_gone();
+            graphs_.push_back(new GraphHold{capture, {}});
+            it = graphs_.end() - 1;
+            hipUserObject_t object;
+            const bool owned = known && hipUserObjectCreate(&object, *it, graph_gone, 1, hipUserObjectNoDestructorSync) == hipSuccess &&
+                               hipGraphRetainUserObject(graph, object, 1, hipGraphUserObjectMove) == hipSuccess;
+            if (!owned) (void)hipGetLastError();  // (nothing will say when the graph is gone: held for good)
+        }
+        for (const Tensor& t : (*it)->held)
+            if (t.is_same(memory)) return;
+        (*it)->held.push_back(memory);
     }
 
 public:
@@ -69,38 +101,36 @@ public:
         const bool capturing = status != hipStreamCaptureStatusNone;
         std::lock_guard<std::mutex> lock(mutex_);
         auto it = pool_.find(key);
-        if (it != pool_.end() && it->second.memory.numel() >= bytes) {
-            it->second.in_graph |= capturing;
-            return it->second.memory;
+        if (it != pool_.end() && it->second.numel() >= bytes) {
+            if (capturing) hold_for_graph(it->second, stream);
+            return it->second;
         }
         int64_t size = std::max(bytes, kFirstWorkspaceBytes);
-        if (it != pool_.end() && !capturing) size = std::max(size, 2 * it->second.memory.numel());
+        if (it != pool_.end() && !capturing) size = std::max(size, 2 * it->second.numel());
         Tensor fresh = at::empty({size}, like.options().dtype(at::kByte));
         const int rc = bfaintb_workspace_init(fresh.data_ptr(), (size_t)size, stream);
         TORCH_CHECK(rc == 0, "bfaintb_workspace_init failed: [", rc, "] ", bfaintb_error_string(rc));
         // (made under capture: the graph's own, filled by the graph's own first node; not for calls outside it)
         if (capturing) return fresh;
+        drop_gone();
         if (it != pool_.end()) {
-            retire(it->second);
-            it->second = Workspace{fresh, false};
+            it->second = fresh;
             return fresh;
         }
         while (pool_.size() >= kMaxWorkspaces) {
-            auto last = pool_.find(recent_.back());
-            retire(last->second);
-            pool_.erase(last);
+            pool_.erase(recent_.back());
             recent_.pop_back();
         }
-        pool_.emplace(key, Workspace{fresh, false});
+        pool_.emplace(key, fresh);
         recent_.push_front(key);
         return fresh;
     }
     void clear()
     {
         std::lock_guard<std::mutex> lock(mutex_);
-        for (auto& kv : pool_) retire(kv.second);
         pool_.clear();
         recent_.clear();
+        drop_gone();
     }
 };
 WorkspacePool& workspaces()
@@ -443,7 +473,7 @@ PyMethodDef g_methods[] = {
     {"linear_forward", (PyCFunction)(void (*)(void))linear_forward, METH_FASTCALL, "QuantLinear's forward pass, or NotImplemented"},
     {"gemm_call", (PyCFunction)(void (*)(void))gemm_call, METH_FASTCALL, "one call of the C ABI: its return code"},
     {"set_error_class", set_error_class, METH_O, "the exception raised for the library's error codes: cls(code, what)"},
-    {"release_workspaces", release_workspaces, METH_NOARGS, "gives the operators' split-K workspaces back (those in captured graphs excepted)"},
+    {"release_workspaces", release_workspaces, METH_NOARGS, "gives the operators' split-K workspaces back (those of graphs that are still there excepted)"},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "_torch_binding", nullptr, -1, g_methods, nullptr, nullptr, nullptr, nullptr};
 

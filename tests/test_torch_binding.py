@@ -1,5 +1,7 @@
 """The native side of the PyTorch binding (awesome_fusion_amd/csrc/torch_binding.cpp): the linear layer's short way against
 the operator it calls, what it hands on to the long way, its errors, and the operators' workspaces."""
+import time
+
 import pytest
 import torch
 
@@ -176,3 +178,47 @@ def test_workspaces_by_stream_growth_and_capture():
             torch.full((64 << 20,), 7, dtype=torch.uint8, device="cuda")
             torch.cuda.synchronize()
             assert torch.equal(big, want_l)
+
+
+@pytest.mark.gpu
+def test_workspaces_of_graphs_are_given_back_with_them():
+    """A program that captures, drops the graph, releases and captures again holds no more memory than after the first round;
+    while a graph is there its workspace is, released, outgrown or not."""
+    torch.manual_seed(6)
+    small, large = _layer(1024, 4096, 8, False), _layer(4096, 8192, 8, False)
+    xs, xl = torch.randn((4, 4096), device="cuda", dtype=torch.bfloat16), torch.randn((256, 8192), device="cuda", dtype=torch.bfloat16)
+    assert 0 < af.workspace_bytes(4, 1024, 4096) <= 4 << 20 < af.workspace_bytes(256, 4096, 8192)
+    want = small(xs)
+    stream = torch.cuda.Stream()
+
+    def held():
+        torch.cuda.synchronize()
+        return torch.cuda.memory_allocated()
+
+    top.release_workspaces()
+    before = held()
+    for rep in range(4):
+        with torch.cuda.stream(stream):
+            small(xs)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            c, d = small(xs), small(xs)
+        if rep % 2:
+            with torch.cuda.stream(stream):
+                large(xl)  # the stream's workspace is replaced by a larger one
+        top.release_workspaces()
+        assert held() - before >= 4 << 20, "the graph's workspace went before the graph"
+        filler = torch.full((8 << 20,), 7, dtype=torch.uint8, device="cuda")
+        for _ in range(2):
+            c.zero_(), d.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(c, want) and torch.equal(d, want)
+        del graph, c, d, filler
+        for _ in range(100):  # (the runtime's own thread says that the graph is gone, a little after its end)
+            top.release_workspaces()
+            if held() - before < 1 << 20:
+                break
+            time.sleep(0.05)
+        assert held() - before < 1 << 20, f"round {rep} left memory behind"
