@@ -55,8 +55,12 @@ struct WorkspaceKeyHash {
 };
 class WorkspacePool {
     std::mutex mutex_;
-    std::list<WorkspaceKey> recent_;  // most recently made first
-    std::unordered_map<WorkspaceKey, Tensor, WorkspaceKeyHash> pool_;
+    struct Workspace {
+        Tensor memory;
+        std::list<WorkspaceKey>::iterator place;  // in recent_
+    };
+    std::list<WorkspaceKey> recent_;  // most recently used first
+    std::unordered_map<WorkspaceKey, Workspace, WorkspaceKeyHash> pool_;
     std::vector<GraphHold*> graphs_;
 
     // (called by the runtime, on a thread and under locks of its own, once the last graph is destroyed and has run: the rest is done
@@ -101,12 +105,13 @@ public:
         const bool capturing = status != hipStreamCaptureStatusNone;
         std::lock_guard<std::mutex> lock(mutex_);
         auto it = pool_.find(key);
-        if (it != pool_.end() && it->second.numel() >= bytes) {
-            if (capturing) hold_for_graph(it->second, stream);
-            return it->second;
+        if (it != pool_.end()) recent_.splice(recent_.begin(), recent_, it->second.place);
+        if (it != pool_.end() && it->second.memory.numel() >= bytes) {
+            if (capturing) hold_for_graph(it->second.memory, stream);
+            return it->second.memory;
         }
         int64_t size = std::max(bytes, kFirstWorkspaceBytes);
-        if (it != pool_.end() && !capturing) size = std::max(size, 2 * it->second.numel());
+        if (it != pool_.end() && !capturing) size = std::max(size, 2 * it->second.memory.numel());
         Tensor fresh = at::empty({size}, like.options().dtype(at::kByte));
         const int rc = bfaintb_workspace_init(fresh.data_ptr(), (size_t)size, stream);
         TORCH_CHECK(rc == 0, "bfaintb_workspace_init failed: [", rc, "] ", bfaintb_error_string(rc));
@@ -114,15 +119,15 @@ public:
         if (capturing) return fresh;
         drop_gone();
         if (it != pool_.end()) {
-            it->second = fresh;
+            it->second.memory = fresh;
             return fresh;
         }
         while (pool_.size() >= kMaxWorkspaces) {
             pool_.erase(recent_.back());
             recent_.pop_back();
         }
-        pool_.emplace(key, fresh);
         recent_.push_front(key);
+        pool_.emplace(key, Workspace{fresh, recent_.begin()});
         return fresh;
     }
     void clear()

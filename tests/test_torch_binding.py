@@ -222,3 +222,34 @@ def test_workspaces_of_graphs_are_given_back_with_them():
                 break
             time.sleep(0.05)
         assert held() - before < 1 << 20, f"round {rep} left memory behind"
+
+
+@pytest.mark.gpu
+def test_a_stream_in_use_keeps_its_workspace():
+    """More streams than workspaces are kept for, and one that is used all along: its workspace is never the one to go."""
+    import ctypes
+    torch.manual_seed(7)
+    layer = _layer(1024, 4096, 8, False)
+    x = torch.randn((4, 4096), device="cuda", dtype=torch.bfloat16)
+    assert af.workspace_bytes(4, 1024, 4096) > 0
+    want = layer(x)
+    torch.cuda.synchronize()
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    handles = [ctypes.c_void_p() for _ in range(72)]
+    assert all(hip.hipStreamCreateWithFlags(ctypes.byref(h), 1) == 0 for h in handles)  # (non-blocking)
+    made = lambda: torch.cuda.memory_stats()["allocation.all.allocated"]
+    top.release_workspaces()
+    layer(x)
+    outs = []
+    for h in handles:
+        with torch.cuda.stream(torch.cuda.ExternalStream(h.value)):
+            outs.append(layer(x))
+        before = made()
+        outs.append(layer(x))
+        assert made() == before + 1, "more was allocated than the output"
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, want) for y in outs)
+    top.release_workspaces()
+    del outs
+    torch.cuda.synchronize()
+    assert all(hip.hipStreamDestroy(h) == 0 for h in handles)
