@@ -1,4 +1,5 @@
-"""ctypes binding of the C ABI in include/bfaintb_gemm.h.
+"""Python binding of the C ABI in include/bfaintb_gemm.h: ctypes, and for gemm and gemm_prepacked the native form of the same
+calls in csrc/torch_binding.cpp where that loads (it is built against the installed torch).
 
 Arguments mirror the reference's launch block {c, a, b, scale, m, n, k, lda, ldb, ldc}
 (/root/reference/bfAintBGemm/bfAintBGemm.cc:119-133).  Tensors are only carriers of device
@@ -7,6 +8,7 @@ pointers (``data_ptr()``); torch supplies device memory and streams, nothing els
 import ctypes as C
 import os
 import subprocess
+import warnings
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB = _PACKAGE_LIB = os.path.join(_HERE, "libbfaintb_gemm.so")
@@ -162,9 +164,10 @@ _binding = None
 
 def binding():
     """The native PyTorch binding (_torch_binding.so): the calls below go through it where torch is installed.  None without
-    torch, and while a library other than the package's own is loaded (an instrumented build)."""
+    torch, while a library other than the package's own is loaded (an instrumented build), and, with a warning, where it
+    does not load (not built, or built against another torch): the same calls then go through ctypes."""
     global _binding
-    if _LIB != _PACKAGE_LIB:
+    if _LIB != _PACKAGE_LIB or _binding is False:
         return None
     if _binding is None:
         lib()  # (raises if it is not built; loads torch first)
@@ -175,8 +178,10 @@ def binding():
         try:
             from . import _torch_binding
         except ImportError as e:
-            raise RuntimeError("awesome_fusion_amd/_torch_binding.so does not load: build it with `make -C awesome_fusion_amd/csrc` "
-                               f"(or __graft_entry__.build()), against the torch that is imported here: {e}") from e
+            warnings.warn("awesome_fusion_amd/_torch_binding.so does not load, so every call takes some 20 us more of host time: build it "
+                          f"with `make -C awesome_fusion_amd/csrc`, against the torch that is imported here ({e})", RuntimeWarning, stacklevel=2)
+            _binding = False
+            return None
         _torch_binding.set_error_class(BfaintbError)
         _binding = _torch_binding
     return _binding

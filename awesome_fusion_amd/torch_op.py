@@ -13,9 +13,9 @@ library:
 [k, n/2] (4-bit, excess-8, even column in the low nibble), ``scale`` bf16 [groups, n], ``bias`` bf16 [n] and
 ``residual`` bf16 [m, n] (added to the fp32 sums before the one rounding, inside the kernel); returns bf16 [m, n].  The
 operators are native code (``csrc/torch_binding.cpp``: the same path written in Python took 21 - 26 us of host time per
-call); this module gives them their shape inference.  torch supplies the output tensor, the current stream and a
-per-(device, stream) split-K workspace; all arithmetic happens in ``libbfaintb_gemm.so``.  There is no CPU
-implementation: on a CPU tensor the operator raises.
+call); this module gives them their shape inference, and their Python form where the native one does not load (with a
+warning).  torch supplies the output tensor, the current stream and a per-(device, stream) split-K workspace; all
+arithmetic happens in ``libbfaintb_gemm.so``.  There is no CPU implementation: on a CPU tensor the operator raises.
 
 ``quantize_weight`` (host-side helper, symmetric round-to-nearest) and ``QuantLinear`` are conveniences
 for trying the kernel on a float model; the quantiser is not part of the reference either.
@@ -24,17 +24,18 @@ from typing import Optional
 
 import torch
 
-from .gemm import (binding as _binding, prepack as _prepack, prepack_bytes as _prepack_bytes, prepack_colmajor as _prepack_colmajor, quantize as _quantize)
+from .gemm import (binding as _binding, gemm as _gemm, gemm_prepacked as _gemm_prepacked, prepack as _prepack, prepack_bytes as _prepack_bytes,
+                   prepack_colmajor as _prepack_colmajor, prepacked_workspace_bytes as _prepacked_workspace_bytes, quantize as _quantize,
+                   workspace_bytes as _workspace_bytes, workspace_init as _workspace_init)
 
 _native = _binding()  # registers the operators (csrc/torch_binding.cpp)
 _OP = "awesome_fusion::bfaintb_gemm"
-bfaintb_gemm = torch.ops.awesome_fusion.bfaintb_gemm
-bfaintb_gemm_prepacked = torch.ops.awesome_fusion.bfaintb_gemm_prepacked
 
 
 def release_workspaces():
     """Gives the operators' split-K workspaces (one per device and stream) back to torch's allocator."""
-    _native.release_workspaces()
+    if _native is not None:
+        _native.release_workspaces()
 
 
 def _check(a, b, scale, weight_bits, group_size, bias=None):
@@ -70,13 +71,6 @@ def _check_residual(residual, m, n):
     return residual
 
 
-@torch.library.register_fake(_OP)
-def _(a, b, scale, weight_bits, group_size, bias=None, residual=None, activation=0):
-    m, n, _k = _check(a, b, scale, weight_bits, group_size, bias)
-    _check_residual(residual, m, _out_cols(n, activation))
-    return a.new_empty((m, _out_cols(n, activation)))
-
-
 def _check_prepacked(a, packed, scale, weight_bits, group_size, bias=None):
     if a.dim() != 2 or scale.dim() != 2 or packed.dim() != 1:
         raise ValueError("bfaintb_gemm_prepacked: a [m, k], packed [k*n*bits/8], scale [groups, n]")
@@ -91,6 +85,54 @@ def _check_prepacked(a, packed, scale, weight_bits, group_size, bias=None):
     if bias is not None and (bias.dtype != torch.bfloat16 or tuple(bias.shape) != (n,)):
         raise ValueError("bfaintb_gemm_prepacked: bias must be bfloat16 [n]")
     return a.shape[0], n, k
+
+
+def _in_python(packed, a, w, scale, weight_bits, group_size, bias, residual, activation):
+    """An operator where the native binding does not load: the same call through ctypes, on a workspace of its own (from the
+    current stream's memory, the graph's under capture)."""
+    m, n, k = (_check_prepacked if packed else _check)(a, w, scale, weight_bits, group_size, bias)
+    n_out = _out_cols(n, activation)
+    _check_residual(residual, m, n_out)
+    if not a.is_cuda:
+        raise RuntimeError(f"bfaintb_gemm{'_prepacked' * packed} runs on the GPU only (no CPU implementation)")
+    if a.stride(1) != 1 or a.stride(0) % 8 or a.data_ptr() % 16:
+        a = a.contiguous()
+    w, scale = w.contiguous(), scale.contiguous()
+    bias, residual = (None if t is None else t.contiguous() for t in (bias, residual))
+    c = torch.empty((m, n_out), dtype=torch.bfloat16, device=a.device)
+    if m == 0 or n == 0:
+        return c
+    with torch.cuda.device(a.device):
+        need = (_prepacked_workspace_bytes if packed else _workspace_bytes)(m, n, k, weight_bits, group_size)
+        ws = torch.empty(need, dtype=torch.uint8, device=a.device) if need else None
+        if need:
+            _workspace_init(ws)
+        (_gemm_prepacked if packed else _gemm)(c, a, w, scale, m, n, k, lda=a.stride(0), weight_bits=weight_bits, group_size=group_size, workspace=ws,
+                                               bias=bias, residual=residual, activation=activation)
+    return c
+
+
+if _native is None:
+    @torch.library.custom_op(_OP, mutates_args=())
+    def _rows(a: torch.Tensor, b: torch.Tensor, scale: torch.Tensor, weight_bits: int, group_size: int, bias: Optional[torch.Tensor] = None,
+              residual: Optional[torch.Tensor] = None, activation: int = 0) -> torch.Tensor:
+        return _in_python(False, a, b, scale, weight_bits, group_size, bias, residual, activation)
+
+    @torch.library.custom_op(_OP + "_prepacked", mutates_args=())
+    def _packed(a: torch.Tensor, packed: torch.Tensor, scale: torch.Tensor, weight_bits: int, group_size: int, bias: Optional[torch.Tensor] = None,
+                residual: Optional[torch.Tensor] = None, activation: int = 0) -> torch.Tensor:
+        return _in_python(True, a, packed, scale, weight_bits, group_size, bias, residual, activation)
+
+
+bfaintb_gemm = torch.ops.awesome_fusion.bfaintb_gemm
+bfaintb_gemm_prepacked = torch.ops.awesome_fusion.bfaintb_gemm_prepacked
+
+
+@torch.library.register_fake(_OP)
+def _(a, b, scale, weight_bits, group_size, bias=None, residual=None, activation=0):
+    m, n, _k = _check(a, b, scale, weight_bits, group_size, bias)
+    _check_residual(residual, m, _out_cols(n, activation))
+    return a.new_empty((m, _out_cols(n, activation)))
 
 
 @torch.library.register_fake(_OP + "_prepacked")
@@ -220,7 +262,7 @@ class QuantLinear(torch.nn.Module):
 
     def forward(self, x, residual=None):
         """``residual`` (same shape as the output, bf16) is added inside the kernel, before the rounding."""
-        if not torch.compiler.is_compiling():
+        if _native is not None and not torch.compiler.is_compiling():
             y = _native.linear_forward(self.__dict__, x, residual)
             if y is not NotImplemented:
                 return y

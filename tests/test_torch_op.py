@@ -20,6 +20,64 @@ def test_operator_is_registered_and_infers_shapes():
     assert out.shape == (5, 48) and out.dtype == torch.bfloat16 and out.device.type == "meta"
 
 
+_WITHOUT_BINDING = """
+import sys, warnings
+import torch
+sys.modules["awesome_fusion_amd._torch_binding"] = None  # as if it did not load
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter("always")
+    import awesome_fusion_amd as af
+    import awesome_fusion_amd.torch_op as top
+    p = 0x10000
+    assert af.gemm(p, p, p, p, 4, 32, 64, lda=8, stream=0, check=False) == -3 == af.gemm_prepacked(p, p, p, p, 4, 32, 64, lda=8, stream=0, check=False)
+assert [w.category for w in seen if "_torch_binding.so" in str(w.message)] == [RuntimeWarning]
+meta = lambda shape, dtype: torch.empty(shape, dtype=dtype, device=where)
+for where in ("meta", "cpu"):
+    a, b, s = meta((4, 128), torch.bfloat16), meta((128, 32), torch.uint8), meta((1, 32), torch.bfloat16)
+    for op, w in ((top.bfaintb_gemm, b), (top.bfaintb_gemm_prepacked, b.reshape(-1))):
+        try:
+            c = op(a, w, s, 8, 0, None, None, 1)
+            assert where == "meta" and c.shape == (4, 16) and c.dtype == torch.bfloat16
+        except RuntimeError as e:
+            assert where == "cpu" and "GPU only" in str(e), e
+top.release_workspaces()
+if sys.argv[1:] == ["gpu"]:
+    torch.manual_seed(1)
+    for m, n, k in ((4, 1024, 4096), (96, 4096, 11008)):
+        assert af.workspace_bytes(m, n, k) > 0
+        layer = top.QuantLinear.from_float(torch.nn.Linear(k, n).cuda(), 8, 0)
+        x, r = torch.randn((2, m // 2, k), device="cuda", dtype=torch.bfloat16), torch.randn((2, m // 2, n), device="cuda", dtype=torch.bfloat16)
+        for ws_bytes in (af.workspace_bytes, af.prepacked_workspace_bytes):
+            y = layer(x, residual=r)
+            need, c = ws_bytes(m, n, k), torch.empty((m, n), device="cuda", dtype=torch.bfloat16)
+            ws = torch.empty(max(need, 256), dtype=torch.uint8, device="cuda")
+            af.workspace_init(ws)
+            args = (c, x, layer.qweight, layer.scales, m, n, k)
+            (af.gemm_prepacked if layer.prepacked else af.gemm)(*args, workspace=ws, bias=layer.bias, residual=r)
+            assert torch.equal(y.reshape(m, n), c) and y.shape == r.shape and bool(c.any())
+            layer.prepack()
+print("fine")
+"""
+
+
+def _without_binding(*argv):
+    import os
+    import subprocess
+    import sys
+    r = subprocess.run([sys.executable, "-c", _WITHOUT_BINDING, *argv], capture_output=True, text=True, timeout=100,
+                       cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert r.returncode == 0 and r.stdout.endswith("fine\n"), r.stderr[-3000:]
+
+
+def test_calls_and_operators_without_the_native_binding():
+    _without_binding()
+
+
+@pytest.mark.gpu
+def test_operators_without_the_native_binding_compute_the_same():
+    _without_binding("gpu")
+
+
 def test_operator_rejects_bad_arguments_and_cpu_tensors():
     a, b, s, bits, g = _args()
     with pytest.raises(RuntimeError):           # no CPU implementation, and no silent fallback
