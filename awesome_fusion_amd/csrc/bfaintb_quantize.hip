@@ -100,9 +100,9 @@ __device__ __forceinline__ uint32_t code_of(float w, float s, float r)
 {
     constexpr int kQmax = BITS == 8 ? 127 : 7;
     const float q = TYPE == kWeightF32 ? w / s : quotient16(w, s, r);
-    int v = (int)rintf(q);  // (v_cvt_i32_f32: a NaN gives 0)
-    v = v < -kQmax - 1 ? -kQmax - 1 : v > kQmax ? kQmax : v;
-    return (uint32_t)(v + kQmax + 1);
+    // (clamped before it becomes an integer: nothing out of an integer's range is converted, and a NaN is the least code until
+    // the caller replaces it)
+    return (uint32_t)((int)fminf(fmaxf(rintf(q), (float)(-kQmax - 1)), (float)kQmax) + kQmax + 1);
 }
 
 struct QuantizeParams {
@@ -123,6 +123,7 @@ template <int BITS, int TYPE, bool FUSED>
 __global__ void __launch_bounds__(512) bfaintb_quantize_kernel(const QuantizeParams p)
 {
     constexpr uint32_t kRows = 32u / BITS;  // rows of W per lane
+    constexpr uint32_t kCode0 = BITS == 8 ? 0x80808080u : 0x88888888u;  // a group without a finite scale (a NaN or an infinity among its weights)
     __shared__ uint32_t tile[kTileK * kTilePitch];
     const uint32_t kq = threadIdx.x & 15u, ng = threadIdx.x >> 4;
     const uint32_t k0 = blockIdx.y * kTileK + 8u * kq, n0 = (blockIdx.x * 32u + ng) * kRows;
@@ -153,17 +154,18 @@ __global__ void __launch_bounds__(512) bfaintb_quantize_kernel(const QuantizePar
                 sb[r] = two & 0xffffu, sb[r + 1] = two >> 16;
             }
         }
-        uint32_t out[8] = {};
+        uint32_t out[8] = {}, finite = 0u;  // (finite: all bits of the rows whose scale is)
 #pragma unroll
         for (uint32_t r = 0; r < kRows; ++r) {
             const float s = bf16_bits_to_f32(sb[r]);
+            finite |= (sb[r] & 0x7f80u) != 0x7f80u ? ((1u << BITS) - 1u) << (BITS * r) : 0u;
             float rcp = __builtin_amdgcn_rcpf(s);
             rcp = fmaf(fmaf(-s, rcp, 1.0f), rcp, rcp);
 #pragma unroll
             for (int i = 0; i < 8; ++i) out[i] |= code_of<BITS, TYPE>(raw_to_f32(raw[r], i), s, rcp) << (BITS * r);
         }
 #pragma unroll
-        for (uint32_t i = 0; i < 8; ++i) tile[(8u * kq + i) * kTilePitch + ng] = out[i];
+        for (uint32_t i = 0; i < 8; ++i) tile[(8u * kq + i) * kTilePitch + ng] = (out[i] & finite) | (kCode0 & ~finite);
     }
     __syncthreads();
     // 16 lanes x 8 bytes = one row's line

@@ -41,6 +41,37 @@ def test_codes_and_scales_are_the_torch_forms(n, k, bits, group, dtype):
     assert torch.equal(b, b1) and torch.equal(s.view(torch.int16), s1.view(torch.int16))
 
 
+@pytest.mark.parametrize("n,k,bits,group", [(48, 384, 4, 128), (144, 192, 8, 64), (272, 1000, 8, 0), (64, 768, 4, 256)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_groups_with_nans_and_infinities_are_code_0(n, k, bits, group, dtype):
+    """A NaN or an infinity makes its group's scale one and all of the group's codes 0; the other groups do not notice.  The
+    largest finite weights stay finite: their group's extreme code times its scale is within half a step of them."""
+    g = torch.Generator(device="cuda").manual_seed(n * k)
+    w = (torch.randn((n, k), generator=g, device="cuda") * 0.05).to(dtype)
+    size, zero = group or k, 128 if bits == 8 else 8
+    codes = lambda b: b if bits == 8 else torch.stack((b & 15, b >> 4), dim=2).reshape(k, n)
+    b0, s0 = top.quantize_weight(w, bits, group)
+    hit = torch.zeros((k // size, n), dtype=torch.bool, device="cuda")
+    x = w.clone()
+    for row, col, value in ((0, 0, float("nan")), (3, k - 1, float("inf")), (4, size - 1, float("-inf")), (n - 1, k // 2, float("nan")), (9, 5, float("nan"))):
+        x[row, col] = value
+        hit[col // size, row] = True
+    x[9, 6] = float("inf")
+    b, s = top.quantize_weight(x, bits, group)
+    assert torch.equal(~s.isfinite(), hit) and bool(s[0, 0].isnan()) and bool(s[0, 9].isnan()) and float(s[(k - 1) // size, 3]) == float("inf") == float(s[0, 4])
+    assert torch.equal(s.view(torch.int16)[~hit], s0.view(torch.int16)[~hit])
+    wide = hit.repeat_interleave(size, dim=0)
+    assert bool((codes(b)[wide] == zero).all()) and torch.equal(codes(b)[~wide], codes(b0)[~wide])
+    top_value = torch.finfo(dtype).max
+    x = w.clone()
+    x[1, 1], x[2, 2] = top_value, -top_value
+    b, s = top.quantize_weight(x, bits, group)
+    assert bool(s.isfinite().all())
+    for row, at in ((1, 1), (2, 2)):
+        value = (int(codes(b)[at, row]) - zero) * float(s[0, row])
+        assert abs(value - float(x[row, at])) <= 0.51 * float(s[0, row])
+
+
 @pytest.mark.parametrize("n,k,bits", [(16, 64, 8), (16, 128, 4), (272, 192, 8), (528, 384, 4), (4112, 64, 8), (48, 2048, 4)])
 def test_packing_is_the_oracles(n, k, bits):
     rng = np.random.default_rng(n + k)
