@@ -381,8 +381,10 @@ static double prefill_estimate_us(uint32_t m, uint32_t n, uint32_t k, int bits, 
 // against 18.1) and loses long ones (8-bit 96 x 4096 x 11008 35.0 / 23.4, 64 rows 24.0 / 19.7; packed 29.6 / 22.6 and 21.5 / 19.5).
 static bool family_leads_tiles(double family_us, uint32_t m, uint32_t n, uint32_t k, int bits, bool packed, bool second_launch)
 {
-    double us = prefill_estimate_us(m, n, k, bits, second_launch);
-    if (prefill_small_tiles(m, n, bits) && tile128_plan(m, n, k, bits, 0, second_launch).finish_launch) {
+    if (!prefill_small_tiles(m, n, bits)) return family_us < prefill_estimate_us(m, n, k, bits, second_launch);
+    const TilePlan t = tile128_plan(m, n, k, bits, 0, second_launch);
+    double us = t.us;
+    if (t.finish_launch) {
         const bool lines = n % (packed ? 128u : 1024u / (uint32_t)bits) == 0;  // (packed: whole workgroups of columns)
         if (packed) us *= bits == 8 ? 0.95 : lines ? 1.06 : 0.95;
         else us *= bits == 8 ? (lines ? 1.06 : 0.84) : (lines ? 1.2 : 1.0);
@@ -1443,9 +1445,10 @@ static double launch_time_us(uint32_t m, uint32_t n, uint32_t k, int bits, bool 
 {
     const double cus = (double)machine_cus(), steps = k / 64.0;
     if (m <= kDecodeAutoMaxM) return 6.0 + (double)n * k * bits / 8.0 / 3.3e6 * (m <= 16u ? 1.0 : 1.25);
-    const int v = packed ? packed_variant(m, n, k, bits, BFAINTB_VARIANT_AUTO) : resolve_variant(m, n, k, bits, BFAINTB_VARIANT_AUTO);
-    if (v == BFAINTB_VARIANT_DECODE)
-        return packed ? packed_family_time_us(m, n, k, bits, packed_family_plan(m, n, k, bits)) : decode_family_time_us(m, n, k, bits, decode_plan(m, n, k, bits, 0));
+    if (m <= kDecodeFamilyAutoMaxM) {  // (beyond 32 rows the library's own choice asks just this)
+        const double family = packed ? packed_family_time_us(m, n, k, bits, packed_family_plan(m, n, k, bits)) : decode_family_time_us(m, n, k, bits, decode_plan(m, n, k, bits, 0));
+        if (family_leads_tiles(family, m, n, k, bits, packed, true)) return family;
+    }
     if (prefill_small_tiles(m, n, bits) || prefill_tall_tiles(m, n, bits)) return prefill_estimate_us(m, n, k, bits);
     const uint32_t tiles = ((m + 255u) / 256u) * ((n + 255u) / 256u);
     const uint32_t thin = bfaintb::thin_round_tiles(tiles, m, machine_cus()), full = tiles - thin;
@@ -1486,10 +1489,17 @@ static uint32_t row_split_rule(uint32_t m, uint32_t n, uint32_t k, int bits, boo
     // as fast on average and none slower; at 0.97 three of 49 are, by 4 - 9 %)
     double best = 0.94 * one;
     uint32_t head = 0;
-    for (const uint64_t c : candidates) {
+    for (size_t i = 0; i < sizeof(candidates) / sizeof(candidates[0]); ++i) {
+        const uint64_t c = candidates[i];
         if (c == 0u || c >= m) continue;
+        bool asked = false;
+        for (size_t j = 0; j < i; ++j) asked = asked || candidates[j] == c;
+        if (asked) continue;
         const uint32_t rows = (uint32_t)c;
-        const double two = launch_time_us(rows, n, k, bits, packed) + launch_time_us(m - rows, n, k, bits, packed) + 1.0;
+        // (no launch is estimated at less than 2 us: most candidates need no look at their rest)
+        const double first = launch_time_us(rows, n, k, bits, packed) + 1.0;
+        if (first + 2.0 >= best) continue;
+        const double two = first + launch_time_us(m - rows, n, k, bits, packed);
         if (two >= best) continue;
         if (row_split_workspace(rows, m - rows, n, k, bits, packed) > BFAINTB_STATIC_SCRATCH_BYTES) continue;
         best = two;
@@ -1499,16 +1509,18 @@ static uint32_t row_split_rule(uint32_t m, uint32_t n, uint32_t k, int bits, boo
 }
 
 // (a call asks two or three times, for its scratch and for its launch, and a model asks about the same few shapes: each
-// thread keeps the last answers, one per slot of a hash of the question)
+// thread keeps the last answers, one per slot of a hash of the question.  A new question costs 0.9 - 1.8 us of host time, where
+// one launch's plan takes 0.15; a known one 0.2, or 0.5 if the answer is two launches.  A prompt of a new length asks once per
+// shape of its layers, as long as no two of them share a slot)
 static uint32_t row_split_head(uint32_t m, uint32_t n, uint32_t k, int bits, bool packed)
 {
     if (m <= 256u) return 0;
     struct Answer {
         uint32_t m, n, k, kind, cus, row_block, head;
     };
-    static thread_local Answer answers[32] = {};
+    static thread_local Answer answers[256] = {};
     const uint32_t kind = (uint32_t)bits * 2u + (packed ? 1u : 0u), cus = machine_cus(), row_block = g_force_row_block.load(std::memory_order_relaxed);
-    Answer& a = answers[((m * 2654435761u) ^ (n * 2246822519u) ^ (k * 3266489917u) ^ kind) >> 27];
+    Answer& a = answers[((m * 2654435761u) ^ (n * 2246822519u) ^ (k * 3266489917u) ^ kind) >> 24];
     if (a.m != m || a.n != n || a.k != k || a.kind != kind || a.cus != cus || a.row_block != row_block)
         a = Answer{m, n, k, kind, cus, row_block, row_split_rule(m, n, k, bits, packed)};
     return a.head;
