@@ -583,12 +583,19 @@ DecodePlan decode_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint32_t fo
         // m = 1 / 8 / 16: 36864 x 4096, 6 splits x 288 blocks = 6.75 rounds, 39.8 / 43.3 / 47.9 us, its best factor, 2, 37.1 /
         // 39.4 / 42.7, wide 31.5 / 33.2 / 35.4; 24576 x 4096, 4 x 192 = 3 rounds, 23.6 / 25.7 / 28.2 against 20.5 / 21.8 / 23.5)
         const bool fills_rounds = narrow_wgs <= cus && narrow_wgs * 20u >= cus * 19u;
-        // 4-bit codes, 17 to 32 rows, up to 192 blocks of 128 columns, and too many of 256 for three splits in a round: that form
-        // makes one thin round of 4-wave workgroups, k split in two; the 128-column form with 4 waves and k split four ways puts two to three on every CU (us at m = 18 / 32:
-        // 22016 x 4096 20.6 / 23.9 against 25.6 / 26.7; 24576 x 4096 24.1 / 27.8 against 26.6 / 27.7; 22016 x 5120 24.2 / 28.3
-        // against 29.1 / 30.0; rows of B that are not whole lines lose 3 - 6 % by it: 24000 x 4608, m = 32: 30.5 / 29.5).
+        // 4-bit codes, 17 to 32 rows, two thirds to three quarters of a round of 128-column blocks (too many 256-column ones for three
+        // splits in a round, so that form makes one thin round of 4-wave workgroups, k split in two).  A launch of 4-wave
+        // workgroups takes its rounds of one per CU over its splits: with s splits whose workgroups stay within s - 1 rounds, (s - 1) /
+        // s of one unsplit pass over k, and here that is s = 4 (us by splits 2 / 3 / 4 / 5 / 6, 22016 x 4096, m = 32: 27.0 / 28.7 / 23.7 /
+        // 27.0 / 30.3; 24064 x 3072, m = 18: 19.5 / 20.7 / 18.3 / 19.9 / 22.4).  Against the 256-column form over the whole range, k = 2176
+        // ... 5120: 1.02 - 1.23 times as fast at 17 to 20 rows, 0.95 - 1.10 at 28 to 32 (22016 x 4096, m = 18 / 32: 25.4 / 26.6 -> 20.6 /
+        // 23.7; 24064 x 5120 28.7 / 29.7 -> 25.1 / 29.1; 23552 x 4352, m = 32: 0.95).  A little past three quarters a fifth split is needed
+        // and the gain is gone (24832 x 4608, m = 18 / 32: 26.5 / 28.0, five splits 25.4 / 29.8).  Rows that start in the same few memory
+        // channels (multiples of 2048 columns) slow the 128-column form: up to 20 rows it is level there or ahead, beyond it loses up
+        // to 10 % (24576 x 5120, m = 18 / 32: 28.9 / 30.5 against 28.7 / 33.5).  Rows that are not whole lines lose 2 - 5 % at 32 (24000 x 4608:
+        // 29.5 / 30.5).
         if (nibbles && !packed && forced_splits == 0 && m > 16u && (n + 255u) / 256u * 3u > cus && narrow_blocks * 4u <= cus * 3u && n % 256u == 0 &&
-            k <= 5120u) {
+            (n % 2048u != 0 || m <= 20u) && k <= 5120u) {
             DecodePlan probe = pl;
             probe.cols = 128u;
             probe.waves = 4u;

@@ -365,3 +365,15 @@ def test_launch_shapes_of_the_decode_family(m, n, k, bits, group, want):
     p = af.plan(m, n, k, bits, group)
     if p.compute_units == 256:
         assert (p.tile_cols, p.waves, p.splits) == want, p.as_dict()
+
+
+@pytest.mark.parametrize("m,n,k,want", [
+    # four splits of 4 waves over two thirds to three quarters of a round of 128-column blocks ...
+    (17, 22016, 5120, (128, 4, 4)), (32, 24320, 2176, (128, 4, 4)), (32, 22528 + 256, 4608, (128, 4, 4)),
+    # ... where rows start in the same few memory channels only up to 20 rows; not past three quarters of a round, nor beyond k = 5120
+    (20, 24576, 4096, (128, 4, 4)), (21, 24576, 4096, (256, 4, 2)), (20, 22528, 5120, (128, 4, 4)), (32, 22528, 5120, (256, 4, 2)),
+    (18, 24832, 4096, (256, 4, 2)), (18, 22016, 5632, (256, 4, 2)), (18, 22032, 4096, (256, 4, 2))])
+def test_four_splits_for_17_to_32_rows_of_4_bit_codes(m, n, k, want):
+    p = af.plan(m, n, k, 4, 128)
+    if p.compute_units == 256:
+        assert (p.tile_cols, p.waves, p.splits) == want, p.as_dict()
