@@ -379,6 +379,10 @@ static double prefill_estimate_us(uint32_t m, uint32_t n, uint32_t k, int bits, 
 // not whole cache lines slow the family's reads by 30 % (8-bit; 127 x 1072 x 6016 18.1 us, tiles 13.6) and the tiles' copies by
 // little; in whole lines the family holds small weights (4-bit 64 x 4096 x 4096 11.7 against 13.6, 128 x 2048 x 8192 16.4
 // against 18.1) and loses long ones (8-bit 96 x 4096 x 11008 35.0 / 23.4, 64 rows 24.0 / 19.7; packed 29.6 / 22.6 and 21.5 / 19.5).
+// How well that picks, over 720 other random shapes with cold weights: 3.6 % over the faster form on average, 146 of them more than
+// 5 % (always the tiles: 5.8 % and 235; always the family: 13.8 % and 355).  What is missing is the family's estimate, which scatters by
+// 10 - 18 % there, the tiles' by 4 - 5 %; other factors (four, fitted on 560 shapes) pick 2.5 % over on average but lose more
+// than 3 % against these on 66 of the 720.
 static bool family_leads_tiles(double family_us, uint32_t m, uint32_t n, uint32_t k, int bits, bool packed, bool second_launch)
 {
     if (!prefill_small_tiles(m, n, bits)) return family_us < prefill_estimate_us(m, n, k, bits, second_launch);
@@ -536,10 +540,12 @@ DecodePlan decode_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint32_t fo
         // rounds; otherwise large matrices stream better in 256-byte row segments.  4-bit codes: wide.
         const bool few = weight_bytes <= (32ull << 20);
         // Up to 8 rows and 24 to 72 MiB of weights, the narrow form runs 4 waves instead of 8: each has twice the steps behind its
-        // first loads, the workgroup half the sums to add through LDS, and k divides into more split factors (us, 8 / 4 waves,
-        // m = 1 / 8: 4096 x 11008 13.2 / 12.0 and 13.9 / 13.1; 8192 x 4096 10.3 / 9.4 and 11.0 / 10.1; 3072 x 8192 9.8 / 9.2 and 10.8 /
-        // 9.9; 8192 x 8192 15.8 / 14.8 and 16.6 / 16.2; 3584 x 18944 15.8 / 15.3 and 17.1 / 16.2; level at 4096 x 14336 and
-        // 11008 x 4096).  Fewer bytes are over before the longer chain pays (4096 x 4096, m = 1: 7.4 / 8.3), more rows want the
+        // first loads, the workgroup half the sums to add through LDS, and k divides into more split factors (one launch after
+        // the other over cold weights, 24 shapes: 1.03 times as fast on average, 0.97 - 1.11; us, 8 / 4 waves, m = 1 / 8: 4096 x 11008
+        // 12.7 / 12.1 and 13.8 / 13.0; 8192 x 4096 10.3 / 9.4 and 11.0 / 10.1; 3072 x 8192 9.8 / 9.2 and 10.8 / 9.9; 8192 x 8192 15.6 / 14.8 and
+        // 16.6 / 16.0; 3584 x 18944 15.9 / 15.3 and 17.1 / 16.2; level at 4096 x 14336, 16384 x 4096 and 11008 x 4096).  In the four
+        // products of a decoder block, replayed as one graph, what is left of it is 0 - 3 % of the step (8 rows; hidden and MLP width 3072 and
+        // 8192: 42.5 -> 41.2; 4096 and 11008: 59.7 -> 59.1; 4096 and 14336: 65.0 -> 65.4).  Fewer bytes are over before the longer chain pays (4096 x 4096, m = 1: 7.4 / 8.3), more rows want the
         // waves to hide their activations behind (m = 16: 3072 x 8192 11.7 / 12.0, 2560 x 10240 11.4 / 13.0).
         // (rows of B that are not whole cache lines: 1 % on average and up to 8 % slower over 24 shapes, so whole lines only)
         const bool four_waves = bits == 8 && !packed && !nibbles && m <= 8u && n % 128u == 0 && weight_bytes >= (24ull << 20) && weight_bytes <= (72ull << 20);
