@@ -219,7 +219,7 @@ BFAINTB_API int bfaintb_init(void* stream);
  * until the process ends.  Same kernels, same variant choice and bit-for-bit the results of bfaintb_gemm.  A shape
  * whose bfaintb_gemm_workspace_bytes exceeds the scratch is refused with BFAINTB_ERR_STATIC_SCRATCH (nothing launched).
  * Every call on a GPU shares that GPU's scratch (each call leaves it in its at-rest state for the next): calls that may
- * overlap on one GPU — different streams, different host threads — race on it and must use bfaintb_gemm with
+ * overlap on one GPU — on different streams, from one host thread or several — race on it and must use bfaintb_gemm with
  * workspaces of their own.  Allocates nothing, on any call.  No counterpart in the reference, whose kernel needs no
  * scratch (no split-K).
  */
