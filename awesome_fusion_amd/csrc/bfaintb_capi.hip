@@ -197,6 +197,18 @@ static double decode_family_time_us(uint32_t m, uint32_t n, uint32_t k, int bits
     return (pl.mb == 4u ? 1.05 : 0.93) * (5.0 + e.core);
 }
 
+// Tall tiles: at most 256 rows x 128 columns; the rows spread evenly over as many tiles as 256 rows each would take, in blocks of 16.
+static uint32_t tall_tile_blocks(uint32_t m)
+{
+    const uint32_t rows_of_tiles = (m + 255u) / 256u, needed = (m + 16u * rows_of_tiles - 1u) / (16u * rows_of_tiles);
+    return needed <= 10u ? 10u : needed <= 12u ? 12u : 16u;
+}
+// Up to a k of 1024 (2048 for tiles of 10 blocks, where launches by rows compete with them) the form that adds an output's products in
+// one chain, as the large tiles do, to the same bits (bfaintb_prefill256x128_wreg_kernel); beyond it the small tiles' kernel with 10 to
+// 16 blocks of 16 rows.  us, one chain / 16 blocks, k = 512 / 1024 / 2048 / 4096: 2048 x 4096 8-bit 17.2 / 16.6, 25.0 / 23.1, 40.2 / 35.6,
+// 70.8 / 63.0; 512 x 11008 4-bit 17.7 / 15.6, 25.4 / 21.2, 40.8 / 31.9, 71.6 / 53.9.
+static bool tall_tiles_in_one_chain(uint32_t m, uint32_t k) { return k <= (tall_tile_blocks(m) == 10u ? 2048u : 1024u); }
+
 // The tiled variant runs 128x128 tiles while those fit one per CU: four times the workgroups of
 // 256x256 tiles, each with a quarter of the work per K-step.  Measured against the large tiles (8-bit, k = 4096, us):
 // m x n = 256 x 4096: 48 / 59, 1024 x 4096: 58 / 66, 512 x 8192 (4-bit, k = 8192): 112 / 137; with more tiles the
@@ -204,7 +216,7 @@ static double decode_family_time_us(uint32_t m, uint32_t n, uint32_t k, int bits
 // (One gap: a few tall tiles more than CUs — 640 x 11008 makes 258 — would go to 129 large tiles on half the machine, 82 us;
 // the small tiles take it in two rounds, 430 of them, in 66 us.  So: also up to two rounds of small tiles where the tall
 // ones do not fit one round and the large ones fill at most 60 % of the CUs.)
-static bool prefill_small_tiles(uint32_t m, uint32_t n, int bits)
+static bool prefill_small_tiles(uint32_t m, uint32_t n, uint32_t k, int bits)
 {
     const uint64_t cus = machine_cus();
     const uint64_t small = (uint64_t)((m + 127u) / 128u) * ((n + 127u) / 128u);
@@ -218,7 +230,7 @@ static bool prefill_small_tiles(uint32_t m, uint32_t n, int bits)
     // kernel converts every weight in two waves; us, small / tall, on two boxes: 1152 x 4096 x 4096, 288 tiles: 65.8 / 70.7
     // and 68.9 / 70.9; 512 x 11008 x 4096, 344: 65.9 / 71.1; with 384 to 448 tiles the second box had them level or the tall
     // ones ahead by 2 %, and packed weights by up to 4 %; 8-bit codes the other way throughout: 63.1 / 59.2 at 288 tiles)
-    if (bits == 4 && small * 20u <= cus * 27u) return true;
+    if (bits == 4 && tall_tiles_in_one_chain(m, k) && small * 20u <= cus * 27u) return true;
     const uint64_t tall = (uint64_t)((m + 255u) / 256u) * ((n + 127u) / 128u);
     const uint64_t large = (uint64_t)((m + 255u) / 256u) * ((n + 255u) / 256u);
     // (0.6 of the CUs at most: 640 x 12032 x 3584, 141 large tiles, 76.2 us; 470 small ones 67.6)
@@ -229,9 +241,9 @@ static bool prefill_small_tiles(uint32_t m, uint32_t n, int bits)
 // occupy a quarter to a half of the CUs there; the tall ones run one per CU at 0.94 us per K-step against the large tiles'
 // 1.02 on twice the work (8-bit, 64 steps, us tall / large: 1536 x 4096: 61.0 / 66.0; 512 x 11008: 60.3 / 64.7; 2048 x 4096:
 // 71.0 / 75.7; 128 steps, 1024 x 8192: 129 / 141; 4-bit, 768 x 8192: 138 / 140).
-static bool prefill_tall_tiles(uint32_t m, uint32_t n, int bits)
+static bool prefill_tall_tiles(uint32_t m, uint32_t n, uint32_t k, int bits)
 {
-    return !prefill_small_tiles(m, n, bits) && (uint64_t)((m + 255u) / 256u) * ((n + 127u) / 128u) <= machine_cus();
+    return !prefill_small_tiles(m, n, k, bits) && (uint64_t)((m + 255u) / 256u) * ((n + 127u) / 128u) <= machine_cus();
 }
 
 static bool is_prefill(int v)
@@ -241,18 +253,17 @@ static bool is_prefill(int v)
 }
 
 // tile size of a tiled-variant launch: forced, or by shape
-static bool use_small_tiles(int v, uint32_t m, uint32_t n, int bits)
+static bool use_small_tiles(int v, uint32_t m, uint32_t n, uint32_t k, int bits)
 {
-    return v == BFAINTB_VARIANT_PREFILL_128 || v == BFAINTB_VARIANT_PREFILL_128_LDS || (v == BFAINTB_VARIANT_PREFILL && prefill_small_tiles(m, n, bits));
+    return v == BFAINTB_VARIANT_PREFILL_128 || v == BFAINTB_VARIANT_PREFILL_128_LDS || (v == BFAINTB_VARIANT_PREFILL && prefill_small_tiles(m, n, k, bits));
 }
 
-// Rough time of the tiled variant (prefill_estimate_us, below the plan of the small tiles).  Small tiles: a K-step takes 0.40 us on an empty machine and 0.55 us with a workgroup on every CU (the kernel that
-// keeps the weights in registers), whichever order the weights are stored in.
 // The small-tile kernel may split k: grid y walks the splits, each workgroup runs its share of
 // the K-steps and the workgroup of the last split adds the others' sums (same workspace and protocol as the decode
 // family).  Worth it while tiles x splits still fit one workgroup per CU.
 struct TilePlan {
     uint32_t k_per_wg, splits;
+    uint32_t blocks;  // of 16 rows of a tile
     uint32_t finish_launch;  // 1: every split's sums go to the workspace and a second launch adds them
     double us;
 };
@@ -269,60 +280,78 @@ static size_t split_workspace_bytes(uint32_t splits, uint32_t m, uint32_t n)
 // (with a second launch the last split's sums lie there as well)
 static size_t tile_workspace_bytes(const TilePlan& t, uint32_t m, uint32_t n) { return split_workspace_bytes(t.splits + t.finish_launch, m, n); }
 
+// A K-step of a tile of 16 x blocks rows and 128 columns, in us, with `load` of the CUs holding a workgroup: what is issued beside the
+// matrix instructions, the matrix instructions, and the clock that gives way to the board's power.  8-bit, us a step at 96 / 256
+// workgroups, 4 / 6 / 8 / 10 / 12 / 16 blocks: 0.33 / 0.39 / 0.44 / 0.50 / 0.52 / 0.60 and 0.33 / 0.40 / 0.46 / 0.60 / 0.66 / 0.82; 4-bit and
+// grouped scales within 7 %.  One row of tiles reads each code once, from memory, which costs some
+// 0.05 on a full machine, at 6 TB/s at most (8-bit, 256 workgroups, 4 / 6 / 8 blocks: 0.34 / 0.45 / 0.55).
+static double tile_step_us(uint32_t blocks, uint32_t m, int bits, double load)
+{
+    const double issue = 0.23 + 0.0255 * blocks + 0.00105 * blocks * blocks * load * load * load;
+    if (m > 16u * blocks) return issue;
+    const double stream = load * machine_cus() * 1024.0 * bits / 6.0e6;
+    return issue + 0.05 * load > stream ? issue + 0.05 * load : stream;
+}
+// The beginning and the end of a launch of such tiles (8 / 16 blocks: 6 / 9 us in a run of launches).
+static double tile_ends_us(uint32_t blocks) { return 3.3 + 0.34 * blocks; }
+
 // second_launch: whether the plan may be one whose sums a second launch adds.  Here and below, false is for the caller who
 // brings less scratch than such a plan needs (all splits' sums) and gets what the library does without it.
 static TilePlan tile128_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint32_t forced_splits, bool second_launch = true)
 {
     const uint32_t ksteps = (k + 63u) / 64u;
-    const double tiles = (double)((m + 127u) / 128u) * (double)((n + 127u) / 128u);
+    // blocks of 16 rows of a tile: the rows, spread evenly over as many tiles as 128 rows each would take
+    const uint32_t rows_of_tiles = (m + 127u) / 128u, needed = (m + 16u * rows_of_tiles - 1u) / (16u * rows_of_tiles);
+    const uint32_t blocks = needed <= 4u ? 4u : needed <= 6u ? 6u : 8u;
+    const double tiles = (double)rows_of_tiles * (double)((n + 127u) / 128u);
     const double cus = (double)machine_cus();
     const double fill = (double)m / (double)((m + 127u) / 128u * 128u);  // the share of the tiles' rows that exist
     auto shape = [&](uint32_t want) {
         TilePlan t;
         t.finish_launch = 0u;
+        t.blocks = blocks;
         if (want > kMaxTileSplits) want = kMaxTileSplits;
         if (want < 1u) want = 1u;
         const uint32_t per = (ksteps + want - 1u) / want;
         t.k_per_wg = per * 64u;
         t.splits = (ksteps + per - 1u) / per;
-        // the hand-over: the producers' device-scope stores have to arrive, then the reducing workgroup fetches the rows
-        // of a tile that exist, per split, through its one CU, slower the more CUs do so at once.  What the measured times
-        // leave after the K-steps (8-bit, us): 48 / 64 / 96 / 128 x 4096 x 4096, 4 splits of 32 tiles: 7.0 / 8.0 / 9.7 / 11.4;
-        // 384 x 2048 x 8192, 4 x 48: 9.6; 384 x 4096 x 4096, 2 x 96: 4.5; 256 x 8192 x 8192, 2 x 128: 5.9; 512 x 4096 x
-        // 4096, 2 x 128: 7.6.
-        const double hand_over = t.splits > 1u ? 3.0 + (t.splits - 1.0) * (0.6 + 1.6 * fill + 0.008 * tiles) : 0.0;
-        // a K-step (two waves per column group): 0.40 us (4-bit codes 0.41) on a nearly empty machine, rising with the
-        // cube of the share of the CUs that hold a workgroup as the clock gives way (8-bit, n = k = 4096, us per step at
-        // 160 / 192 / 224 / 256 workgroups: 0.425 / 0.44 / 0.50 / 0.55; 4-bit g128: 0.49 at 224, 0.55 - 0.56 at 256);
-        // rows of a tile that do not exist are not copied (28672 x 8192 4-bit, m = 64 / 96 / 128: 0.435 / 0.45 / 0.48)
+        // the hand-over: the producers' device-scope stores have to arrive, then the reducing workgroup fetches the rows of a tile that
+        // exist, per split, through its one CU, slower the more CUs do so at once (fitted, with the steps' factor, on 60 shapes of 33 ...
+        // 577 rows, both code widths and weight orders, 2 to 4 splits: 7 % rms)
+        const double hand_over = t.splits > 1u ? 1.8 + (t.splits - 1.0) * (2.5 * fill + 0.024 * tiles) : 0.0;
         const double wgs = tiles * t.splits;
-        auto step_us = [&](double load) { return ((bits == 4 ? 0.41 : 0.40) + 0.15 * load * load * load) * (0.8 + 0.2 * fill); };
-        // (more small tiles than CUs: whole rounds of them and a last one at the pace of its own load — 96 x 36864 x 8192, 288
-        // tiles: 128 us, 122 over packed weights; 640 x 11008 x 4096, 430: 66; 96 x 50304 x 4096, 393: 72; beyond two rounds the
-        // steps take 10 - 18 % longer than this: 64 / 96 / 128 x 128256 x 4096, four rounds: 152 / 162 / 171 us with 8-bit
-        // codes, 148 / 154 / 163 with 4-bit ones)
         const double whole = (double)(uint64_t)(wgs / cus), rest = wgs - whole * cus;
-        const double steps_us = whole * step_us(1.0) + (rest > 0.0 ? step_us(rest / cus) : 0.0);
-        t.us = 4.0 + (wgs > 2.0 * cus ? 1.12 : 1.0) * per * steps_us + hand_over;
+        if (!second_launch) {
+            // (a caller who brings the scratch that a call needed before there were second launches is served with that much: the
+            // choice among these plans, and between them and the family, goes by the estimates of that time)
+            auto step_us = [&](double load) { return ((bits == 4 ? 0.41 : 0.40) + 0.15 * load * load * load) * (0.8 + 0.2 * fill); };
+            t.us = 4.0 + (wgs > 2.0 * cus ? 1.12 : 1.0) * per * (whole * step_us(1.0) + (rest > 0.0 ? step_us(rest / cus) : 0.0)) +
+                   (t.splits > 1u ? 3.0 + (t.splits - 1.0) * (0.6 + 1.6 * fill + 0.008 * tiles) : 0.0);
+            if (t.splits > 2u) t.us *= 1.07;
+            return t;
+        }
+        const double steps_us = whole * tile_step_us(blocks, m, bits, 1.0) + (rest > 0.0 ? tile_step_us(blocks, m, bits, rest / cus) : 0.0);
+        // (further rounds of tiles begin behind the ones before them, each at four fifths of a launch's beginning and end)
+        t.us = tile_ends_us(blocks) * (0.2 + 0.8 * (whole + (rest > 0.0 ? 1.0 : 0.0))) + 0.94 * per * steps_us + hand_over;
         // (three splits and more: the hand-over scatters more than this says, and where the row-blocked family is about as
         // fast it is the safer pick — 192 x 4096 x 4096: 25.5 against 22.9 us, 128 x 4096 x 11008: 39.0 against 34.3)
         if (t.splits > 2u) t.us *= 1.07;
         return t;
     };
     if (forced_splits) return shape(forced_splits);
-    // with the second launch: the steps as above, 6.75 us for the two launches' beginnings and ends (one more where a
-    // thread fetches twice, beyond eight splits), and the words' way through
-    // memory (fitted on 70 shapes, m = 33 .. 352, n = 1040 .. 5300, k = 2048 .. 15500, both code widths and weight orders: within
-    // 5 % rms; 8-bit, us, measured / this: 220 x 2464 x 4480, 6 splits 18.2 / 17.5; 64 x 2832 x 14976, 8 splits 22.1 / 21.1)
+    // with the second launch: the two launches' beginnings and ends (a little more where a thread fetches twice, beyond eight splits), the
+    // steps, and the words' way through memory (fitted on the same shapes, 6 to 16 splits, 102 times: 5 % rms)
     auto finish_us = [&](const TilePlan& t) {
-        const double load = tiles * t.splits / cus;
-        const double step = ((bits == 4 ? 0.41 : 0.40) + 0.15 * load * load * load) * (0.8 + 0.2 * fill);
-        return (t.splits > 8u ? 7.75 : 6.75) + t.k_per_wg / 64u * step + t.splits * (double)m * n * 4.0 / 2.36e6;
+        return 7.8 - 0.2 * blocks + (t.splits > 8u ? 0.7 : 0.0) + 1.1 * (t.k_per_wg / 64u) * tile_step_us(blocks, m, bits, tiles * t.splits / cus) +
+               0.54e-6 * t.splits * (double)m * n * 4.0;
     };
     TilePlan best = shape(1);
     static const uint32_t kCandidates[] = {2, 3, 4, 6, 7, 8, 10, 12, 14, 16};
     for (uint32_t s : kCandidates) {
         if (tiles * s > cus) break;
+        // (one launch deals a split's tiles out in eights: 85 tiles x 3 are 33 workgroups on seven of the XCDs of 32 CUs, 54 us at 515 x 2080 x
+        // 8192, two splits 40)
+        if ((!second_launch || s < kFinishLaunchSplits) && (double)(((uint32_t)tiles + 7u) / 8u * 8u) * s > cus) continue;
         TilePlan t = shape(s);
         if (t.splits != s) continue;  // k does not divide that way
         // from six splits on their sums are added by a second launch, if all of them fit the scratch of the entry point that
@@ -358,13 +387,14 @@ static TilePlan tile128_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint3
 
 static double prefill_estimate_us(uint32_t m, uint32_t n, uint32_t k, int bits, bool second_launch = true)
 {
-    if (prefill_small_tiles(m, n, bits)) return tile128_plan(m, n, k, bits, 0, second_launch).us;
+    if (prefill_small_tiles(m, n, k, bits)) return tile128_plan(m, n, k, bits, 0, second_launch).us;
     const double cus = (double)machine_cus();
-    if (prefill_tall_tiles(m, n, bits)) {
-        // one tile of 256 rows x 128 columns per CU at most (8-bit, us per K-step: 512 x 11008 x 4096, 172 tiles: 0.87;
-        // 768 x 8192 x 8192 and 1536 x 4096 x 4096, 192: 0.84 and 0.88; 2048 x 4096 x 4096 and x 11008, 256: 1.02 and 0.98)
-        const double tiles = (double)((m + 255u) / 256u) * (double)((n + 127u) / 128u);
-        const double load = tiles / cus;
+    if (prefill_tall_tiles(m, n, k, bits)) {
+        const double load = (double)((m + 255u) / 256u) * (double)((n + 127u) / 128u) / cus;
+        const uint32_t blocks = tall_tile_blocks(m);
+        if (!tall_tiles_in_one_chain(m, k)) return tile_ends_us(blocks) + (k / 64.0) * tile_step_us(blocks, m, bits, load);
+        // the form of one chain (8-bit, us per K-step: 512 x 11008 x 4096, 172 tiles: 0.87; 768 x 8192 x 8192 and 1536 x 4096 x 4096,
+        // 192: 0.84 and 0.88; 2048 x 4096 x 4096 and x 11008, 256: 1.02 and 0.98)
         return 4.0 + (k / 64.0) * (0.83 + 0.17 * load * load * load);
     }
     // whole rounds of 256x256 tiles at what the board's power allows (4096^3: 1.55 us per K-step and round)
@@ -373,27 +403,27 @@ static double prefill_estimate_us(uint32_t m, uint32_t n, uint32_t k, int bits, 
     return 4.0 + rounds * (k / 64.0) * 1.5;
 }
 
-// Whether the row-blocked family, at its estimated time, is the one to run.  Tiles whose sums a second launch adds are estimated
-// within 5 %; the family's estimate is not that good where it meets them, which one factor per kind of weights makes up
-// for (the ratio of the two estimates above which the tiles were the faster form, over 180 measured shapes).  Rows of B that are
-// not whole cache lines slow the family's reads by 30 % (8-bit; 127 x 1072 x 6016 18.1 us, tiles 13.6) and the tiles' copies by
-// little; in whole lines the family holds small weights (4-bit 64 x 4096 x 4096 11.7 against 13.6, 128 x 2048 x 8192 16.4
-// against 18.1) and loses long ones (8-bit 96 x 4096 x 11008 35.0 / 23.4, 64 rows 24.0 / 19.7; packed 29.6 / 22.6 and 21.5 / 19.5).
-// How well that picks, over 720 other random shapes with cold weights: 3.6 % over the faster form on average, 146 of them more than
-// 5 % (always the tiles: 5.8 % and 235; always the family: 13.8 % and 355).  What is missing is the family's estimate, which scatters by
-// 10 - 18 % there, the tiles' by 4 - 5 %; other factors (four, fitted on 560 shapes) pick 2.5 % over on average but lose more
-// than 3 % against these on 66 of the 720.
+// The family's estimate, corrected to what it takes where it meets the tiles (fitted on 665 random shapes with cold weights, 33 ... 1500
+// rows; it then scatters by 13 - 21 %, most of all for codes in rows of which a workgroup's 128 are not whole; the tiles' estimate by 6 -
+// 8 %).  The lower of the two picks 2 % over the faster form on average (always the tiles 4.5 %, always the family 26 %).
+static double family_beside_tiles_us(double us, uint32_t m, uint32_t n, int bits, bool packed)
+{
+    const double ragged = n % 128u == 0 ? 0.0 : 1.0;
+    if (packed) return bits == 8 ? 1.19 * us - 0.7 + 0.0037 * m : 0.97 * us + 1.8 + 0.0044 * m;
+    return bits == 8 ? (1.035 + 0.165 * ragged) * us + 0.7 * (ragged - 1.0) + 0.0016 * m : (0.80 + 0.2 * ragged) * us + 2.3;
+}
+
+// Whether the row-blocked family, at its estimated time, is the one to run.
 static bool family_leads_tiles(double family_us, uint32_t m, uint32_t n, uint32_t k, int bits, bool packed, bool second_launch)
 {
-    if (!prefill_small_tiles(m, n, bits)) return family_us < prefill_estimate_us(m, n, k, bits, second_launch);
+    if (!prefill_small_tiles(m, n, k, bits)) return family_us < prefill_estimate_us(m, n, k, bits, second_launch);
     const TilePlan t = tile128_plan(m, n, k, bits, 0, second_launch);
-    double us = t.us;
-    if (t.finish_launch) {
-        const bool lines = n % (packed ? 128u : 1024u / (uint32_t)bits) == 0;  // (packed: whole workgroups of columns)
-        if (packed) us *= bits == 8 ? 0.95 : lines ? 1.06 : 0.95;
-        else us *= bits == 8 ? (lines ? 1.06 : 0.84) : (lines ? 1.2 : 1.0);
-    }
-    return family_us < us;
+    if (!second_launch) return family_us < t.us;  // (the estimates of the time before: see tile128_plan)
+    // (packed 4-bit codes in one 64-row block of the family, which reads each code once as a tile does, against split tiles that leave
+    // a third of the CUs idle: level, 48 x 11008 x 8192 33.9 against 32.7)
+    const uint64_t wgs = (uint64_t)((n + 127u) / 128u) * t.splits, cus = machine_cus();
+    const double level = packed && bits == 4 && m <= 64u && t.splits > 1u && !t.finish_launch && wgs * 10u <= cus * 7u ? 1.12 : 1.0;
+    return family_beside_tiles_us(family_us, m, n, bits, packed) < level * t.us;
 }
 
 // The decode family in row blocks: grid z walks blocks of 16*mb rows.  128 columns x 64 rows (mb = 4, 4 waves: one
@@ -727,13 +757,13 @@ int resolve_variant(uint32_t m, uint32_t n, uint32_t k, int bits, int variant, b
 }
 
 // whether a tiled-variant launch over row-major weights goes to the small-tile kernel that can split k
-static bool tiled_may_split(int v, uint32_t m, uint32_t n, int bits) { return use_small_tiles(v, m, n, bits) && v != BFAINTB_VARIANT_PREFILL_128_LDS; }
+static bool tiled_may_split(int v, uint32_t m, uint32_t n, uint32_t k, int bits) { return use_small_tiles(v, m, n, k, bits) && v != BFAINTB_VARIANT_PREFILL_128_LDS; }
 
 size_t workspace_need(uint32_t m, uint32_t n, uint32_t k, int bits, int variant, uint32_t forced_split)
 {
     if (m == 0 || n == 0) return 0;
     if (variant == BFAINTB_VARIANT_DECODE) return split_workspace_bytes(decode_plan(m, n, k, bits, forced_split).splits, m, n);
-    if (is_prefill(variant) && tiled_may_split(variant, m, n, bits)) return tile_workspace_bytes(tile128_plan(m, n, k, bits, forced_split), m, n);
+    if (is_prefill(variant) && tiled_may_split(variant, m, n, k, bits)) return tile_workspace_bytes(tile128_plan(m, n, k, bits, forced_split), m, n);
     return 0;
 }
 
@@ -879,7 +909,7 @@ uint32_t bfaintb_gemm_split_k(uint32_t m, uint32_t n, uint32_t k, int weight_bit
         }
     }
     if (v == BFAINTB_VARIANT_DECODE) return decode_plan(m, n, k, weight_bits, 0).splits;
-    if (v == BFAINTB_VARIANT_PREFILL && tiled_may_split(v, m, n, weight_bits)) return tile128_plan(m, n, k, weight_bits, 0).splits;
+    if (v == BFAINTB_VARIANT_PREFILL && tiled_may_split(v, m, n, k, weight_bits)) return tile128_plan(m, n, k, weight_bits, 0).splits;
     return 1;
 }
 
@@ -1115,11 +1145,12 @@ static int gemm_impl(void* c, const void* a, const void* b, const void* scale, c
         return (int)bfaintb::launch_prefill(p, weight_bits, st, v != BFAINTB_VARIANT_PREFILL_256_LDS);
 #endif
         // row-major weights on small tiles: that form, unless the other one is asked for by name
-        small_wreg = tiled_may_split(v, m, n, weight_bits) && bfaintb::prefill128_wreg_serves(p);
+        small_wreg = tiled_may_split(v, m, n, k, weight_bits) && bfaintb::prefill128_wreg_serves(p);
         if (small_wreg) {
             const TilePlan tp = tile128_plan(m, n, k, weight_bits, split_k, second_launch);
             p.k_per_wg = tp.k_per_wg;
             p.splits = tp.splits;
+            p.tile_blocks = tp.blocks;
             p.finish_launch = tp.finish_launch;
         }
     } else {
@@ -1159,9 +1190,14 @@ static int gemm_impl(void* c, const void* a, const void* b, const void* scale, c
     if (p.splits > 1) in_order = std::unique_lock<std::mutex>(workspace_order(p.ws_header));
     if (tiled) {
         if (small_wreg) return (int)bfaintb::launch_prefill128_wreg(p, weight_bits, false, st);
-        if ((v == BFAINTB_VARIANT_PREFILL_256X128 || (v == BFAINTB_VARIANT_PREFILL && prefill_tall_tiles(m, n, weight_bits))) && !p.reference_arith)
+        if (v == BFAINTB_VARIANT_PREFILL && !tall_tiles_in_one_chain(m, k) && prefill_tall_tiles(m, n, k, weight_bits) && bfaintb::prefill128_wreg_serves(p)) {
+            p.tile_blocks = tall_tile_blocks(m);
+            p.k_per_wg = (k + 63u) / 64u * 64u;  // (whole K-steps)
+            return (int)bfaintb::launch_prefill128_wreg(p, weight_bits, false, st);
+        }
+        if ((v == BFAINTB_VARIANT_PREFILL_256X128 || (v == BFAINTB_VARIANT_PREFILL && prefill_tall_tiles(m, n, k, weight_bits))) && !p.reference_arith)
             return (int)bfaintb::launch_prefill256x128_wreg(p, weight_bits, false, st);
-        if (use_small_tiles(v, m, n, weight_bits)) return (int)bfaintb::launch_prefill128(p, weight_bits, false, st);
+        if (use_small_tiles(v, m, n, k, weight_bits)) return (int)bfaintb::launch_prefill128(p, weight_bits, false, st);
         return (int)bfaintb::launch_prefill(p, weight_bits, st, v != BFAINTB_VARIANT_PREFILL_256_LDS);
     }
 #ifdef BFAINTB_TRACE
@@ -1437,7 +1473,7 @@ int bfaintb_gemm_prepacked_variant(uint32_t m, uint32_t n, uint32_t k, int weigh
 static size_t packed_workspace_need(uint32_t m, uint32_t n, uint32_t k, int bits, int v, bool second_launch = true)
 {
     if (m == 0 || n == 0) return 0;
-    if (is_prefill(v)) return tiled_may_split(v, m, n, bits) ? tile_workspace_bytes(tile128_plan(m, n, k, bits, 0, second_launch), m, n) : 0;
+    if (is_prefill(v)) return tiled_may_split(v, m, n, k, bits) ? tile_workspace_bytes(tile128_plan(m, n, k, bits, 0, second_launch), m, n) : 0;
     if (v != BFAINTB_VARIANT_DECODE || packed_uses_slab(m, n, k, bits)) return 0;
     const DecodePlan pl = packed_family_plan(m, n, k, bits);
     if (pl.splits <= 1) return 0;
@@ -1460,9 +1496,10 @@ static double launch_time_us(uint32_t m, uint32_t n, uint32_t k, int bits, bool 
     if (m <= kDecodeAutoMaxM) return 6.0 + (double)n * k * bits / 8.0 / 3.3e6 * (m <= 16u ? 1.0 : 1.25);
     if (m <= kDecodeFamilyAutoMaxM) {  // (beyond 32 rows the library's own choice asks just this)
         const double family = packed ? packed_family_time_us(m, n, k, bits, packed_family_plan(m, n, k, bits)) : decode_family_time_us(m, n, k, bits, decode_plan(m, n, k, bits, 0));
-        if (family_leads_tiles(family, m, n, k, bits, packed, true)) return family;
+        if (family_leads_tiles(family, m, n, k, bits, packed, true))
+            return prefill_small_tiles(m, n, k, bits) ? family_beside_tiles_us(family, m, n, bits, packed) : family;
     }
-    if (prefill_small_tiles(m, n, bits) || prefill_tall_tiles(m, n, bits)) return prefill_estimate_us(m, n, k, bits);
+    if (prefill_small_tiles(m, n, k, bits) || prefill_tall_tiles(m, n, k, bits)) return prefill_estimate_us(m, n, k, bits);
     const uint32_t tiles = ((m + 255u) / 256u) * ((n + 255u) / 256u);
     const uint32_t thin = bfaintb::thin_round_tiles(tiles, m, machine_cus()), full = tiles - thin;
     auto round_us = [&](double load) { return steps * (bits == 8 ? 1.0 + 0.5 * load : 1.1 + 0.45 * load); };
@@ -1612,12 +1649,13 @@ static int gemm_prepacked_impl(void* c, const void* a, const void* packed_b, con
         // a tile's 16 column blocks and a 256-row panel of A are addressed through 32-bit buffer extents
         if ((uint64_t)k * 256u * (uint32_t)weight_bits / 8u >= (1ull << 31) || (uint64_t)256 * lda * 2u >= (1ull << 31))
             return BFAINTB_ERR_BAD_SHAPE;
-        if (tiled_may_split(v, m, n, weight_bits) && bfaintb::prefill128_wreg_serves(p)) {
+        if (tiled_may_split(v, m, n, k, weight_bits) && bfaintb::prefill128_wreg_serves(p)) {
             // small tiles: the kernel that keeps the weights in registers, with the plan (split along k included) and the
             // workspace protocol of the row-major path
             const TilePlan tp = tile128_plan(m, n, k, weight_bits, 0, second_launch);
             p.k_per_wg = tp.k_per_wg;
             p.splits = tp.splits;
+            p.tile_blocks = tp.blocks;
             p.finish_launch = tp.finish_launch;
             std::unique_lock<std::mutex> in_order;
             if (p.splits > 1) {
@@ -1627,12 +1665,16 @@ static int gemm_prepacked_impl(void* c, const void* a, const void* packed_b, con
             }
             return (int)bfaintb::launch_prefill128_wreg(p, weight_bits, true, st);
         }
-        if (v == BFAINTB_VARIANT_PREFILL_256X128 || (v == BFAINTB_VARIANT_PREFILL && prefill_tall_tiles(m, n, weight_bits))) {
+        if (v == BFAINTB_VARIANT_PREFILL_256X128 || (v == BFAINTB_VARIANT_PREFILL && prefill_tall_tiles(m, n, k, weight_bits))) {
             p.k_per_wg = k;
             p.splits = 1;
+            if (v == BFAINTB_VARIANT_PREFILL && !tall_tiles_in_one_chain(m, k)) {
+                p.tile_blocks = tall_tile_blocks(m);
+                return (int)bfaintb::launch_prefill128_wreg(p, weight_bits, true, st);
+            }
             return (int)bfaintb::launch_prefill256x128_wreg(p, weight_bits, true, st);
         }
-        if (use_small_tiles(v, m, n, weight_bits)) return (int)bfaintb::launch_prefill128(p, weight_bits, true, st);
+        if (use_small_tiles(v, m, n, k, weight_bits)) return (int)bfaintb::launch_prefill128(p, weight_bits, true, st);
         return (int)bfaintb::launch_prefill_packed(p, weight_bits, st, v != BFAINTB_VARIANT_PREFILL_256_LDS);
     }
     if (!packed_uses_slab(m, n, k, weight_bits)) {
@@ -1808,7 +1850,7 @@ static int plan_whole(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint3
         return BFAINTB_OK;
     }
     // the tiled kernels
-    if (use_small_tiles(v, m, n, weight_bits)) {
+    if (use_small_tiles(v, m, n, k, weight_bits)) {
         out->variant = BFAINTB_VARIANT_PREFILL_128;
         out->tile_rows = out->tile_cols = 128u;
         const bool wreg = v != BFAINTB_VARIANT_PREFILL_128_LDS;
@@ -1824,12 +1866,13 @@ static int plan_whole(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint3
         out->workgroups = ((m + 127u) / 128u) * ((n + 127u) / 128u) * out->splits;
         return BFAINTB_OK;
     }
-    if (v == BFAINTB_VARIANT_PREFILL_256X128 || (v == BFAINTB_VARIANT_PREFILL && prefill_tall_tiles(m, n, weight_bits))) {
-        out->variant = BFAINTB_VARIANT_PREFILL_256X128;
-        out->kernel = BFAINTB_KERNEL_TILES_256X128;
+    if (v == BFAINTB_VARIANT_PREFILL_256X128 || (v == BFAINTB_VARIANT_PREFILL && prefill_tall_tiles(m, n, k, weight_bits))) {
+        const bool one_chain = v == BFAINTB_VARIANT_PREFILL_256X128 || tall_tiles_in_one_chain(m, k);
+        out->variant = one_chain ? BFAINTB_VARIANT_PREFILL_256X128 : BFAINTB_VARIANT_PREFILL;
+        out->kernel = one_chain ? BFAINTB_KERNEL_TILES_256X128 : BFAINTB_KERNEL_TILES_128;
         out->tile_rows = 256u;
         out->tile_cols = 128u;
-        out->waves = 4u;
+        out->waves = one_chain ? 4u : 8u;
         out->workgroups = ((m + 255u) / 256u) * ((n + 127u) / 128u);
         return BFAINTB_OK;
     }
@@ -1880,8 +1923,8 @@ int bfaintb_gemm_plan(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint3
     return plan_whole(m, n, k, weight_bits, group_size, packed, variant, split_k, out);
 }
 
-uint32_t bfaintb_prefill_tile(uint32_t m, uint32_t n) { return prefill_small_tiles(m, n, 8) ? 128u : 256u; }
-uint32_t bfaintb_prefill_tile_cols(uint32_t m, uint32_t n) { return (prefill_small_tiles(m, n, 8) || prefill_tall_tiles(m, n, 8)) ? 128u : 256u; }
+uint32_t bfaintb_prefill_tile(uint32_t m, uint32_t n) { return prefill_small_tiles(m, n, 4096u, 8) ? 128u : 256u; }
+uint32_t bfaintb_prefill_tile_cols(uint32_t m, uint32_t n) { return (prefill_small_tiles(m, n, 4096u, 8) || prefill_tall_tiles(m, n, 4096u, 8)) ? 128u : 256u; }
 
 const char* bfaintb_kernel_name(int variant, int weight_bits, uint32_t group_size, uint32_t m)
 {

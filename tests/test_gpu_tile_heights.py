@@ -1,0 +1,91 @@
+"""Tiles of 128 columns and 64 to 256 rows (bfaintb_prefill128_wreg_kernel): every height, stage count, weight order and scale grouping, at
+the steps, rows and columns where they can go wrong.  The oracle is the repository's: 2 bf16 units of the fp32 sum."""
+import numpy as np
+import pytest
+
+import helpers
+from helpers import Problem, assert_close_gated, assert_close_ulp, from_dev_u16, run_gemm, to_dev
+
+pytestmark = pytest.mark.gpu
+
+FORMATS = [(8, 0), (8, 64), (8, 32), (4, 0), (4, 128), (4, 32)]
+
+
+def run(af, p, packed, which):
+    import torch
+    if not packed:
+        return run_gemm(p, which=which)
+    w = torch.empty(af.prepack_bytes(p.n, p.k, p.bits), dtype=torch.uint8, device="cuda")
+    af.prepack(w, to_dev(p.b_bytes), p.n, p.k, weight_bits=p.bits)
+    c = torch.zeros((p.m, p.n), dtype=torch.int16, device="cuda")
+    ws = helpers._ws.get(af.prepacked_workspace_bytes(p.m, p.n, p.k, p.bits, p.group_size, which))
+    af.gemm_prepacked(c, to_dev(p.a_bf), w, to_dev(p.s_bf), p.m, p.n, p.k, weight_bits=p.bits, group_size=p.group_size, workspace=ws, which=which)
+    torch.cuda.synchronize()
+    return from_dev_u16(c)
+
+
+# 4, 6 and 8 blocks of 16 rows (33 .. 64, .. 96, .. 128 rows a tile), one tile and several, the last one of one row; one K-step, fewer than the
+# stages, as many, one more, and several rounds of them
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("bits,group", FORMATS)
+@pytest.mark.parametrize("m,n,k", [(33, 128, 128), (64, 272, 384), (65, 144, 512), (96, 128, 640), (97, 400, 256), (128, 272, 1408), (129, 128, 384), (257, 144, 1152)])
+def test_small_tiles(m, n, k, bits, group, packed):
+    import awesome_fusion_amd as af
+    p = Problem(m, n, k, bits, group, seed=m + n + k + bits)
+    c = run(af, p, packed, af.PREFILL_128)
+    assert_close_ulp(p, c, f"{m}x{n}x{k} bits={bits} g={group} packed={packed}")
+    assert np.array_equal(run(af, p, packed, af.PREFILL_128), c), "not reproducible"
+
+
+# 10, 12 and 16 blocks: the tall tiles of the library's own choice, planned for few compute units
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("bits,group", FORMATS)
+@pytest.mark.parametrize("m,n,k,blocks", [(320, 640, 2176, 10), (305, 528, 2304, 10), (384, 640, 1152, 12), (353, 528, 1280, 12), (512, 640, 1152, 16), (391, 656, 1408, 16)])
+def test_tall_tiles(m, n, k, blocks, bits, group, packed):
+    import awesome_fusion_amd as af
+    try:
+        af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 14)
+        pl = af.plan(m, n, k, bits, group, packed=packed, which=af.PREFILL)
+        assert (pl.kernel, pl.tile_rows, pl.tile_cols, pl.waves, pl.splits) == (af.KERNEL_TILES_128, 256, 128, 8, 1), pl.as_dict()
+        p = Problem(m, n, k, bits, group, seed=m + k + bits)
+        c = run(af, p, packed, af.PREFILL)
+        assert_close_ulp(p, c, f"{blocks} blocks: {m}x{n}x{k} bits={bits} g={group} packed={packed}")
+        assert np.array_equal(run(af, p, packed, af.PREFILL), c), "not reproducible"
+    finally:
+        af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 0)
+
+
+def test_tall_tiles_take_the_epilogues_and_strides():
+    import awesome_fusion_amd as af
+    try:
+        af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 14)
+        for (m, n, k, bits, group) in ((500, 656, 1064, 8, 0), (300, 640, 2304, 4, 128)):   # (a last K-step that is not whole)
+            assert af.variant(m, n, k, bits, group) == af.PREFILL and af.plan(m, n, k, bits, group).kernel == af.KERNEL_TILES_128
+            p = Problem(m, n, k, bits, group, seed=m)
+            c = run_gemm(p)
+            wide = run_gemm(p, ldc=n + 24, c_fill=0x1234)
+            assert np.array_equal(wide[:, :n], c) and (wide[:, n:] == 0x1234).all()
+            p.with_bias().with_residual()
+            assert_close_ulp(p, run_gemm(p), "bias and residual")
+            g = Problem(m, n, k, bits, group, seed=3, scale_lo=0.002, scale_hi=0.02 if bits == 8 else 0.2).with_bias()
+            assert_close_gated(g, run_gemm(g, activation=af.ACT_SILU_GATE), "gated")
+    finally:
+        af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 0)
+
+
+@pytest.mark.parametrize("bits,group,packed", [(8, 0, False), (8, 64, True), (4, 32, False), (4, 128, True)])
+def test_scales_of_any_sign_and_size(bits, group, packed):
+    """The conversion's two terms, (1024 + code) s and (1024 + excess) s, are exact whatever the scale: negative, zero, subnormal, large."""
+    import awesome_fusion_amd as af
+    import oracle
+    p = Problem(70, 144, 512, bits, group, seed=4)
+    s = np.random.default_rng(6).uniform(-1.0, 1.0, size=p.s_bf.shape).astype(np.float32)
+    s[:, 0::6] *= np.float32(2.0 ** -120)
+    s[:, 1::6] *= np.float32(2.0 ** 90)
+    s[:, 2::6] = 0.0
+    p.s_bf, p._w = oracle.f32_to_bf16_rne(s), None
+    c = helpers.widen(run(af, p, packed, af.PREFILL_128)).astype(np.float64)
+    w = helpers.widen(p.w_bf).astype(np.float64)
+    exact, absum = helpers.widen(p.a_bf).astype(np.float64) @ w, np.abs(helpers.widen(p.a_bf).astype(np.float64)) @ np.abs(w)
+    # (one rounding to bf16, 2^-8, and an fp32 sum of 512 terms, at most 512 x 2^-24 of the sum of their magnitudes)
+    assert (np.abs(c - exact) <= 2.0 ** -8 * np.abs(exact) + 512 * 2.0 ** -24 * absum + 1e-38).all()
