@@ -302,7 +302,7 @@ static TilePlan tile128_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint3
     const uint32_t ksteps = (k + 63u) / 64u;
     // blocks of 16 rows of a tile: the rows, spread evenly over as many tiles as 128 rows each would take
     const uint32_t rows_of_tiles = (m + 127u) / 128u, needed = (m + 16u * rows_of_tiles - 1u) / (16u * rows_of_tiles);
-    const uint32_t blocks = needed <= 4u ? 4u : needed <= 6u ? 6u : 8u;
+    const uint32_t blocks = needed <= 2u ? 2u : needed <= 4u ? 4u : needed <= 6u ? 6u : 8u;
     const double tiles = (double)rows_of_tiles * (double)((n + 127u) / 128u);
     const double cus = (double)machine_cus();
     const double fill = (double)m / (double)((m + 127u) / 128u * 128u);  // the share of the tiles' rows that exist
@@ -756,6 +756,44 @@ int resolve_variant(uint32_t m, uint32_t n, uint32_t k, int bits, int variant, b
     return BFAINTB_ERR_BAD_VARIANT;
 }
 
+// 17 to 32 rows whose launch by the library's own choice goes to tiles of 32 rows x 128 columns, unsplit, instead of the family (which
+// keeps its place for calls that name it, and its scratch is asked for all the same).  pitch: codes from one row of B to the next.
+// us, family / tiles (32 rows of A unless said; B cold):
+// Over 174 random shapes that it takes, 17 ... 32 rows, 1.12 times as fast as the family.
+//   - nine sixteenths of a round of tiles at least; with fewer the family's split fills the machine (128 tiles, k = 4096: 8-bit 19.9 /
+//     24.6, 4-bit 18.0 / 24.3).
+//   - packed 4-bit codes, however many rounds: 22016 x 4096 23.5 / 21.1, 32768 x 4096 27.4 / 22.7, 27008 x 1280 12.7 / 10.8, 50304 x
+//     4096 44.9 / 40.6; level at k = 6144 (29.5 / 29.3), behind at 8192 (36.2 / 38.6), where the family's longer walk amortises its
+//     start; and where k is 2048, at which every column block begins in the same memory channels (22016 columns, 20 rows 12.5 / 13.0).
+//   - packed 8-bit codes: 20480 x 4096 22.9 / 20.7, 22016 x 5120 28.6 / 26.5, 50304 x 4096 47.5 / 44.0; a short k has too few steps to
+//     fill the pipeline (22016 x 2048 15.6 / 17.3), a long one is level or behind (28672 x 6144, 20 rows 31.4 / 33.3), and so are several rounds with one scale per column
+//     (50944 x 3456, 20 rows 38.4 / 40.5, 34560 x 3584, 29 rows 38.5 / 40.3; groups of 128, 47344 x 4096, 30 rows 49.2 / 44.1).
+//   - codes in rows: one round of tiles at most (36864 x 4096, 288 tiles: 8-bit 41.9 / 45.3, 4-bit 37.8 / 43.8), and not where the rows lie
+//     a multiple of 1024 codes apart, which crowds the memory channels and which whole rows of 128 columns feel more than the family's
+//     blocks do (8-bit 20480 x 4096 27.3 / 28.7, 18432 x 4096 26.1 / 26.9, 23552 x 5880, 29 rows 37.8 / 43.3).  Otherwise 8-bit 22016 x 4096 26.5 / 24.3, 18560 x
+//     2432 20.7 / 15.5, 31328 x 1152, 24 rows, 14.3 / 12.0, 27808 x 4992, 17 rows, 36.3 / 30.6; 4-bit 22016 x 4096 23.7 / 21.5, 27728 x
+//     5504, 20 rows, 32.8 / 27.6.  Up to two thirds of a round only where the family does not split a long k three ways (20272 x 1536 8-bit
+//     16.6 / 13.8, 19216 x 2560 4-bit 20.7 / 15.8; 18944 x 4192 8-bit 23.4 / 25.3, 18560 x 6272 4-bit 26.7 / 29.3).  Up to 20 rows of 4-bit codes only where rows are not whole lines (22016 x 5120, 20 rows: 24.4 / 25.0).
+static bool few_rows_on_tiles(uint32_t m, uint32_t n, uint32_t k, int bits, bool grouped, bool packed, uint32_t pitch)
+{
+    const uint32_t cus = machine_cus(), tiles = n / 128u + (n % 128u != 0u);
+    if (m < 17u || m > 32u || tiles * 16ull < cus * 9ull) return false;
+    if (packed && bits == 4) return k > 1024u && k <= 5120u && k != 2048u;
+    if (packed) return k >= 3072u && k <= 5632u && (tiles <= cus || grouped);
+    if (tiles * 3ull <= cus * 2ull && k > 4096u) return false;
+    if (tiles > cus || pitch % 1024u == 0u || k <= 1024u || k >= 8192u) return false;
+    return bits == 8 || m > 20u || pitch % 256u != 0u;
+}
+
+static hipError_t launch_few_rows_on_tiles(GemmParams p, int bits, bool packed, hipStream_t stream)
+{
+    p.k_per_wg = (p.k + 63u) / 64u * 64u;  // (whole K-steps)
+    p.splits = 1u;
+    p.tile_blocks = 2u;
+    p.finish_launch = 0u;
+    return bfaintb::launch_prefill128_wreg(p, bits, packed, stream);
+}
+
 // whether a tiled-variant launch over row-major weights goes to the small-tile kernel that can split k
 static bool tiled_may_split(int v, uint32_t m, uint32_t n, uint32_t k, int bits) { return use_small_tiles(v, m, n, k, bits) && v != BFAINTB_VARIANT_PREFILL_128_LDS; }
 
@@ -1186,6 +1224,10 @@ static int gemm_impl(void* c, const void* a, const void* b, const void* scale, c
         e = attach_workspace(p, workspace, BFAINTB_STATIC_SCRATCH_BYTES, need);
         if (e) return e;
     }
+    // (the tiled kernel addresses B and the rows of A through 32-bit buffer extents; the reference's arithmetic has no such form)
+    if (variant == BFAINTB_VARIANT_AUTO && !tiled && split_k == 0 && !ep.reference_arith && few_rows_on_tiles(m, n, k, weight_bits, group_size != 0, false, ldb) &&
+        (uint64_t)k * p.ldb_bytes < (1ull << 31) && (uint64_t)256 * lda * 2u < (1ull << 31))
+        return (int)launch_few_rows_on_tiles(p, weight_bits, false, st);
     std::unique_lock<std::mutex> in_order;
     if (p.splits > 1) in_order = std::unique_lock<std::mutex>(workspace_order(p.ws_header));
     if (tiled) {
@@ -1695,6 +1737,8 @@ static int gemm_prepacked_impl(void* c, const void* a, const void* packed_b, con
         DeviceState* dev = nullptr;
         e = device_state(st, &dev);
         if (e) return e;
+        if (variant == BFAINTB_VARIANT_AUTO && few_rows_on_tiles(m, n, k, weight_bits, group_size != 0, true, n) && (uint64_t)256 * lda * 2u < (1ull << 31))
+            return (int)launch_few_rows_on_tiles(p, weight_bits, true, st);
         std::unique_lock<std::mutex> in_order;
         if (p.splits > 1) in_order = std::unique_lock<std::mutex>(workspace_order(p.ws_header));
         return (int)bfaintb::launch_decode_family_packed(p, weight_bits, st);
@@ -1820,7 +1864,6 @@ static int plan_whole(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint3
                       bfaintb_plan* out)
 {
     memset(out, 0, sizeof(*out));
-    (void)group_size;
     const int v = packed ? packed_variant(m, n, k, weight_bits, variant) : resolve_variant(m, n, k, weight_bits, variant);
     if (v < 0) return v;
     out->compute_units = machine_cus();
@@ -1839,6 +1882,8 @@ static int plan_whole(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint3
             return BFAINTB_OK;
         }
         const DecodePlan pl = packed ? packed_family_plan(m, n, k, weight_bits) : decode_plan(m, n, k, weight_bits, split_k);
+        if (variant == BFAINTB_VARIANT_AUTO && (packed || split_k == 0) && few_rows_on_tiles(m, n, k, weight_bits, group_size != 0, packed != 0, n))
+            out->tiles_instead = (n + 127u) / 128u;
         out->kernel = BFAINTB_KERNEL_DECODE_FAMILY;
         out->tile_rows = 16u * pl.mb;
         out->tile_cols = pl.cols;

@@ -1,4 +1,4 @@
-// Tiled variant, tiles of 128 columns and 64 to 256 rows, weights kept in registers: the small-tile and the tall-tile kernel, for
+// Tiled variant, tiles of 128 columns and 32 to 256 rows, weights kept in registers: the small-tile and the tall-tile kernel, for
 // row-major B and for B in the packed order (PACKED).
 //
 // Same job and the same reference kernel replaced as bfaintb_prefill128_kernel
@@ -22,12 +22,18 @@
 // too few of those, what the conversion (36 to 46 vector instructions a wave) and the reads add.  Hence
 //   - the tall tiles: 16 blocks share one conversion.  us, 4 waves of 128 x 64 (bfaintb_prefill256x128_wreg_kernel) / this: 2048 x 4096 x
 //     4096 8-bit 70.8 / 63.0; 512 x 11008 x 4096 8-bit 63.0 / 52.1, 4-bit 71.6 / 53.9; 512 x 13824 x 5120 packed 4-bit 85.4 / 73.1.
-//   - no row blocks that do not exist: MT = 4, 6, 8, 10, 12, 16, the rows spread evenly over the tiles (96 x 20480 x 4096 packed 8-bit 32.9
+//   - no row blocks that do not exist: MT = 2, 4, 6, 8, 10, 12, 16, the rows spread evenly over the tiles (96 x 20480 x 4096 packed 8-bit 32.9
 //     with eight blocks / 29.1 with six).
 //   - the conversion by half-precision magic numbers (see there) and codes by transposing reads: 42 vector and 16 LDS instructions a wave
 //     and step before, 34 and 10 now (64 x 4096 x 11008 8-bit unsplit, codes in the last-level cache: 55.9 -> 49.2).
 //   - more stages the fewer rows there are, since such launches read their codes from memory and wait for it: 64 x 4096 x 11008 8-bit
 //     unsplit, codes cold, 4 / 8 stages 69.2 / 63.1; 96 rows 4-bit g128, 4 / 6 stages 88.9 / 78.6.
+//   - for 17 to 32 rows, whose calls read every code once, from memory: the copying wave and eight stages whatever the codes (32 x 22016 x
+//     4096, one row of 172 tiles, us with / without: 4-bit g128 in rows 21.5 / 23.9; 8-bit in rows 24.3 / 24.1), and a walk over k that each
+//     tile of packed 8-bit codes starts at a step of its own, so that the column blocks, a power of two apart, are not all read at the
+//     same place at once (22016 x 4096 22.5 without / 21.3, 28672 x 8192 44.6 / 43.5; 4-bit codes lose by it, 38.6 / 39.9).  A step of
+//     two row blocks takes 0.25 to 0.3 us: 16 waves in two halves of k, each with stages of its own, were no faster (32 x 22016 x 4096 8-bit
+//     in rows 27.1, 28672 x 8192 packed 4-bit 41.9 against 38.9): the vector instructions of the conversion bound it, not a wait.
 // With a workgroup on every CU the clock gives way to the board's power on top (16 blocks: 0.60 us a step on 96 CUs, 0.82 on 256).
 // Accumulator (mt, j), register r of lane (c16 = lane % 16, q = lane / 16): row 16 mt + 4 q + r, column 32 w + 16 j + c16 of the tile.
 // Epilogue: as bfaintb_prefill128_kernel — fp32 sums staged in LDS in [m][n] order, each thread finishes 8 neighbouring
@@ -76,11 +82,12 @@ __shared__ __attribute__((aligned(1024))) uint8_t tw_lds[BYTES];
 template <int BITS, bool GROUPED, bool PACKED, bool SCALES, int MT, int NS, bool COPIER>
 __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, const uint32_t n0, const uint32_t ks)
 {
-    static_assert(MT >= 4 && MT <= 16, "blocks of 16 rows");
-    static_assert((NS == 4 || NS == 6 || NS == 8) && NS * MT % 4 == 0, "the fragments' rotation comes round with the stages");
+    static_assert(MT >= 2 && MT <= 16, "blocks of 16 rows");
+    constexpr uint32_t kAhead = MT < 4 ? MT : 4;       // units that the fragments of A are read ahead
+    static_assert((NS == 4 || NS == 6 || NS == 8) && NS * MT % kAhead == 0, "the fragments' rotation comes round with the stages");
     constexpr uint32_t kRows = 16u * MT;               // rows of a tile
     constexpr uint32_t kACopies = (MT + 3u) / 4u;      // of A, per wave and step: 8 rows each
-    constexpr uint32_t kStageRows = 64u * kACopies;    // rows of a stage of A (those past the tile's are zero and not read)
+    constexpr uint32_t kStageRows = MT < 4 ? kRows : 64u * kACopies;  // rows of a stage of A (those past the tile's are zero and not read)
     constexpr uint32_t kRowBytes = 128u * BITS / 8u;   // a tile row of codes
     constexpr bool kScalesInLds = GROUPED && SCALES;   // group scales come by the copy engine as well
     using C0 = std::integral_constant<uint32_t, 0>;
@@ -124,23 +131,36 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
     const uint32_t ksteps = p.k_per_wg / kTwK < ksteps_all - kbase ? p.k_per_wg / kTwK : ksteps_all - kbase;
     const uint32_t last_chunks = (p.k - (ksteps_all - 1u) * kTwK) / 8u;  // valid 16-byte chunks per row of A in the last step
     auto clamp = [&](uint32_t t) { return t < ksteps ? t : ksteps - 1u; };
+    // The K-step of the whole matrix that step t of the share is.  Few rows of packed 8-bit codes: each tile starts its walk at a step of its
+    // own (see the head of the file).
+    const uint32_t rotate = PACKED && BITS == 8 && MT < 4 ? (n0 / kTw) % ksteps : 0u;
+    auto at_step = [&](uint32_t t) -> uint32_t {
+        if constexpr (PACKED && BITS == 8 && MT < 4) {
+            const uint32_t r = t + rotate;
+            return kbase + (r < ksteps ? r : r - ksteps);
+        } else {
+            return kbase + t;
+        }
+    };
 
     // A copy: instruction j of wave w fills rows 8 (kACopies w + j) .. + 7; lane l lands at row + l / 8, chunk position l % 8, so
     // it fetches chunk (l % 8) ^ ((row >> 1) & 7) = (l % 8) ^ (l / 16) for even kACopies w + j and that ^ 4 for odd ones; the row
     // advance of j and the K advance sit in the scalar offset.  A chunk past the end of k (partial last step) is fetched from
     // beyond the extent and reads as zero; rows of B past k read as zero codes, finite weights, and multiply those zeros.
-    const uint32_t a_row = 8u * kACopies * wave + (lane >> 3);
-    const uint32_t chunk_e = (lane & 7u) ^ ((lane >> 4) & 7u) ^ (4u * (kACopies & wave & 1u)), chunk_o = chunk_e ^ 4u;
+    // (a stage of fewer than 64 rows: several waves copy the same 8 rows to the same place, so that all have as many requests in flight)
+    const uint32_t a_block = kStageRows < 64u ? wave & (kStageRows / 8u - 1u) : kACopies * wave;  // the wave's first 8 rows
+    const uint32_t a_row = 8u * a_block + (lane >> 3);
+    const uint32_t chunk_e = (lane & 7u) ^ ((lane >> 4) & 7u) ^ (4u * (a_block & 1u)), chunk_o = chunk_e ^ 4u;
     const uint32_t a_voff_e = (a_row * p.lda + chunk_e * 8u) * 2u, a_voff_o = (a_row * p.lda + chunk_o * 8u) * 2u;
     const uint32_t a_last_e = chunk_e < last_chunks ? a_voff_e : a_extent, a_last_o = chunk_o < last_chunks ? a_voff_o : a_extent;
     auto dma_a = [&](auto stage_c, uint32_t kt) {
-        uint8_t* base = a_tile(stage_c) + wave * (1024u * kACopies);
-        const bool last = kbase + kt + 1u == ksteps_all;
+        uint8_t* base = a_tile(stage_c) + a_block * 1024u;
+        const bool last = at_step(kt) + 1u == ksteps_all;
         const uint32_t ve = last ? a_last_e : a_voff_e, vo = last ? a_last_o : a_voff_o;
 #pragma unroll
         for (uint32_t j = 0; j < kACopies; ++j)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (__attribute__((address_space(3))) void*)(base + j * 1024u), 16,
-                                                     (j & 1u) ? vo : ve, (kbase + kt) * kTwK * 2u + j * 16u * p.lda, 0, 0);
+                                                     (j & 1u) ? vo : ve, at_step(kt) * kTwK * 2u + j * 16u * p.lda, 0, 0);
     };
 
     // W codes.  Copy: a 16-byte-per-lane instruction fills 1024 bytes = kRowsPerCopy rows of the stage; the step's 64
@@ -169,7 +189,7 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
     constexpr uint32_t w_shift = (PACKED && BITS == 4) ? 1u : 0u;
     auto dma_w = [&](uint8_t* stage, uint32_t kt) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (__attribute__((address_space(3))) void*)(stage + wave * 1024u), 16, w_voff,
-                                                 ((kbase + kt) >> w_shift) * w_step, 0, 0);
+                                                 (at_step(kt) >> w_shift) * w_step, 0, 0);
     };
     // Read: lane (c16, kq) of the wave takes, of its block of 32 k, rows 8 kq .. 8 kq + 7 of columns 16 j + c16, j = 0, 1, of the
     // wave's 32: 8 bytes (8-bit codes) or 4 for each.
@@ -206,7 +226,7 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
             }
         } else if constexpr (PACKED) {
 #pragma unroll
-            for (uint32_t j = 0; j < 2; ++j) c.d[j][0] = *reinterpret_cast<const uint32_t*>(stage + w_rd[j] + 8u * ((kbase + kt) & 1u));
+            for (uint32_t j = 0; j < 2; ++j) c.d[j][0] = *reinterpret_cast<const uint32_t*>(stage + w_rd[j] + 8u * (at_step(kt) & 1u));
         } else {
             const v2i v = __builtin_amdgcn_ds_read_tr4_b64_v2i32((lds_v2i)(const_cast<uint8_t*>(stage) + w_rd[0]));
             c.d[0][0] = (uint32_t)v[0], c.d[1][0] = (uint32_t)v[1];
@@ -228,7 +248,7 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
         for (uint32_t j = 0; j < 2; ++j) sr.s[j] = __builtin_amdgcn_raw_buffer_load_b16(rsrc_s, s_voff + 32u * j, row_off, 0);
     };
     auto group_offset = [&](uint32_t kt, uint32_t block) {  // of the scale row of a block of 32 k of step kt
-        uint32_t g = group_of_row(p, (kbase + kt) * kTwK + 32u * block);
+        uint32_t g = group_of_row(p, at_step(kt) * kTwK + 32u * block);
         if (g >= scale_rows) g = scale_rows - 1u;  // rows past k in a partial last step: any scale will do
         return g * p.lds * 2u;
     };
@@ -259,12 +279,12 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
         }
         constexpr uint32_t kStepCopies = kStageRows / 8u + kCodeCopies + (kScalesInLds ? 2u : 0u);
         auto copy_step = [&](auto stage_c, uint32_t kt) {
-            const bool last = kbase + kt + 1u == ksteps_all;
+            const bool last = at_step(kt) + 1u == ksteps_all;
             const uint32_t ve = last ? pl_e : pa_e, vo = last ? pl_o : pa_o;
 #pragma unroll
             for (uint32_t j = 0; j < kCodeCopies; ++j)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (__attribute__((address_space(3))) void*)(w_tile(stage_c) + j * 1024u), 16, pw[j],
-                                                         ((kbase + kt) >> w_shift) * w_step, 0, 0);
+                                                         (at_step(kt) >> w_shift) * w_step, 0, 0);
             if constexpr (kScalesInLds) {
 #pragma unroll
                 for (uint32_t h = 0; h < 2; ++h)
@@ -274,7 +294,7 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
 #pragma unroll
             for (uint32_t j = 0; j < kStageRows / 8u; ++j)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (__attribute__((address_space(3))) void*)(a_tile(stage_c) + j * 1024u), 16, (j & 1u) ? vo : ve,
-                                                         (kbase + kt) * kTwK * 2u + j * 16u * p.lda, 0, 0);
+                                                         at_step(kt) * kTwK * 2u + j * 16u * p.lda, 0, 0);
         };
         barrier_no_fence();  // (the first steps' copies are shared out over the computing waves: see the prologue)
         uint32_t kt = 0;
@@ -378,7 +398,6 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
         for (int j = 0; j < 2; ++j) acc[mt][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
     // fragment mt: row 16 mt + c16 of the tile, chunk 4 kh + kq (the swizzle repeats every 16 rows)
-    constexpr uint32_t kAhead = 4;
     bf16x8_t af[kAhead];  // the fragments of the next few units, carried from step to step
     const uint32_t a_rd = tw_swz(c16, 4u * kh + kq);
 
@@ -408,9 +427,9 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
         if constexpr (!COPIER) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((kDepth - 2u) * kRequests + (kRing ? 2u : 0u)) : "memory");
         barrier_no_fence();  // (a fenced barrier would also wait for the copies of the steps ahead)
         const uint32_t kt3 = clamp(kt + kDepth);
-        const bool last3 = kbase + kt3 + 1u == ksteps_all;
+        const bool last3 = at_step(kt3) + 1u == ksteps_all;
         const uint32_t ve = last3 ? a_last_e : a_voff_e, vo = last3 ? a_last_o : a_voff_o;
-        uint8_t* const a_dst = a_tile(Target{}) + wave * (1024u * kACopies);
+        uint8_t* const a_dst = a_tile(Target{}) + a_block * 1024u;
         const uint8_t* const a_src = a_tile(stage_c) + a_rd;
         const uint8_t* const a_nxt = a_tile(Next{}) + a_rd;
         const uint8_t* const w_src = w_tile(Next{});
@@ -451,15 +470,16 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
                 if (kRing && u == 0u) {
                     const uint32_t off = group_offset(clamp(kt + NS), kh);
                     load_scales(ring[S], off);
-                } else if (COPIER) {
-                } else if (u >= kFirstCopy && u < kFirstCopy + kACopies) {
-                    const uint32_t q = u - kFirstCopy;
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (__attribute__((address_space(3))) void*)(a_dst + q * 1024u), 16, (q & 1u) ? vo : ve,
-                                                             (kbase + kt3) * kTwK * 2u + q * 16u * p.lda, 0, 0);
-                } else if (u == kFirstCopy + kACopies) {
-                    dma_w(w_tile(Target{}), kt3);
-                } else if (kScalesInLds && u == kFirstCopy + kACopies + 1u) {
-                    dma_s(s_tile(Target{}), kt3);
+                }
+                // (tiles of fewer units than a step has requests: the rest with the last)
+#pragma unroll
+                for (uint32_t q = 0; q < (COPIER ? 0u : kRequests); ++q) {
+                    if ((kFirstCopy + q < (uint32_t)MT ? kFirstCopy + q : (uint32_t)MT - 1u) != u) continue;
+                    if (q < kACopies)
+                        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (__attribute__((address_space(3))) void*)(a_dst + q * 1024u), 16, (q & 1u) ? vo : ve,
+                                                                 at_step(kt3) * kTwK * 2u + q * 16u * p.lda, 0, 0);
+                    else if (q == kACopies) dma_w(w_tile(Target{}), kt3);
+                    else dma_s(s_tile(Target{}), kt3);
                 }
             }
 #pragma unroll
@@ -851,6 +871,7 @@ static hipError_t launch_prefill128_wreg_rows(const GemmParams& p, hipStream_t s
         }
     }
     switch (p.tile_blocks) {
+        case 2: return launch_prefill128_wreg_t<BITS, GROUPED, PACKED, 2, 8, true>(p, stream);  // (see the head of the file)
         case 10: return launch_prefill128_wreg_t<BITS, GROUPED, PACKED, 10, 4>(p, stream);
         case 12: return launch_prefill128_wreg_t<BITS, GROUPED, PACKED, 12, 4>(p, stream);
         case 16: return launch_prefill128_wreg_t<BITS, GROUPED, PACKED, 16, 4>(p, stream);

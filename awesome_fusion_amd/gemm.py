@@ -271,10 +271,10 @@ class Plan(C.Structure):
     """bfaintb_plan: what a call would launch."""
     _fields_ = [("variant", C.c_int32), ("kernel", _u32), ("tile_rows", _u32), ("tile_cols", _u32), ("waves", _u32), ("splits", _u32),
                 ("k_per_workgroup", _u32), ("workgroups", _u32), ("tail_workgroups", _u32), ("launches", _u32), ("compute_units", _u32),
-                ("reserved", _u32), ("workspace_bytes", C.c_uint64)]
+                ("tiles_instead", _u32), ("workspace_bytes", C.c_uint64)]
 
     def as_dict(self):
-        return {f: getattr(self, f) for f, _ in self._fields_ if f != "reserved"}
+        return {f: getattr(self, f) for f, _ in self._fields_}
 
 
 KERNEL_DECODE_FAMILY, KERNEL_DECODE_SLAB, KERNEL_TILES_128, KERNEL_TILES_128_LDS, KERNEL_TILES_256X128, KERNEL_TILES_256, KERNEL_TILES_256_LDS = range(1, 8)

@@ -370,7 +370,9 @@ typedef struct bfaintb_plan {
     uint32_t tail_workgroups;  /* of further launches over a last, thin round of tiles or over the last rows, or 0 */
     uint32_t launches;         /* kernels launched: 1, or more with a tail or with split sums added by a launch of their own */
     uint32_t compute_units;    /* what the plan was made for */
-    uint32_t reserved;
+    uint32_t tiles_instead;    /* 17 to 32 rows by the library's own choice: so many tiles of 32 rows x 128 columns, unsplit, run in place
+                                  of the launch that the fields above describe (which a call that names the variant, asks for the
+                                  reference's arithmetic or has rows too far apart for 32-bit extents gets); 0: they do not */
     uint64_t workspace_bytes;  /* what bfaintb_gemm[_prepacked]_workspace_bytes_ex reports for the same arguments */
 } bfaintb_plan;
 BFAINTB_API int bfaintb_gemm_plan(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint32_t group_size, int packed, int variant,

@@ -1,4 +1,4 @@
-"""Tiles of 128 columns and 64 to 256 rows (bfaintb_prefill128_wreg_kernel): every height, stage count, weight order and scale grouping, at
+"""Tiles of 128 columns and 32 to 256 rows (bfaintb_prefill128_wreg_kernel): every height, stage count, weight order and scale grouping, at
 the steps, rows and columns where they can go wrong.  The oracle is the repository's: 2 bf16 units of the fp32 sum."""
 import numpy as np
 import pytest
@@ -89,3 +89,50 @@ def test_scales_of_any_sign_and_size(bits, group, packed):
     exact, absum = helpers.widen(p.a_bf).astype(np.float64) @ w, np.abs(helpers.widen(p.a_bf).astype(np.float64)) @ np.abs(w)
     # (one rounding to bf16, 2^-8, and an fp32 sum of 512 terms, at most 512 x 2^-24 of the sum of their magnitudes)
     assert (np.abs(c - exact) <= 2.0 ** -8 * np.abs(exact) + 512 * 2.0 ** -24 * absum + 1e-38).all()
+
+
+# 2 blocks: fewer rows than a tile, one K-step, fewer than the stages, as many, one more, several rounds and an odd rest; a ragged last tile
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("bits,group", FORMATS)
+@pytest.mark.parametrize("m,n,k", [(1, 128, 128), (16, 144, 384), (17, 272, 512), (32, 128, 640), (31, 400, 1408)])
+def test_tiles_of_32_rows(m, n, k, bits, group, packed):
+    import awesome_fusion_amd as af
+    p = Problem(m, n, k, bits, group, seed=m + n + k + bits)
+    c = run(af, p, packed, af.PREFILL_128)
+    assert_close_ulp(p, c, f"{m}x{n}x{k} bits={bits} g={group} packed={packed}")
+    assert np.array_equal(run(af, p, packed, af.PREFILL_128), c), "not reproducible"
+
+
+# ... and as the library's own choice for 17 to 32 rows, planned for 8 compute units: 5 tiles (nine sixteenths of a round) to 8 and, of packed
+# codes, more; k that is no multiple of a K-step; the family beside it agrees with the same oracle
+@pytest.mark.parametrize("m,n,k,bits,group,packed", [(17, 656, 1032, 8, 0, False), (32, 1008, 1088, 8, 64, False), (21, 592, 1032, 4, 0, False),
+                                                     (32, 1008, 1664, 4, 128, False), (24, 656, 3136, 8, 0, True), (32, 1552, 3072, 8, 64, True),
+                                                     (17, 592, 1152, 4, 128, True), (32, 1552, 1280, 4, 0, True)])
+def test_few_rows_choose_tiles(m, n, k, bits, group, packed):
+    import awesome_fusion_amd as af
+    try:
+        af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 8)
+        pl = af.plan(m, n, k, bits, group, packed=packed)
+        assert pl.variant == af.DECODE and pl.tiles_instead == (n + 127) // 128, pl.as_dict()
+        assert af.plan(m, n, k, bits, group, packed=packed, which=af.DECODE).tiles_instead == 0
+        p = Problem(m, n, k, bits, group, seed=m + n + k)
+        c = run(af, p, packed, af.AUTO)
+        assert_close_ulp(p, c, "tiles")
+        assert_close_ulp(p, run(af, p, packed, af.DECODE), "family")
+        if not packed:
+            wide = run_gemm(p, ldc=n + 24, c_fill=0x1234)
+            assert np.array_equal(wide[:, :n], c) and (wide[:, n:] == 0x1234).all()
+            p.with_bias().with_residual()
+            assert_close_ulp(p, run_gemm(p), "bias and residual")
+            g = Problem(m, n, k, bits, group, seed=3, scale_lo=0.002, scale_hi=0.02 if bits == 8 else 0.2).with_bias()
+            assert_close_gated(g, run_gemm(g, activation=af.ACT_SILU_GATE), "gated")
+    finally:
+        af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 0)
+
+
+@pytest.mark.parametrize("m,n,k,group", [(18, 22016, 2560, 128), (32, 22016, 2176, 0)])
+def test_the_familys_four_splits_by_name(m, n, k, group):
+    """4-bit codes, 17 to 32 rows: the launch that the plan describes is what a call that names the family runs."""
+    import awesome_fusion_amd as af
+    p = Problem(m, n, k, 4, group, seed=m + k)
+    assert_close_ulp(p, run_gemm(p, which=af.DECODE), f"{m}x{n}x{k} g={group}")
