@@ -407,3 +407,18 @@ def test_hip_graph_replays_match_eager(af):
         for i, d in enumerate(bufs):
             assert np.array_equal(from_dev_u16(d["c"]), eager[i]), f"replay {replay}, problem {i}"
         run_prepacked(af, probs[0])  # unrelated eager work between replays
+
+
+@pytest.mark.parametrize("bits,k,n,ldb", [(8, 128, 256, None), (8, 64, 240, 512), (8, 192, 784, 800), (4, 256, 512, None), (4, 128, 496, 1024), (4, 384, 1296, 1312)])
+def test_pack_at_the_edges_of_its_workgroups(af, bits, k, n, ldb):
+    """256 (8-bit) or 512 columns a workgroup: whole ones, one that lacks a column block, a rest; nothing past the packed codes is written."""
+    import torch
+    p = Problem(1, n, k, bits, 0, seed=k + n + bits)
+    wide = np.full((k, (ldb or n) * bits // 8), 0xAB, np.uint8)
+    wide[:, :n * bits // 8] = p.b_bytes
+    need = af.prepack_bytes(n, k, bits)
+    pk = torch.full((need + 4096,), 0x5A, dtype=torch.uint8, device="cuda")
+    af.prepack(pk, to_dev(wide), n, k, ldb=ldb, weight_bits=bits)
+    torch.cuda.synchronize()
+    assert np.array_equal(pk[:need].cpu().numpy(), oracle.pack_mfma16(p.b_bytes, k, n, bits).reshape(-1))
+    assert (pk[need:] == 0x5A).all()
