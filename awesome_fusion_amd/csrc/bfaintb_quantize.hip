@@ -5,7 +5,7 @@
 //
 // Bound by memory: every weight read once (twice where a group is longer than a tile, the second time mostly from the
 // 256 MB cache), every code written once.  As a chain of framework operations the same work is 17 passes over fp32 copies:
-// 11008 x 4096, groups of 128, 4-bit, quantised and packed: 1200 us; with this kernel and the packing one 40 us.
+// 11008 x 4096, groups of 128, 4-bit, quantised and packed: 1200 us; with this kernel and the packing one 33 us.
 #include <type_traits>
 #include "bfaintb_device.hpp"
 
@@ -95,14 +95,17 @@ __device__ __forceinline__ float quotient16(float w, float s, float r)
     return fmaf(fmaf(-q, s, w), r, q);
 }
 
+// The code is left in the low bits of 2^23 + code: adding 2^23 + excess (an even number) to the quotient rounds it to an integer, half to
+// even, and puts it into the significand.  7 instructions a weight with the unpacking, where a rounding, two comparisons, a
+// conversion and an addition made it 10.  (Clamped first, which changes no code: the bounds are whole numbers.  A NaN becomes the least
+// code — v_med3_f32 gives the least of the other two — until the caller replaces it.)
+constexpr uint32_t kMagic = 0x4b000000u;  // the bits of 2^23
 template <int BITS, int TYPE>
-__device__ __forceinline__ uint32_t code_of(float w, float s, float r)
+__device__ __forceinline__ uint32_t code_in_float(float w, float s, float r)
 {
-    constexpr int kQmax = BITS == 8 ? 127 : 7;
+    constexpr float kExcess = BITS == 8 ? 128.0f : 8.0f;
     const float q = TYPE == kWeightF32 ? w / s : quotient16(w, s, r);
-    // (clamped before it becomes an integer: nothing out of an integer's range is converted, and a NaN is the least code until
-    // the caller replaces it)
-    return (uint32_t)((int)fminf(fmaxf(rintf(q), (float)(-kQmax - 1)), (float)kQmax) + kQmax + 1);
+    return __float_as_uint(__builtin_amdgcn_fmed3f(q, -kExcess, kExcess - 1.0f) + (8388608.0f + kExcess));
 }
 
 struct QuantizeParams {
@@ -115,7 +118,10 @@ struct QuantizeParams {
 constexpr uint32_t kTileK = 128, kTileBytes = 128;  // a workgroup's tile of codes: 128 rows of k, one cache line of each
 constexpr uint32_t kTilePitch = kTileBytes / 4u + 1u;  // dwords: the 16 lanes that write 8 rows apart fall into different banks
 
-// One workgroup: 128 k x 256 columns (4-bit; 128 columns for 8-bit codes).  A lane holds 8 consecutive k of as many rows of
+// One workgroup: 128 k x 256 columns (4-bit; 128 columns for 8-bit codes), neighbours along k: they read whole rows of W between them,
+// where neighbours along n would all read the same 256 bytes of rows that often lie a power of two apart, in few memory channels
+// (28672 x 4096 4-bit g64 72 us so, 60 now; 11008 x 4096 4-bit g128 30.4 and 26.1, 4.3 TB/s; only 8-bit codes whose scales were made
+// before, and whose weights come from the cache therefore, are 2 % faster along n: 11008 x 4096 41.5 / 42.4).  A lane holds 8 consecutive k of as many rows of
 // W as a dword holds codes, so that it makes whole dwords of the output's rows; the tile is turned through LDS and leaves
 // in full 128-byte lines.  FUSED: groups lie within the tile (32, 64 or 128 weights = 4, 8 or 16 lanes) and the scales
 // are made here, over the row of lanes; otherwise they have been made by scale_kernel.
@@ -125,8 +131,12 @@ __global__ void __launch_bounds__(512) bfaintb_quantize_kernel(const QuantizePar
     constexpr uint32_t kRows = 32u / BITS;  // rows of W per lane
     constexpr uint32_t kCode0 = BITS == 8 ? 0x80808080u : 0x88888888u;  // a group without a finite scale (a NaN or an infinity among its weights)
     __shared__ uint32_t tile[kTileK * kTilePitch];
+    constexpr bool kAlongK = FUSED || BITS == 4;
+    const uint32_t fast = kAlongK ? (p.k + kTileK - 1u) / kTileK : (p.n + 32u * kRows - 1u) / (32u * kRows);  // tiles of the direction that neighbours walk
+    const uint32_t slow_tile = blockIdx.x / fast, fast_tile = blockIdx.x - slow_tile * fast;
+    const uint32_t tile_k = kAlongK ? fast_tile : slow_tile, tile_n = kAlongK ? slow_tile : fast_tile;
     const uint32_t kq = threadIdx.x & 15u, ng = threadIdx.x >> 4;
-    const uint32_t k0 = blockIdx.y * kTileK + 8u * kq, n0 = (blockIdx.x * 32u + ng) * kRows;
+    const uint32_t k0 = tile_k * kTileK + 8u * kq, n0 = (tile_n * 32u + ng) * kRows;
     if (k0 < p.k && n0 < p.n) {  // (whole groups of lanes: n is a multiple of kRows, and k of 8 and of the group)
         Raw8<TYPE> raw[kRows];
 #pragma unroll
@@ -154,7 +164,10 @@ __global__ void __launch_bounds__(512) bfaintb_quantize_kernel(const QuantizePar
                 sb[r] = two & 0xffffu, sb[r + 1] = two >> 16;
             }
         }
-        uint32_t out[8] = {}, finite = 0u;  // (finite: all bits of the rows whose scale is)
+        uint32_t out[8], finite = 0u;  // (finite: all bits of the rows whose scale is)
+        constexpr uint32_t kMagics = BITS == 8 ? kMagic : (uint32_t)(kMagic * 0x11111111ull);  // what the 2^23s of all rows add up to
+#pragma unroll
+        for (int i = 0; i < 8; ++i) out[i] = 0u - kMagics;
 #pragma unroll
         for (uint32_t r = 0; r < kRows; ++r) {
             const float s = bf16_bits_to_f32(sb[r]);
@@ -162,18 +175,18 @@ __global__ void __launch_bounds__(512) bfaintb_quantize_kernel(const QuantizePar
             float rcp = __builtin_amdgcn_rcpf(s);
             rcp = fmaf(fmaf(-s, rcp, 1.0f), rcp, rcp);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) out[i] |= code_of<BITS, TYPE>(raw_to_f32(raw[r], i), s, rcp) << (BITS * r);
+            for (int i = 0; i < 8; ++i) out[i] += code_in_float<BITS, TYPE>(raw_to_f32(raw[r], i), s, rcp) << (BITS * r);
         }
 #pragma unroll
         for (uint32_t i = 0; i < 8; ++i) tile[(8u * kq + i) * kTilePitch + ng] = (out[i] & finite) | (kCode0 & ~finite);
     }
     __syncthreads();
     // 16 lanes x 8 bytes = one row's line
-    const uint32_t row_bytes = p.n * BITS / 8u, col = blockIdx.x * kTileBytes + 8u * kq;
+    const uint32_t row_bytes = p.n * BITS / 8u, col = tile_n * kTileBytes + 8u * kq;
     if (col >= row_bytes) return;
 #pragma unroll
     for (uint32_t i = 0; i < 4; ++i) {
-        const uint32_t kr = 32u * i + ng, row = blockIdx.y * kTileK + kr;
+        const uint32_t kr = 32u * i + ng, row = tile_k * kTileK + kr;
         if (row >= p.k) break;
         const uint32_t* src = tile + kr * kTilePitch + 2u * kq;
         *reinterpret_cast<uint2*>(p.b + (size_t)row * p.ldb_bytes + col) = make_uint2(src[0], src[1]);
@@ -207,7 +220,7 @@ template <int BITS, int TYPE>
 hipError_t launch_quantize_t(const QuantizeParams& p, hipStream_t stream)
 {
     constexpr uint32_t kCols = 32u * (32u / BITS);
-    const dim3 grid((p.n + kCols - 1u) / kCols, (p.k + kTileK - 1u) / kTileK, 1);
+    const dim3 grid(((p.k + kTileK - 1u) / kTileK) * ((p.n + kCols - 1u) / kCols), 1, 1);
     // groups of 32, 64 or 128 lie within one tile, and within one row of 16 lanes
     if (p.group_size == 32u || p.group_size == 64u || p.group_size == 128u)
         return launch_kernel(bfaintb_quantize_kernel<BITS, TYPE, true>, grid, dim3(512, 1, 1), 0, stream, p);
