@@ -36,9 +36,10 @@ def test_launch_shapes_of_the_whole_machine_match_oracle(m, n, k, bits, group, w
     assert np.array_equal(run_gemm(problem), c)
 
 
-@pytest.mark.parametrize("m,n,k,group,packed", [(5, 144, 512, 32, False), (16, 272, 640, 128, False), (9, 144, 512, 64, True), (32, 272, 1024, 128, False)])
+@pytest.mark.parametrize("m,n,k,group,packed", [(5, 144, 512, 32, False), (16, 272, 640, 128, False), (9, 144, 512, 64, True), (32, 272, 1024, 128, False),
+                                                  (2, 144, 512, 128, True), (5, 272, 640, 0, True)])
 def test_scales_of_any_sign_and_size(m, n, k, group, packed):
-    """4-bit codes with grouped scales: the conversion's two terms, (1024 + code) s and (1024 + 8) s, are exact whatever the scale:
+    """4-bit codes by halves (the family with grouped scales, the slab kernel with a scale for each chunk): the conversion's two terms, (1024 + code) s and (1024 + 8) s, are exact whatever the scale:
     negative, zero, subnormal, large."""
     import torch
     import awesome_fusion_amd as af
