@@ -855,14 +855,21 @@ static hipError_t launch_prefill128_wreg_rows(const GemmParams& p, hipStream_t s
     // the copying wave, and the fewer stages that its wait counts reach, over packed weights with grouped scales or 4-bit codes (us,
     // without / with: 128 x 20480 x 4096 4-bit g128 35.1 / 31.7, 64 rows 28.1 / 24.9; 8-bit g64 35.6 / 34.7 and 28.0 / 26.2; 4-bit, one scale
     // per column, 33.5 / 31.6 and 23.6 / 22.9; not 8-bit, one scale per column: 34.6 / 36.4 and 25.3 / 26.1, nor codes in rows: 38.7 / 39.2)
-    if constexpr (PACKED && (GROUPED || BITS == 4)) {
-        switch (p.tile_blocks) {
-            case 4: return launch_prefill128_wreg_t<BITS, GROUPED, PACKED, 4, 6, true>(p, stream);
-            case 6: return launch_prefill128_wreg_t<BITS, GROUPED, PACKED, 6, 4, true>(p, stream);
-            case 8: return launch_prefill128_wreg_t<BITS, GROUPED, PACKED, 8, 4, true>(p, stream);
-            default: break;
+    // Codes in rows with grouped scales: where several rows of tiles split k into shares of up to 64 steps (without / with: 785 x 1440 x 4480
+    // 8-bit 26.3 / 25.0, 4-bit 26.7 / 25.5; 400 x 2560 x 2560 19.9 / 18.8 and 20.3 / 19.2; 900 x 2048 x 8192 44.4 / 42.5 and 43.3 / 42.1; longer
+    // shares lose what the start gains, 384 x 4096 x 11008 52.6 / 54.5 and 50.7 / 53.9, and so do unsplit ones, 640 x 4096 x 4096 8-bit 34.2 /
+    // 35.9, and one row of tiles, 128 x 11008 x 4096 8-bit 26.7 / 28.5).
+    constexpr bool kCopierOnly = PACKED && (GROUPED || BITS == 4), kCopierToo = !PACKED && GROUPED;
+    if (kCopierOnly || (kCopierToo && p.splits > 1u && p.m > 256u && p.k_per_wg <= 64u * kTwK)) {
+        if constexpr (kCopierOnly || kCopierToo) {
+            switch (p.tile_blocks) {
+                case 4: return launch_prefill128_wreg_t<BITS, GROUPED, PACKED, 4, 6, true>(p, stream);
+                case 6: return launch_prefill128_wreg_t<BITS, GROUPED, PACKED, 6, 4, true>(p, stream);
+                case 8: return launch_prefill128_wreg_t<BITS, GROUPED, PACKED, 8, 4, true>(p, stream);
+                default: break;
+            }
         }
-    } else {
+    } else if constexpr (!kCopierOnly) {
         switch (p.tile_blocks) {
             case 4: return launch_prefill128_wreg_t<BITS, GROUPED, PACKED, 4, 8>(p, stream);
             case 6: return launch_prefill128_wreg_t<BITS, GROUPED, PACKED, 6, 6>(p, stream);

@@ -136,3 +136,14 @@ def test_the_familys_four_splits_by_name(m, n, k, group):
     import awesome_fusion_amd as af
     p = Problem(m, n, k, 4, group, seed=m + k)
     assert_close_ulp(p, run_gemm(p, which=af.DECODE), f"{m}x{n}x{k} g={group}")
+
+
+# more than two rows of tiles with grouped scales over codes in rows, k split: the copying wave there too (up to 64 steps a share)
+@pytest.mark.parametrize("bits,group", [(8, 64), (8, 32), (4, 128), (4, 32)])
+@pytest.mark.parametrize("m,n,k,splits", [(257, 272, 1152, 2), (300, 144, 640, 3), (520, 128, 8448, 2)])
+def test_split_tiles_of_several_rows(m, n, k, splits, bits, group):
+    p = Problem(m, n, k, bits, group, seed=m + n + bits)
+    import awesome_fusion_amd as af
+    c = run_gemm(p, which=af.PREFILL_128, force_split_k=splits)
+    assert_close_ulp(p, c, f"{m}x{n}x{k} bits={bits} g={group} splits={splits}")
+    assert np.array_equal(run_gemm(p, which=af.PREFILL_128, force_split_k=splits), c), "not reproducible"
