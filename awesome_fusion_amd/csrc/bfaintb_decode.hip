@@ -50,10 +50,7 @@ __device__ __forceinline__ float value_f32(const uint32_t (&row)[PD])
 
 // How a kernel makes its weights.  Two ways, to the same bits:
 //   - the code as an fp32 number by a conversion that reads it where it lies, times the scale, rounded by the pack;
-//   - HALVES: the code goes into the low bits of a half-precision 1024 (1024 + c, exact), two at a time, and one fused operation that
-//     reads a half-precision operand does the rest, (1024 + c) s - (1024 + excess) s, exact in fp32 (bfaintb_prefill128_wreg.hip has the
-//     argument).  4-bit codes also at four bits up, (1024 + 16 c) (s / 16) - (64 + excess) s, where there are registers for two
-//     multipliers more (128 columns).  17 instructions for 8 weights instead of 22.
+//   - HALVES: the conversion by halves (bfaintb_device.hpp has the argument), 17 instructions for 8 weights instead of 22.
 // HALVES is what 4-bit codes with grouped scales do: those kernels are bound by the instructions they issue (us, before / with it, groups of
 // 128: 28672 x 8192 packed, 8 and 16 rows 31.1 / 28.8 and 31.4 / 29.1; in rows 30.8 / 29.8; 22016 x 4096, 16 rows, 19.4 / 18.4 either order).
 // 8-bit codes, which wait for memory, gain nothing (28672 x 8192 packed g128, 8 rows, 44.2 / 45.6); with one scale per column the compiler
@@ -61,51 +58,17 @@ __device__ __forceinline__ float value_f32(const uint32_t (&row)[PD])
 // over packed codes (22016 x 4096, 32 rows, 23.4 / 26.3).
 __host__ __device__ constexpr bool decode_by_halves(int bits, bool grouped, bool packed, int mb) { return bits == 4 && grouped && !(packed && mb >= 2); }
 
-template <int BITS, int CPL, bool HALVES>
+// (256 columns: no registers for two multipliers more)
+__host__ __device__ constexpr int half_upper(int cpl) { return cpl == 8 ? 1024 : 0; }
+
+template <int CPL, bool HALVES>
 struct Multipliers {
-    static constexpr bool kUpper = HALVES && CPL == 8;
     float s[CPL];  // the scale (the conversion of 4-bit codes divides by 16: 16 times the scale)
-    float o[HALVES ? CPL : 1];
-    float s4[kUpper ? CPL : 1], o4[kUpper ? CPL : 1];
 };
-
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-
-// Constants of the conversion by halves, kept in registers, one of each instruction's in a scalar one: as literals they cost an
-// instruction more.
-struct HalfConstants {
-    uint32_t low, up, one_k;
+template <int CPL>
+struct Multipliers<CPL, true> {
+    HalfMultipliers<4, half_upper(CPL)> h[CPL];
 };
-template <bool HALVES>
-__device__ __forceinline__ HalfConstants half_constants()
-{
-    HalfConstants k{0x000f000fu, 0x00f000f0u, 0x64006400u};
-    if constexpr (HALVES) {
-        asm("" : "+s"(k.low), "+s"(k.up));
-        asm("" : "+v"(k.one_k));
-    }
-    return k;
-}
-
-// Eight 4-bit codes as halves of 1024 + code: codes i and i + 4 in out[i] (UPPER: of i = 1 and 3 four bits up)
-template <bool UPPER>
-__device__ __forceinline__ void codes4_to_halves(uint32_t* out, uint32_t x, const HalfConstants& k)
-{
-    const uint32_t y = x >> 8;
-    out[0] = (x & k.low) | k.one_k;
-    out[1] = UPPER ? (x & k.up) | k.one_k : ((x >> 4) & k.low) | k.one_k;
-    out[2] = (y & k.low) | k.one_k;
-    out[3] = UPPER ? (y & k.up) | k.one_k : ((x >> 12) & k.low) | k.one_k;
-}
-
-// Code I's weight of column c
-template <int CPL, int I>
-__device__ __forceinline__ float weight_of(const uint32_t* halves, const Multipliers<4, CPL, true>& mu, int c)
-{
-    const float v = (float)__builtin_bit_cast(half2_t, halves[I & 3])[I >> 2];
-    if constexpr (Multipliers<4, CPL, true>::kUpper && (I & 1)) return __builtin_fmaf(v, mu.s4[c], mu.o4[c]);
-    else return __builtin_fmaf(v, mu.s[c], mu.o[c]);
-}
 
 // Non-temporal loads: the weights are read once, and marked so they stream through the caches without displacing the
 // activations, the scales, the workspace and the kernel's own code (measured on the fetch alone: 16 MiB in 3.9 us
@@ -162,13 +125,14 @@ __device__ __forceinline__ void mac_column(const uint32_t (&rows)[8][CPL / 4], c
 
 // The same by halves, rows[r]: row r's codes as such; columns in the order in which a dword's halves hold them, 0, 4, 1, 5, ...
 template <int CPL, int MB, int I>
-__device__ __forceinline__ void mac_column_halves(const uint32_t (&rows)[8][CPL / 2], const Multipliers<4, CPL, true>& mu, const uint4 (&afrag)[MB],
+__device__ __forceinline__ void mac_column_halves(const uint32_t (&rows)[8][CPL / 2], const Multipliers<CPL, true>& mu, const uint4 (&afrag)[MB],
                                                   f32x4_t (&acc)[MB][CPL])
 {
     constexpr int kCode = (I & 1) * 4 + (I >> 1 & 3), kDword = I / 8, kC = 8 * kDword + kCode;
     float v[8];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) v[r] = weight_of<CPL, kCode>(rows[r] + 4 * kDword, mu, kC);
+    for (int r = 0; r < 8; ++r)
+        v[r] = weight_of_half<kCode & 3>(rows[r][4 * kDword + (kCode & 3)], kCode >> 2, mu.h[kC]);
     const uint4 w = make_uint4(pack_bf16_rne(v[0], v[1]), pack_bf16_rne(v[2], v[3]), pack_bf16_rne(v[4], v[5]), pack_bf16_rne(v[6], v[7]));
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
@@ -176,22 +140,26 @@ __device__ __forceinline__ void mac_column_halves(const uint32_t (&rows)[8][CPL 
 }
 
 template <int BITS, int CPL, int MB, bool REF, bool HALVES, int... Cs>
-__device__ __forceinline__ void mac_step(const RawStep<BITS, CPL>& raw, const Multipliers<BITS, CPL, HALVES>& mu, const HalfConstants& k, const uint4 (&afrag)[MB],
-                                         f32x4_t (&acc)[MB][CPL], std::integer_sequence<int, Cs...>)
+__device__ __forceinline__ void mac_step(const RawStep<BITS, CPL>& raw, const Multipliers<CPL, HALVES>& mu, const HalfConstants<4, half_upper(CPL)>& k,
+                                         const uint4 (&afrag)[MB], f32x4_t (&acc)[MB][CPL], std::integer_sequence<int, Cs...>)
 {
     if constexpr (HALVES) {
-        uint32_t halves[8][CPL / 2];
+        uint32_t hv[8][CPL / 2];
 #pragma unroll
         for (int r = 0; r < 8; ++r)
 #pragma unroll
-            for (int i = 0; i < CPL / 8; ++i) codes4_to_halves<Multipliers<BITS, CPL, true>::kUpper>(halves[r] + 4 * i, raw.d[r][i], k);
-        (mac_column_halves<CPL, MB, Cs>(halves, mu, afrag, acc), ...);
-        return;
-    }
-    uint32_t rows[8][CPL / 4];
+            for (int i = 0; i < CPL / 8; ++i) {
+                const uint32_t x = raw.d[r][i];
+                hv[r][4 * i] = halves<0>(x, k), hv[r][4 * i + 1] = halves<1>(x, k);
+                hv[r][4 * i + 2] = halves<2>(x, k), hv[r][4 * i + 3] = halves<3>(x, k);
+            }
+        (mac_column_halves<CPL, MB, Cs>(hv, mu, afrag, acc), ...);
+    } else {
+        uint32_t rows[8][CPL / 4];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) prepare_row<BITS, CPL>(rows[r], raw.d[r]);
-    (mac_column<BITS, CPL, MB, REF, Cs>(rows, mu.s, afrag, acc), ...);
+        for (int r = 0; r < 8; ++r) prepare_row<BITS, CPL>(rows[r], raw.d[r]);
+        (mac_column<BITS, CPL, MB, REF, Cs>(rows, mu.s, afrag, acc), ...);
+    }
 }
 
 // ---- the same step over weights in the packed order (bfaintb_packed.hip): the workgroup's CPL column blocks of 16 take
@@ -252,34 +220,15 @@ __device__ __forceinline__ void load_packed_chunk4(PackedStep<4, CPL> (&blocks)[
 }
 
 template <int BITS, int CPL, int MB, bool HALVES>
-__device__ __forceinline__ void mac_step_packed(const PackedStep<BITS, CPL>& raw, const Multipliers<BITS, CPL, HALVES>& mu, const HalfConstants& k,
+__device__ __forceinline__ void mac_step_packed(const PackedStep<BITS, CPL>& raw, const Multipliers<CPL, HALVES>& mu, const HalfConstants<4, half_upper(CPL)>& k,
                                                 const uint4 (&afrag)[MB], f32x4_t (&acc)[MB][CPL])
 {
 #pragma unroll
     for (int c = 0; c < CPL; ++c) {
-        const float s = mu.s[c];
         uint4 w;
-        if constexpr (HALVES) {
-            uint32_t h[4];
-            codes4_to_halves<Multipliers<BITS, CPL, true>::kUpper>(h, raw.d[c][0], k);
-            w.x = pack_bf16_rne(weight_of<CPL, 0>(h, mu, c), weight_of<CPL, 1>(h, mu, c));
-            w.y = pack_bf16_rne(weight_of<CPL, 2>(h, mu, c), weight_of<CPL, 3>(h, mu, c));
-            w.z = pack_bf16_rne(weight_of<CPL, 4>(h, mu, c), weight_of<CPL, 5>(h, mu, c));
-            w.w = pack_bf16_rne(weight_of<CPL, 6>(h, mu, c), weight_of<CPL, 7>(h, mu, c));
-        } else if constexpr (BITS == 8) {
-            const uint32_t lo = codes8_to_s8(raw.d[c][0]), hi = codes8_to_s8(raw.d[c][1]);
-            w.x = pack_bf16_rne(sbyte_to_f32<0>(lo) * s, sbyte_to_f32<1>(lo) * s);
-            w.y = pack_bf16_rne(sbyte_to_f32<2>(lo) * s, sbyte_to_f32<3>(lo) * s);
-            w.z = pack_bf16_rne(sbyte_to_f32<0>(hi) * s, sbyte_to_f32<1>(hi) * s);
-            w.w = pack_bf16_rne(sbyte_to_f32<2>(hi) * s, sbyte_to_f32<3>(hi) * s);
-        } else {
-            uint32_t ev, od;
-            codes4_to_nibbles(raw.d[c][0], ev, od);
-            w.x = pack_bf16_rne(nibble_to_f32_sixteenth<0>(ev) * s, nibble_to_f32_sixteenth<0>(od) * s);
-            w.y = pack_bf16_rne(nibble_to_f32_sixteenth<1>(ev) * s, nibble_to_f32_sixteenth<1>(od) * s);
-            w.z = pack_bf16_rne(nibble_to_f32_sixteenth<2>(ev) * s, nibble_to_f32_sixteenth<2>(od) * s);
-            w.w = pack_bf16_rne(nibble_to_f32_sixteenth<3>(ev) * s, nibble_to_f32_sixteenth<3>(od) * s);
-        }
+        if constexpr (HALVES) w = weights4_by_halves(raw.d[c][0], k, mu.h[c]);
+        else if constexpr (BITS == 8) w = weights8(raw.d[c][0], raw.d[c][1], mu.s[c]);
+        else w = weights4(raw.d[c][0], mu.s[c]);
         const bf16x8_t wf = __builtin_bit_cast(bf16x8_t, w);
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
@@ -308,28 +257,23 @@ __device__ __forceinline__ void load_scales(uint4 (&sraw)[CPL / 8], const uint16
     for (int i = 0; i < CPL / 8; ++i) sraw[i] = *reinterpret_cast<const uint4*>(src + 16 * i);
 }
 
+// most: the largest magnitude among the lane's scales (by halves)
 template <int BITS, int CPL, bool HALVES>
-__device__ __forceinline__ void apply_scales(Multipliers<BITS, CPL, HALVES>& mu, const uint4 (&sraw)[CPL / 8])
+__device__ __forceinline__ void apply_scales(Multipliers<CPL, HALVES>& mu, float& most, const uint4 (&sraw)[CPL / 8])
 {
     uint32_t d[CPL / 2];
 #pragma unroll
     for (int i = 0; i < CPL / 8; ++i) {
         d[4 * i] = sraw[i].x; d[4 * i + 1] = sraw[i].y; d[4 * i + 2] = sraw[i].z; d[4 * i + 3] = sraw[i].w;
     }
-#pragma unroll
-    for (int i = 0; i < CPL / 2; ++i) {
-        mu.s[2 * i] = HALVES ? bf16_bits_to_f32(d[i] & 0xffffu) : make_col_scale_nibble<BITS>(d[i] & 0xffffu);
-        mu.s[2 * i + 1] = HALVES ? bf16_bits_to_f32(d[i] >> 16) : make_col_scale_nibble<BITS>(d[i] >> 16);
-    }
     if constexpr (HALVES) {
 #pragma unroll
-        for (int c = 0; c < CPL; ++c) {
-            mu.o[c] = -1032.0f * mu.s[c];
-            if constexpr (Multipliers<BITS, CPL, true>::kUpper) {
-                mu.s4[c] = 0.0625f * mu.s[c];
-                mu.o4[c] = -72.0f * mu.s[c];
-            }
-        }
+        for (int c = 0; c < CPL; ++c) mu.h[c] = HalfMultipliers<4, half_upper(CPL)>(bf16_bits_to_f32(c & 1 ? d[c / 2] >> 16 : d[c / 2] & 0xffffu));
+#pragma unroll
+        for (int c = 0; c < CPL; c += 2) largest_scale(most, mu.h[c].s, mu.h[c + 1].s);
+    } else {
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) mu.s[c] = make_col_scale_nibble<BITS>(c & 1 ? d[c / 2] >> 16 : d[c / 2] & 0xffffu);
     }
 }
 
@@ -633,6 +577,8 @@ bfaintb_decode_kernel(const GemmParams p)
 #pragma unroll
         for (int c = 0; c < CPL; ++c) acc[mb][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
+    constexpr bool kHalves = decode_by_halves(BITS, GROUPED, PACKED, MB);
+    float most = 0.f;
     if (nsteps > 0 || tail_rows != 0u) {
         // Two register stages, used alternately: the loads of step s+1 are issued before step s is
         // computed.  A step is KB blocks of 32 rows, so that a lane has 128 bytes of B in flight per
@@ -645,9 +591,9 @@ bfaintb_decode_kernel(const GemmParams p)
             uint4 af[KB][MB];
             uint4 sraw[KB][CPL / 8];
         };
-        constexpr bool kHalves = decode_by_halves(BITS, GROUPED, PACKED, MB);
-        Multipliers<BITS, CPL, kHalves> mu;
-        const HalfConstants half_k = half_constants<kHalves>();
+        Multipliers<CPL, kHalves> mu;
+        HalfConstants<4, half_upper(CPL)> half_k;
+        if constexpr (kHalves) half_k.keep();
         const uint16_t* sptr = p.scale;
         // packed weights with grouped scales: the wave's transposition table in LDS, behind the reduction area, and
         // the columns whose scales this lane fetches (kept inside the scale row)
@@ -749,9 +695,9 @@ bfaintb_decode_kernel(const GemmParams p)
                             uint4 mine[CPL / 8];
 #pragma unroll
                             for (int i = 0; i < CPL / 8; ++i) mine[i] = *reinterpret_cast<const uint4*>(sc_table + (uint32_t)nl * CPL + 8u * i);
-                            apply_scales<BITS, CPL, kHalves>(mu, mine);
+                            apply_scales<BITS, CPL, kHalves>(mu, most, mine);
                         } else {
-                            apply_scales<BITS, CPL, kHalves>(mu, st.sraw[q]);
+                            apply_scales<BITS, CPL, kHalves>(mu, most, st.sraw[q]);
                         }
                         blocks_to_group = next_group_blocks;
                         next_group_blocks = p.group_size / 32u;
@@ -779,7 +725,7 @@ bfaintb_decode_kernel(const GemmParams p)
             Stage s0, s1;
             request_scales(s0);
             load_stage(s0, 0);
-            if constexpr (!GROUPED && !REF) apply_scales<BITS, CPL, kHalves>(mu, s0.sraw[0]);
+            if constexpr (!GROUPED && !REF) apply_scales<BITS, CPL, kHalves>(mu, most, s0.sraw[0]);
             int s = 0;
             for (; s + 2 < nsteps; s += 2) {
                 load_stage(s1, s + 1);
@@ -802,7 +748,7 @@ bfaintb_decode_kernel(const GemmParams p)
                 Stage st;
                 if (nsteps == 0) {
                     request_scales(st);
-                    if constexpr (!REF) apply_scales<BITS, CPL, kHalves>(mu, st.sraw[0]);
+                    if constexpr (!REF) apply_scales<BITS, CPL, kHalves>(mu, most, st.sraw[0]);
                 }
                 const uint32_t krow = kb + 32u * (uint32_t)nsteps + 8u * (uint32_t)kg;
                 const bool live = krow < p.k;
@@ -813,6 +759,46 @@ bfaintb_decode_kernel(const GemmParams p)
                     if (live) st.af[0][mb] = *reinterpret_cast<const uint4*>(aptr[mb] + (size_t)nsteps * 32);
                 }
                 compute_stage(st);
+            }
+        }
+    }
+    // A scale beyond the conversion by halves: the wave's sums once more, in the same order, by the other conversion, a block of 32 rows at a time
+    if constexpr (kHalves) {
+        if (__builtin_expect(beyond_halves(most), 0)) {
+            uint32_t again = cb;
+            asm volatile("" : "+s"(again)::"memory");  // (nothing of the walk above is kept in registers for this one)
+#pragma unroll
+            for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                for (int c = 0; c < CPL; ++c) acc[mb][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (uint32_t blk = 0; blk < (uint32_t)(nsteps * KB); ++blk) {
+                std::conditional_t<PACKED, PackedStep<BITS, CPL>, RawStep<BITS, CPL>> raw;
+                uint4 af[MB], sraw[CPL / 8];
+                const uint16_t* srow = p.scale + (size_t)group_of_row(p, kb + 32u * blk) * p.lds;
+                if constexpr (PACKED) {
+                    const uint8_t* slabs[CPL];
+                    uint32_t cols[CPL];
+#pragma unroll
+                    for (int c = 0; c < CPL; ++c) {
+                        uint32_t gb = again * CPL + (uint32_t)c;
+                        if (gb >= p.n / 16u) gb = p.n / 16u - 1u;
+                        slabs[c] = p.b + (size_t)gb * p.k * 8u;
+                        cols[c] = 16u * gb + (uint32_t)nl;
+                    }
+                    load_packed<BITS, CPL>(raw, slabs, (uint32_t)lane * 16u + (kblock0 + blk) / kBlocksPerChunk * 1024u + (kblock0 + blk) % kBlocksPerChunk * kBlockBytes);
+                    load_scales_packed<CPL>(sraw, srow, cols);
+                } else {
+                    load_raw<BITS, CPL>(raw, bptr + blk * bstep, b_lane, p.ldb_bytes);
+                    load_scales<CPL>(sraw, srow, n_ld);
+                }
+#pragma unroll
+                for (int mb = 0; mb < MB; ++mb) af[mb] = *reinterpret_cast<const uint4*>(aptr[mb] + (size_t)blk * 32);
+                Multipliers<CPL, false> mu;
+                float unused = 0.f;
+                apply_scales<BITS, CPL, false>(mu, unused, sraw);
+                if constexpr (PACKED) mac_step_packed<BITS, CPL, MB, false>(raw, mu, {}, af, acc);
+                else mac_step<BITS, CPL, MB, REF, false>(raw, mu, {}, af, acc, std::make_integer_sequence<int, CPL>{});
             }
         }
     }

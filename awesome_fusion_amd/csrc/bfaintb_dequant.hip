@@ -1,5 +1,6 @@
-// Dequantised-weight dump: W[k,n] = bf16(float(q) * float(scale)) written to memory, through the
-// same device routines (codes*_to_s8*, sbyte_to_f32, make_col_scale, pack_bf16_rne) the GEMM kernels use.
+// Dequantised-weight dump: W[k,n] = bf16(float(q) * float(scale)) written to memory, through the device routines of the
+// conversion (codes*_to_s8*, sbyte_to_f32, make_col_scale, pack_bf16_rne).  The GEMM kernels that make their weights by halves
+// (bfaintb_device.hpp) come to the same weights but for the sign of a zero; products with one-hot rows hold them against this dump.
 // Successor of the reference's ASM_PRINT channel (/root/reference/bfAintBGemm/bfAintBGemm.cc:113-118,
 // 156-169; bf16gemm_kernel_gfx90a.s:2-16): the way to look at in-kernel dequantised values.
 #include "bfaintb_device.hpp"

@@ -290,6 +290,107 @@ __device__ __forceinline__ float make_col_scale(uint32_t scale_bf16_bits)
     return BITS == 8 ? s : s * 0.0625f;
 }
 
+// Eight weights of a column, rows 0 .. 7, as the 8-element operand of the matrix instruction: codes as fp32 by a conversion that reads
+// the signed byte where it lies, times the scale, rounded by the pack.  lo, hi: rows 0 .. 3 and 4 .. 7 of 8-bit codes, as stored.
+__device__ __forceinline__ uint4 weights8(uint32_t lo, uint32_t hi, float s)
+{
+    lo = codes8_to_s8(lo), hi = codes8_to_s8(hi);
+    return make_uint4(pack_bf16_rne(sbyte_to_f32<0>(lo) * s, sbyte_to_f32<1>(lo) * s), pack_bf16_rne(sbyte_to_f32<2>(lo) * s, sbyte_to_f32<3>(lo) * s),
+                      pack_bf16_rne(sbyte_to_f32<0>(hi) * s, sbyte_to_f32<1>(hi) * s), pack_bf16_rne(sbyte_to_f32<2>(hi) * s, sbyte_to_f32<3>(hi) * s));
+}
+
+// The same for a dword of 4-bit codes, row i in nibble i (s16: 16 times the scale)
+__device__ __forceinline__ uint4 weights4(uint32_t x, float s16)
+{
+    uint32_t ev, od;
+    codes4_to_nibbles(x, ev, od);
+    return make_uint4(pack_bf16_rne(nibble_to_f32_sixteenth<0>(ev) * s16, nibble_to_f32_sixteenth<0>(od) * s16),
+                      pack_bf16_rne(nibble_to_f32_sixteenth<1>(ev) * s16, nibble_to_f32_sixteenth<1>(od) * s16),
+                      pack_bf16_rne(nibble_to_f32_sixteenth<2>(ev) * s16, nibble_to_f32_sixteenth<2>(od) * s16),
+                      pack_bf16_rne(nibble_to_f32_sixteenth<3>(ev) * s16, nibble_to_f32_sixteenth<3>(od) * s16));
+}
+
+// ---- The conversion by halves.  A code goes into the low bits of a half-precision 1024 (1024 + c, exact: 0x6400 | c), two at a time, and
+// one fused operation that reads a half-precision operand does the rest: (1024 + c) s - (1024 + excess) s.  Both products and their
+// difference (c - excess) s are exact in fp32 (11 x 8, 8 x 8 and 8 x 8 significant bits), so it is the product q s of the signed code, bit
+// for bit, and is rounded once, to bf16, by the pack that follows (a zero code gives +0 where q s gives -0 for a negative scale: no sum can
+// tell).  4-bit codes also at four bits up: (1024 + 16 c) (s / 16) - (64 + excess) s.
+// Instructions for eight weights, pack included: 16 (8-bit) and 17 (4-bit), where a conversion, a multiplication and the pack take 20 to 28.
+//
+// The second product has to be finite, and the format allows scales up to 2^120.  Two ways, each where it is the faster one:
+//   - (tiles, decode family) a wave keeps the largest magnitude among the scales that its lanes have used, half an instruction a scale, and
+//     walks its k a second time with the conversion above if it finds one from kHalvesLimit on at the end: never with quantised weights;
+//   - (slab kernel) 4-bit codes four bits up in halves of 64, 64 + c, all of them: 72 s is finite below 2^121, and two more shifts for eight
+//     weights cost less than the second walk's code, which a launch of a few microseconds notices.
+// What that costs, the time without any care for such scales being 1: 28672 x 8192 packed 4-bit g128, 16 rows (28.9 us), in the family 1.005 by a
+// second walk and 1.04 in halves of 64; 4096 x 4096, 1 row (4.24 us), in the slab kernel 1.23 and 1.01.  A branch to the other conversion in
+// every step spills in the family (48 x 11008 x 4096 4-bit 20.5 / 25.0 us) and costs tiles with group scales 3 to 5 % (577 x 13824 x 5120 packed 4-bit
+// 94.8 / 98.3 us; by a second walk 1.00, and 1.01 for 32 x 22016 x 4096 4-bit at 20.0 us).
+constexpr float kHalvesLimit = 0x1p117f;
+typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void largest_scale(float& most, float s0, float s1) { asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(s0), "v"(s1)); }
+__device__ __forceinline__ bool beyond_halves(float most) { return __builtin_amdgcn_ballot_w64(!(most < kHalvesLimit)) != 0u; }
+
+// UPPER, the odd ones of 4-bit codes: 0, left where the even ones are; 1024, four bits up in halves of 1024; 64, all codes in halves of 64.
+// A scale's multipliers:
+template <int BITS, int UPPER>
+struct HalfMultipliers {
+    float s, o;    // the scale, and what the excess costs
+    float s4, o4;  // (4-bit codes, UPPER = 1024: for codes four bits up)
+    HalfMultipliers() = default;
+    __device__ __forceinline__ explicit HalfMultipliers(float scale)
+    {
+        s = scale;
+        o = (BITS == 8 ? -1152.0f : UPPER == 64 ? -72.0f : -1032.0f) * scale;
+        if constexpr (BITS == 4 && UPPER == 1024) s4 = 0.0625f * scale, o4 = -72.0f * scale;
+    }
+};
+// The conversion's constants, kept in registers, one of each instruction's in a scalar one: as literals they cost an instruction more.
+template <int BITS, int UPPER>
+struct HalfConstants {
+    uint32_t low = BITS == 8 ? 0x00ff00ffu : 0x000f000fu, up = BITS == 8 ? 0x64646464u : 0x00f000f0u;
+    uint32_t one = UPPER == 64 ? 0x54005400u : 0x64006400u, odd_bytes = 0x04030401u;
+    __device__ __forceinline__ void keep()
+    {
+        asm("" : "+s"(low), "+s"(up));
+        asm("" : "+v"(one), "+v"(odd_bytes));
+    }
+};
+// Two codes of a dword as halves: 8-bit, bytes I and I + 2; 4-bit, nibbles I and I + 4
+template <int I, int BITS, int UPPER>
+__device__ __forceinline__ uint32_t halves(uint32_t x, const HalfConstants<BITS, UPPER>& k)
+{
+    if constexpr (BITS == 8) {
+        if constexpr (I == 1) return __builtin_amdgcn_perm(k.up, x, k.odd_bytes);  // bytes {1, 0x64, 3, 0x64}
+        return (x & k.low) | k.one;
+    } else {
+        if constexpr (UPPER == 64 && I == 0) return ((x << 4) & k.up) | k.one;
+        if constexpr (UPPER == 64 || (UPPER == 1024 && (I & 1))) return ((x >> (4 * I - 4)) & k.up) | k.one;
+        return ((x >> (4 * I)) & k.low) | k.one;
+    }
+}
+// The weight of the code in half `part` of halves<I>
+template <int I, int BITS, int UPPER>
+__device__ __forceinline__ float weight_of_half(uint32_t h, uint32_t part, const HalfMultipliers<BITS, UPPER>& mu)
+{
+    const float v = (float)__builtin_bit_cast(half2_t, h)[part];
+    if constexpr (BITS == 4 && UPPER == 1024 && (I & 1)) return __builtin_fmaf(v, mu.s4, mu.o4);
+    return __builtin_fmaf(v, mu.s, mu.o);
+}
+// weights4 by halves
+template <int UPPER>
+__device__ __forceinline__ uint4 weights4_by_halves(uint32_t x, const HalfConstants<4, UPPER>& k, const HalfMultipliers<4, UPPER>& mu)
+{
+    const uint32_t h0 = halves<0>(x, k), h1 = halves<1>(x, k), h2 = halves<2>(x, k), h3 = halves<3>(x, k);
+    uint32_t w[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i) {
+        w[2 * i] = pack_bf16_rne(weight_of_half<0>(h0, i, mu), weight_of_half<1>(h1, i, mu));
+        w[2 * i + 1] = pack_bf16_rne(weight_of_half<2>(h2, i, mu), weight_of_half<3>(h3, i, mu));
+    }
+    return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
 // A workgroup barrier without the memory fence that __syncthreads() carries.  That fence makes the compiler wait, before
 // the barrier, for EVERY asynchronous global -> LDS copy issued so far — also the ones meant to land steps later — which
 // turns a pipeline of several stages into one of a single stage.  The caller states what must have completed with

@@ -270,13 +270,9 @@ __device__ __forceinline__ void decode_packed_body(const GemmParams& p)
     // per column, 4096 x 11008 10.03 / 9.53, 28672 x 8192 31.4 / 29.8; groups of 128, 4096 x 4096 4.55 / 4.27; groups of 64, 8 rows, 4096 x
     // 4096 5.13 / 5.33).
     constexpr bool kHalves = BITS == 4 && SCALES != kScalePerBlock;
-    if constexpr (!GROUPED) cs = kHalves ? bf16_bits_to_f32(*sptr) : make_col_scale<BITS>(*sptr);
-    typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-    uint32_t low = 0x000f000fu, up = 0x00f000f0u, one_k = 0x64006400u;  // (in registers: as literals they cost an instruction more)
-    if constexpr (kHalves) {
-        asm("" : "+s"(low), "+s"(up));
-        asm("" : "+v"(one_k));
-    }
+    if constexpr (!GROUPED) cs = bf16_bits_to_f32(*sptr);
+    HalfConstants<4, 64> half_k;
+    if constexpr (kHalves) half_k.keep();
 
     f32x4_t acc[MB];
 #pragma unroll
@@ -323,24 +319,9 @@ __device__ __forceinline__ void decode_packed_body(const GemmParams& p)
                     }
                     uint4 w;
                     if constexpr (BITS == 8) {
-                        const uint32_t lo = codes8_to_s8(wd[2 * h]), hi = codes8_to_s8(wd[2 * h + 1]);
-                        w.x = pack_bf16_rne(sbyte_to_f32<0>(lo) * s, sbyte_to_f32<1>(lo) * s);
-                        w.y = pack_bf16_rne(sbyte_to_f32<2>(lo) * s, sbyte_to_f32<3>(lo) * s);
-                        w.z = pack_bf16_rne(sbyte_to_f32<0>(hi) * s, sbyte_to_f32<1>(hi) * s);
-                        w.w = pack_bf16_rne(sbyte_to_f32<2>(hi) * s, sbyte_to_f32<3>(hi) * s);
+                        w = weights8(wd[2 * h], wd[2 * h + 1], s);
                     } else if constexpr (kHalves) {
-                        // rows i and i + 4 as halves of 1024 + code (1 and 3 of them four bits up), and one fused operation for each weight, as
-                        // in bfaintb_decode_kernel
-                        const uint32_t x = wd[h], y = x >> 8;
-                        const uint32_t half[4] = {(x & low) | one_k, (x & up) | one_k, (y & low) | one_k, (y & up) | one_k};
-                        const float o = -1032.0f * s, s4 = 0.0625f * s, o4 = -72.0f * s;
-                        float v[8];
-#pragma unroll
-                        for (int r = 0; r < 8; ++r) {
-                            const float f = (float)__builtin_bit_cast(half2_t, half[r & 3])[r >> 2];
-                            v[r] = r & 1 ? __builtin_fmaf(f, s4, o4) : __builtin_fmaf(f, s, o);
-                        }
-                        w = make_uint4(pack_bf16_rne(v[0], v[1]), pack_bf16_rne(v[2], v[3]), pack_bf16_rne(v[4], v[5]), pack_bf16_rne(v[6], v[7]));
+                        w = weights4_by_halves(wd[h], half_k, HalfMultipliers<4, 64>(s));
                     } else {
                         // nibble r of the dword is row r: even rows from the low nibbles, odd rows from the high ones
                         uint32_t ev, od;

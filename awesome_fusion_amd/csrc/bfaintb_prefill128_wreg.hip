@@ -316,58 +316,37 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
         return;           // (a wave that has ended no longer counts at the barriers that follow)
     }
 
-    // ---- Conversion.  A code c goes into the low bits of a half-precision 1024 (1024 + c, exact: 0x6400 | c), two at a time, and one
-    // fused operation that reads a half-precision operand does the rest: (1024 + c) s - (1024 + excess) s.  Both products and their
-    // difference (c - excess) s are exact in fp32 (11 x 8, 8 x 8 and 8 x 8 significant bits), so it is the product q s of the signed
-    // code, bit for bit, and is rounded once, to bf16, by the pack that follows (a zero code gives +0 where q s gives -0 for a negative
-    // scale: no sum can tell; an infinite scale, or one beyond 2^117, gives NaN where q s would be infinite or, up to 2^120,
-    // finite).  4-bit codes also at four bits up: (1024 + 16 c) (s / 16) - (64 + excess) s.
-    // 4 (8-bit) and 4.25 (4-bit) instructions for two weights, where a conversion, a multiplication and the pack take 5 to 7: the step
-    // is bound by the instructions a SIMD issues, some 4 cycles each beside its matrix instructions.
+    // ---- Conversion by halves (bfaintb_device.hpp has the argument): 4 (8-bit) and 4.25 (4-bit) instructions for two weights, where a
+    // conversion, a multiplication and the pack take 5 to 7; the step is bound by the instructions a SIMD issues, some 4 cycles each
+    // beside its matrix instructions.
     struct Multipliers {
-        float s[2], o[2];    // scale, and what the excess costs
-        float s4[2], o4[2];  // the same for codes four bits up
+        HalfMultipliers<BITS, 1024> h[2];
     };
+    float most = 0.f;  // the largest magnitude among the lane's scales
     auto multipliers = [&](Multipliers& mu, const Scales& sr) {
 #pragma unroll
         for (uint32_t j = 0; j < 2; ++j) {
             uint32_t bits = sr.s[j];
             asm volatile("" : "+v"(bits));  // (or the widening moves up to the load, a step's wait with it)
-            mu.s[j] = bf16_bits_to_f32(bits);
-            if constexpr (BITS == 8) {
-                mu.o[j] = -1152.0f * mu.s[j];
-            } else {
-                mu.o[j] = -1032.0f * mu.s[j];
-                mu.s4[j] = 0.0625f * mu.s[j];
-                mu.o4[j] = -72.0f * mu.s[j];
-            }
+            mu.h[j] = HalfMultipliers<BITS, 1024>(bf16_bits_to_f32(bits));
         }
+        largest_scale(most, mu.h[0].s, mu.h[1].s);
     };
-    typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-    // (constants kept in registers, one of each instruction's in a scalar one: as literals they cost an instruction more)
-    uint32_t mask_low = BITS == 8 ? 0x00ff00ffu : 0x000f000fu, mask_up = BITS == 8 ? 0x64646464u : 0x00f000f0u;
-    uint32_t one_k = 0x64006400u, odd_bytes = 0x04030401u;
-    asm("" : "+s"(mask_low), "+s"(mask_up));
-    asm("" : "+v"(one_k), "+v"(odd_bytes));
+    HalfConstants<BITS, 1024> half_k;
+    half_k.keep();
     struct Halves {
         uint32_t e[2], d[2];  // 8-bit: rows 0 and 2 (+ 4 h), rows 1 and 3 [h]; 4-bit: [0]: rows 0 and 4, 1 and 5; [1]: 2 and 6, 3 and 7
     };
     // what pairs 2 h and 2 h + 1 (8-bit), or h and h + 2 (4-bit), need
     auto extract = [&](Halves& hv, const uint32_t (&c)[BITS / 4], uint32_t h) {
-        if constexpr (BITS == 8) {
-            hv.e[h] = (c[h] & mask_low) | one_k;
-            hv.d[h] = __builtin_amdgcn_perm(mask_up, c[h], odd_bytes);  // bytes {1, 0x64, 3, 0x64}
-        } else {
-            const uint32_t x = h == 0 ? c[0] : c[0] >> 8;
-            hv.e[h] = (x & mask_low) | one_k;
-            hv.d[h] = (x & mask_up) | one_k;
-        }
+        const uint32_t x = BITS == 8 ? c[h] : h == 0 ? c[0] : c[0] >> 8;
+        hv.e[h] = halves<0>(x, half_k);
+        hv.d[h] = halves<1>(x, half_k);
     };
     // rows 2 pr and 2 pr + 1 of column j, times its scale
     auto weight = [&](const Halves& hv, const Multipliers& mu, uint32_t j, uint32_t pr, bool odd) -> float {
         const uint32_t h = BITS == 8 ? pr >> 1 : pr & 1u, part = BITS == 8 ? pr & 1u : pr >> 1;
-        const float v = (float)__builtin_bit_cast(half2_t, odd ? hv.d[h] : hv.e[h])[part];
-        return BITS == 4 && odd ? __builtin_fmaf(v, mu.s4[j], mu.o4[j]) : __builtin_fmaf(v, mu.s[j], mu.o[j]);
+        return odd ? weight_of_half<1>(hv.d[h], part, mu.h[j]) : weight_of_half<0>(hv.e[h], part, mu.h[j]);
     };
     struct Ops {
         uint32_t w[2][4];  // [column j][dword]: the 8-element operand as 4 packed pairs
@@ -545,8 +524,53 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
     };
     run_rest(C0{}), run_rest(C1{}), run_rest(C2{}), run_rest(C3{}), run_rest(C4{}), run_rest(C5{}), run_rest(C6{});
 
-    // ---- epilogue: fp32 sums -> LDS in [m][n] order (a quarter of a stage's rows in each array), then finish row-wise
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing asynchronous may still be writing LDS
+    // ---- a scale beyond the conversion by halves: the wave's sums once more, in the same order, by the other conversion, everything straight
+    // from memory (the other waves wait at the epilogue's first barrier)
+    if (__builtin_expect(beyond_halves(most), 0)) {
+        tw_settle(acc);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[mt][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+        for (uint32_t t = 0; t < ksteps; ++t) {
+            const uint32_t at = at_step(t), row0 = at * kTwK + 32u * kh + 8u * kq;  // the lane's 8 rows of B
+            Scales sr;
+            load_scales(sr, GROUPED ? group_offset(t, kh) : 0u);
+            bf16x8_t wf[2];
+#pragma unroll
+            for (uint32_t j = 0; j < 2; ++j) {
+                uint32_t c[2] = {0u, 0u};
+                if constexpr (PACKED) {
+                    const uint32_t off = (2u * wc + j) * slab_bytes + (at >> w_shift) * w_step + lane * 16u + (BITS == 8 ? 8u * kh : 8u * (at & 1u) + 4u * kh);
+                    c[0] = __builtin_amdgcn_raw_buffer_load_b32(rsrc_b, off, 0, 0);
+                    if constexpr (BITS == 8) c[1] = __builtin_amdgcn_raw_buffer_load_b32(rsrc_b, off + 4u, 0, 0);
+                } else {
+                    const uint32_t col = wcol + 16u * j;
+#pragma unroll
+                    for (uint32_t r = 0; r < 8; ++r) {
+                        const uint32_t byte = __builtin_amdgcn_raw_buffer_load_b8(rsrc_b, (row0 + r) * p.ldb_bytes + (BITS == 8 ? col : col / 2u), 0, 0);
+                        if constexpr (BITS == 8) c[r >> 2] |= byte << (8u * (r & 3u));
+                        else c[0] |= (byte >> (4u * (col & 1u)) & 15u) << (4u * r);
+                    }
+                }
+                const float s = bf16_bits_to_f32(sr.s[j]);
+                wf[j] = __builtin_bit_cast(bf16x8_t, BITS == 8 ? weights8(c[0], c[1], s) : weights4(c[0], 16.0f * s));
+            }
+            const bool past_k = at + 1u == ksteps_all && 4u * kh + kq >= last_chunks;
+#pragma unroll
+            for (uint32_t mt = 0; mt < (uint32_t)MT; ++mt) {
+                const uint32_t off = past_k ? a_extent : ((16u * mt + c16) * p.lda + row0) * 2u;
+                const bf16x8_t a = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, off, 0, 0));
+                // (the compiler's own instruction: its operands are written just before, which tw_mfma is not made for)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[mt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, wf[j], acc[mt][j], 0, 0, 0);
+            }
+        }
+    }
+
+    // ---- epilogue: fp32 sums -> LDS in [m][n] order (a quarter of a stage's rows in each array), then finish row-wise
     tw_settle(acc);                                       // the last matrix instructions have written their sums
     __syncthreads();                                   // ... and every wave is done reading the stages
     constexpr uint32_t kArrayRows = kStageRows / 4u;

@@ -396,8 +396,8 @@ BFAINTB_API uint32_t bfaintb_prefill_tile_cols(uint32_t m, uint32_t n);
 BFAINTB_API uint32_t bfaintb_gemm_split_k(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint32_t group_size);
 
 /*
- * Writes the dequantised weights W[k,n] as bf16 to w (row stride ldw elements), using the same
- * device dequantisation routine as the GEMM kernels.  Successor of the reference's ASM_PRINT debug
+ * Writes the dequantised weights W[k,n] as bf16 to w (row stride ldw elements): the weights that the GEMM
+ * kernels multiply by (some of which make a zero of a negative scale +0, not -0).  Successor of the reference's ASM_PRINT debug
  * channel (bfAintBGemm.cc:113-118,156-169; bf16gemm_kernel_gfx90a.s:2-16), which was its only way
  * to look at in-kernel values.
  */

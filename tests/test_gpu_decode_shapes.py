@@ -36,34 +36,31 @@ def test_launch_shapes_of_the_whole_machine_match_oracle(m, n, k, bits, group, w
     assert np.array_equal(run_gemm(problem), c)
 
 
-@pytest.mark.parametrize("m,n,k,group,packed", [(5, 144, 512, 32, False), (16, 272, 640, 128, False), (9, 144, 512, 64, True), (32, 272, 1024, 128, False),
-                                                  (2, 144, 512, 128, True), (5, 272, 640, 0, True)])
-def test_scales_of_any_sign_and_size(m, n, k, group, packed):
-    """4-bit codes by halves (the family with grouped scales, the slab kernel with a scale for each chunk): the conversion's two terms, (1024 + code) s and (1024 + 8) s, are exact whatever the scale:
-    negative, zero, subnormal, large."""
+# the family in rows and packed (one and two row blocks, 128 and 256 columns), the slab kernel with a scale for each column, chunk and block of
+# rows, and the other tiled kernels
+@pytest.mark.parametrize("which,m,n,k,bits,group,packed", [
+    ("DECODE", 5, 144, 512, 4, 32, False), ("DECODE", 16, 272, 640, 4, 128, False), ("DECODE", 32, 272, 1024, 4, 128, False),
+    ("DECODE", 2, 8192, 8192, 4, 128, False), ("DECODE", 40, 272, 640, 4, 0, False), ("DECODE", 9, 144, 512, 4, 64, True),
+    ("DECODE", 2, 144, 512, 4, 128, True), ("DECODE", 5, 272, 640, 4, 0, True), ("DECODE", 16, 8192, 4096, 4, 128, True),
+    ("DECODE", 5, 144, 512, 8, 64, False), ("DECODE", 3, 144, 512, 8, 0, True), ("DECODE", 40, 272, 640, 8, 32, True),
+    ("PREFILL_256", 70, 272, 512, 8, 64, False), ("PREFILL_256", 70, 272, 512, 4, 128, True), ("PREFILL_256X128", 70, 272, 512, 8, 0, False),
+    ("PREFILL_256X128", 70, 272, 512, 4, 64, True), ("PREFILL_128_LDS", 70, 272, 512, 8, 32, False), ("PREFILL_256_LDS", 70, 272, 512, 4, 64, False)])
+def test_scales_of_any_sign_and_size(which, m, n, k, bits, group, packed):
+    """A weight is q s, rounded once, whatever the scale: negative, zero, subnormal, and up to the format's limit of 2^120."""
     import torch
     import awesome_fusion_amd as af
     import helpers
-    import oracle
-    p = Problem(m, n, k, 4, group, seed=4)
-    s = np.random.default_rng(6).uniform(-1.0, 1.0, size=p.s_bf.shape).astype(np.float32)
-    s[:, 0::6] *= np.float32(2.0 ** -120)
-    s[:, 1::6] *= np.float32(2.0 ** 90)
-    s[:, 2::6] = 0.0
-    p.s_bf, p._w = oracle.f32_to_bf16_rne(s), None
+    which = getattr(af, which)
+    p = helpers.scales_of_any_sign_and_size(Problem(m, n, k, bits, group, seed=4))
     if packed:
         to_dev = helpers.to_dev
-        w = torch.empty(af.prepack_bytes(n, k, 4), dtype=torch.uint8, device="cuda")
-        af.prepack(w, to_dev(p.b_bytes), n, k, weight_bits=4)
+        w = torch.empty(af.prepack_bytes(n, k, bits), dtype=torch.uint8, device="cuda")
+        af.prepack(w, to_dev(p.b_bytes), n, k, weight_bits=bits)
         c = torch.zeros((m, n), dtype=torch.int16, device="cuda")
-        ws = helpers._ws.get(af.prepacked_workspace_bytes(m, n, k, 4, group, af.DECODE))
-        af.gemm_prepacked(c, to_dev(p.a_bf), w, to_dev(p.s_bf), m, n, k, weight_bits=4, group_size=group, workspace=ws, which=af.DECODE)
+        ws = helpers._ws.get(af.prepacked_workspace_bytes(m, n, k, bits, group, which))
+        af.gemm_prepacked(c, to_dev(p.a_bf), w, to_dev(p.s_bf), m, n, k, weight_bits=bits, group_size=group, workspace=ws, which=which)
         torch.cuda.synchronize()
         c = helpers.from_dev_u16(c)
     else:
-        c = run_gemm(p, which=af.DECODE)
-    c = helpers.widen(c).astype(np.float64)
-    w, a = helpers.widen(p.w_bf).astype(np.float64), helpers.widen(p.a_bf).astype(np.float64)
-    exact, absum = a @ w, np.abs(a) @ np.abs(w)
-    # (one rounding to bf16, 2^-8, and an fp32 sum of k terms, at most k x 2^-24 of the sum of their magnitudes)
-    assert (np.abs(c - exact) <= 2.0 ** -8 * np.abs(exact) + k * 2.0 ** -24 * absum + 1e-38).all()
+        c = run_gemm(p, which=which)
+    helpers.assert_close_at_any_scale(p, c, f"{m}x{n}x{k} bits={bits} g={group} packed={packed}")

@@ -73,22 +73,23 @@ def test_tall_tiles_take_the_epilogues_and_strides():
         af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 0)
 
 
-@pytest.mark.parametrize("bits,group,packed", [(8, 0, False), (8, 64, True), (4, 32, False), (4, 128, True)])
-def test_scales_of_any_sign_and_size(bits, group, packed):
-    """The conversion's two terms, (1024 + code) s and (1024 + excess) s, are exact whatever the scale: negative, zero, subnormal, large."""
+# every height with (by 14 compute units, the tall ones) and without the copying wave
+@pytest.mark.parametrize("bits,group,packed", [(8, 0, False), (8, 0, True), (8, 64, False), (8, 64, True), (4, 0, False), (4, 32, False), (4, 0, True), (4, 128, True)])
+@pytest.mark.parametrize("m,n,k", [(20, 144, 512), (40, 144, 640), (70, 144, 512), (128, 272, 512), (320, 640, 2176), (384, 640, 1152), (512, 640, 1152)])
+def test_scales_of_any_sign_and_size(m, n, k, bits, group, packed):
+    """The conversion by halves gives q s whatever the scale, up to the format's limit: beyond 2^117 its second product is not finite for 8-bit
+    codes, which then go another way."""
     import awesome_fusion_amd as af
-    import oracle
-    p = Problem(70, 144, 512, bits, group, seed=4)
-    s = np.random.default_rng(6).uniform(-1.0, 1.0, size=p.s_bf.shape).astype(np.float32)
-    s[:, 0::6] *= np.float32(2.0 ** -120)
-    s[:, 1::6] *= np.float32(2.0 ** 90)
-    s[:, 2::6] = 0.0
-    p.s_bf, p._w = oracle.f32_to_bf16_rne(s), None
-    c = helpers.widen(run(af, p, packed, af.PREFILL_128)).astype(np.float64)
-    w = helpers.widen(p.w_bf).astype(np.float64)
-    exact, absum = helpers.widen(p.a_bf).astype(np.float64) @ w, np.abs(helpers.widen(p.a_bf).astype(np.float64)) @ np.abs(w)
-    # (one rounding to bf16, 2^-8, and an fp32 sum of 512 terms, at most 512 x 2^-24 of the sum of their magnitudes)
-    assert (np.abs(c - exact) <= 2.0 ** -8 * np.abs(exact) + 512 * 2.0 ** -24 * absum + 1e-38).all()
+    try:
+        which = af.PREFILL_128
+        if m > 128:
+            af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 14)
+            which = af.PREFILL
+            assert af.plan(m, n, k, bits, group, packed=packed, which=which).kernel == af.KERNEL_TILES_128
+        p = helpers.scales_of_any_sign_and_size(Problem(m, n, k, bits, group, seed=4))
+        helpers.assert_close_at_any_scale(p, run(af, p, packed, which), f"{m}x{n}x{k} bits={bits} g={group} packed={packed}")
+    finally:
+        af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 0)
 
 
 # 2 blocks: fewer rows than a tile, one K-step, fewer than the stages, as many, one more, several rounds and an odd rest; a ragged last tile
