@@ -199,13 +199,13 @@ def assert_close_ulp(p, c_bits, what, rows=None, threads=8):
 
 def scales_of_any_sign_and_size(p, seed=6):
     """Gives p scales over all that the format allows: negative, zero, subnormal, and up to the limit of 2^120 (in every other group, so
-    that a kernel meets them from one group to the next).  The activations are small enough for the sums to stay finite."""
+    that a kernel meets them from one group to the next; every seventh column, so that each place in a dword of codes meets each kind).  The activations are small enough for the sums to stay finite."""
     rng = np.random.default_rng(seed)
     s = rng.uniform(-1.0, 1.0, size=p.s_bf.shape).astype(np.float32)
-    s[:, 0::6] *= np.float32(2.0 ** -120)
-    s[0::2, 1::6] = np.where(s[0::2, 1::6] < 0, -1, 1) * rng.uniform(2.0 ** 117, 0.99 * 2.0 ** 120, size=s[0::2, 1::6].shape).astype(np.float32)
-    s[:, 2::6] = 0.0
-    s[:, 3::6] *= np.float32(2.0 ** 117)
+    s[:, 0::7] *= np.float32(2.0 ** -120)
+    s[0::2, 1::7] = np.where(s[0::2, 1::7] < 0, -1, 1) * rng.uniform(2.0 ** 117, 0.99 * 2.0 ** 120, size=s[0::2, 1::7].shape).astype(np.float32)
+    s[:, 2::7] = 0.0
+    s[:, 3::7] *= np.float32(2.0 ** 117)
     p.s_bf, p._w = oracle.f32_to_bf16_rne(s), None
     p.a_bf = oracle.f32_to_bf16_rne(widen(p.a_bf) * np.float32(2.0 ** -8))
     return p
@@ -218,7 +218,7 @@ def assert_close_at_any_scale(p, c_bits, what):
     exact, absum = a @ w, np.abs(a) @ np.abs(w)
     off = ~(np.abs(c - exact) <= 2.0 ** -8 * np.abs(exact) + p.k * 2.0 ** -24 * absum + 1e-38)
     assert np.abs(exact).max() < 2.0 ** 127 and not off.any(), \
-        f"{what}: {int(off.sum())} of {off.size} outputs off, {int((~np.isfinite(c)).sum())} not finite, in columns {np.unique(np.nonzero(off)[1] % 6)} mod 6"
+        f"{what}: {int(off.sum())} of {off.size} outputs off, {int((~np.isfinite(c)).sum())} not finite, in columns {np.unique(np.nonzero(off)[1] % 7)} mod 7"
 
 
 def gated_reference(p, rows=None, threads=8):
