@@ -30,6 +30,7 @@ hipError_t launch_prefill_packed(const GemmParams& p, int bits, hipStream_t stre
 hipError_t launch_prefill128(const GemmParams& p, int bits, bool packed, hipStream_t stream);
 hipError_t launch_prefill128_wreg(const GemmParams& p, int bits, bool packed, hipStream_t stream);
 bool prefill128_wreg_serves(const GemmParams& p);
+bool prefill128_wreg_copier(const GemmParams& p, int bits, bool packed);
 hipError_t launch_prefill256x128_wreg(const GemmParams& p, int bits, bool packed, hipStream_t stream);
 hipError_t launch_decode_family_packed(const GemmParams& p, int bits, hipStream_t stream);
 hipError_t decode_prepare_device();
@@ -1871,6 +1872,21 @@ static int plan_whole(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint3
     out->splits = 1;
     out->k_per_workgroup = k;
     if (m == 0 || n == 0) return BFAINTB_OK;
+    auto tiles_of_128_columns = [&](uint32_t blocks, uint32_t splits, uint32_t k_per_wg) {
+        GemmParams p{};
+        p.m = m;
+        p.group_size = group_size;
+        p.tile_blocks = blocks;
+        p.splits = splits;
+        p.k_per_wg = k_per_wg;
+        out->kernel = BFAINTB_KERNEL_TILES_128;
+        out->tile_rows = 16u * blocks;
+        out->tile_cols = 128u;
+        out->waves = bfaintb::prefill128_wreg_copier(p, weight_bits, packed != 0) ? 9u : 8u;
+        out->splits = splits;
+        out->k_per_workgroup = k_per_wg;
+        out->workgroups = ((m + out->tile_rows - 1u) / out->tile_rows) * ((n + 127u) / 128u) * splits;
+    };
     if (v == BFAINTB_VARIANT_DECODE) {
         out->variant = v;
         if (packed && packed_uses_slab(m, n, k, weight_bits)) {
@@ -1882,8 +1898,12 @@ static int plan_whole(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint3
             return BFAINTB_OK;
         }
         const DecodePlan pl = packed ? packed_family_plan(m, n, k, weight_bits) : decode_plan(m, n, k, weight_bits, split_k);
-        if (variant == BFAINTB_VARIANT_AUTO && (packed || split_k == 0) && few_rows_on_tiles(m, n, k, weight_bits, group_size != 0, packed != 0, n))
-            out->tiles_instead = (n + 127u) / 128u;
+        out->workspace_bytes = split_workspace_bytes(pl.splits, m, n);
+        if (variant == BFAINTB_VARIANT_AUTO && (packed || split_k == 0) && few_rows_on_tiles(m, n, k, weight_bits, group_size != 0, packed != 0, n)) {
+            tiles_of_128_columns(2u, 1u, (k + 63u) / 64u * 64u);
+            out->tiles_instead = out->workgroups;
+            return BFAINTB_OK;
+        }
         out->kernel = BFAINTB_KERNEL_DECODE_FAMILY;
         out->tile_rows = 16u * pl.mb;
         out->tile_cols = pl.cols;
@@ -1891,33 +1911,35 @@ static int plan_whole(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint3
         out->splits = pl.splits;
         out->k_per_workgroup = pl.k_per_wg;
         out->workgroups = ((n + pl.cols - 1u) / pl.cols) * pl.splits * ((m + 16u * pl.mb - 1u) / (16u * pl.mb));
-        out->workspace_bytes = split_workspace_bytes(pl.splits, m, n);
         return BFAINTB_OK;
     }
     // the tiled kernels
     if (use_small_tiles(v, m, n, k, weight_bits)) {
         out->variant = BFAINTB_VARIANT_PREFILL_128;
-        out->tile_rows = out->tile_cols = 128u;
-        const bool wreg = v != BFAINTB_VARIANT_PREFILL_128_LDS;
-        out->kernel = wreg ? BFAINTB_KERNEL_TILES_128 : BFAINTB_KERNEL_TILES_128_LDS;
-        out->waves = wreg ? 4u : 8u;
-        if (wreg) {
+        if (v != BFAINTB_VARIANT_PREFILL_128_LDS) {
             const TilePlan tp = tile128_plan(m, n, k, weight_bits, packed ? 0u : split_k);
-            out->splits = tp.splits;
+            tiles_of_128_columns(tp.blocks, tp.splits, tp.k_per_wg);
             out->launches = 1u + tp.finish_launch;
             out->workspace_bytes = tile_workspace_bytes(tp, m, n);
-            out->k_per_workgroup = tp.k_per_wg;
+            return BFAINTB_OK;
         }
-        out->workgroups = ((m + 127u) / 128u) * ((n + 127u) / 128u) * out->splits;
+        out->kernel = BFAINTB_KERNEL_TILES_128_LDS;
+        out->tile_rows = out->tile_cols = 128u;
+        out->waves = 8u;
+        out->workgroups = ((m + 127u) / 128u) * ((n + 127u) / 128u);
         return BFAINTB_OK;
     }
     if (v == BFAINTB_VARIANT_PREFILL_256X128 || (v == BFAINTB_VARIANT_PREFILL && prefill_tall_tiles(m, n, k, weight_bits))) {
-        const bool one_chain = v == BFAINTB_VARIANT_PREFILL_256X128 || tall_tiles_in_one_chain(m, k);
-        out->variant = one_chain ? BFAINTB_VARIANT_PREFILL_256X128 : BFAINTB_VARIANT_PREFILL;
-        out->kernel = one_chain ? BFAINTB_KERNEL_TILES_256X128 : BFAINTB_KERNEL_TILES_128;
+        if (v == BFAINTB_VARIANT_PREFILL && !tall_tiles_in_one_chain(m, k)) {
+            out->variant = v;  // (no variant names these tiles)
+            tiles_of_128_columns(tall_tile_blocks(m), 1u, (k + 63u) / 64u * 64u);
+            return BFAINTB_OK;
+        }
+        out->variant = BFAINTB_VARIANT_PREFILL_256X128;
+        out->kernel = BFAINTB_KERNEL_TILES_256X128;
         out->tile_rows = 256u;
         out->tile_cols = 128u;
-        out->waves = one_chain ? 4u : 8u;
+        out->waves = 4u;
         out->workgroups = ((m + 255u) / 256u) * ((n + 127u) / 128u);
         return BFAINTB_OK;
     }

@@ -873,18 +873,27 @@ static hipError_t launch_prefill128_wreg_t(const GemmParams& p, hipStream_t stre
     return launch_kernel(bfaintb_split_finish_kernel, dim3((p.m * (p.n / 4u) + 255u) / 256u, 1, 1), dim3(256, 1, 1), 0, stream, p);
 }
 
+// Whether a launch has the copying wave (p: the tile's blocks, the rows, the split and its share of k, the group size).  Always with two
+// blocks (see the head of the file), never with more than eight.  Otherwise, and with the fewer stages that its wait counts reach:
+// Over packed weights with grouped scales or 4-bit codes (us, without / with: 128 x 20480 x 4096 4-bit g128 35.1 / 31.7, 64 rows 28.1 / 24.9;
+// 8-bit g64 35.6 / 34.7 and 28.0 / 26.2; 4-bit, one scale per column, 33.5 / 31.6 and 23.6 / 22.9; not 8-bit, one scale per column: 34.6 /
+// 36.4 and 25.3 / 26.1, nor codes in rows: 38.7 / 39.2).
+// Codes in rows with grouped scales: where several rows of tiles split k into shares of up to 64 steps (without / with: 785 x 1440 x 4480
+// 8-bit 26.3 / 25.0, 4-bit 26.7 / 25.5; 400 x 2560 x 2560 19.9 / 18.8 and 20.3 / 19.2; 900 x 2048 x 8192 44.4 / 42.5 and 43.3 / 42.1; longer
+// shares lose what the start gains, 384 x 4096 x 11008 52.6 / 54.5 and 50.7 / 53.9, and so do unsplit ones, 640 x 4096 x 4096 8-bit 34.2 /
+// 35.9, and one row of tiles, 128 x 11008 x 4096 8-bit 26.7 / 28.5).
+bool prefill128_wreg_copier(const GemmParams& p, int bits, bool packed)
+{
+    const bool grouped = p.group_size != 0u;
+    if (p.tile_blocks == 2u || p.tile_blocks > 8u) return p.tile_blocks == 2u;
+    return packed ? grouped || bits == 4 : grouped && p.splits > 1u && p.m > 256u && p.k_per_wg <= 64u * kTwK;
+}
+
 template <int BITS, bool GROUPED, bool PACKED>
 static hipError_t launch_prefill128_wreg_rows(const GemmParams& p, hipStream_t stream)
 {
-    // the copying wave, and the fewer stages that its wait counts reach, over packed weights with grouped scales or 4-bit codes (us,
-    // without / with: 128 x 20480 x 4096 4-bit g128 35.1 / 31.7, 64 rows 28.1 / 24.9; 8-bit g64 35.6 / 34.7 and 28.0 / 26.2; 4-bit, one scale
-    // per column, 33.5 / 31.6 and 23.6 / 22.9; not 8-bit, one scale per column: 34.6 / 36.4 and 25.3 / 26.1, nor codes in rows: 38.7 / 39.2)
-    // Codes in rows with grouped scales: where several rows of tiles split k into shares of up to 64 steps (without / with: 785 x 1440 x 4480
-    // 8-bit 26.3 / 25.0, 4-bit 26.7 / 25.5; 400 x 2560 x 2560 19.9 / 18.8 and 20.3 / 19.2; 900 x 2048 x 8192 44.4 / 42.5 and 43.3 / 42.1; longer
-    // shares lose what the start gains, 384 x 4096 x 11008 52.6 / 54.5 and 50.7 / 53.9, and so do unsplit ones, 640 x 4096 x 4096 8-bit 34.2 /
-    // 35.9, and one row of tiles, 128 x 11008 x 4096 8-bit 26.7 / 28.5).
     constexpr bool kCopierOnly = PACKED && (GROUPED || BITS == 4), kCopierToo = !PACKED && GROUPED;
-    if (kCopierOnly || (kCopierToo && p.splits > 1u && p.m > 256u && p.k_per_wg <= 64u * kTwK)) {
+    if (prefill128_wreg_copier(p, BITS, PACKED)) {
         if constexpr (kCopierOnly || kCopierToo) {
             switch (p.tile_blocks) {
                 case 4: return launch_prefill128_wreg_t<BITS, GROUPED, PACKED, 4, 6, true>(p, stream);

@@ -57,13 +57,15 @@ enum {
 enum {
     BFAINTB_VARIANT_AUTO = 0,   /* decode up to m = 32; beyond, whichever the library estimates faster for (m, n, k) */
     BFAINTB_VARIANT_DECODE = 1, /* split-K weight-streaming kernel (HBM-bound); m > 32 in row blocks; accepts m <= 32768 */
-    BFAINTB_VARIANT_PREFILL = 2, /* LDS-tiled MFMA kernels (MFMA-bound): 256x256 tiles, or 128x128 tiles while m x n
-                                  * holds at most 256 of those (the large tiles would leave most CUs idle); while even
+    BFAINTB_VARIANT_PREFILL = 2, /* LDS-tiled MFMA kernels (MFMA-bound): 256x256 tiles, or small tiles of 128 columns and at
+                                  * most 128 rows while m x n holds at most 256 of those (the large tiles would leave most
+                                  * CUs idle), or tall ones of 128 columns and 160 to 256 rows in between; while even
                                   * the small tiles leave CUs idle, their kernel splits k between workgroups (same
                                   * workspace and hand-over as the decode family's split-K) */
     BFAINTB_VARIANT_PREFILL_256 = 3, /* the tiled kernel with 256x256 tiles, whatever the shape (tests, tuning) */
-    BFAINTB_VARIANT_PREFILL_128 = 4, /* the tiled kernel with 128x128 tiles, whatever the shape (tests, tuning).  Its fp32
-                                      * sums are those of two chains of matrix instructions added at the end (even and odd
+    BFAINTB_VARIANT_PREFILL_128 = 4, /* the tiled kernel with small tiles, whatever the shape (tests, tuning): 128 columns and
+                                      * 32, 64, 96 or 128 rows, the rows of A spread evenly over as many tiles as 128 each
+                                      * would take.  Its fp32 sums are those of two chains of matrix instructions added at the end (even and odd
                                       * blocks of 32 k), so it agrees with the other tiled forms to rounding, not in
                                       * every bit; like every form it gives the same bits on every run */
     BFAINTB_VARIANT_PREFILL_256_LDS = 5, /* 256x256 tiles with both operands staged in LDS — the older form, which the
@@ -73,8 +75,11 @@ enum {
                                           * reference's arithmetic; otherwise the form that keeps the weights in
                                           * registers runs (tests, tuning) */
     BFAINTB_VARIANT_PREFILL_256X128 = 7  /* tiles of 256 rows x 128 columns, weights in registers (this library's
-                                          * arithmetic), whatever the shape (tests, tuning): what PREFILL runs
-                                          * where 128x128 tiles would need a second round and 256x256 tiles leave CUs idle */
+                                          * arithmetic), whatever the shape (tests, tuning): with k up to 1024 (2048 for tiles
+                                          * of 160 rows) what PREFILL runs where small tiles would need a second round and
+                                          * 256x256 tiles leave CUs idle.  Each output is one chain of ascending k, as in the
+                                          * 256x256 tiles, so the bits are theirs; beyond that k PREFILL runs the small tiles'
+                                          * kernel there with 160, 192 or 256 rows, which is faster and adds two chains */
 };
 
 /*
@@ -352,27 +357,29 @@ BFAINTB_API int bfaintb_packed_header_check(const bfaintb_packed_header* h);
 enum {
     BFAINTB_KERNEL_DECODE_FAMILY = 1, /* weight streaming with split-K, in row blocks beyond 32 rows of A */
     BFAINTB_KERNEL_DECODE_SLAB = 2,   /* packed weights: one column block of 16 per workgroup, no split */
-    BFAINTB_KERNEL_TILES_128 = 3,     /* 128 x 128 tiles, weights in registers, may split k */
+    BFAINTB_KERNEL_TILES_128 = 3,     /* tiles of 128 columns and 32 to 256 rows, weights in registers; up to 128 rows may split k */
     BFAINTB_KERNEL_TILES_128_LDS = 4, /* 128 x 128 tiles, both operands through LDS */
-    BFAINTB_KERNEL_TILES_256X128 = 5, /* tiles of 256 rows x 128 columns, weights in registers */
+    BFAINTB_KERNEL_TILES_256X128 = 5, /* tiles of 256 rows x 128 columns, weights in registers, one chain of products an output */
     BFAINTB_KERNEL_TILES_256 = 6,     /* 256 x 256 tiles, weights in registers */
     BFAINTB_KERNEL_TILES_256_LDS = 7  /* 256 x 256 tiles, both operands through LDS */
 };
 typedef struct bfaintb_plan {
-    int32_t variant;           /* BFAINTB_VARIANT_DECODE, or the tiled variant with its tile size resolved */
+    int32_t variant;           /* BFAINTB_VARIANT_DECODE, or the tiled variant with its tile size resolved (PREFILL where no variant names it) */
     uint32_t kernel;           /* BFAINTB_KERNEL_* */
     uint32_t tile_rows;        /* rows of A per workgroup */
     uint32_t tile_cols;        /* columns of B per workgroup */
-    uint32_t waves;            /* waves per workgroup */
+    uint32_t waves;            /* waves per workgroup, one that only copies included */
     uint32_t splits;           /* workgroups along k per tile */
     uint32_t k_per_workgroup;  /* rows of k one workgroup covers */
     uint32_t workgroups;       /* of the launch (the first one, if there are two) */
     uint32_t tail_workgroups;  /* of further launches over a last, thin round of tiles or over the last rows, or 0 */
     uint32_t launches;         /* kernels launched: 1, or more with a tail or with split sums added by a launch of their own */
     uint32_t compute_units;    /* what the plan was made for */
-    uint32_t tiles_instead;    /* 17 to 32 rows by the library's own choice: so many tiles of 32 rows x 128 columns, unsplit, run in place
-                                  of the launch that the fields above describe (which a call that names the variant, asks for the
-                                  reference's arithmetic or has rows too far apart for 32-bit extents gets); 0: they do not */
+    uint32_t tiles_instead;    /* 17 to 32 rows by the library's own choice: so many tiles of 32 rows x 128 columns, unsplit, run instead of the
+                                  decode family, and the fields above describe them (variant stays BFAINTB_VARIANT_DECODE, as
+                                  bfaintb_gemm_variant answers, and the scratch is the family's); else 0.  The plan takes the rows
+                                  of B to lie n codes apart; a call decides by its own ldb.  A call that names the variant, asks for
+                                  the reference's arithmetic or has rows too far apart for 32-bit extents runs the family */
     uint64_t workspace_bytes;  /* what bfaintb_gemm[_prepacked]_workspace_bytes_ex reports for the same arguments */
 } bfaintb_plan;
 BFAINTB_API int bfaintb_gemm_plan(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint32_t group_size, int packed, int variant,
@@ -381,14 +388,15 @@ BFAINTB_API int bfaintb_gemm_plan(uint32_t m, uint32_t n, uint32_t k, int weight
 /* Which variant bfaintb_gemm would run (BFAINTB_VARIANT_*), or a negative error. */
 BFAINTB_API int bfaintb_gemm_variant(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint32_t group_size);
 
-/* Rows (bfaintb_prefill_tile) and columns of the tiles BFAINTB_VARIANT_PREFILL runs an m x n output of row-major
- * weights with: 128 x 128 while that makes at most 256 tiles (one per CU); else 256 rows x 128 columns while that
+/* Rows (bfaintb_prefill_tile) and columns of the kind of tiles BFAINTB_VARIANT_PREFILL runs an m x n output of row-major
+ * weights with: small, 128 x 128, while that makes at most 256 tiles (one per CU); else tall, 256 rows x 128 columns, while that
  * makes at most 256; else 256 x 256 (256 = the device's compute units: one tile per unit) — except that up to 512
- * tiles of 128 x 128 run in two rounds where the 256 x 128 ones just miss one round and the 256 x 256 ones would fill
- * at most 60 % of the units (640 x 11008), and that up to 128 rows always run 128 x 128 tiles, in as many rounds as it
- * takes (taller tiles would be half empty).  The two functions answer for 8-bit codes; 4-bit codes keep the 128 x 128
- * tiles up to 345 of them (their 256 x 128 kernel is the weaker one); bfaintb_gemm_plan answers for either.  Pre-packed
- * weights run the same tiles.  (The reference arithmetic has no 256 x 128 form: 256 x 256 there.) */
+ * small tiles run in two rounds where the tall ones just miss one round and the 256 x 256 ones would fill
+ * at most 60 % of the units (640 x 11008), and that up to 128 rows always run small tiles, in as many rounds as it
+ * takes (taller tiles would be half empty).  Small and tall tiles are of at most that many rows: the rows of A are spread evenly
+ * over them, in steps of 32 or 64 (bfaintb_gemm_plan has the number).  The two functions answer for 8-bit codes and a k of 4096; 4-bit
+ * codes with a short k keep the small tiles up to 345 of them; bfaintb_gemm_plan answers for either.  Pre-packed
+ * weights run the same tiles.  (The reference arithmetic has no tall form: 256 x 256 there.) */
 BFAINTB_API uint32_t bfaintb_prefill_tile(uint32_t m, uint32_t n);
 BFAINTB_API uint32_t bfaintb_prefill_tile_cols(uint32_t m, uint32_t n);
 

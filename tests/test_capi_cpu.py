@@ -208,13 +208,13 @@ def test_plan_query_agrees_with_the_other_queries_and_follows_the_compute_units(
         assert (t.kernel, t.splits, t.workgroups) == (af.KERNEL_TILES_128, 3, 432) and t.workspace_bytes == 256 + 2 * 48 * 18432 * 4
         assert af.plan(48, 18432, 4096).splits == 1 and af.plan(128, 18432, 8192).splits == 1 and af.plan(48, 21760, 8192).splits == 1
         assert af.plan(96, 18432, 8192).workspace_bytes <= af.lib().bfaintb_gemm_static_scratch_bytes()
-        # one row of tiles is always 128 x 128 tiles, whatever their number; more rows go back to large tiles
+        # one row of tiles is always small tiles, whatever their number, of no more rows than there are in steps of 32; more rows go back to large tiles
         assert (af.prefill_tile(96, 36864), af.prefill_tile(128, 128256), af.prefill_tile(129, 36864)) == (128, 128, 256)
         for packed in (False, True):
             t = af.plan(96, 36864, 8192, packed=packed)
-            assert (t.tile_rows, t.tile_cols, t.workgroups) == (128, 128, 288), (packed, t.as_dict())
+            assert (t.tile_rows, t.tile_cols, t.workgroups) == (96, 128, 288), (packed, t.as_dict())
             t = af.plan(64, 128256, 4096, 4, 128, packed=packed)
-            assert t.workgroups == 1002 and (t.tile_rows == 128) == (not packed), (packed, t.as_dict())
+            assert (t.kernel == af.KERNEL_TILES_128, t.tile_rows, t.workgroups) == (not packed, 64, 1002), (packed, t.as_dict())
     try:
         for cus in (64, 304):
             af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, cus)
@@ -362,7 +362,7 @@ def test_product_does_not_reach_for_the_oracle():
     # 4-bit codes, 17 to 32 rows: four splits of 4 waves; not where three splits of 256 columns fit a round
     (32, 22016, 4096, 4, 128, (128, 4, 4)), (32, 21760, 4096, 4, 128, (256, 4, 3)), (32, 24576, 5248, 4, 128, (256, 4, 2))])
 def test_launch_shapes_of_the_decode_family(m, n, k, bits, group, want):
-    p = af.plan(m, n, k, bits, group)
+    p = af.plan(m, n, k, bits, group, which=af.DECODE)   # (by name: 17 to 32 rows run tiles by the library's own choice)
     if p.compute_units == 256:
         assert (p.tile_cols, p.waves, p.splits) == want, p.as_dict()
 
@@ -374,6 +374,6 @@ def test_launch_shapes_of_the_decode_family(m, n, k, bits, group, want):
     (20, 24576, 4096, (128, 4, 4)), (21, 24576, 4096, (256, 4, 2)), (20, 22528, 5120, (128, 4, 4)), (32, 22528, 5120, (256, 4, 2)),
     (18, 24832, 4096, (256, 4, 2)), (18, 22016, 5632, (256, 4, 2)), (18, 22032, 4096, (256, 4, 2))])
 def test_four_splits_for_17_to_32_rows_of_4_bit_codes(m, n, k, want):
-    p = af.plan(m, n, k, 4, 128)
+    p = af.plan(m, n, k, 4, 128, which=af.DECODE)
     if p.compute_units == 256:
         assert (p.tile_cols, p.waves, p.splits) == want, p.as_dict()

@@ -15,12 +15,12 @@ def test_launch_shapes_match_oracle(m, n, k, bits, group, want):
     import awesome_fusion_amd as af
     try:
         af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 16)
-        p = af.plan(m, n, k, bits, group)
+        p = af.plan(m, n, k, bits, group, which=af.DECODE)   # (by name: 17 to 32 rows run tiles by the library's own choice)
         assert (p.tile_cols, p.waves, p.splits) == want, p.as_dict()
         problem = Problem(m, n, k, bits, group, seed=m + k)
-        c = run_gemm(problem)
+        c = run_gemm(problem, which=af.DECODE)
         assert_close_ulp(problem, c, f"{m}x{n}x{k} bits={bits} g={group}")
-        assert np.array_equal(run_gemm(problem), c)
+        assert np.array_equal(run_gemm(problem, which=af.DECODE), c)
     finally:
         af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 0)
 
@@ -28,12 +28,12 @@ def test_launch_shapes_match_oracle(m, n, k, bits, group, want):
 @pytest.mark.parametrize("m,n,k,bits,group,want", [(3, 3072, 8192, 8, 0, (128, 4, 10)), (18, 22016, 2560, 4, 128, (128, 4, 4)), (32, 22016, 2176, 4, 0, (128, 4, 4))])
 def test_launch_shapes_of_the_whole_machine_match_oracle(m, n, k, bits, group, want):
     import awesome_fusion_amd as af
-    p = af.plan(m, n, k, bits, group)
+    p = af.plan(m, n, k, bits, group, which=af.DECODE)
     assert p.compute_units != 256 or (p.tile_cols, p.waves, p.splits) == want, p.as_dict()
     problem = Problem(m, n, k, bits, group, seed=m + k)
-    c = run_gemm(problem)
+    c = run_gemm(problem, which=af.DECODE)
     assert_close_ulp(problem, c, f"{m}x{n}x{k} bits={bits} g={group}")
-    assert np.array_equal(run_gemm(problem), c)
+    assert np.array_equal(run_gemm(problem, which=af.DECODE), c)
 
 
 # the family in rows and packed (one and two row blocks, 128 and 256 columns), the slab kernel with a scale for each column, chunk and block of

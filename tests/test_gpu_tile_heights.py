@@ -46,7 +46,7 @@ def test_tall_tiles(m, n, k, blocks, bits, group, packed):
     try:
         af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 14)
         pl = af.plan(m, n, k, bits, group, packed=packed, which=af.PREFILL)
-        assert (pl.kernel, pl.tile_rows, pl.tile_cols, pl.waves, pl.splits) == (af.KERNEL_TILES_128, 256, 128, 8, 1), pl.as_dict()
+        assert (pl.kernel, pl.tile_rows, pl.tile_cols, pl.waves, pl.splits) == (af.KERNEL_TILES_128, 16 * blocks, 128, 8, 1), pl.as_dict()
         p = Problem(m, n, k, bits, group, seed=m + k + bits)
         c = run(af, p, packed, af.PREFILL)
         assert_close_ulp(p, c, f"{blocks} blocks: {m}x{n}x{k} bits={bits} g={group} packed={packed}")
@@ -114,8 +114,10 @@ def test_few_rows_choose_tiles(m, n, k, bits, group, packed):
     try:
         af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 8)
         pl = af.plan(m, n, k, bits, group, packed=packed)
-        assert pl.variant == af.DECODE and pl.tiles_instead == (n + 127) // 128, pl.as_dict()
-        assert af.plan(m, n, k, bits, group, packed=packed, which=af.DECODE).tiles_instead == 0
+        assert pl.variant == af.DECODE and pl.tiles_instead == pl.workgroups == (n + 127) // 128, pl.as_dict()
+        assert (pl.kernel, pl.tile_rows, pl.tile_cols, pl.splits) == (af.KERNEL_TILES_128, 32, 128, 1), pl.as_dict()
+        by_name = af.plan(m, n, k, bits, group, packed=packed, which=af.DECODE)
+        assert by_name.tiles_instead == 0 and by_name.kernel == af.KERNEL_DECODE_FAMILY and by_name.workspace_bytes == pl.workspace_bytes
         p = Problem(m, n, k, bits, group, seed=m + n + k)
         c = run(af, p, packed, af.AUTO)
         assert_close_ulp(p, c, "tiles")

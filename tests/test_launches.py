@@ -73,6 +73,42 @@ def test_reference_arithmetic_takes_the_kernel_it_has(tmp_path):
         assert bare[:2] == (0, 1) and (family.splits == 1 or bare[2] < workgroups)
 
 
+# (shape, code width, group, packed, tile rows): the family, the slab kernel, every height of tiles with and without the copying wave, split k in
+# one launch and in two, the large tiles and their thin last round, a product in two launches by rows
+PLANS = [((1, 4096, 4096), 8, 0, 0, 16), ((8, 4096, 4096), 4, 128, 1, 16), ((32, 4096, 4096), 8, 0, 1, 16), ((40, 4096, 4096), 8, 0, 0, None),
+         ((17, 22016, 2048), 8, 0, 0, 32), ((32, 22016, 4096), 4, 128, 0, 32), ((32, 22016, 4096), 4, 128, 1, 32), ((20, 20480, 4096), 8, 0, 1, 32),
+         ((96, 4096, 11008), 8, 0, 0, 96), ((64, 20480, 4096), 4, 128, 1, 64), ((96, 36864, 8192), 8, 0, 0, 96), ((128, 20480, 4096), 8, 64, 1, 128),
+         ((48, 18432, 8192), 8, 0, 0, 64), ((640, 4096, 4096), 8, 64, 0, 128), ((785, 1440, 4480), 8, 32, 0, 128), ((320, 16384, 4096), 8, 0, 0, 160),
+         ((384, 16384, 4096), 4, 128, 1, 192), ((512, 11008, 4096), 8, 0, 0, 256), ((512, 11008, 512), 8, 0, 0, 256), ((4096, 4096, 4096), 8, 0, 0, 256),
+         ((2048, 28672, 8192), 4, 128, 0, 256), ((577, 13824, 5120), 4, 128, 1, None)]
+
+
+def test_the_plan_describes_what_is_launched(tmp_path):
+    """Rows of a tile, waves, workgroups (the tiled kernels launch a whole number of them per XCD, an eighth each) and launches; and the same
+    for every variant by name."""
+    import awesome_fusion_amd as af
+    asked = [(s, b, g, pk, rows, v) for s, b, g, pk, rows in PLANS
+             for v in (af.AUTO, af.DECODE, af.PREFILL, af.PREFILL_128, af.PREFILL_256, af.PREFILL_256X128, af.PREFILL_128_LDS, af.PREFILL_256_LDS)]
+    r = on_stand_in(tmp_path, "plan_launches", "\n".join("%d %d %d %d %d %d %d" % (*s, b, g, pk, v) for s, b, g, pk, _, v in asked))
+    assert r.returncode == 0
+    answers = [tuple(map(int, line.split())) for line in r.stdout.split("\n") if line]
+    assert len(answers) == len(asked)
+    kinds = set()
+    for q, (variant, kernel, rows, cols, waves, splits, wgs, tail, launches, rc, did, did_waves, did_wgs, did_others) in zip(asked, answers):
+        (m, n, k), bits, group, packed, want, which = q
+        what = (q, rows, cols, waves, splits, wgs, tail, launches, did, did_waves, did_wgs, did_others)
+        assert (rc, did, did_waves) == (0, launches, waves), what
+        first = wgs or tail   # (fewer large tiles than half a round are all cut in halves: the thin round is all there is)
+        assert first <= did_wgs < first + 8 * splits, what
+        assert which != af.AUTO or want is None or rows == want, what
+        two_by_rows = which == af.AUTO and tail and kernel not in (af.KERNEL_TILES_256, af.KERNEL_TILES_256_LDS)
+        if not (two_by_rows or kernel in (af.KERNEL_TILES_256, af.KERNEL_TILES_256_LDS)):
+            assert wgs == -(-m // rows) * -(-n // cols) * splits, what
+        assert tail <= did_others or wgs == 0, what
+        kinds.add((kernel, rows))
+    assert {(af.KERNEL_TILES_128, r) for r in (32, 64, 96, 128, 160, 192, 256)} <= kinds and (af.KERNEL_TILES_256X128, 256) in kinds
+
+
 @pytest.mark.gpu
 def test_two_threads_share_a_stream():
     """The operators' workspace is one per stream: products in two launches and split decode calls from two threads."""
