@@ -903,7 +903,7 @@ int static_scratch(DeviceState& st, hipStream_t stream, void** out)
 
 extern "C" {
 
-static uint32_t row_split_head(uint32_t m, uint32_t n, uint32_t k, int bits, bool packed);
+static uint32_t row_split_head(uint32_t m, uint32_t n, uint32_t k, int bits, bool packed, bool grouped);
 static size_t row_split_workspace(uint32_t head, uint32_t rest, uint32_t n, uint32_t k, int bits, bool packed);
 
 int bfaintb_version(void) { return BFAINTB_VERSION; }
@@ -941,7 +941,7 @@ uint32_t bfaintb_gemm_split_k(uint32_t m, uint32_t n, uint32_t k, int weight_bit
 {
     int v = bfaintb_gemm_variant(m, n, k, weight_bits, group_size);
     if (v >= 0) {
-        const uint32_t head = row_split_head(m, n, k, weight_bits, false);
+        const uint32_t head = row_split_head(m, n, k, weight_bits, false, group_size != 0);
         if (head != 0u) {
             m = head;
             v = resolve_variant(m, n, k, weight_bits, BFAINTB_VARIANT_AUTO);
@@ -959,7 +959,7 @@ size_t bfaintb_gemm_workspace_bytes_ex(uint32_t m, uint32_t n, uint32_t k, int w
     const int v = resolve_variant(m, n, k, weight_bits, variant);
     if (v < 0) return 0;
     if (variant == BFAINTB_VARIANT_AUTO && split_k == 0) {
-        const uint32_t head = row_split_head(m, n, k, weight_bits, false);
+        const uint32_t head = row_split_head(m, n, k, weight_bits, false, group_size != 0);
         if (head != 0u) return row_split_workspace(head, m - head, n, k, weight_bits, false);
     }
     return workspace_need(m, n, k, weight_bits, v, split_k);
@@ -1140,7 +1140,7 @@ static int gemm_impl(void* c, const void* a, const void* b, const void* scale, c
     if (misaligned16(c) || misaligned16(a) || misaligned16(b) || misaligned16(scale) || misaligned16(bias) || misaligned16(ep.residual))
         return BFAINTB_ERR_ALIGNMENT;
     if (!whole && variant == BFAINTB_VARIANT_AUTO && split_k == 0 && !ep.reference_arith) {
-        const uint32_t head = row_split_head(m, n, k, weight_bits, false);
+        const uint32_t head = row_split_head(m, n, k, weight_bits, false, group_size != 0);
         if (head != 0u && row_split_served(workspace, workspace_bytes, row_split_workspace(head, m - head, n, k, weight_bits, false), use_static_scratch,
                                            static_cast<hipStream_t>(stream))) {
             e = gemm_impl(c, a, b, scale, ep, head, n, k, lda, ldb, ldc, weight_bits, group_size, workspace, workspace_bytes, stream, variant, 0,
@@ -1533,9 +1533,12 @@ static size_t packed_workspace_need(uint32_t m, uint32_t n, uint32_t k, int bits
 // kernels are asked about: the large tiles by their number (a round at a load below one CU each runs at a higher clock; us per
 // K-step at 162 / 216 / 256 tiles, 4-bit 1.39 / 1.49 / 1.55, 8-bit, at 172 / 256, 1.26 / 1.52), the thin last round as the half tiles
 // it runs as; up to 32 rows the stream of the weights.
-static double launch_time_us(uint32_t m, uint32_t n, uint32_t k, int bits, bool packed)
+// (17 to 32 rows on tiles: by the tiles' estimate, 0.88 - 1.07 of the measured time by kind of weights, 9 % rms over 340 shapes; the stream at
+// this rate would be 1.15 (4-bit) to 1.69 (8-bit) times it.  For rows of B that lie n codes apart, as the scratch is asked for.)
+static double launch_time_us(uint32_t m, uint32_t n, uint32_t k, int bits, bool packed, bool grouped)
 {
     const double cus = (double)machine_cus(), steps = k / 64.0;
+    if (few_rows_on_tiles(m, n, k, bits, grouped, packed, n)) return tile128_plan(m, n, k, bits, 1).us;
     if (m <= kDecodeAutoMaxM) return 6.0 + (double)n * k * bits / 8.0 / 3.3e6 * (m <= 16u ? 1.0 : 1.25);
     if (m <= kDecodeFamilyAutoMaxM) {  // (beyond 32 rows the library's own choice asks just this)
         const double family = packed ? packed_family_time_us(m, n, k, bits, packed_family_plan(m, n, k, bits)) : decode_family_time_us(m, n, k, bits, decode_plan(m, n, k, bits, 0));
@@ -1567,7 +1570,7 @@ static size_t row_split_workspace(uint32_t head, uint32_t rest, uint32_t n, uint
 }
 
 // Rows of the first launch, or 0 for one launch over all of them.
-static uint32_t row_split_rule(uint32_t m, uint32_t n, uint32_t k, int bits, bool packed)
+static uint32_t row_split_rule(uint32_t m, uint32_t n, uint32_t k, int bits, bool packed, bool grouped)
 {
     if (m <= 256u || n < 16u || g_force_row_block.load(std::memory_order_relaxed) != 0u) return 0;
     const uint64_t cus = machine_cus();
@@ -1577,7 +1580,7 @@ static uint32_t row_split_rule(uint32_t m, uint32_t n, uint32_t k, int bits, boo
     const uint64_t rounds = (uint64_t)((m + 255u) / 256u) * cols256 / cus;
     const uint64_t candidates[] = {rounds * cus / cols256 * 256u, cus / cols128 * 256u, cus / cols128 * 128u, (m - 1u) / 256u * 256u,
                                    (m - 1u) / 256u * 256u - 256u};
-    const double one = launch_time_us(m, n, k, bits, packed);
+    const double one = launch_time_us(m, n, k, bits, packed, grouped);
     // (0.94: the estimates' error.  Of 200 shapes, m = 257 .. 4096, 25 go in two launches so, 1.25 times
     // as fast on average and none slower; at 0.97 three of 49 are, by 4 - 9 %)
     double best = 0.94 * one;
@@ -1590,9 +1593,9 @@ static uint32_t row_split_rule(uint32_t m, uint32_t n, uint32_t k, int bits, boo
         if (asked) continue;
         const uint32_t rows = (uint32_t)c;
         // (no launch is estimated at less than 2 us: most candidates need no look at their rest)
-        const double first = launch_time_us(rows, n, k, bits, packed) + 1.0;
+        const double first = launch_time_us(rows, n, k, bits, packed, grouped) + 1.0;
         if (first + 2.0 >= best) continue;
-        const double two = first + launch_time_us(m - rows, n, k, bits, packed);
+        const double two = first + launch_time_us(m - rows, n, k, bits, packed, grouped);
         if (two >= best) continue;
         if (row_split_workspace(rows, m - rows, n, k, bits, packed) > BFAINTB_STATIC_SCRATCH_BYTES) continue;
         best = two;
@@ -1605,17 +1608,17 @@ static uint32_t row_split_rule(uint32_t m, uint32_t n, uint32_t k, int bits, boo
 // thread keeps the last answers, one per slot of a hash of the question.  A new question costs 0.9 - 1.8 us of host time, where
 // one launch's plan takes 0.15; a known one 0.2, or 0.5 if the answer is two launches.  A prompt of a new length asks once per
 // shape of its layers, as long as no two of them share a slot)
-static uint32_t row_split_head(uint32_t m, uint32_t n, uint32_t k, int bits, bool packed)
+static uint32_t row_split_head(uint32_t m, uint32_t n, uint32_t k, int bits, bool packed, bool grouped)
 {
     if (m <= 256u) return 0;
     struct Answer {
         uint32_t m, n, k, kind, cus, row_block, head;
     };
     static thread_local Answer answers[256] = {};
-    const uint32_t kind = (uint32_t)bits * 2u + (packed ? 1u : 0u), cus = machine_cus(), row_block = g_force_row_block.load(std::memory_order_relaxed);
+    const uint32_t kind = (uint32_t)bits * 4u + (packed ? 2u : 0u) + (grouped ? 1u : 0u), cus = machine_cus(), row_block = g_force_row_block.load(std::memory_order_relaxed);
     Answer& a = answers[((m * 2654435761u) ^ (n * 2246822519u) ^ (k * 3266489917u) ^ kind) >> 24];
     if (a.m != m || a.n != n || a.k != k || a.kind != kind || a.cus != cus || a.row_block != row_block)
-        a = Answer{m, n, k, kind, cus, row_block, row_split_rule(m, n, k, bits, packed)};
+        a = Answer{m, n, k, kind, cus, row_block, row_split_rule(m, n, k, bits, packed, grouped)};
     return a.head;
 }
 
@@ -1625,7 +1628,7 @@ size_t bfaintb_gemm_prepacked_workspace_bytes_ex(uint32_t m, uint32_t n, uint32_
     const int v = packed_variant(m, n, k, weight_bits, variant);
     if (v < 0) return 0;
     if (variant == BFAINTB_VARIANT_AUTO) {
-        const uint32_t head = row_split_head(m, n, k, weight_bits, true);
+        const uint32_t head = row_split_head(m, n, k, weight_bits, true, group_size != 0);
         if (head != 0u) return row_split_workspace(head, m - head, n, k, weight_bits, true);
     }
     return packed_workspace_need(m, n, k, weight_bits, v);
@@ -1656,7 +1659,7 @@ static int gemm_prepacked_impl(void* c, const void* a, const void* packed_b, con
         misaligned16(ep.residual))
         return BFAINTB_ERR_ALIGNMENT;
     if (!whole && variant == BFAINTB_VARIANT_AUTO) {
-        const uint32_t head = row_split_head(m, n, k, weight_bits, true);
+        const uint32_t head = row_split_head(m, n, k, weight_bits, true, group_size != 0);
         if (head != 0u && row_split_served(workspace, workspace_bytes, row_split_workspace(head, m - head, n, k, weight_bits, true), false,
                                            static_cast<hipStream_t>(stream))) {
             e = gemm_prepacked_impl(c, a, packed_b, scale, ep, head, n, k, lda, ldc, weight_bits, group_size, workspace, workspace_bytes, stream, variant,
@@ -1975,7 +1978,7 @@ int bfaintb_gemm_plan(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint3
     const int v = packed ? packed_variant(m, n, k, weight_bits, variant) : resolve_variant(m, n, k, weight_bits, variant);
     if (v < 0) return v;
     if (variant == BFAINTB_VARIANT_AUTO && (packed || split_k == 0)) {
-        const uint32_t head = row_split_head(m, n, k, weight_bits, packed != 0);
+        const uint32_t head = row_split_head(m, n, k, weight_bits, packed != 0, group_size != 0);
         if (head != 0u) {  // the first launch, described as such; of the second one its workgroups
             bfaintb_plan rest;
             e = plan_whole(head, n, k, weight_bits, group_size, packed, variant, 0, out);
