@@ -204,18 +204,20 @@ static uint32_t tall_tile_blocks(uint32_t m)
     const uint32_t rows_of_tiles = (m + 255u) / 256u, needed = (m + 16u * rows_of_tiles - 1u) / (16u * rows_of_tiles);
     return needed <= 10u ? 10u : needed <= 12u ? 12u : 16u;
 }
-// Up to a k of 1024 (2048 for tiles of 10 blocks, where launches by rows compete with them) the form that adds an output's products in
-// one chain, as the large tiles do, to the same bits (bfaintb_prefill256x128_wreg_kernel); beyond it the small tiles' kernel with 10 to
-// 16 blocks of 16 rows.  us, one chain / 16 blocks, k = 512 / 1024 / 2048 / 4096: 2048 x 4096 8-bit 17.2 / 16.6, 25.0 / 23.1, 40.2 / 35.6,
-// 70.8 / 63.0; 512 x 11008 4-bit 17.7 / 15.6, 25.4 / 21.2, 40.8 / 31.9, 71.6 / 53.9.
+// Up to a k of 1024 (2048 for tiles of 10 blocks) the form that adds an output's products in one chain of ascending k, as the large tiles do:
+// a product of a short k has the bits of the large tiles, whichever of the two its size picks (bfaintb_prefill256x128_wreg_kernel).  That is
+// the whole reason: beyond it the small tiles' kernel with 10 to 16 blocks of 16 rows, which adds two chains, runs, and below it it would
+// mostly be the faster one as well.  us, one chain / the other, k = 512 / 1024 / 2048 / 4096: 16 blocks, 2048 x 4096 8-bit 17.3 / 17.0, 24.8 /
+// 24.1, 40.2 / 35.5, 70.9 / 63.3; 512 x 11008 4-bit 17.2 / 15.1, 24.9 / 20.5, 40.7 / 31.5, 71.8 / 54.2; 10 blocks, 300 x 12288 8-bit 15.2 / 11.0, 22.0 /
+// 15.8, 35.0 / 24.6, 61.9 / 41.4; the other way round where 8-bit rows lie a large power of two apart and k is 512 (384 x 16384 16.0 / 21.4).
 static bool tall_tiles_in_one_chain(uint32_t m, uint32_t k) { return k <= (tall_tile_blocks(m) == 10u ? 2048u : 1024u); }
 
-// The tiled variant runs 128x128 tiles while those fit one per CU: four times the workgroups of
-// 256x256 tiles, each with a quarter of the work per K-step.  Measured against the large tiles (8-bit, k = 4096, us):
-// m x n = 256 x 4096: 48 / 59, 1024 x 4096: 58 / 66, 512 x 8192 (4-bit, k = 8192): 112 / 137; with more tiles the
-// large ones win (1536 x 4096: 81 / 72, 512 x 11008: 80 / 68).
-// (One gap: a few tall tiles more than CUs — 640 x 11008 makes 258 — would go to 129 large tiles on half the machine, 82 us;
-// the small tiles take it in two rounds, 430 of them, in 66 us.  So: also up to two rounds of small tiles where the tall
+// The tiled variant runs small tiles, of 128 columns and at most 128 rows, while those fit one per CU: four times the workgroups of
+// 256x256 tiles, each with a quarter of the work per K-step.  Measured against the tall and the large tiles (8-bit, k = 4096, us,
+// small / tall / large): 256 x 4096: 33.7 / 48.2 / 58.5, 1024 x 4096: 41.1 / 50.6 / 60.0, 512 x 8192 (4-bit, k = 8192): 78.2 / 95.6 / 133; with more
+// tiles the others win (1536 x 4096: 67.4 / 54.7 / 60.8, 512 x 11008: 67.2 / 54.5 / 60.7).
+// (One gap: a few tall tiles more than CUs — 640 x 11008 makes 258, two rounds, 98.5 us — would go to 129 large tiles on half the machine,
+// 85.7 us; the small tiles take it in two rounds, 430 of them, in 70.8 us.  So: also up to two rounds of small tiles where the tall
 // ones do not fit one round and the large ones fill at most 60 % of the CUs.)
 static bool prefill_small_tiles(uint32_t m, uint32_t n, uint32_t k, int bits)
 {
@@ -223,25 +225,25 @@ static bool prefill_small_tiles(uint32_t m, uint32_t n, uint32_t k, int bits)
     const uint64_t small = (uint64_t)((m + 127u) / 128u) * ((n + 127u) / 128u);
     if (small <= cus) return true;
     // One row of tiles: 256-row tiles would spend half their matrix instructions or more on rows that do not exist, however
-    // many rounds the small ones take (us, small / large, 8-bit and 4-bit codes: 64 x 128256 x 4096, 1002 small tiles, 152 / 187
-    // and 148 / 203; 128 x 128256 x 4096 171 / 202 and 163 / 210; 96 x 50304 x 4096, 393 tiles, 71 / 86 and 69 / 101;
-    // 128 x 36864 x 8192, 288 tiles, 134 / 157 and 135 / 135; from 129 rows on the large tiles win: 192 x 50304 x 4096 132 / 97)
+    // many rounds the small ones take (us, small / large, 8-bit and 4-bit codes: 64 x 128256 x 4096, 1002 small tiles, 126 / 187
+    // and 119 / 203; 128 x 128256 x 4096 169 / 204 and 163 / 210; 96 x 50304 x 4096, 393 tiles, 66.5 / 86.5 and 65.1 / 102;
+    // 128 x 36864 x 8192, 288 tiles, 135 / 158 and 133 / 193; from 129 rows on the large tiles win: 192 x 50304 x 4096 123 / 98)
     if (m <= 128u) return true;
-    // 4-bit codes: two rounds of small tiles beat one of tall ones while the second round is about a third full (the tall
-    // kernel converts every weight in two waves; us, small / tall, on two boxes: 1152 x 4096 x 4096, 288 tiles: 65.8 / 70.7
-    // and 68.9 / 70.9; 512 x 11008 x 4096, 344: 65.9 / 71.1; with 384 to 448 tiles the second box had them level or the tall
-    // ones ahead by 2 %, and packed weights by up to 4 %; 8-bit codes the other way throughout: 63.1 / 59.2 at 288 tiles)
+    // 4-bit codes where the tall tiles would be those of one chain, whose kernel converts every weight in two waves: small ones while a
+    // second round of them is about a third full.  Made when a long k ran so as well (k = 4096, us, small / one chain: 1152 x 4096, 288 tiles,
+    // 67.2 / 71.0; 512 x 11008, 344, 69.7 / 72.0); at the k that is left of it the two are level to a tenth apart (k = 1024: 25.2 / 24.5 and 25.1 /
+    // 24.9; k = 512: 18.4 / 16.7 and 18.5 / 17.1), and the rule goes with the tall tiles' (8-bit codes: 23.4 / 21.5 at 1152 x 4096 x 1024).
     if (bits == 4 && tall_tiles_in_one_chain(m, k) && small * 20u <= cus * 27u) return true;
     const uint64_t tall = (uint64_t)((m + 255u) / 256u) * ((n + 127u) / 128u);
     const uint64_t large = (uint64_t)((m + 255u) / 256u) * ((n + 255u) / 256u);
-    // (0.6 of the CUs at most: 640 x 12032 x 3584, 141 large tiles, 76.2 us; 470 small ones 67.6)
+    // (0.6 of the CUs at most: 640 x 12032 x 3584, 141 large tiles, 76.5 us; 470 small ones 66.5)
     return small <= 2u * cus && tall > cus && large * 5u <= cus * 3u;
 }
 
 // Between the two: more small tiles than CUs, but at most one tile of 256 rows x 128 columns per CU.  The large tiles would
-// occupy a quarter to a half of the CUs there; the tall ones run one per CU at 0.94 us per K-step against the large tiles'
-// 1.02 on twice the work (8-bit, 64 steps, us tall / large: 1536 x 4096: 61.0 / 66.0; 512 x 11008: 60.3 / 64.7; 2048 x 4096:
-// 71.0 / 75.7; 128 steps, 1024 x 8192: 129 / 141; 4-bit, 768 x 8192: 138 / 140).
+// occupy a quarter to a half of the CUs there; the tall ones run one per CU and share one conversion among 10 to 16 blocks of rows
+// (us, tall / large, 8-bit, 64 steps: 1536 x 4096: 54.7 / 60.8; 512 x 11008: 54.5 / 60.7; 2048 x 4096: 63.4 / 72.3; 128 steps,
+// 1024 x 8192: 117 / 133; 4-bit, 768 x 8192: 103 / 134).
 static bool prefill_tall_tiles(uint32_t m, uint32_t n, uint32_t k, int bits)
 {
     return !prefill_small_tiles(m, n, k, bits) && (uint64_t)((m + 255u) / 256u) * ((n + 127u) / 128u) <= machine_cus();
@@ -323,8 +325,10 @@ static TilePlan tile128_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint3
         const double wgs = tiles * t.splits;
         const double whole = (double)(uint64_t)(wgs / cus), rest = wgs - whole * cus;
         if (!second_launch) {
-            // (a caller who brings the scratch that a call needed before there were second launches is served with that much: the
-            // choice among these plans, and between them and the family, goes by the estimates of that time)
+            // (A caller who brings the scratch that a call needed before there were second launches, or none, is served with that much.  So these
+            // plans, and the choice between them and the family, go by the steps' times of then, not by what the kernels take now: the
+            // estimate decides how much scratch such a caller has to bring, and by today's steps 206 of 8000 random calls without any, 33 ...
+            // 1500 rows, would be refused that are served.  What it costs is a slower plan for a caller with too little scratch.)
             auto step_us = [&](double load) { return ((bits == 4 ? 0.41 : 0.40) + 0.15 * load * load * load) * (0.8 + 0.2 * fill); };
             t.us = 4.0 + (wgs > 2.0 * cus ? 1.12 : 1.0) * per * (whole * step_us(1.0) + (rest > 0.0 ? step_us(rest / cus) : 0.0)) +
                    (t.splits > 1u ? 3.0 + (t.splits - 1.0) * (0.6 + 1.6 * fill + 0.008 * tiles) : 0.0);
@@ -371,10 +375,10 @@ static TilePlan tile128_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint3
     }
     // One row of tiles that leaves a third or more of the CUs idle (half to five eighths of a round) and a long k: three
     // splits, as the decode family does on such widths — the estimate has the two forms level, the machine does not (us,
-    // unsplit / three splits, 8-bit and 4-bit codes: 48 x 18432 x 8192, 144 tiles, 56.0 / 47.2 and 50.3 / 42.9; 96 x 18432 x
-    // 8192 62.1 / 57.3 and 59.2 / 54.0; 48 x 20480 x 8192, 160 tiles, 60.3 / 51.1 and 50.6 / 43.1).  The launch rounds a split's
-    // workgroups up to a multiple of 8, and three splits must stay clear of two rounds: 170 tiles make 528 and lose (57.9 /
-    // 69.7).  A shorter k gains little or loses (k = 6144: 35.3 / 33.4 at 48 rows, 42.5 / 43.4 at 96; k = 4096: 25.1 / 27.2).
+    // unsplit / three splits, 8-bit and 4-bit codes: 48 x 18432 x 8192, 144 tiles, 51.9 / 47.3 and 51.8 / 45.2; 96 x 18432 x
+    // 8192 63.8 / 59.0 and 58.6 / 53.9; 48 x 20480 x 8192, 160 tiles, 56.2 / 51.8 and 52.1 / 45.7).  The launch rounds a split's
+    // workgroups up to a multiple of 8, and three splits must stay clear of two rounds: 170 tiles make 528 and lose (44.7 /
+    // 65.5).  A shorter k gains little or loses (k = 6144: 40.5 / 40.3 and 40.3 / 37.6 at 48 rows, 49.5 / 49.4 at 96; k = 4096: 29.2 / 31.6).
     // (While the partial sums stay within the 14 MiB of the note above.)
     const double per_split = (double)(uint64_t)((tiles + 7.0) / 8.0) * 8.0;
     if (best.splits == 1u && m <= 128u && tiles * 2.0 > cus && per_split * 3.0 * 16.0 <= cus * 31.0 && k >= 8192u &&
@@ -765,7 +769,9 @@ int resolve_variant(uint32_t m, uint32_t n, uint32_t k, int bits, int variant, b
 //     24.6, 4-bit 18.0 / 24.3).
 //   - packed 4-bit codes, however many rounds: 22016 x 4096 23.5 / 21.1, 32768 x 4096 27.4 / 22.7, 27008 x 1280 12.7 / 10.8, 50304 x
 //     4096 44.9 / 40.6; level at k = 6144 (29.5 / 29.3), behind at 8192 (36.2 / 38.6), where the family's longer walk amortises its
-//     start; and where k is 2048, at which every column block begins in the same memory channels (22016 columns, 20 rows 12.5 / 13.0).
+//     start.  The family walks in whole steps of 1024 rows and is at its best where k is just those and they are few: over 24 calls each, 18432 to
+//     50304 columns, family / tiles on average 1.09 at k = 1536, 1.00 at 1920, 0.985 at 2048 (0.945 - 1.03), 1.15 at 2176 (a third step), 1.14
+//     at 2560, 1.06 at 3072, 1.11 at 4096, 1.03 at 5120: so not at 2048, its two whole steps.
 //   - packed 8-bit codes: 20480 x 4096 22.9 / 20.7, 22016 x 5120 28.6 / 26.5, 50304 x 4096 47.5 / 44.0; a short k has too few steps to
 //     fill the pipeline (22016 x 2048 15.6 / 17.3), a long one is level or behind (28672 x 6144, 20 rows 31.4 / 33.3), and so are several rounds with one scale per column
 //     (50944 x 3456, 20 rows 38.4 / 40.5, 34560 x 3584, 29 rows 38.5 / 40.3; groups of 128, 47344 x 4096, 30 rows 49.2 / 44.1).
@@ -1370,7 +1376,9 @@ static DecodePlan packed_family_plan(uint32_t m, uint32_t n, uint32_t k, int bit
 // 5120 x 13824, m = 16: slab 31.0, family 17.2; 13824 x 5120: 26.0 / 15.5; 4096 x 2048, m = 32: 5.5 / 6.9; 1024 x 16384,
 // m = 1: 10.5 / 9.0.  8-bit codes, m = 8: 5120 x 13824 23.2 / 16.3; 13824 x 5120 20.2 / 15.0; 5120 x 5120 11.3 / 9.2;
 // 2048 x 4096, m = 12: 5.5 / 6.9).  Picks on the scan, weights cold: 4-bit 9 of 252 more than 5 % off the faster kernel
-// (worst 12 %), 8-bit 12 of 252 (worst 14 %); fixed row limits, as before: 22 of 196, up to 42 %.
+// (worst 12 %), 8-bit 12 of 252 (worst 14 %); fixed row limits, as before: 22 of 196, up to 42 %.  With the conversion by halves both
+// 4-bit kernels are 1 - 9 % faster than fitted, and the picks hold: over the 28 shapes, 10 row counts and groups of 128 or none, 16 of 560 more
+// than 5 % off, 0.4 % over the faster kernel on average (worst 8192 x 28672, 1 row: slab 35.9, family 29.0).
 static double packed_slab_walks(uint32_t n)
 {
     const double cus = (double)machine_cus();
