@@ -11,6 +11,15 @@ pytestmark = pytest.mark.gpu
 FORMATS = [(8, 0), (8, 64), (8, 32), (4, 0), (4, 128), (4, 32)]
 
 
+def run_padded(p, pad_a, ldb, which=0, split=0):
+    """run_gemm with rows of A pad_a elements longer (NaNs there) and rows of B ldb codes apart (codes there that must not count)."""
+    a = np.full((p.m, p.k + pad_a), 0x7FC0, np.uint16)
+    a[:, :p.k] = p.a_bf
+    b = np.random.default_rng(9).integers(0, 256, size=(p.k, ldb * p.bits // 8), dtype=np.uint8)
+    b[:, :p.n * p.bits // 8] = np.asarray(p.b_bytes).reshape(p.k, -1)
+    return run_gemm(p, which=which, force_split_k=split, lda=p.k + pad_a, ldb=ldb, a_dev=to_dev(a), b_dev=to_dev(b))
+
+
 def run(af, p, packed, which):
     import torch
     if not packed:
@@ -51,6 +60,25 @@ def test_tall_tiles(m, n, k, blocks, bits, group, packed):
         c = run(af, p, packed, af.PREFILL)
         assert_close_ulp(p, c, f"{blocks} blocks: {m}x{n}x{k} bits={bits} g={group} packed={packed}")
         assert np.array_equal(run(af, p, packed, af.PREFILL), c), "not reproducible"
+    finally:
+        af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 0)
+
+
+# the same over rows of A and B that are longer than they need be, for columns of which the last 16 are half (8-bit codes), a k that is no multiple
+# of a K-step, and the small tiles beside them
+@pytest.mark.parametrize("m,n,k,rows", [(305, 648, 2184, 160), (384, 648, 1160, 192), (391, 648, 1416, 256), (512, 648, 1160, 256), (300, 264, 1160, 128), (70, 136, 520, 96), (40, 136, 520, 64)])
+@pytest.mark.parametrize("bits,group", [(8, 0), (4, 0)])
+def test_longer_rows_and_ragged_columns(m, n, k, rows, bits, group):
+    import awesome_fusion_amd as af
+    n += 8 if bits == 4 else 0
+    try:
+        af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 14)
+        pl = af.plan(m, n, k, bits, group, which=af.PREFILL)
+        assert (pl.kernel, pl.tile_rows, n % 16) == (af.KERNEL_TILES_128, rows, 8 if bits == 8 else 0), pl.as_dict()
+        p = Problem(m, n, k, bits, group, seed=m + k + bits)
+        c = run_padded(p, 24, (n + 40) // 16 * 16, af.PREFILL)
+        assert_close_ulp(p, c, f"{rows} rows: {m}x{n}x{k} bits={bits}")
+        assert np.array_equal(run_padded(p, 0, (n + 15) // 16 * 16, af.PREFILL), c)
     finally:
         af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 0)
 
@@ -129,6 +157,60 @@ def test_few_rows_choose_tiles(m, n, k, bits, group, packed):
             assert_close_ulp(p, run_gemm(p), "bias and residual")
             g = Problem(m, n, k, bits, group, seed=3, scale_lo=0.002, scale_hi=0.02 if bits == 8 else 0.2).with_bias()
             assert_close_gated(g, run_gemm(g, activation=af.ACT_SILU_GATE), "gated")
+    finally:
+        af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 0)
+
+
+# ... over longer rows of A and B: the choice goes by the call's own distance of rows, a multiple of 1024 codes gets the family, any other the tiles
+# (test_launches.py); a k that is no multiple of a K-step, columns of which the last 16 are half
+@pytest.mark.parametrize("m,n,k,bits,group", [(17, 648, 1032, 8, 0), (32, 1000, 1088, 8, 64), (21, 592, 1032, 4, 0), (32, 1008, 1664, 4, 128)])
+def test_few_rows_over_longer_rows(m, n, k, bits, group):
+    import awesome_fusion_amd as af
+    try:
+        af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 8)
+        p = Problem(m, n, k, bits, group, seed=m + n + k)
+        tiles, family = run_padded(p, 40, 2048 + 16), run_padded(p, 40, 2048)
+        assert_close_ulp(p, tiles, "tiles")
+        assert_close_ulp(p, family, "family")
+        assert np.array_equal(run_padded(p, 0, (n + 15) // 16 * 16, af.PREFILL_128, 1), tiles) and np.array_equal(run_padded(p, 0, 1024, af.DECODE), family)
+    finally:
+        af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 0)
+
+
+@pytest.mark.parametrize("m,n,k,bits,group,packed", [(17, 656, 1032, 8, 0, False), (32, 1552, 3072, 8, 64, True), (24, 592, 1152, 4, 128, True)])
+def test_few_rows_on_tiles_under_capture(m, n, k, bits, group, packed):
+    """Recorded into a graph and replayed over new activations, other work on the same scratch between the replays."""
+    import torch
+    import awesome_fusion_amd as af
+    try:
+        af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 8)
+        assert af.plan(m, n, k, bits, group, packed=packed).tiles_instead
+        problems = [Problem(m, n, k, bits, group, seed=s) for s in (1, 2, 3)]
+        b, s = to_dev(problems[0].b_bytes), to_dev(problems[0].s_bf)
+        if packed:
+            w = torch.empty(af.prepack_bytes(n, k, bits), dtype=torch.uint8, device="cuda")
+            af.prepack(w, b, n, k, weight_bits=bits)
+            b = w
+        a, c = to_dev(problems[0].a_bf), torch.zeros((m, n), dtype=torch.int16, device="cuda")
+        ws = helpers._ws.get(max(af.workspace_bytes(m, n, k, bits, group), af.prepacked_workspace_bytes(m, n, k, bits, group) if packed else 0, af.workspace_bytes(4, n, 4096)))
+        call = af.gemm_prepacked if packed else af.gemm
+        af.init()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            call(c, a, b, s, m, n, k, weight_bits=bits, group_size=group, workspace=ws)
+        for i, q in enumerate(problems):
+            a.copy_(to_dev(q.a_bf))
+            c.fill_(0x7FC0)
+            graph.replay()
+            torch.cuda.synchronize()
+            got = from_dev_u16(c)
+            q.q, q.b_bytes, q.s_bf, q._w = problems[0].q, problems[0].b_bytes, problems[0].s_bf, None
+            assert_close_ulp(q, got, f"replay {i}")
+            call(c, a, b, s, m, n, k, weight_bits=bits, group_size=group, workspace=ws)
+            torch.cuda.synchronize()
+            assert np.array_equal(from_dev_u16(c), got)
+            run_gemm(Problem(4, n, 4096, 8, 0, seed=5))   # a split call on the same scratch
     finally:
         af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 0)
 

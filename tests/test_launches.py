@@ -89,7 +89,7 @@ def test_the_plan_describes_what_is_launched(tmp_path):
     import awesome_fusion_amd as af
     asked = [(s, b, g, pk, rows, v) for s, b, g, pk, rows in PLANS
              for v in (af.AUTO, af.DECODE, af.PREFILL, af.PREFILL_128, af.PREFILL_256, af.PREFILL_256X128, af.PREFILL_128_LDS, af.PREFILL_256_LDS)]
-    r = on_stand_in(tmp_path, "plan_launches", "\n".join("%d %d %d %d %d %d %d" % (*s, b, g, pk, v) for s, b, g, pk, _, v in asked))
+    r = on_stand_in(tmp_path, "plan_launches", "\n".join("%d %d %d %d %d %d %d 0" % (*s, b, g, pk, v) for s, b, g, pk, _, v in asked))
     assert r.returncode == 0
     answers = [tuple(map(int, line.split())) for line in r.stdout.split("\n") if line]
     assert len(answers) == len(asked)
@@ -107,6 +107,23 @@ def test_the_plan_describes_what_is_launched(tmp_path):
         assert tail <= did_others or wgs == 0, what
         kinds.add((kernel, rows))
     assert {(af.KERNEL_TILES_128, r) for r in (32, 64, 96, 128, 160, 192, 256)} <= kinds and (af.KERNEL_TILES_256X128, 256) in kinds
+
+
+def test_few_rows_choose_by_the_calls_own_distance_of_rows(tmp_path):
+    """17 to 32 rows over codes in rows: rows a multiple of 1024 codes apart get the family's launch, whatever n; others the tiles'."""
+    import awesome_fusion_amd as af
+    asked, wants = [], []
+    for m, n, k, bits, group in ((17, 22016, 2048, 8, 0), (32, 22016, 4096, 8, 128), (32, 22528, 4096, 8, 0), (32, 22016, 4096, 4, 128), (20, 22016, 4096, 4, 128)):
+        family, tiles = af.plan(m, n, k, bits, group, which=af.DECODE), (n + 127) // 128
+        for ldb in (0, n + 16, n + 128, n // 1024 * 1024 + 1024, 32768):
+            pitch = ldb or n   # (up to 20 rows of 4-bit codes: only where rows are not whole lines)
+            on_tiles = pitch % 1024 != 0 and (bits == 8 or m > 20 or pitch % 256 != 0)
+            asked.append("%d %d %d %d %d 0 0 %d" % (m, n, k, bits, group, ldb))
+            wants.append((9, (tiles + 7) // 8 * 8) if on_tiles else (family.waves, family.workgroups))
+    r = on_stand_in(tmp_path, "plan_launches", "\n".join(asked))
+    assert r.returncode == 0
+    got = [tuple(int(x) for x in line.split()[11:13]) for line in r.stdout.split("\n") if line]
+    assert got == wants, [x for x in zip(asked, got, wants) if x[1] != x[2]]
 
 
 @pytest.mark.gpu
