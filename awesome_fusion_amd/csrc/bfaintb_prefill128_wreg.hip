@@ -24,8 +24,9 @@
 //     4096 8-bit 70.8 / 63.0; 512 x 11008 x 4096 8-bit 63.0 / 52.1, 4-bit 71.6 / 53.9; 512 x 13824 x 5120 packed 4-bit 85.4 / 73.1.
 //   - no row blocks that do not exist: MT = 2, 4, 6, 8, 10, 12, 16, the rows spread evenly over the tiles (96 x 20480 x 4096 packed 8-bit 32.9
 //     with eight blocks / 29.1 with six).
-//   - the conversion by half-precision magic numbers (see there) and codes by transposing reads: 42 vector and 16 LDS instructions a wave
-//     and step before, 34 and 10 now (64 x 4096 x 11008 8-bit unsplit, codes in the last-level cache: 55.9 -> 49.2).
+//   - the conversion by half-precision magic numbers (bfaintb_device.hpp) and codes by transposing reads: 42 vector and 16 LDS instructions a
+//     wave and step of eight blocks before, 34 and 10 now, counted in the compiled loop for 8-bit codes and a scale for each column (64 x 4096 x
+//     11008 8-bit unsplit, codes in the last-level cache: 55.9 -> 49.2); 43 to 45 vector ones with group scales, whose multipliers are new every step.
 //   - more stages the fewer rows there are, since such launches read their codes from memory and wait for it: 64 x 4096 x 11008 8-bit
 //     unsplit, codes cold, 4 / 8 stages 69.2 / 63.1; 96 rows 4-bit g128, 4 / 6 stages 88.9 / 78.6.
 //   - for 17 to 32 rows, whose calls read every code once, from memory: the copying wave and eight stages whatever the codes (32 x 22016 x

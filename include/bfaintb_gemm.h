@@ -6,6 +6,11 @@
  * A, C: bf16, row-major.  B: packed integer codes q, row-major K x N.  fp32 accumulation, one
  * rounding (to nearest even) when W is formed and one when C is stored.
  *
+ * The order in which an output's products are added in fp32 follows from the call's arguments, the device's plan and
+ * the output's place, never from timing: the same call gives the same bits.  It does depend on the place: equal columns
+ * of W in different column blocks may differ in the last bit (over pre-packed 8-bit codes each column block starts its
+ * walk along k at a step of its own), and so may equal rows of A in calls of another m or in a product made in two launches.
+ *
  * The entry points replace the raw module launch of the reference driver
  * (/root/reference/bfAintBGemm/bfAintBGemm.cc:65-66 hipModuleLoad/hipModuleGetFunction and
  * :119-152 packed kernarg + hipModuleLaunchKernel).  The argument order of bfaintb_gemm is that
