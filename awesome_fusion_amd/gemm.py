@@ -14,10 +14,10 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB = _PACKAGE_LIB = os.path.join(_HERE, "libbfaintb_gemm.so")
 
 AUTO, DECODE, PREFILL = 0, 1, 2
-PREFILL_256, PREFILL_128 = 3, 4  # the tiled variant with its tile size forced (tests, tuning)
+PREFILL_256, PREFILL_128 = 3, 4  # the tiled variant with its tile size forced, 256 x 256 or small (tests, tuning)
 PREFILL_256_LDS = 5               # ... and its form with both operands in LDS forced
-PREFILL_128_LDS = 6               # the same for the 128-tile kernel
-PREFILL_256X128 = 7               # tiles of 256 rows x 128 columns, weights in registers
+PREFILL_128_LDS = 6               # the same for the small tiles, of 128 x 128
+PREFILL_256X128 = 7               # tiles of 256 rows x 128 columns in one chain, weights in registers
 ACT_NONE, ACT_SILU_GATE = 0, 1
 
 
