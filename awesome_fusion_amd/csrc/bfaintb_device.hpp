@@ -102,7 +102,7 @@ struct GemmParams {
     uint32_t decode_mb;    // blocks of 16 rows of A per workgroup of the decode variant (1, 2 or 4)
     uint32_t decode_scale_lds;  // byte offset, in dynamic LDS, of the waves' scale tables (packed weights, grouped scales)
     uint32_t splits;     // workgroups along k
-    uint32_t tile_blocks;  // tiles of 128 columns: blocks of 16 rows of a tile
+    uint32_t tile_blocks;  // tiles of 128 columns, and of 256 (0: 16): blocks of 16 rows of a tile
     uint32_t finish_launch;  // small tiles: every split leaves its sums in `partials` (then [splits][m][n]) for a second launch to finish
     unsigned long long* partials;  // [splits - 1][m][n] fp32 partial sums; kEmptyWord wherever none is waiting
     uint32_t partial_bytes;        // size of that area (below 2^31)

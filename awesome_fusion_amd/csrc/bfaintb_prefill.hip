@@ -618,6 +618,12 @@ template <int BITS, bool GROUPED, bool PACKED, bool REF = false>
 static hipError_t launch_prefill_t(const GemmParams& p0, hipStream_t stream, bool wreg = false)
 {
     GemmParams p = p0;
+    if (p.tile_blocks != 0u) {  // tiles of fewer rows (the kernel that keeps the weights in registers only), all of them in one launch
+        if (!wreg || REF) return hipErrorInvalidValue;
+        p.tile_first = 0;
+        p.tile_count = ((p.m + 16u * p.tile_blocks - 1u) / (16u * p.tile_blocks)) * ((p.n + kBN - 1) / kBN);
+        return launch_prefill_wreg(p, BITS, PACKED, stream);
+    }
     const uint32_t tiles = ((p.m + kBM - 1) / kBM) * ((p.n + kBN - 1) / kBN);
     // whole rounds of one workgroup per CU run 256x256 tiles; a last round that would fill at most half of the
     // CUs runs as twice as many half tiles instead (also when there is no whole round at all)
