@@ -390,8 +390,69 @@ static TilePlan tile128_plan(uint32_t m, uint32_t n, uint32_t k, int bits, uint3
     return best;
 }
 
+// Tiles of 256 columns and 16 x blocks rows, all in one launch: the rows spread evenly over the tiles, and as many rows of tiles as make the
+// rounds of one tile per CU come out best (blocks 0: not such tiles).
+struct WideTiles {
+    uint32_t blocks, rows_of_tiles;
+    double us;
+};
+// What they take, in us: fitted to 24000 timings of 7269 random shapes (33 ... 4096 rows, both code widths and weight orders, weights cold), 4.3 %
+// rms.  A K-step is 128 cycles of matrix instructions a block and some 770 (8-bit) or 840 (4-bit codes, mostly with group scales) beside
+// them, at 2.39 GHz while few CUs hold few rows, and at what the board's power leaves otherwise: 0.83 of it with 14 blocks on every CU.
+static double wide_tiles_us(uint32_t blocks, double tiles, uint32_t k, int bits)
+{
+    const double cus = (double)machine_cus();
+    auto step_us = [&](double load) {
+        const double heat = blocks * load, slower = heat <= 7.0 ? 1.0 : heat <= 10.0 ? 1.0 + 0.040 * (heat - 7.0) : 1.12 + 0.012 * (heat - 10.0);
+        return (128.0 * blocks + (bits == 8 ? 770.0 : 840.0) + (blocks < 14u ? 22.0 * (14u - blocks) * load * load : 0.0)) / 2390.0 * slower;
+    };
+    const double whole = (double)(uint64_t)(tiles / cus), rest = tiles - whole * cus;
+    return 6.5 + 0.234 * blocks + 7.3 * (whole + (rest > 0.0 ? 1.0 : 0.0) - 1.0) + (double)((k + 63u) / 64u) * (whole * step_us(1.0) + (rest > 0.0 ? step_us(rest / cus) : 0.0));
+}
+static WideTiles wide_tiles_best(uint32_t m, uint32_t n, uint32_t k, int bits)
+{
+    WideTiles best{0u, 0u, 0.0};
+    const double cols = (double)((n + 255u) / 256u);
+    for (uint32_t blocks = 8; blocks <= 16u; blocks += 2u) {
+        const uint32_t rows = (m + 16u * blocks - 1u) / (16u * blocks);
+        const double us = wide_tiles_us(blocks, rows * cols, k, bits);
+        if (best.blocks == 0u || us < best.us) best = WideTiles{blocks, rows, us};
+    }
+    return best;
+}
+// The 256x256 tiles whose last round, if it is thin, runs as half tiles in a launch of its own (fitted to the same timings: 4 % rms).
+static double square_tiles_us(uint32_t m, uint32_t n, uint32_t k, int bits)
+{
+    const uint32_t tiles = ((m + 255u) / 256u) * ((n + 255u) / 256u), thin = bfaintb::thin_round_tiles(tiles, m, machine_cus());
+    const double load = 2.0 * thin / (double)machine_cus();
+    return (tiles != thin ? wide_tiles_us(16u, tiles - thin, k, bits) : 0.0) + (thin != 0u ? 12.4 + (double)((k + 63u) / 64u) * (0.81 + 0.135 * load * load * load) : 0.0);
+}
+// Whether a tiled launch of the library's own choice goes to them: where neither small nor tall tiles fit one round, unless the 256x256 tiles
+// and their thin last round are estimated faster; and for 97 to 128 rows that make more small tiles than CUs.  Of 7269 random shapes the tall tiles, and
+// the small ones within a round, lead on all but a few; where the 256x256 tiles ran, these are 1.15 times as fast (geometric mean of 1854; 1741 of
+// them faster), where a product ran as two launches by rows 1.07 times.  By this rule, over 4484 other random shapes of 33 ... 4096 rows: 1.046 times
+// as fast on the whole, 871 more than 10 % faster, 9 more than 5 % slower, worst 0.90 (778 x 18976 x 11552 8-bit 329 / 366).  us, before / now: 148 x 43680 x
+// 4096 8-bit g128 101 / 70; 418 x 17728 x 9728 packed 8-bit g128 205 / 150; 577 x 13824 x 5120 packed 4-bit g128 93.0 / 82.8; 913 x 9296 x 3328 packed 8-bit 70.3 /
+// 55.5; 1010 x 17776 x 1024 8-bit 56.8 / 46.0.
+// (At least 96 of them: the estimates are for a machine's worth of tiles.)
+static WideTiles wide_tiles(uint32_t m, uint32_t n, uint32_t k, int bits)
+{
+    const WideTiles none{0u, 0u, 0.0};
+    const uint64_t cus = machine_cus();
+    if (prefill_small_tiles(m, n, k, bits)) {
+        if ((uint64_t)((n + 127u) / 128u) <= cus || m <= 96u || m > 128u || k < 1024u) return none;
+        const WideTiles w = wide_tiles_best(m, n, k, bits);
+        return w.us < 0.95 * tile128_plan(m, n, k, bits, 0).us ? w : none;
+    }
+    if (prefill_tall_tiles(m, n, k, bits)) return none;
+    const WideTiles w = wide_tiles_best(m, n, k, bits);
+    return w.rows_of_tiles * ((n + 255u) / 256u) >= 96u && w.us < square_tiles_us(m, n, k, bits) ? w : none;
+}
+
 static double prefill_estimate_us(uint32_t m, uint32_t n, uint32_t k, int bits, bool second_launch = true)
 {
+    const WideTiles wide = wide_tiles(m, n, k, bits);
+    if (wide.blocks != 0u && second_launch) return wide.us;
     if (prefill_small_tiles(m, n, k, bits)) return tile128_plan(m, n, k, bits, 0, second_launch).us;
     const double cus = (double)machine_cus();
     if (prefill_tall_tiles(m, n, k, bits)) {
@@ -421,6 +482,8 @@ static double family_beside_tiles_us(double us, uint32_t m, uint32_t n, int bits
 // Whether the row-blocked family, at its estimated time, is the one to run.
 static bool family_leads_tiles(double family_us, uint32_t m, uint32_t n, uint32_t k, int bits, bool packed, bool second_launch)
 {
+    // (the family is estimated at 0.8 of what it takes on the shapes that meet the tiles of 256 columns, those at what they take)
+    if (second_launch && wide_tiles(m, n, k, bits).blocks != 0u) return 1.15 * family_us < wide_tiles(m, n, k, bits).us;
     if (!prefill_small_tiles(m, n, k, bits)) return family_us < prefill_estimate_us(m, n, k, bits, second_launch);
     const TilePlan t = tile128_plan(m, n, k, bits, 0, second_launch);
     if (!second_launch) return family_us < t.us;  // (the estimates of the time before: see tile128_plan)
@@ -802,7 +865,10 @@ static hipError_t launch_few_rows_on_tiles(GemmParams p, int bits, bool packed, 
 }
 
 // whether a tiled-variant launch over row-major weights goes to the small-tile kernel that can split k
-static bool tiled_may_split(int v, uint32_t m, uint32_t n, uint32_t k, int bits) { return use_small_tiles(v, m, n, k, bits) && v != BFAINTB_VARIANT_PREFILL_128_LDS; }
+static bool tiled_may_split(int v, uint32_t m, uint32_t n, uint32_t k, int bits)
+{
+    return use_small_tiles(v, m, n, k, bits) && v != BFAINTB_VARIANT_PREFILL_128_LDS && !(v == BFAINTB_VARIANT_PREFILL && wide_tiles(m, n, k, bits).blocks != 0u);
+}
 
 size_t workspace_need(uint32_t m, uint32_t n, uint32_t k, int bits, int variant, uint32_t forced_split)
 {
@@ -1239,6 +1305,10 @@ static int gemm_impl(void* c, const void* a, const void* b, const void* scale, c
     if (p.splits > 1) in_order = std::unique_lock<std::mutex>(workspace_order(p.ws_header));
     if (tiled) {
         if (small_wreg) return (int)bfaintb::launch_prefill128_wreg(p, weight_bits, false, st);
+        if (v == BFAINTB_VARIANT_PREFILL && !p.reference_arith) {
+            p.tile_blocks = wide_tiles(m, n, k, weight_bits).blocks;
+            if (p.tile_blocks != 0u) return (int)bfaintb::launch_prefill(p, weight_bits, st, true);
+        }
         if (v == BFAINTB_VARIANT_PREFILL && !tall_tiles_in_one_chain(m, k) && prefill_tall_tiles(m, n, k, weight_bits) && bfaintb::prefill128_wreg_serves(p)) {
             p.tile_blocks = tall_tile_blocks(m);
             p.k_per_wg = (k + 63u) / 64u * 64u;  // (whole K-steps)
@@ -1545,7 +1615,6 @@ static size_t packed_workspace_need(uint32_t m, uint32_t n, uint32_t k, int bits
 // this rate would be 1.15 (4-bit) to 1.69 (8-bit) times it.  For rows of B that lie n codes apart, as the scratch is asked for.)
 static double launch_time_us(uint32_t m, uint32_t n, uint32_t k, int bits, bool packed, bool grouped)
 {
-    const double cus = (double)machine_cus(), steps = k / 64.0;
     if (few_rows_on_tiles(m, n, k, bits, grouped, packed, n)) return tile128_plan(m, n, k, bits, 1).us;
     if (m <= kDecodeAutoMaxM) return 6.0 + (double)n * k * bits / 8.0 / 3.3e6 * (m <= 16u ? 1.0 : 1.25);
     if (m <= kDecodeFamilyAutoMaxM) {  // (beyond 32 rows the library's own choice asks just this)
@@ -1553,17 +1622,10 @@ static double launch_time_us(uint32_t m, uint32_t n, uint32_t k, int bits, bool 
         if (family_leads_tiles(family, m, n, k, bits, packed, true))
             return prefill_small_tiles(m, n, k, bits) ? family_beside_tiles_us(family, m, n, bits, packed) : family;
     }
+    const WideTiles wide = wide_tiles(m, n, k, bits);
+    if (wide.blocks != 0u) return wide.us;
     if (prefill_small_tiles(m, n, k, bits) || prefill_tall_tiles(m, n, k, bits)) return prefill_estimate_us(m, n, k, bits);
-    const uint32_t tiles = ((m + 255u) / 256u) * ((n + 255u) / 256u);
-    const uint32_t thin = bfaintb::thin_round_tiles(tiles, m, machine_cus()), full = tiles - thin;
-    auto round_us = [&](double load) { return steps * (bits == 8 ? 1.0 + 0.5 * load : 1.1 + 0.45 * load); };
-    const uint32_t whole = full / machine_cus(), rest = full - whole * machine_cus();
-    double us = 4.0 + whole * round_us(1.0) + (rest != 0u ? round_us(rest / cus) : 0.0);
-    if (thin != 0u) {
-        const double load = 2.0 * thin / cus;
-        us += 4.0 + steps * (0.83 + 0.17 * load * load * load);
-    }
-    return us;
+    return square_tiles_us(m, n, k, bits);
 }
 
 static size_t row_split_workspace(uint32_t head, uint32_t rest, uint32_t n, uint32_t k, int bits, bool packed)
@@ -1591,7 +1653,9 @@ static uint32_t row_split_rule(uint32_t m, uint32_t n, uint32_t k, int bits, boo
     const double one = launch_time_us(m, n, k, bits, packed, grouped);
     // (0.94: the estimates' error.  Of 200 shapes, m = 257 .. 4096, 25 go in two launches so, 1.25 times
     // as fast on average and none slower; at 0.97 three of 49 are, by 4 - 9 %)
-    double best = 0.94 * one;
+    // (0.985 where the one launch is of tiles of 256 columns and as many rows as suit it, whose estimate is nearer)
+    const bool wide = m > kDecodeFamilyAutoMaxM || (packed ? packed_variant(m, n, k, bits, BFAINTB_VARIANT_AUTO) : resolve_variant(m, n, k, bits, BFAINTB_VARIANT_AUTO)) == BFAINTB_VARIANT_PREFILL;
+    double best = (wide && wide_tiles(m, n, k, bits).blocks != 0u ? 0.985 : 0.94) * one;
     uint32_t head = 0;
     for (size_t i = 0; i < sizeof(candidates) / sizeof(candidates[0]); ++i) {
         const uint64_t c = candidates[i];
@@ -1718,6 +1782,10 @@ static int gemm_prepacked_impl(void* c, const void* a, const void* packed_b, con
                 in_order = std::unique_lock<std::mutex>(workspace_order(p.ws_header));
             }
             return (int)bfaintb::launch_prefill128_wreg(p, weight_bits, true, st);
+        }
+        if (v == BFAINTB_VARIANT_PREFILL) {
+            p.tile_blocks = wide_tiles(m, n, k, weight_bits).blocks;
+            if (p.tile_blocks != 0u) return (int)bfaintb::launch_prefill_packed(p, weight_bits, st, true);
         }
         if (v == BFAINTB_VARIANT_PREFILL_256X128 || (v == BFAINTB_VARIANT_PREFILL && prefill_tall_tiles(m, n, k, weight_bits))) {
             p.k_per_wg = k;
@@ -1925,6 +1993,18 @@ static int plan_whole(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint3
         return BFAINTB_OK;
     }
     // the tiled kernels
+    if (v == BFAINTB_VARIANT_PREFILL) {
+        const WideTiles w = wide_tiles(m, n, k, weight_bits);
+        if (w.blocks != 0u) {
+            out->variant = v;  // (no variant names these tiles)
+            out->kernel = BFAINTB_KERNEL_TILES_256;
+            out->tile_rows = 16u * w.blocks;
+            out->tile_cols = 256u;
+            out->waves = 4u;
+            out->workgroups = w.rows_of_tiles * ((n + 255u) / 256u);
+            return BFAINTB_OK;
+        }
+    }
     if (use_small_tiles(v, m, n, k, weight_bits)) {
         out->variant = BFAINTB_VARIANT_PREFILL_128;
         if (v != BFAINTB_VARIANT_PREFILL_128_LDS) {

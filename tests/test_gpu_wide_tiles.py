@@ -1,0 +1,90 @@
+"""Tiles of 256 columns and 128 to 256 rows (bfaintb_prefill_wreg_kernel), every height: at the K-steps where the stages of LDS, the operand sets and
+the fragments' rotation come round or do not, and at partial steps, rows and columns.  On plans for 64 compute units, where small products make
+enough of them.  An output is one chain of products in ascending k, whatever the tile: the form that stages both operands in LDS has its bits."""
+import numpy as np
+import pytest
+
+import helpers
+from helpers import Problem, assert_close_gated, assert_close_ulp, from_dev_u16, run_gemm, to_dev
+
+pytestmark = pytest.mark.gpu
+
+# rows of A one past a row of tiles, so that the last row of tiles holds one (or few) rows; columns half a column block past a tile
+HEIGHTS = [(128, 257, 8208), (160, 385, 8208), (192, 481, 8208), (224, 577, 8208), (256, 673, 12304)]
+# one step, two, three and a partial one, four, five, six, seven and a partial one, thirteen, seven
+STEPS = [(8, 0, 64), (8, 64, 128), (8, 0, 200), (8, 32, 256), (4, 0, 320), (4, 128, 384), (8, 0, 456), (4, 64, 832), (4, 32, 448)]
+
+
+@pytest.fixture
+def units64():
+    import awesome_fusion_amd as af
+    af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 64)
+    yield af
+    af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 0)
+
+
+def run_packed(af, p, which=0, **kw):
+    import torch
+    w = torch.empty(af.prepack_bytes(p.n, p.k, p.bits), dtype=torch.uint8, device="cuda")
+    af.prepack(w, to_dev(p.b_bytes), p.n, p.k, weight_bits=p.bits)
+    c = torch.zeros((p.m, p.n), dtype=torch.int16, device="cuda")
+    af.gemm_prepacked(c, to_dev(p.a_bf), w, to_dev(p.s_bf), p.m, p.n, p.k, weight_bits=p.bits, group_size=p.group_size, which=which, **kw)
+    torch.cuda.synchronize()
+    return from_dev_u16(c)
+
+
+def is_wide(af, rows, p, packed=False):
+    pl = af.plan(p.m, p.n, p.k, p.bits, p.group_size, packed=packed, which=af.PREFILL)
+    assert (pl.kernel, pl.variant, pl.tile_rows, pl.tile_cols, pl.launches, pl.workspace_bytes) == (af.KERNEL_TILES_256, af.PREFILL, rows, 256, 1, 0), pl.as_dict()
+
+
+@pytest.mark.parametrize("rows,m,n", HEIGHTS)
+@pytest.mark.parametrize("bits,group,k", STEPS)
+def test_every_height_has_the_bits_of_the_form_through_lds(units64, rows, m, n, bits, group, k):
+    af = units64
+    p = Problem(m, n, k, bits, group, seed=m + k)
+    is_wide(af, rows, p)
+    c = run_gemm(p, which=af.PREFILL)
+    assert np.array_equal(c, run_gemm(p, which=af.PREFILL_256_LDS))
+    if rows == 160 or k == 200:
+        assert_close_ulp(p, c, f"{rows} rows: {m}x{n}x{k} bits={bits} g={group}")
+    if k % (64 if bits == 8 else 128) == 0:
+        is_wide(af, rows, p, True)
+        assert np.array_equal(run_packed(af, p, af.PREFILL), c), "packed"
+
+
+@pytest.mark.parametrize("rows,m,n", HEIGHTS)
+@pytest.mark.parametrize("bits,group", [(8, 0), (4, 128)])
+def test_epilogues_and_strides(units64, rows, m, n, bits, group):
+    """Bias and residual, the gate, rows of C, A and B that are longer than they need be."""
+    af, k = units64, 384
+    p = Problem(m, n, k, bits, group, seed=rows)
+    is_wide(af, rows, p)
+    assert af.plan(m, n, k, bits, group).as_dict() == af.plan(m, n, k, bits, group, which=af.PREFILL).as_dict()  # (the fused calls name no variant)
+    c = run_gemm(p, which=af.PREFILL)
+    wide = run_gemm(p, which=af.PREFILL, ldc=n + 24, c_fill=0x1234)
+    assert np.array_equal(wide[:, :n], c) and (wide[:, n:] == 0x1234).all()
+    a = np.full((m, k + 24), 0x7FC0, np.uint16)
+    a[:, :k] = p.a_bf
+    b = np.random.default_rng(9).integers(0, 256, size=(k, (n + 32) * bits // 8), dtype=np.uint8)
+    b[:, :n * bits // 8] = np.asarray(p.b_bytes).reshape(k, -1)
+    assert np.array_equal(run_gemm(p, which=af.PREFILL, lda=k + 24, ldb=n + 32, a_dev=to_dev(a), b_dev=to_dev(b)), c)
+    p.with_bias()
+    assert_close_ulp(p, run_gemm(p), "bias", threads=16)
+    p.with_residual()
+    assert_close_ulp(p, run_gemm(p), "bias and residual", threads=16)
+    g = Problem(m, n, k, bits, group, seed=3, scale_lo=0.002, scale_hi=0.02 if bits == 8 else 0.2).with_bias()
+    assert_close_gated(g, run_gemm(g, activation=af.ACT_SILU_GATE), "gated")
+
+
+# beyond 2^117 8-bit codes go a second way along k
+@pytest.mark.parametrize("rows,m,n", HEIGHTS)
+@pytest.mark.parametrize("bits,group,k", [(8, 0, 200), (8, 64, 384), (4, 0, 320), (4, 128, 384)])
+def test_scales_of_any_sign_and_size(units64, rows, m, n, bits, group, k):
+    af = units64
+    p = helpers.scales_of_any_sign_and_size(Problem(m, n, k, bits, group, seed=4))
+    is_wide(af, rows, p)
+    c = run_gemm(p, which=af.PREFILL)
+    helpers.assert_close_at_any_scale(p, c, f"{rows} rows: {m}x{n}x{k} bits={bits} g={group}")
+    if k % 128 == 0:
+        helpers.assert_close_at_any_scale(p, run_packed(af, p, af.PREFILL), f"{rows} rows, packed: {m}x{n}x{k} bits={bits} g={group}")
