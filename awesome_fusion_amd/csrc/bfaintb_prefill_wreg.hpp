@@ -18,14 +18,15 @@
 // Accumulator (mt, j), register r of lane (c16, q = lane / 16): row 16 mt + 4 q + r, column 64 w + 16 j + c16 of the tile.
 //
 // What bounds it: on a full machine the board's power (1.4 kW: the clock gives way to 1.9 GHz); below that what one wave a SIMD issues in order.
-// Measured by switching parts off, cycles a step of 16 blocks (2048 of them the matrix pipe's): the bare loop 2233; LDS reads nothing; one
-// vector instruction in every slot some 1, a second one in a slot 8; a memory request 17 (four waves make theirs at the same time).  Hence
+// Measured by switching parts off, cycles a step of 16 blocks (2048 of them the matrix pipe's): the bare loop 2110; LDS reads 70; one
+// vector instruction in every slot some 1, a second one in a slot 8; a memory request 7 if the step's are spread evenly, 17 to 33 one behind the other
+// (four waves make theirs at the same time, and a copy of 16 bytes a lane takes the memory path 16 cycles).  Hence
 //   - few vector instructions, one a slot: the conversion by halves (128 a step for 8-bit codes, 168 for 4-bit ones with group scales; a
 //     conversion, a multiplication and half a pack were 194 and 250), every one held in the slot it is written for;
-//   - few requests: codes in rows through LDS, 4 or 2 copies a wave and step (16 loads of a dword or less before), the copies of A apart from them;
+//   - few requests, spread over the step: codes in rows through LDS, 4 or 2 copies a wave and step (16 loads of a dword or less before);
 //   - waits that cover many registers at once.
-// Cycles a step, 8-bit codes in rows, one scale a column / 4-bit, groups of 128: 2632 / 3070 before; 2605 / 2790 now with 16 blocks, 2385 / 2455 with 14, 2150 /
-// 2290 with 12, 1920 / 2090 with 10.  us, before / now: 4096 x 4096 x 4096 8-bit in rows 106.7 / 106.6, packed 104.1 / 100.8, 4-bit g128 106.2 / 102.4,
+// Cycles a step, 8-bit codes in rows, one scale a column / 4-bit, groups of 128: 2632 / 3070 before; 2520 / 2700 now with 16 blocks, 1930
+// / 2070 with 10.  us, before / now: 4096 x 4096 x 4096 8-bit in rows 106.7 / 106.6, packed 104.1 / 100.8, 4-bit g128 106.2 / 102.4,
 // packed 107.4 / 102.6; 2048 x 28672 x 8192 4-bit g128 754 / 717, packed 734 / 708; 2560 x 4096 x 4096 4-bit g128 94.5 / 89.0.
 // Fewer blocks: rows spread evenly over the tiles (wide_tiles in bfaintb_capi.hip), so that no matrix instruction is spent on rows
 // that do not exist and the tiles make whole rounds.  us, tiles of 256 rows / as few blocks as serve: 384 x 22016 x 4096 4-bit g128 94.7 / 73.4, 8-bit
@@ -429,28 +430,49 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
     // step ago) or from the code stage S + 1; `raw2` receives the packed codes of step kt + 2.
     // With one wave per SIMD nothing overlaps by itself: the wave issues in order, and the matrix pipe idles whenever the
     // wave is busy issuing something else for longer than a matrix instruction runs (16 cycles).  One vector instruction and one LDS read fit
-    // beside a matrix instruction, a second vector instruction costs some 8 cycles, a memory request some 17 (four waves make theirs at
+    // beside a matrix instruction, a second vector instruction costs some 8 cycles, a memory request 7 or more (four waves make theirs at
     // the same time).  So the step is written as 8 MT fenced slots of one matrix instruction, with everything else spread evenly over them: slot
     // 4 u + j is unit u (row block u % MT of the block of 32 k u / MT), column block j.
     //   fragments of A: a group of four units waits once, for its own, and reads those of the group after the next, one in each unit;
     //   quads: read a quarter of a step before they are prepared, the first two at the end of the step before;
     //   conversion: one instruction after the other (Schedule);
-    //   memory: codes and group scales (rows: of step kt + 3, packed codes: of kt + 2) before the barrier, the copies of A of step kt + 2 behind it.
-    // The step's one barrier stands 32 slots before its end, where the next step's first fragments and codes are about to be read: before it
-    // the wave makes sure that its part of them has landed (what may still be in flight then is this step's own requests).  Behind it
-    // every wave's part has, and every wave has read the last of the stage that this step's copies of A go to (step kt - 1's) and of the code
-    // stage that the next step's go to.
-    constexpr uint32_t kUnits = 2u * MT, kSlots = 8u * MT, kBarrierSlot = kSlots - 32u;
-    constexpr uint32_t kEarly = (GROUPED ? 1u : 0u) + (PACKED ? 4u : kCodeCopies);  // requests before the barrier
-    auto early_slot = [](uint32_t r) constexpr -> uint32_t { return 2u + r * (kBarrierSlot - 2u) / kEarly; };
-    auto copy_slot = [](uint32_t r) constexpr -> uint32_t { return kBarrierSlot + 1u + r * 31u / kACopies; };
-    // LDS reads behind the last fragment of group g and before the group begins: another group's fragments, and quads
+    //   memory: codes and group scales (rows: of step kt + 3, packed codes: of kt + 2) and the copies of A of step kt + 2, evenly over the step.
+    // The step's one barrier stands 24 slots before its end, where the next step's first fragments and codes are about to be read: before it
+    // the wave makes sure that its part of them has landed (requested in the step before: what may still be in flight then is this step's own)
+    // and that it has the fragments of this step.  Behind it every wave's part has landed, and nobody reads this step's stage of A,
+    // or the codes of the next one, any more: the next step's copies go there.
+    constexpr uint32_t kUnits = 2u * MT, kSlots = 8u * MT, kBarrierSlot = kSlots - 24u;
+    // Requests: codes and group scales in their order, the copies of A spread among them.
+    constexpr uint32_t kCodes = (GROUPED ? 1u : 0u) + (PACKED ? 4u : kCodeCopies), kRequests = kCodes + kACopies;
+    auto copies_before = [](uint32_t r) constexpr -> uint32_t { return r * kACopies / kRequests; };
+    auto request_slot = [](uint32_t r) constexpr -> uint32_t { return 2u + r * (kSlots - 2u) / kRequests; };
+    constexpr uint32_t kBeforeBarrier = first_at_least<kRequests>(request_slot, kBarrierSlot);
+    constexpr uint32_t kBehindCodes = [=]() constexpr {  // of a step's requests
+        uint32_t r = 0;
+        while (r - copies_before(r) < kCodes) ++r;
+        return kRequests - r;
+    }();
+    // LDS reads: of unit un's fragment (un < 8: the next step's), of a quad
+    auto frag_slot = [](uint32_t un) constexpr -> uint32_t { return un >= 8u ? 4u * (un - 8u) : kBarrierSlot + 3u * un; };
+    auto quad_slot = [](uint32_t quad) constexpr -> uint32_t {
+        return quad >= 2u ? (quad - 2u) * MT : (quad + 6u) * MT > kBarrierSlot ? (quad + 6u) * MT : kBarrierSlot + 1u;
+    };
+    auto reads_at = [=](uint32_t slot) constexpr -> uint32_t {
+        uint32_t n = 0;
+        for (uint32_t un = 0; un < kUnits; ++un) n += frag_slot(un) == slot ? 1u : 0u;
+        for (uint32_t quad = 0; quad < 8u; ++quad) n += quad_slot(quad) == slot ? kQuadReads[quad & 1u] : 0u;
+        return n;
+    };
+    // ... behind the last fragment of group g and before the group begins; and behind the step's own last one and before the barrier
     auto in_flight = [=](uint32_t g) constexpr -> uint32_t {
-        uint32_t n = 4u;
-        for (uint32_t i = 0; i < 20u; ++i) {
-            const uint32_t slot = (16u * g + kSlots - 20u + i) % kSlots;
-            if (slot % MT == 0u) n += kQuadReads[(slot / MT) & 1u];
-        }
+        uint32_t n = 0;
+        const uint32_t last = frag_slot(4u * g + 3u);
+        for (uint32_t slot = last + 1u; slot < 16u * g + (g < 2u ? kSlots : 0u); ++slot) n += reads_at(slot % kSlots);
+        return n;
+    };
+    auto in_flight_at_barrier = [=]() constexpr -> uint32_t {
+        uint32_t n = 0;
+        for (uint32_t slot = frag_slot(kUnits - 1u) + 1u; slot < kBarrierSlot; ++slot) n += reads_at(slot);
         return n;
     };
     bf16x8_t af[12];
@@ -464,7 +486,7 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
         const uint32_t a_ve = last ? a_last_e : a_voff_e, a_vo = last ? a_last_o : a_voff_o;
         uint32_t a_soff = kt2 * kWrK * 2u;
         Conversion w;
-        if constexpr (PACKED) wait_vm<kACopies>();  // raw1's
+        if constexpr (PACKED) wait_vm<kBehindCodes>();  // raw1's
         __builtin_amdgcn_sched_barrier(0);
         for_each_const<kSlots>([&](auto slot_c) {
             constexpr uint32_t slot = decltype(slot_c)::value;
@@ -473,31 +495,40 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
             mfma16<4u * mt + j>(af[(u + kTurn) % 12u],
                                 __builtin_bit_cast(bf16x8_t, make_uint4(cur.w[blk][j][0], cur.w[blk][j][1], cur.w[blk][j][2], cur.w[blk][j][3])));
             if constexpr (slot == kBarrierSlot) {
-                wait_vm<kEarly>();
+                wait_vm<kBeforeBarrier>();
+                wait_lds<in_flight_at_barrier()>();
                 barrier_no_fence();  // (a fenced barrier would also wait for the copies this step has just started)
             }
-            if constexpr (j == 0u) {  // the fragment of the unit two groups on (the last two groups': the next step's first)
-                constexpr uint32_t un = u + 8u;
-                if constexpr (un < kUnits) af[(un + kTurn) % 12u] = read_frag(Now{}, un / MT, un % MT);
-                else af[(un + kTurn) % 12u] = read_frag(Next{}, 0, un - kUnits);
-            }
-            if constexpr (slot % MT == 0u) {
-                constexpr uint32_t quad = (slot / MT + 2u) & 7u;
-                if constexpr (slot / MT < 6u) read_quad(Next{}, std::integral_constant<uint32_t, quad>{});
-                else read_quad(After{}, std::integral_constant<uint32_t, quad>{});
-            }
+            for_each_const<2u>([&](auto next_c) {  // a fragment: of the unit two groups on; behind the barrier the next step's first
+                constexpr bool next = decltype(next_c)::value != 0u;
+                constexpr uint32_t un = next ? (slot - kBarrierSlot) / 3u : slot / 4u + 8u;
+                if constexpr (next ? slot >= kBarrierSlot && un < 8u && frag_slot(un) == slot : un < kUnits && frag_slot(un) == slot) {
+                    if constexpr (next) af[(un + kUnits + kTurn) % 12u] = read_frag(Next{}, 0, un);
+                    else af[(un + kTurn) % 12u] = read_frag(Now{}, un / MT, un % MT);
+                }
+            });
+            for_each_const<8u>([&](auto quad_c) {
+                if constexpr (quad_slot(decltype(quad_c)::value) == slot) {
+                    if constexpr (decltype(quad_c)::value < 2u) read_quad(After{}, quad_c);
+                    else read_quad(Next{}, quad_c);
+                }
+            });
             constexpr uint32_t from = slot * Schedule::kOps / kSlots, to = (slot + 1u) * Schedule::kOps / kSlots;
             for_each_const<to - from>([&](auto i_c) { convert_op(nxt, w, raw1, std::integral_constant<uint32_t, from + decltype(i_c)::value>{}); });
-            constexpr uint32_t r = first_at_least<kEarly>(early_slot, slot), c = first_at_least<kACopies>(copy_slot, slot);
-            if constexpr (r < kEarly && early_slot(r) == slot) {
-                if constexpr (GROUPED && r == 0u) copy_scales(Now{}, kt3);
-                else if constexpr (PACKED) load_codes(raw2, kt2, std::integral_constant<uint32_t, r - (GROUPED ? 1u : 0u)>{});
-                else copy_codes(Now{}, std::integral_constant<uint32_t, r - (GROUPED ? 1u : 0u)>{}, kt3);
-            }
-            if constexpr (c < kACopies && copy_slot(c) == slot) {
-                copy_a(After{}, std::integral_constant<uint32_t, c>{}, a_ve, a_vo, a_soff);
-                a_soff += 16u * p.lda;
-                asm("" : "+s"(a_soff));  // (or each request gets a multiplication of its own)
+            constexpr uint32_t r = first_at_least<kRequests>(request_slot, slot);
+            if constexpr (r < kRequests && request_slot(r) == slot) {
+                constexpr uint32_t c = copies_before(r), q = r - c;
+                if constexpr (copies_before(r + 1u) != c) {
+                    copy_a(After{}, std::integral_constant<uint32_t, c>{}, a_ve, a_vo, a_soff);
+                    a_soff += 16u * p.lda;
+                    asm("" : "+s"(a_soff));  // (or each request gets a multiplication of its own)
+                } else if constexpr (GROUPED && q == 0u) {
+                    copy_scales(Now{}, kt3);
+                } else if constexpr (PACKED) {
+                    load_codes(raw2, kt2, std::integral_constant<uint32_t, q - (GROUPED ? 1u : 0u)>{});
+                } else {
+                    copy_codes(Now{}, std::integral_constant<uint32_t, q - (GROUPED ? 1u : 0u)>{}, kt3);
+                }
             }
             __builtin_amdgcn_sched_barrier(0);
         });
@@ -536,6 +567,8 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
             });
         });
     }
+    // (the first step's copies of codes and scales go to stage 0: every wave has read it)
+    if constexpr (!PACKED || GROUPED) barrier_no_fence();
     read_quad(C1{}, C0{}), read_quad(C1{}, C1{});
 
 #ifdef BFAINTB_TRACE
