@@ -391,6 +391,38 @@ __device__ __forceinline__ uint4 weights4_by_halves(uint32_t x, const HalfConsta
     return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+// Two weights, of the codes in half PART of h0 and of h1, and their pack, as one piece of assembly: three instructions that stay in the slot of a step they
+// are written in, without the idle cycle that the compiler puts between a v_fma_mix_f32 and whatever reads its result next.
+template <uint32_t PART>
+__device__ __forceinline__ uint32_t pair_of_halves(uint32_t h0, uint32_t h1, float s0, float o0, float s1, float o1)
+{
+    uint32_t w, odd;
+    if constexpr (PART == 0u)
+        asm volatile("v_fma_mix_f32 %0, %2, %4, %5 op_sel_hi:[1,0,0]\n\tv_fma_mix_f32 %1, %3, %6, %7 op_sel_hi:[1,0,0]\n\tv_cvt_pk_bf16_f32 %0, %0, %1"
+                     : "=&v"(w), "=&v"(odd) : "v"(h0), "v"(h1), "v"(s0), "v"(o0), "v"(s1), "v"(o1));
+    else
+        asm volatile("v_fma_mix_f32 %0, %2, %4, %5 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\tv_fma_mix_f32 %1, %3, %6, %7 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\tv_cvt_pk_bf16_f32 %0, %0, %1"
+                     : "=&v"(w), "=&v"(odd) : "v"(h0), "v"(h1), "v"(s0), "v"(o0), "v"(s1), "v"(o1));
+    return w;
+}
+// A value is made here, and not where it is used.
+template <typename T>
+__device__ __forceinline__ void hold(T& v) { asm volatile("" : "+v"(v)); }
+
+// f(0), f(1) .. f(N - 1), the argument a compile-time constant
+template <typename F, size_t... I>
+__device__ __forceinline__ void for_each_const(F&& f, std::index_sequence<I...>) { (f(std::integral_constant<uint32_t, (uint32_t)I>{}), ...); }
+template <uint32_t N, typename F>
+__device__ __forceinline__ void for_each_const(F&& f) { for_each_const(f, std::make_index_sequence<N>{}); }
+// The first of 0 .. N - 1 whose slot is not before `slot`, or N
+template <uint32_t N, typename F>
+__host__ __device__ constexpr uint32_t first_at_least(F slot_of, uint32_t slot)
+{
+    uint32_t v = 0;
+    while (v < N && slot_of(v) < slot) ++v;
+    return v;
+}
+
 // A workgroup barrier without the memory fence that __syncthreads() carries.  That fence makes the compiler wait, before
 // the barrier, for EVERY asynchronous global -> LDS copy issued so far — also the ones meant to land steps later — which
 // turns a pipeline of several stages into one of a single stage.  The caller states what must have completed with

@@ -26,7 +26,12 @@
 //     with eight blocks / 29.1 with six).
 //   - the conversion by half-precision magic numbers (bfaintb_device.hpp) and codes by transposing reads: 42 vector and 16 LDS instructions a
 //     wave and step of eight blocks before, 34 and 10 now, counted in the compiled loop for 8-bit codes and a scale for each column (64 x 4096 x
-//     11008 8-bit unsplit, codes in the last-level cache: 55.9 -> 49.2); 43 to 45 vector ones with group scales, whose multipliers are new every step.
+//     11008 8-bit unsplit, codes in the last-level cache: 55.9 -> 49.2); 38 to 43 vector ones with group scales, whose multipliers are new every step.
+//   - the conversion spread over the slots an instruction or a pair of weights at a time, each where the schedule below puts it, and none
+//     where the codes are still on their way: a pair's two products and its rounding pack are one piece of assembly, so that the compiler, which
+//     fenced them with idle cycles (8 to 11 a step, each of the next instruction's time), sees one result; 2 to 4 are left.  The copies'
+//     requests are spread likewise.  us before / after: 128 x 20480 x 4096 packed 4-bit g128 31.7 / 29.7, 192 x 16384 x 4096 32.6 / 31.5, 64 x
+//     20480 x 4096 packed 4-bit 22.6 / 21.5; over 40000 random shapes of 17 to 700 rows 1.3 % on average, 2.2 % for 33 to 64 rows.
 //   - more stages the fewer rows there are, since such launches read their codes from memory and wait for it: 64 x 4096 x 11008 8-bit
 //     unsplit, codes cold, 4 / 8 stages 69.2 / 63.1; 96 rows 4-bit g128, 4 / 6 stages 88.9 / 78.6.
 //   - for 17 to 32 rows, whose calls read every code once, from memory: the copying wave and eight stages whatever the codes (32 x 22016 x
@@ -72,6 +77,35 @@ __device__ __forceinline__ void tw_settle(f32x4_t (&acc)[MT][2])
         for (int j = 0; j < 2; ++j) asm volatile("" : "+a"(acc[mt][j]));
 }
 }  // namespace
+
+// The order of a step's conversion: what column 0 needs, then its pairs with the instructions that column 1 needs between them, then column 1's pairs.
+struct TwOp {
+    bool pair;  // three instructions, or one
+    uint32_t column, index;
+};
+template <uint32_t PREPARE>
+struct TwSchedule {
+    static constexpr uint32_t kCount = 2u * PREPARE + 8u, kInstructions = 2u * PREPARE + 24u;
+    static constexpr TwOp op(uint32_t at)
+    {
+        if (at < PREPARE) return TwOp{false, 0u, at};
+        at -= PREPARE;
+        for (uint32_t b = 0; b < 4u; ++b) {
+            const uint32_t from = b * PREPARE / 4u, to = (b + 1u) * PREPARE / 4u;
+            if (at == 0u) return TwOp{true, 0u, b};
+            at -= 1u;
+            if (at < to - from) return TwOp{false, 1u, from + at};
+            at -= to - from;
+        }
+        return TwOp{true, 1u, at};
+    }
+    static constexpr uint32_t before(uint32_t at)  // instructions
+    {
+        uint32_t n = 0;
+        for (uint32_t i = 0; i < at; ++i) n += op(i).pair ? 3u : 1u;
+        return n;
+    }
+};
 
 // The LDS of a workgroup, one array for each stage and kind (A, codes, scales): the compiler then sees that a stage's reads do not
 // depend on the copies into the others.
@@ -320,35 +354,21 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
     // ---- Conversion by halves (bfaintb_device.hpp has the argument): 4 (8-bit) and 4.25 (4-bit) instructions for two weights, where a
     // conversion, a multiplication and the pack take 5 to 7; the step is bound by the instructions a SIMD issues, some 4 cycles each
     // beside its matrix instructions.
+    // (4-bit codes with group scales, whose multipliers are new every step: two of them and two shifts more, good for every scale of the format)
+    constexpr int kUpper = BITS == 4 && GROUPED ? 64 : 1024;
+    constexpr bool kLimited = kUpper == 1024;  // scales beyond the conversion go a second way along k
+    typedef HalfMultipliers<BITS, kUpper> Multiplier;
     struct Multipliers {
-        HalfMultipliers<BITS, 1024> h[2];
+        Multiplier h[2];
     };
     float most = 0.f;  // the largest magnitude among the lane's scales
     auto multipliers = [&](Multipliers& mu, const Scales& sr) {
 #pragma unroll
-        for (uint32_t j = 0; j < 2; ++j) {
-            uint32_t bits = sr.s[j];
-            asm volatile("" : "+v"(bits));  // (or the widening moves up to the load, a step's wait with it)
-            mu.h[j] = HalfMultipliers<BITS, 1024>(bf16_bits_to_f32(bits));
-        }
-        largest_scale(most, mu.h[0].s, mu.h[1].s);
+        for (uint32_t j = 0; j < 2; ++j) mu.h[j] = Multiplier(bf16_bits_to_f32(sr.s[j]));
+        if constexpr (kLimited) largest_scale(most, mu.h[0].s, mu.h[1].s);
     };
-    HalfConstants<BITS, 1024> half_k;
+    HalfConstants<BITS, kUpper> half_k;
     half_k.keep();
-    struct Halves {
-        uint32_t e[2], d[2];  // 8-bit: rows 0 and 2 (+ 4 h), rows 1 and 3 [h]; 4-bit: [0]: rows 0 and 4, 1 and 5; [1]: 2 and 6, 3 and 7
-    };
-    // what pairs 2 h and 2 h + 1 (8-bit), or h and h + 2 (4-bit), need
-    auto extract = [&](Halves& hv, const uint32_t (&c)[BITS / 4], uint32_t h) {
-        const uint32_t x = BITS == 8 ? c[h] : h == 0 ? c[0] : c[0] >> 8;
-        hv.e[h] = halves<0>(x, half_k);
-        hv.d[h] = halves<1>(x, half_k);
-    };
-    // rows 2 pr and 2 pr + 1 of column j, times its scale
-    auto weight = [&](const Halves& hv, const Multipliers& mu, uint32_t j, uint32_t pr, bool odd) -> float {
-        const uint32_t h = BITS == 8 ? pr >> 1 : pr & 1u, part = BITS == 8 ? pr & 1u : pr >> 1;
-        return odd ? weight_of_half<1>(hv.d[h], part, mu.h[j]) : weight_of_half<0>(hv.e[h], part, mu.h[j]);
-    };
     struct Ops {
         uint32_t w[2][4];  // [column j][dword]: the 8-element operand as 4 packed pairs
     };
@@ -363,12 +383,62 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
         if constexpr (GROUPED) multipliers(mu, sr);
 #pragma unroll
         for (uint32_t j = 0; j < 2; ++j) {
-            Halves hv;
-            extract(hv, c.d[j], 0);
-            extract(hv, c.d[j], 1);
+            if constexpr (BITS == 4) {
+                const uint4 w = weights4_by_halves(c.d[j][0], half_k, mu.h[j]);
+                ops.w[j][0] = w.x, ops.w[j][1] = w.y, ops.w[j][2] = w.z, ops.w[j][3] = w.w;
+            } else {
 #pragma unroll
-            for (uint32_t pr = 0; pr < 4u; ++pr) ops.w[j][pr] = pack_bf16_rne(weight(hv, mu, j, pr, false), weight(hv, mu, j, pr, true));
+                for (uint32_t pr = 0; pr < 4u; ++pr)
+                    ops.w[j][pr] = pack_bf16_rne(weight_of_half<0>(halves<0>(c.d[j][pr >> 1], half_k), pr & 1u, mu.h[j]),
+                                                 weight_of_half<1>(halves<1>(c.d[j][pr >> 1], half_k), pr & 1u, mu.h[j]));
+            }
         }
+    };
+    // In a step: what a column needs before its products, one vector instruction at a time, each held where it is written, and its four pairs of
+    // rows (4-bit codes: pairs 0, 2, 1, 3, as the halves lie).
+    struct Conversion {
+        uint32_t h[2][4], x[3];
+        Multiplier mu[2];
+    };
+    constexpr uint32_t kHalvesOps = BITS == 8 ? 4u : kUpper == 64 ? 7u : 5u, kPrepareOps = kHalvesOps + (GROUPED ? 2u : 0u);
+    auto prepare = [&](Conversion& w, const Codes& c, const Scales& sr, auto j_c, auto op_c) {
+        constexpr uint32_t j = decltype(j_c)::value, at = decltype(op_c)::value;
+        // (group scales: the widening first, the offset three instructions on)
+        constexpr uint32_t kWiden = 100u, kOffset = 101u;
+        constexpr uint32_t op = !GROUPED ? at : at == 0u ? kWiden : at == 3u ? kOffset : at < 3u ? at - 1u : at - 2u;
+        uint32_t (&h)[4] = w.h[j];
+        if constexpr (op == kWiden) {
+            uint32_t bits = sr.s[j];
+            hold(bits);  // (or the widening moves up to the load, a step's wait with it)
+            w.mu[j].s = bf16_bits_to_f32(bits), hold(w.mu[j].s);
+        } else if constexpr (op == kOffset) {
+            w.mu[j].o = Multiplier(w.mu[j].s).o, hold(w.mu[j].o);
+            if constexpr (kLimited && j == 1u) largest_scale(most, w.mu[0].s, w.mu[1].s);
+        } else if constexpr (BITS == 8) {
+            h[op] = (op & 1u) == 0u ? halves<0>(c.d[j][op >> 1], half_k) : halves<1>(c.d[j][op >> 1], half_k);
+            hold(h[op]);
+        } else if constexpr (kUpper == 64) {
+            if constexpr (op == 0u) w.x[0] = c.d[j][0] << 4, hold(w.x[0]);
+            if constexpr (op == 1u) w.x[1] = c.d[j][0] >> 4, hold(w.x[1]);
+            if constexpr (op == 2u) h[0] = halves<1>(w.x[0], half_k), hold(h[0]);
+            if constexpr (op == 3u) w.x[2] = c.d[j][0] >> 8, hold(w.x[2]);
+            if constexpr (op == 4u) h[1] = halves<1>(c.d[j][0], half_k), hold(h[1]);
+            if constexpr (op == 5u) h[2] = halves<1>(w.x[1], half_k), hold(h[2]);
+            if constexpr (op == 6u) h[3] = halves<1>(w.x[2], half_k), hold(h[3]);
+        } else {
+            if constexpr (op == 0u) w.x[0] = c.d[j][0] >> 8, hold(w.x[0]);
+            if constexpr (op == 1u) h[0] = halves<0>(c.d[j][0], half_k), hold(h[0]);
+            if constexpr (op == 2u) h[1] = halves<1>(c.d[j][0], half_k), hold(h[1]);
+            if constexpr (op == 3u) h[2] = halves<0>(w.x[0], half_k), hold(h[2]);
+            if constexpr (op == 4u) h[3] = halves<1>(w.x[0], half_k), hold(h[3]);
+        }
+    };
+    auto make_pair = [&](Ops& ops, const Conversion& w, auto j_c, auto b_c) {
+        constexpr uint32_t j = decltype(j_c)::value, b = decltype(b_c)::value;
+        const Multiplier& mu = GROUPED ? w.mu[j] : fixed.h[j];
+        uint32_t& to = ops.w[j][BITS == 8 ? b : (b & 1u) * 2u + (b >> 1)];
+        if constexpr (BITS == 4 && kUpper == 1024) to = pair_of_halves<(b & 1u)>(w.h[j][b & 2u], w.h[j][(b & 2u) + 1u], mu.s, mu.o, mu.s4, mu.o4);
+        else to = pair_of_halves<(b & 1u)>(w.h[j][b & 2u], w.h[j][(b & 2u) + 1u], mu.s, mu.o, mu.s, mu.o);
     };
 
     f32x4_t acc[MT][2];
@@ -389,13 +459,25 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
     //   slot 0 of unit u: the A fragment of unit u + kAhead (the last kAhead units fetch the next step's first
     //          fragments: its stage is complete, see the wait below)
     //   slot 1 of unit u: one memory request (with group scales: those first, in unit 0; then the copies)
-    // The step's eight conversion pairs (two weights) are spread evenly over the slots: the codes' halves and the two products of a pair in
-    // one slot, the rounding pack in the slot behind it.
+    // The conversion's instructions and the requests are spread evenly over the slots (several waves' requests behind one another hold all of
+    // them up).
     // (fragments rotate through af[]: MT units leave the rotation MT % 4 further on, and four steps bring it back)
     constexpr uint32_t kSlots = 2u * MT;
     Scales ring[NS];  // group scales that do not go through LDS: those of step kt in ring[kt % NS]
     constexpr bool kRing = GROUPED && !kScalesInLds;
     constexpr uint32_t kRequests = kACopies + 1u + (kScalesInLds ? 1u : 0u);  // copies of a wave and step
+    typedef TwSchedule<kPrepareOps> Schedule;
+    // The first slots are left to the codes' read: five of six blocks' twelve, where two of them waited for it (284 x 10624 x 2560 packed 4-bit, us
+    // with 2 / 3 / 5 / 6: 21.2 / 20.0 / 19.6 / 19.4; 259 x 4960 x 14208 packed 8-bit g128 59.0 / 56.4 / 56.0 / 55.6; sixteen blocks don't mind).
+    // With fewer blocks there are none to spare: three where the multipliers or the packed order's reads come first, none for 8-bit codes in
+    // rows (64 x 4096 x 11008 20.5 with none, 20.9 with three; packed 4-bit 64 x 20480 x 4096 21.7 / 21.5).
+    constexpr uint32_t kFree = MT >= 6 ? 5u : MT >= 4 ? (GROUPED || PACKED || BITS == 4 ? 3u : 0u) : 1u;
+    auto op_slot = [](uint32_t i) constexpr -> uint32_t { return kFree + Schedule::before(i) * (kSlots - kFree) / Schedule::kInstructions; };
+    // (few blocks: as early as they can be, since those launches wait for memory: 40 x 4096 x 11008 8-bit 19.2 spread / 18.7)
+    auto request_unit = [](uint32_t q) constexpr -> uint32_t {
+        constexpr uint32_t first = kRing ? 1u : 0u, units = (uint32_t)MT - first;
+        return first + (MT >= 6 ? q * units / kRequests : q < units ? q : units - 1u);
+    };
     auto step = [&](auto stage_c, uint32_t kt, const Ops& cur, Ops& nxt) {
         constexpr uint32_t S = decltype(stage_c)::value;
         constexpr uint32_t kTurn = S * (uint32_t)MT % kAhead;
@@ -414,62 +496,46 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
         const uint8_t* const a_nxt = a_tile(Next{}) + a_rd;
         const uint8_t* const w_src = w_tile(Next{});
         Codes code;  // of step kt + 1
-        Halves hv[2];
-        Multipliers mu = fixed;
-        float f0[8], f1[8];
+        Conversion conv;
         Scales sr;
         if constexpr (kScalesInLds) read_scales(sr, s_tile(Next{}));
         else sr = ring[(S + 1u) % NS];
-        // pair v: rows 2 (v / 2), + 1 of column v % 2
-        auto convert_first = [&](uint32_t v) {
-            const uint32_t pr = v >> 1, j = v & 1u;
-            if (BITS == 8 ? (pr & 1u) == 0u : pr < 2u) extract(hv[j], code.d[j], BITS == 8 ? pr >> 1 : pr);
-            f0[v] = weight(hv[j], mu, j, pr, false);
-            f1[v] = weight(hv[j], mu, j, pr, true);
-            asm volatile("" : "+v"(f0[v]), "+v"(f1[v]));  // here, and not where the pair is packed
-        };
-        auto convert_second = [&](uint32_t v) { nxt.w[v & 1u][v >> 1] = pack_bf16_rne(f0[v], f1[v]); };
         read_codes(code, w_src, kt + 1u);
-        if constexpr (GROUPED) multipliers(mu, sr);
         __builtin_amdgcn_sched_barrier(0);
         const bf16x8_t wf0 = __builtin_bit_cast(bf16x8_t, make_uint4(cur.w[0][0], cur.w[0][1], cur.w[0][2], cur.w[0][3]));
         const bf16x8_t wf1 = __builtin_bit_cast(bf16x8_t, make_uint4(cur.w[1][0], cur.w[1][1], cur.w[1][2], cur.w[1][3]));
         bf16x8_t a_now;
-#pragma unroll
-        for (uint32_t slot = 0; slot < kSlots; ++slot) {
-            const uint32_t u = slot >> 1;
-            if ((slot & 1u) == 0u) {
-                const uint32_t at = (u + kTurn) % kAhead;
+        for_each_const<kSlots>([&](auto slot_c) {
+            constexpr uint32_t slot = decltype(slot_c)::value, u = slot >> 1;
+            if constexpr ((slot & 1u) == 0u) {
+                constexpr uint32_t at = (u + kTurn) % kAhead;
                 a_now = af[at];
                 tw_mfma(acc[u][0], a_now, wf0);
-                if (u + kAhead < (uint32_t)MT) af[at] = *reinterpret_cast<const bf16x8_t*>(a_src + (u + kAhead) * 2048u);
+                if constexpr (u + kAhead < (uint32_t)MT) af[at] = *reinterpret_cast<const bf16x8_t*>(a_src + (u + kAhead) * 2048u);
                 else af[at] = *reinterpret_cast<const bf16x8_t*>(a_nxt + (u + kAhead - (uint32_t)MT) * 2048u);
             } else {
                 tw_mfma(acc[u][1], a_now, wf1);
-                constexpr uint32_t kFirstCopy = kRing ? 1u : 0u;
-                if (kRing && u == 0u) {
-                    const uint32_t off = group_offset(clamp(kt + NS), kh);
-                    load_scales(ring[S], off);
-                }
-                // (tiles of fewer units than a step has requests: the rest with the last)
-#pragma unroll
-                for (uint32_t q = 0; q < (COPIER ? 0u : kRequests); ++q) {
-                    if ((kFirstCopy + q < (uint32_t)MT ? kFirstCopy + q : (uint32_t)MT - 1u) != u) continue;
-                    if (q < kACopies)
+                if constexpr (kRing && u == 0u) load_scales(ring[S], group_offset(clamp(kt + NS), kh));
+                constexpr uint32_t from = COPIER ? 0u : first_at_least<kRequests>(request_unit, u), to = COPIER ? 0u : first_at_least<kRequests>(request_unit, u + 1u);
+                for_each_const<to - from>([&](auto i_c) {
+                    constexpr uint32_t q = from + decltype(i_c)::value;
+                    if constexpr (q < kACopies)
                         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (__attribute__((address_space(3))) void*)(a_dst + q * 1024u), 16, (q & 1u) ? vo : ve,
                                                                  at_step(kt3) * kTwK * 2u + q * 16u * p.lda, 0, 0);
-                    else if (q == kACopies) dma_w(w_tile(Target{}), kt3);
+                    else if constexpr (q == kACopies) dma_w(w_tile(Target{}), kt3);
                     else dma_s(s_tile(Target{}), kt3);
-                }
+                });
             }
-#pragma unroll
-            for (uint32_t v = 0; v < 8u; ++v) {
-                const uint32_t first = v * (kSlots - 2u) / 7u;  // (0 .. kSlots - 2)
-                if (slot == first + 1u) convert_second(v);
-                if (slot == first) convert_first(v);
-            }
+            constexpr uint32_t from = first_at_least<Schedule::kCount>(op_slot, slot), to = first_at_least<Schedule::kCount>(op_slot, slot + 1u);
+            for_each_const<to - from>([&](auto i_c) {
+                constexpr TwOp o = Schedule::op(from + decltype(i_c)::value);
+                using Column = std::integral_constant<uint32_t, o.column>;
+                using Index = std::integral_constant<uint32_t, o.index>;
+                if constexpr (o.pair) make_pair(nxt, conv, Column{}, Index{});
+                else prepare(conv, code, sr, Column{}, Index{});
+            });
             __builtin_amdgcn_sched_barrier(0);
-        }
+        });
     };
 
     // ---- prologue: A tiles and codes of steps 0, 1, 2 -> stages 0, 1, 2; operands of step 0
@@ -528,7 +594,7 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // nothing asynchronous may still be writing LDS
     // ---- a scale beyond the conversion by halves: the wave's sums once more, in the same order, by the other conversion, everything straight
     // from memory (the other waves wait at the epilogue's first barrier)
-    if (__builtin_expect(beyond_halves(most), 0)) {
+    if (kLimited && __builtin_expect(beyond_halves(most), 0)) {
         tw_settle(acc);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)

@@ -99,29 +99,12 @@ __device__ __forceinline__ void wait_vm()
 template <uint32_t IN_FLIGHT>
 __device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xc07f | IN_FLIGHT << 8); }  // lgkmcnt
 
-// A value is made here, and not where it is used.
-template <typename T>
-__device__ __forceinline__ void hold(T& v) { asm volatile("" : "+v"(v)); }
 // The weight of the code in half PART of h: as assembly, which stays in the slot it is written in.
 template <uint32_t PART>
 __device__ __forceinline__ void weight_in_place(float& w, uint32_t h, float s, float o)
 {
     if constexpr (PART == 0u) asm volatile("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[1,0,0]" : "=v"(w) : "v"(h), "v"(s), "v"(o));
     else asm volatile("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(w) : "v"(h), "v"(s), "v"(o));
-}
-
-// f(0), f(1) .. f(N - 1), the argument a compile-time constant
-template <typename F, size_t... I>
-__device__ __forceinline__ void for_each_const(F&& f, std::index_sequence<I...>) { (f(std::integral_constant<uint32_t, (uint32_t)I>{}), ...); }
-template <uint32_t N, typename F>
-__device__ __forceinline__ void for_each_const(F&& f) { for_each_const(f, std::make_index_sequence<N>{}); }
-// The first of 0 .. N - 1 whose slot is not before `slot`, or N
-template <uint32_t N, typename F>
-__host__ __device__ constexpr uint32_t first_at_least(F slot_of, uint32_t slot)
-{
-    uint32_t v = 0;
-    while (v < N && slot_of(v) < slot) ++v;
-    return v;
 }
 
 // The order of a step's conversion instructions (see convert_op).
