@@ -168,7 +168,7 @@ static double decode_family_time_us(uint32_t m, uint32_t n, uint32_t k, int bits
         // 128-column form at m = 40 / 48 / 64 against the tiles, us: 11008 x 8192 32.4 / 36.3, 33.6 / 36.5, 36.5 / 36.8;
         // 32000 x 4096 31.1 / 32.6, 32.1 / 32.6, 34.9 / 33.1; 16384 x 8192 34.4 / 36.8, 37.0 / 37.0, 40.6 / 38.8)
         const double block_rows = 16.0 * pl.mb;
-        if (m <= block_rows && pl.cols == 128u) {
+        if (m <= block_rows && pl.cols <= 128u) {
             // (and CUs left idle slow the stream less than in proportion, as over packed weights: 86 column blocks x 2 splits)
             const double wgs = (double)((n + pl.cols - 1u) / pl.cols) * pl.splits, cus = (double)machine_cus();
             // (not below 0.65 of a round: 144 and 160 column blocks, unsplit, take all the estimate says and more — 18432 x 6144,
@@ -1478,7 +1478,11 @@ static double packed8_family_time_us(uint32_t m, uint32_t n, uint32_t k, const D
     // (a long k streams faster, the workgroups' starts and hand-overs weighing less: 6 x 15104 x 11008 28.8 us, 6 x 7168 x 14336
     // 20.6, where 5.63 TB/s would say 34.1 and 23.3)
     const double long_k = k <= 4096u ? 0.0 : k >= 12288u ? 1.0 : (k - 4096.0) / 8192.0;
-    const double stream_us = (double)n * k / 1.0e6 / (5.63 * (1.0 + 0.12 * long_k) * pow(packed_family_fill(m, n, pl), 0.638));
+    // (many splits: the hand-over, not the stream, is what narrower workgroups leave — 5 x 1456 x 6912, 14 splits, 8.7 us with eight column blocks,
+    // 8.9 with six; 4 x 1296 x 6400 8.6 / 8.1, five; the slab kernel 7.7 and 7.5)
+    DecodePlan at = pl;
+    if (pl.splits > 8u) at.cols = 128u;
+    const double stream_us = (double)n * k / 1.0e6 / (5.63 * (1.0 + 0.12 * long_k) * pow(packed_family_fill(m, n, at), 0.638));
     return 3.0 + 0.0885 * m + 0.118 * (pl.splits - 1.0) + stream_us * (1.0 - 0.0037 * m + (m > 16u ? 0.1076 : 0.0)) * (pl.cols == 256u ? 1.1 : 1.0);
 }
 static double packed4_slab_time_us(uint32_t m, uint32_t n, uint32_t k)
@@ -1490,7 +1494,9 @@ static double packed4_slab_time_us(uint32_t m, uint32_t n, uint32_t k)
     // (from the third walk on a walk never takes less than 1.45 us, as for 8-bit codes: k = 2048, 12 x 10240 9.6 us, 8 x 9984 8.3)
     const double walks = packed_slab_walks(n);
     const double per_walk = (k / 1975.0 > 1.45 || walks <= 2.0) ? k / 1975.0 : 1.45;
-    return 2.58 + many * walks * per_walk * rows;
+    // (more than 96 Mi weights: 10 % more on average over 310 shapes, and up to 25 % — 24272 x 9216, m = 1: 35.6 us, 31392 x 8960, m = 3: 43.6)
+    const double large = (uint64_t)n * k > (96ull << 20) ? 1.1 : 1.0;
+    return 2.58 + many * large * walks * per_walk * rows;
 }
 static double packed4_family_time_us(uint32_t m, uint32_t n, uint32_t k, const DecodePlan& pl)
 {
@@ -1498,15 +1504,43 @@ static double packed4_family_time_us(uint32_t m, uint32_t n, uint32_t k, const D
     // m = 16: 37.4 / 75.4 / 91.5)
     const double wgs = (double)((n + pl.cols - 1u) / pl.cols) * pl.splits * ((m + 16u * pl.mb - 1u) / (16u * pl.mb));
     const double stream_us = (double)n * k / 2.0e6 / (4.37 * pow(packed_family_fill(m, n, pl), 0.58)) * (wgs > (double)machine_cus() ? 1.08 : 1.0);
-    return 4.71 + 0.067 * m + 0.144 * (pl.splits - 1.0) + stream_us * (1.0 + 0.0003 * m + (m > 16u ? 0.258 : 0.0));
+    // (narrower workgroups on few weights: what they gain is the stream's, not the start's — 1 x 9296 x 1408 6.4, the slab kernel 6.0; 2 x 10576 x 1408
+    // 7.1 / 6.3; 21 x 3584 x 4224 9.9 / 8.7)
+    const double few = pl.cols < 128u && (uint64_t)n * k < (24ull << 20) ? 1.08 : 1.0;
+    return 4.71 + 0.067 * m + 0.144 * (pl.splits - 1.0) + few * stream_us * (1.0 + 0.0003 * m + (m > 16u ? 0.258 : 0.0));
 }
 static bool packed_uses_slab(uint32_t m, uint32_t n, uint32_t k, int bits)
 {
     if (m > kDecodeAutoMaxM) return false;
     const DecodePlan pl = packed_family_plan(m, n, k, bits);
     if (bits == 8) return packed8_slab_time_us(m, n, k) <= packed8_family_time_us(m, n, k, pl);
-    if (pl.cols != 128u) return m <= 8u;
+    if (pl.cols > 128u) return m <= 8u;
     return packed4_slab_time_us(m, n, k) <= packed4_family_time_us(m, n, k, pl);
+}
+
+// Columns of a workgroup over packed weights, by whole column blocks of 16: eight, or as few as make the launch shorter by the fullest CU's share,
+// rounds of workgroups times columns.  A workgroup has one CU's LDS and waves to itself while it runs, and eight blocks fill the CUs where
+// n / 128 times the splits happens to be 256 or a little less (us, eight blocks / the rule's, 16 rows: 22016 x 4096 4-bit g128 18.8 / 16.5, six;
+// 8-bit 20.3 / 17.5, six; 11008 x 4096 4-bit 11.5 / 10.3, six; 28672 x 8192 4-bit 31.6 / 29.2, seven; more
+// than a round of eight: 34560 x 7936 4-bit, 4 rows, 53.7 / 36.2, five).  Over 3900 random shapes of 1 to 32 rows the family is faster by 15 % where it takes
+// five blocks, 11 % six, 3 % seven; against the best of the four at each shape the rule is 0.5 % off.
+// Seven only unsplit and from 13 rows, where the gain is up to 7 % (28672 x 8192); and a split of more than 128 Mi weights as it was, 12288 x
+// 12288 for one: callers have those plans.
+// (k up to 1024, which is over before its workgroups have filled: 13 x 16336 x 1024 8-bit 7.5 with eight, 8.1 with five; and more than 12 splits, where the
+// hand-over is most of it: 8 x 1024 x 15872 4-bit 9.9 / 10.7.)
+// (More than 32 rows take their row blocks again for every workgroup: not looked at.)
+static DecodePlan fitted_to_cus(DecodePlan pl, uint32_t m, uint32_t n, uint32_t k)
+{
+    if (m > kDecodeAutoMaxM || pl.mb > 2u || pl.waves != 8u || (pl.splits > 1u && (uint64_t)n * k > (128ull << 20)) || k <= 1024u || pl.splits > 12u) return pl;
+    const uint64_t blocks = n / 16u, others = (uint64_t)pl.splits * ((m + 16u * pl.mb - 1u) / (16u * pl.mb)), cus = machine_cus();
+    auto share = [&](uint32_t c) { return ((blocks + c - 1u) / c * others + cus - 1u) / cus * c; };
+    // (a tenth less at least: three rounds of five blocks are no better than two of eight — 59680 x 1024 4-bit, 6 rows, 14.6 / 13.2)
+    uint64_t least = share(8u) * 9u / 10u + 1u;
+    for (uint32_t c = 7u; c >= 5u; --c) {
+        if (share(c) >= least || (c == 7u && (m <= 12u || pl.splits > 1u))) continue;
+        least = share(c), pl.cols = 16u * c;
+    }
+    return pl;
 }
 
 // The family's plan over packed weights.  8-bit codes: the one row-major weights get, as long as it uses the 128 columns
@@ -1516,7 +1550,7 @@ static DecodePlan packed_family_plan(uint32_t m, uint32_t n, uint32_t k, int bit
 {
     if (bits == 8) {
         const DecodePlan pl = decode_plan(m, n, k, bits, 0, true);
-        if (pl.cols == 128u) return pl;
+        if (pl.cols == 128u) return fitted_to_cus(pl, m, n, k);
     }
     // 4-bit codes: the 128-column form (8 column blocks of 16 per workgroup, 8 waves) with the launch shape 8-bit codes
     // would get, wherever that shape has 128 columns.  Against the 256-column form, whose kernels over packed 4-bit codes
@@ -1526,7 +1560,7 @@ static DecodePlan packed_family_plan(uint32_t m, uint32_t n, uint32_t k, int bit
     // other way round at most 6 % (16384 x 8192, m = 12: 29.5 / 27.8; 32000 x 4096: 27.6 / 26.3).
     if (bits == 4) {
         const DecodePlan pl = decode_plan(m, n, k, 8, 0, true, true);
-        if (pl.cols == 128u) return pl;
+        if (pl.cols == 128u) return fitted_to_cus(pl, m, n, k);
     }
     return decode_plan_row_blocks(m, n, k, bits, 0, true);
 }
@@ -1551,7 +1585,7 @@ static double packed_family_time_us(uint32_t m, uint32_t n, uint32_t k, int bits
         const double wgs_ = (double)((n + pl.cols - 1u) / pl.cols) * (double)((m + 16u * pl.mb - 1u) / (16u * pl.mb));
         if (wgs_ > 2.0 * (double)machine_cus()) return 5.0 + e.core;
     }
-    if (bits == 4) return (pl.cols == 128u ? 0.70 : 0.84) * ranked;  // (the 128-column form measures 0.52 - 0.79 of its estimate)
+    if (bits == 4) return (pl.cols <= 128u ? 0.70 : 0.84) * ranked;  // (the 128-column form measures 0.52 - 0.79 of its estimate)
     // (a row block that is not full costs less: 64-row blocks at m = 40 / 48 / 64 measure 0.87 / 0.91 / 1.0 of the tiles' time
     // over 11 weight shapes where the estimate had them level — the rows past m are neither converted for nor multiplied)
     const double block_rows = 16.0 * pl.mb;

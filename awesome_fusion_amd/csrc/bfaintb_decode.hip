@@ -5,8 +5,8 @@
 // each MFMA at m = 1 and launches only n/64 workgroups with no split along k.
 //
 // Work decomposition
-//   grid  = (ceil(n/COLS), splits); block = 4 or 8 waves.  CPL = weights per lane and row (16 or 8),
-//   COLS = 16*CPL columns per workgroup (256 or 128).
+//   grid  = (ceil(n/COLS), splits); block = 4 or 8 waves.  CPL = weights per lane and row (16 or 8; over packed weights,
+//   where a lane has one column of each of CPL blocks of 16, also 7, 6 and 5), COLS = 16*CPL columns per workgroup.
 //   A workgroup owns COLS consecutive columns and k_per_wg rows of B; each wave owns an equal share of
 //   those rows and walks them in steps of 32 rows.
 //   Within a wave, lane = (kg, nl) with nl = lane%16, kg = lane/16.  Per step the lane loads, from
@@ -59,7 +59,7 @@ __device__ __forceinline__ float value_f32(const uint32_t (&row)[PD])
 __host__ __device__ constexpr bool decode_by_halves(int bits, bool grouped, bool packed, int mb) { return bits == 4 && grouped && !(packed && mb >= 2); }
 
 // (256 columns: no registers for two multipliers more)
-__host__ __device__ constexpr int half_upper(int cpl) { return cpl == 8 ? 1024 : 0; }
+__host__ __device__ constexpr int half_upper(int cpl) { return cpl <= 8 ? 1024 : 0; }
 
 template <int CPL, bool HALVES>
 struct Multipliers {
@@ -233,24 +233,27 @@ __device__ __forceinline__ void mac_step_packed(const PackedStep<BITS, CPL>& raw
 #pragma unroll
         for (int mb = 0; mb < MB; ++mb)
             acc[mb][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, __builtin_bit_cast(bf16x8_t, afrag[mb]), acc[mb][c], 0, 0, 0);
+        // (the compiler draws the conversions of several blocks together here, and spills: 24 x 12464 x 2816 15.4 us, 13.1 with blocks of eight)
+        if constexpr (BITS == 8 && CPL == 7 && MB == 2) __builtin_amdgcn_sched_barrier(0);
     }
 }
 
 // the lane's CPL scales in packed mode: column col[c] of a scale row, as raw bf16 pairs in the layout load_scales
 // produces (scale c in half c % 2 of dword c / 2)
 template <int CPL>
-__device__ __forceinline__ void load_scales_packed(uint4 (&sraw)[CPL / 8], const uint16_t* srow, const uint32_t (&col)[CPL])
+__device__ __forceinline__ void load_scales_packed(uint4 (&sraw)[(CPL + 7) / 8], const uint16_t* srow, const uint32_t (&col)[CPL])
 {
-    uint32_t d[CPL / 2];
+    constexpr int kVectors = (CPL + 7) / 8;
+    uint32_t d[4 * kVectors] = {};
 #pragma unroll
-    for (int i = 0; i < CPL / 2; ++i) d[i] = (uint32_t)srow[col[2 * i]] | ((uint32_t)srow[col[2 * i + 1]] << 16);
+    for (int c = 0; c < CPL; ++c) d[c / 2] |= (uint32_t)srow[col[c]] << (16 * (c & 1));
 #pragma unroll
-    for (int i = 0; i < CPL / 8; ++i) sraw[i] = make_uint4(d[4 * i], d[4 * i + 1], d[4 * i + 2], d[4 * i + 3]);
+    for (int i = 0; i < kVectors; ++i) sraw[i] = make_uint4(d[4 * i], d[4 * i + 1], d[4 * i + 2], d[4 * i + 3]);
 }
 
 // `srow`: a row of scales, the same for every lane; `first_col`: the lane's first column
 template <int CPL>
-__device__ __forceinline__ void load_scales(uint4 (&sraw)[CPL / 8], const uint16_t* srow, uint32_t first_col)
+__device__ __forceinline__ void load_scales(uint4 (&sraw)[(CPL + 7) / 8], const uint16_t* srow, uint32_t first_col)
 {
     const uint8_t* src = reinterpret_cast<const uint8_t*>(srow) + first_col * 2u;
 #pragma unroll
@@ -259,18 +262,19 @@ __device__ __forceinline__ void load_scales(uint4 (&sraw)[CPL / 8], const uint16
 
 // most: the largest magnitude among the lane's scales (by halves)
 template <int BITS, int CPL, bool HALVES>
-__device__ __forceinline__ void apply_scales(Multipliers<CPL, HALVES>& mu, float& most, const uint4 (&sraw)[CPL / 8])
+__device__ __forceinline__ void apply_scales(Multipliers<CPL, HALVES>& mu, float& most, const uint4 (&sraw)[(CPL + 7) / 8])
 {
-    uint32_t d[CPL / 2];
+    constexpr int kVectors = (CPL + 7) / 8;
+    uint32_t d[4 * kVectors];
 #pragma unroll
-    for (int i = 0; i < CPL / 8; ++i) {
+    for (int i = 0; i < kVectors; ++i) {
         d[4 * i] = sraw[i].x; d[4 * i + 1] = sraw[i].y; d[4 * i + 2] = sraw[i].z; d[4 * i + 3] = sraw[i].w;
     }
     if constexpr (HALVES) {
 #pragma unroll
         for (int c = 0; c < CPL; ++c) mu.h[c] = HalfMultipliers<4, half_upper(CPL)>(bf16_bits_to_f32(c & 1 ? d[c / 2] >> 16 : d[c / 2] & 0xffffu));
 #pragma unroll
-        for (int c = 0; c < CPL; c += 2) largest_scale(most, mu.h[c].s, mu.h[c + 1].s);
+        for (int c = 0; c < CPL; c += 2) largest_scale(most, mu.h[c].s, mu.h[c + 1 < CPL ? c + 1 : c].s);
     } else {
 #pragma unroll
         for (int c = 0; c < CPL; ++c) mu.s[c] = make_col_scale_nibble<BITS>(c & 1 ? d[c / 2] >> 16 : d[c / 2] & 0xffffu);
@@ -283,12 +287,22 @@ __device__ __forceinline__ void apply_scales(Multipliers<CPL, HALVES>& mu, float
 #define TRACE_MARK(i) do { } while (0)
 #endif
 
+constexpr uint32_t next_power_of_two(uint32_t x)
+{
+    uint32_t p = 1u;
+    while (p < x) p *= 2u;
+    return p;
+}
+
 // Blocks of 16 rows whose per-wave tiles fit in LDS together (4 waves; 8 waves run MB <= 2).
 __host__ __device__ constexpr int decode_rows16_per_pass(int cpl, int mb)
 {
-    const int fit = cpl == 8 ? 4 : 2;  // 4 waves x 64 rows x 132 floats, or 4 waves x 32 rows x 260 floats: 133 KiB
+    const int fit = cpl <= 8 ? 4 : 2;  // 4 waves x 64 rows x 132 floats, or 4 waves x 32 rows x 260 floats: 133 KiB
     return mb < fit ? mb : fit;
 }
+
+// Columns of a wave's table of scales in LDS (a row is read in pieces of 16 bytes).
+__host__ __device__ constexpr uint32_t decode_table_stride(int cpl) { return cpl <= 8 ? 8u : 16u; }
 
 // Dynamic LDS of one workgroup, in floats: the waves' tiles [waves][rows of one pass][COLS + 4].
 __host__ __device__ inline uint32_t decode_red_floats(uint32_t waves, uint32_t rows, uint32_t cols)
@@ -484,13 +498,15 @@ __device__ __forceinline__ void reduce_splits_two_in_flight(const GemmParams& p,
 template <int BITS, int CPL, int MB, bool GROUPED, bool PACKED, bool REF>
 // (packed 4-bit codes always run 4 waves: with 8 — their registers would allow it for one block of 16 rows — the 256-column
 // kernel over packed weights is slower, 28672 x 8192, m = 16: 55 against 42 us)
-__global__ void __launch_bounds__((MB <= 2 && (CPL == 8 || MB == 1) && !(PACKED && BITS == 4 && CPL == 16)) ? 512 : 256)
+__global__ void __launch_bounds__((MB <= 2 && (CPL <= 8 || MB == 1) && !(PACKED && BITS == 4 && CPL == 16)) ? 512 : 256)
 bfaintb_decode_kernel(const GemmParams p)
 {
+    static_assert(CPL == 16 || CPL == 8 || (PACKED && CPL >= 5 && CPL < 8 && MB <= 2), "the forms there are");
     static_assert(!REF || (BITS == 8 && !GROUPED && !PACKED), "the reference's arithmetic: 8-bit codes, row-major, one scale per column");
     constexpr int KB = decode_blocks_per_step(BITS, CPL, PACKED, MB);  // blocks of 32 rows per pipeline step
     constexpr uint32_t kCols = 16u * CPL;             // columns per workgroup
     constexpr uint32_t kRedStride = kCols + 4u;       // floats per row of a wave's tile in LDS (+4: spreads rows over banks)
+    constexpr uint32_t kTableStride = decode_table_stride(CPL);
     constexpr uint32_t kLaneBytes = CPL * BITS / 8;   // bytes of one row a lane loads
     extern __shared__ __attribute__((aligned(16))) float red[];
 
@@ -539,7 +555,7 @@ bfaintb_decode_kernel(const GemmParams p)
     constexpr uint32_t kBlocksPerChunk = BITS == 8 ? 2u : 4u;
     constexpr uint32_t kBlockBytes = 16u / kBlocksPerChunk;
     // column block c of the workgroup (blocks past the last one re-read it; what they compute is never stored)
-    constexpr bool kUniformSlabs = BITS == 8 || (CPL == 8 && MB == 2);
+    constexpr bool kUniformSlabs = BITS == 8 || (CPL <= 8 && MB == 2);
     const uint8_t* slab[CPL];
     uint32_t pk_col[CPL];
     if constexpr (PACKED) {
@@ -558,7 +574,7 @@ bfaintb_decode_kernel(const GemmParams p)
         }
     }
     const uint32_t kblock0 = kb / 32u;  // first K-block of this wave
-    static_assert(kLaneBytes == 16 || kLaneBytes == 8 || kLaneBytes == 4, "row-major weights: a lane loads 16, 8 or (4-bit codes, 128 columns) 4 bytes of a row");
+    static_assert(PACKED || kLaneBytes == 16 || kLaneBytes == 8 || kLaneBytes == 4, "row-major weights: a lane loads 16, 8 or (4-bit codes, 128 columns) 4 bytes of a row");
 
     // activation operand: row mi = 16*mb + lane%16, 8 consecutive k starting at k0 + 8*kg.
     // Lanes whose row is past the last one re-read the last one; their accumulator columns are never stored.
@@ -589,7 +605,7 @@ bfaintb_decode_kernel(const GemmParams p)
         struct Stage {
             std::conditional_t<PACKED, PackedStep<BITS, CPL>, RawStep<BITS, CPL>> raw[KB];
             uint4 af[KB][MB];
-            uint4 sraw[KB][CPL / 8];
+            uint4 sraw[KB][(CPL + 7) / 8];
         };
         Multipliers<CPL, kHalves> mu;
         HalfConstants<4, half_upper(CPL)> half_k;
@@ -597,7 +613,7 @@ bfaintb_decode_kernel(const GemmParams p)
         const uint16_t* sptr = p.scale;
         // packed weights with grouped scales: the wave's transposition table in LDS, behind the reduction area, and
         // the columns whose scales this lane fetches (kept inside the scale row)
-        uint16_t* sc_table = reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(red) + p.decode_scale_lds) + (uint32_t)wave * 16u * CPL;
+        uint16_t* sc_table = reinterpret_cast<uint16_t*>(reinterpret_cast<uint8_t*>(red) + p.decode_scale_lds) + (uint32_t)wave * 16u * kTableStride;
         uint32_t sc_col = cb * kCols + 4u * (uint32_t)lane;
         if (sc_col + 4u > p.n) sc_col = p.n - 4u;
         // Packed 8-bit codes: a workgroup starts its walk along k at a step of its own (and wraps round).  Slabs lie k x 16 bytes apart; when that is a large power of two, every workgroup's loads of a step
@@ -689,12 +705,12 @@ bfaintb_decode_kernel(const GemmParams p)
 #pragma unroll
                                 for (uint32_t e = 0; e < 4; ++e) {
                                     const uint32_t cix = 4u * (uint32_t)lane + e;
-                                    sc_table[(cix & 15u) * CPL + (cix >> 4)] = (uint16_t)(e & 1u ? d[e >> 1] >> 16 : d[e >> 1] & 0xffffu);
+                                    sc_table[(cix & 15u) * kTableStride + (cix >> 4)] = (uint16_t)(e & 1u ? d[e >> 1] >> 16 : d[e >> 1] & 0xffffu);
                                 }
                             }
-                            uint4 mine[CPL / 8];
+                            uint4 mine[(CPL + 7) / 8];
 #pragma unroll
-                            for (int i = 0; i < CPL / 8; ++i) mine[i] = *reinterpret_cast<const uint4*>(sc_table + (uint32_t)nl * CPL + 8u * i);
+                            for (int i = 0; i < (CPL + 7) / 8; ++i) mine[i] = *reinterpret_cast<const uint4*>(sc_table + (uint32_t)nl * kTableStride + 8u * i);
                             apply_scales<BITS, CPL, kHalves>(mu, most, mine);
                         } else {
                             apply_scales<BITS, CPL, kHalves>(mu, most, st.sraw[q]);
@@ -774,7 +790,7 @@ bfaintb_decode_kernel(const GemmParams p)
 #pragma unroll 1
             for (uint32_t blk = 0; blk < (uint32_t)(nsteps * KB); ++blk) {
                 std::conditional_t<PACKED, PackedStep<BITS, CPL>, RawStep<BITS, CPL>> raw;
-                uint4 af[MB], sraw[CPL / 8];
+                uint4 af[MB], sraw[(CPL + 7) / 8];
                 const uint16_t* srow = p.scale + (size_t)group_of_row(p, kb + 32u * blk) * p.lds;
                 if constexpr (PACKED) {
                     const uint8_t* slabs[CPL];
@@ -809,9 +825,12 @@ bfaintb_decode_kernel(const GemmParams p)
     //      row 16*mb + nl, local column (4*kg + r)*CPL + c.
     constexpr int kMBC = decode_rows16_per_pass(CPL, MB);
     constexpr uint32_t kQuads = kCols / 4u;
-    constexpr uint32_t kMaxR = 16u * kMBC * kQuads / 256u;      // rows per thread and pass with 4 waves (half that with 8)
+    // rows per thread and pass with 4 waves (half that with 8), up to a power of two
+    constexpr uint32_t kRowsAtOnce = 256u / kQuads, kMaxR = (uint32_t)next_power_of_two((16u * kMBC + kRowsAtOnce - 1u) / kRowsAtOnce);
     // thread t: 4 consecutive columns (cg = t % (kCols/4)) of rows t / (kCols/4), + threads/(kCols/4), ...
-    const uint32_t cg = threadIdx.x % kQuads, rs = threadIdx.x / kQuads, nrs = blockDim.x / kQuads;
+    const uint32_t cg = threadIdx.x % kQuads, nrs = blockDim.x / kQuads;
+    uint32_t rs = threadIdx.x / kQuads;
+    if (kQuads * kRowsAtOnce != 256u && rs >= nrs) rs = 1u << 16;  // (fewer threads than a further row has: none of the pass's rows)
     const uint32_t col = cb * kCols + 4u * cg;
     const bool col_ok = col < p.n;
 
@@ -902,7 +921,7 @@ bfaintb_decode_kernel(const GemmParams p)
             // never arrives leaves a NaN in the output instead of hanging the kernel.
             // Rows a thread has in this pass: a power of two up to kMaxR; the fewer, the more splits are fetched at once.
             const uint32_t rows_per_thread = (rows_out + nrs - 1u) / nrs;
-            constexpr bool kTwoAttempts = CPL == 8;  // (see reduce_splits_two_in_flight)
+            constexpr bool kTwoAttempts = CPL <= 8;  // (see reduce_splits_two_in_flight)
             if (kTwoAttempts && rows_per_thread <= 1u && p.splits <= 2u) reduce_splits_two_in_flight<1>(p, sum, first_row, rows_out, rs, col, col_ok);
             else if (kTwoAttempts && rows_per_thread <= 1u && p.splits <= 3u) reduce_splits_two_in_flight<2>(p, sum, first_row, rows_out, rs, col, col_ok);
             else if (kTwoAttempts && rows_per_thread <= 1u && p.splits <= 5u) reduce_splits_two_in_flight<4>(p, sum, first_row, rows_out, rs, col, col_ok);
@@ -929,8 +948,8 @@ static hipError_t launch_decode_t(const GemmParams& p, hipStream_t stream)
     size_t lds = (size_t)decode_red_floats(waves, p.m < pass_rows ? p.m : pass_rows, kCols) * sizeof(float);
     GemmParams q = p;
     if (PACKED && GROUPED) {
-        q.decode_scale_lds = (uint32_t)lds;     // each wave's 16 x CPL table of bf16 scales sits behind the reduction area
-        lds += (size_t)waves * 16u * CPL * 2u;
+        q.decode_scale_lds = (uint32_t)lds;     // each wave's table of bf16 scales, 16 x CPL, sits behind the reduction area
+        lds += (size_t)waves * 16u * decode_table_stride(CPL) * 2u;
     }
     if (lds > 160 * 1024 - 64) return hipErrorInvalidValue;
     void (*kernel)(const GemmParams) = bfaintb_decode_kernel<BITS, CPL, MB, GROUPED, PACKED, REF>;
@@ -977,12 +996,16 @@ hipError_t launch_decode(const GemmParams& p, int bits, hipStream_t stream)
     return p.decode_cols == 128u ? launch_decode_b<4, 8, false>(p, stream) : launch_decode_b<4, 16, false>(p, stream);
 }
 
-// The same family over weights in the packed order (p.b = the packed buffer): the shapes the plan uses beyond 32 rows of A,
-// 128 columns for 8-bit and 256 for 4-bit codes.  n must hold at least one such group of column blocks.
+// The same family over weights in the packed order (p.b = the packed buffer): five to eight column blocks of 16, or, for 4-bit codes, 16.
 hipError_t launch_decode_family_packed(const GemmParams& p, int bits, hipStream_t stream)
 {
-    if (bits == 8) return p.decode_cols == 128u ? launch_decode_b<8, 8, true>(p, stream) : hipErrorInvalidValue;
-    return p.decode_cols == 128u ? launch_decode_b<4, 8, true>(p, stream) : launch_decode_b<4, 16, true>(p, stream);
+    switch (p.decode_cols) {
+        case 80: return bits == 8 ? launch_decode_b<8, 5, true>(p, stream) : launch_decode_b<4, 5, true>(p, stream);
+        case 96: return bits == 8 ? launch_decode_b<8, 6, true>(p, stream) : launch_decode_b<4, 6, true>(p, stream);
+        case 112: return bits == 8 ? launch_decode_b<8, 7, true>(p, stream) : launch_decode_b<4, 7, true>(p, stream);
+        case 128: return bits == 8 ? launch_decode_b<8, 8, true>(p, stream) : launch_decode_b<4, 8, true>(p, stream);
+        default: return bits == 8 ? hipErrorInvalidValue : launch_decode_b<4, 16, true>(p, stream);
+    }
 }
 
 // Allows every kernel of the family its largest dynamic LDS size on the current device.  Runs once per device, from the
@@ -1014,6 +1037,12 @@ hipError_t decode_prepare_device()
     if (e == hipSuccess) e = allow_lds_b<8, 16, false>();
     if (e == hipSuccess) e = allow_lds_b<4, 16, false>();
     if (e == hipSuccess) e = allow_lds_b<8, 8, true>();
+    if (e == hipSuccess) e = allow_lds_b<8, 7, true>();
+    if (e == hipSuccess) e = allow_lds_b<4, 7, true>();
+    if (e == hipSuccess) e = allow_lds_b<8, 6, true>();
+    if (e == hipSuccess) e = allow_lds_b<4, 6, true>();
+    if (e == hipSuccess) e = allow_lds_b<8, 5, true>();
+    if (e == hipSuccess) e = allow_lds_b<4, 5, true>();
     if (e == hipSuccess) e = allow_lds_b<4, 16, true>();
     if (e == hipSuccess) e = allow_lds<8, 8, 1, false, false, true>();
     if (e == hipSuccess) e = allow_lds<8, 8, 2, false, false, true>();

@@ -70,7 +70,7 @@ inline void fill_argv(void** argv, Tuple& t, std::index_sequence<I...>)
 // 9 - 14 % faster on matrices from 32 MiB).
 __host__ __device__ constexpr int decode_blocks_per_step(int bits, int cpl, bool packed, int mb)
 {
-    return packed ? (bits == 4 && cpl == 8 && mb <= 2 ? 4 : 2) : 1;
+    return packed ? (bits == 4 && cpl <= 8 && mb <= 2 ? 4 : 2) : 1;
 }
 
 struct GemmParams {
@@ -98,7 +98,7 @@ struct GemmParams {
     // split-K (decode variant only)
     uint32_t k_per_wg;   // rows of k one workgroup covers (multiple of 32 * decode_blocks_per_step * decode_waves)
     uint32_t decode_waves; // waves per workgroup of the decode variant (4 or 8)
-    uint32_t decode_cols;  // columns per workgroup of the decode variant (256, or 128 for 8-bit codes)
+    uint32_t decode_cols;  // columns per workgroup of the decode variant (256 or 128; packed weights also 112, 96, 80)
     uint32_t decode_mb;    // blocks of 16 rows of A per workgroup of the decode variant (1, 2 or 4)
     uint32_t decode_scale_lds;  // byte offset, in dynamic LDS, of the waves' scale tables (packed weights, grouped scales)
     uint32_t splits;     // workgroups along k
