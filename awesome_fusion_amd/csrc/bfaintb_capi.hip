@@ -1431,7 +1431,7 @@ int bfaintb_prepack_colmajor(void* packed, const void* b, uint32_t n, uint32_t k
 // of 16 rows of A converts the slab again) or the decode family reading packed slabs (128 or 256 columns per workgroup,
 // split along k).  The slab kernel wins while the rows are few; how few depends on the shape, so packed_uses_slab
 // compares what each was measured to take.
-static DecodePlan packed_family_plan(uint32_t m, uint32_t n, uint32_t k, int bits);
+static DecodePlan packed_family_plan(uint32_t m, uint32_t n, uint32_t k, int bits, bool fitted = true);
 
 // The slab kernel against the family, by what each was measured to take: 28 weight shapes from 256 x 7168 to 28672 x 8192,
 // m = 1 .. 32, both code widths; least-squares fits, 7 - 9 % rms (us).
@@ -1485,7 +1485,7 @@ static double packed8_family_time_us(uint32_t m, uint32_t n, uint32_t k, const D
     const double stream_us = (double)n * k / 1.0e6 / (5.63 * (1.0 + 0.12 * long_k) * pow(packed_family_fill(m, n, at), 0.638));
     return 3.0 + 0.0885 * m + 0.118 * (pl.splits - 1.0) + stream_us * (1.0 - 0.0037 * m + (m > 16u ? 0.1076 : 0.0)) * (pl.cols == 256u ? 1.1 : 1.0);
 }
-static double packed4_slab_time_us(uint32_t m, uint32_t n, uint32_t k)
+static double packed4_slab_time_us(uint32_t m, uint32_t n, uint32_t k, bool charge_large)
 {
     const double rows = m <= 6u ? 1.0 + 0.031 * (m - 1.0) : m <= 16u ? 1.155 + 0.078 * (m - 6.0) : 1.267 + 0.0776 * m;
     // (more than seven slabs per CU: 5 % less than that — 32000 / 50304 / 128256 / 151936 x 4096, m = 1: 17.6 / 26.2 / 63.4 / 74.8 us;
@@ -1495,7 +1495,7 @@ static double packed4_slab_time_us(uint32_t m, uint32_t n, uint32_t k)
     const double walks = packed_slab_walks(n);
     const double per_walk = (k / 1975.0 > 1.45 || walks <= 2.0) ? k / 1975.0 : 1.45;
     // (more than 96 Mi weights: 10 % more on average over 310 shapes, and up to 25 % — 24272 x 9216, m = 1: 35.6 us, 31392 x 8960, m = 3: 43.6)
-    const double large = (uint64_t)n * k > (96ull << 20) ? 1.1 : 1.0;
+    const double large = charge_large && (uint64_t)n * k > (96ull << 20) ? 1.1 : 1.0;
     return 2.58 + many * large * walks * per_walk * rows;
 }
 static double packed4_family_time_us(uint32_t m, uint32_t n, uint32_t k, const DecodePlan& pl)
@@ -1509,13 +1509,23 @@ static double packed4_family_time_us(uint32_t m, uint32_t n, uint32_t k, const D
     const double few = pl.cols < 128u && (uint64_t)n * k < (24ull << 20) ? 1.08 : 1.0;
     return 4.71 + 0.067 * m + 0.144 * (pl.splits - 1.0) + few * stream_us * (1.0 + 0.0003 * m + (m > 16u ? 0.258 : 0.0));
 }
-static bool packed_uses_slab(uint32_t m, uint32_t n, uint32_t k, int bits)
+static bool packed_slab_leads(uint32_t m, uint32_t n, uint32_t k, int bits, const DecodePlan& pl, bool large)
 {
     if (m > kDecodeAutoMaxM) return false;
-    const DecodePlan pl = packed_family_plan(m, n, k, bits);
     if (bits == 8) return packed8_slab_time_us(m, n, k) <= packed8_family_time_us(m, n, k, pl);
     if (pl.cols > 128u) return m <= 8u;
-    return packed4_slab_time_us(m, n, k) <= packed4_family_time_us(m, n, k, pl);
+    return packed4_slab_time_us(m, n, k, large) <= packed4_family_time_us(m, n, k, pl);
+}
+// Whether the slab kernel leads the family with eight column blocks: what the choice was before there were fewer.  Such a call has no scratch to
+// ask for and may be a first one under capture, and stays one.
+static bool packed_slab_leads_eight_blocks(uint32_t m, uint32_t n, uint32_t k, int bits)
+{
+    return packed_slab_leads(m, n, k, bits, packed_family_plan(m, n, k, bits, false), false);
+}
+static bool packed_uses_slab(uint32_t m, uint32_t n, uint32_t k, int bits)
+{
+    const DecodePlan pl = packed_family_plan(m, n, k, bits);
+    return packed_slab_leads(m, n, k, bits, pl, true) || (pl.splits > 1u && packed_slab_leads_eight_blocks(m, n, k, bits));
 }
 
 // Columns of a workgroup over packed weights, by whole column blocks of 16: eight, or as few as make the launch shorter by the fullest CU's share,
@@ -1546,11 +1556,11 @@ static DecodePlan fitted_to_cus(DecodePlan pl, uint32_t m, uint32_t n, uint32_t 
 // The family's plan over packed weights.  8-bit codes: the one row-major weights get, as long as it uses the 128 columns
 // per workgroup the packed kernels are built for.  4-bit codes: the row-block plan also below 33 rows of A (measured
 // against the small-m plan: 8192 x 8192, m = 32: 28.9 / 36.4 us; 28672 x 8192, m = 24: 56.9 / 65.6 us).
-static DecodePlan packed_family_plan(uint32_t m, uint32_t n, uint32_t k, int bits)
+static DecodePlan packed_family_plan(uint32_t m, uint32_t n, uint32_t k, int bits, bool fitted)
 {
     if (bits == 8) {
         const DecodePlan pl = decode_plan(m, n, k, bits, 0, true);
-        if (pl.cols == 128u) return fitted_to_cus(pl, m, n, k);
+        if (pl.cols == 128u) return fitted ? fitted_to_cus(pl, m, n, k) : pl;
     }
     // 4-bit codes: the 128-column form (8 column blocks of 16 per workgroup, 8 waves) with the launch shape 8-bit codes
     // would get, wherever that shape has 128 columns.  Against the 256-column form, whose kernels over packed 4-bit codes
@@ -1560,7 +1570,7 @@ static DecodePlan packed_family_plan(uint32_t m, uint32_t n, uint32_t k, int bit
     // other way round at most 6 % (16384 x 8192, m = 12: 29.5 / 27.8; 32000 x 4096: 27.6 / 26.3).
     if (bits == 4) {
         const DecodePlan pl = decode_plan(m, n, k, 8, 0, true, true);
-        if (pl.cols == 128u) return fitted_to_cus(pl, m, n, k);
+        if (pl.cols == 128u) return fitted ? fitted_to_cus(pl, m, n, k) : pl;
     }
     return decode_plan_row_blocks(m, n, k, bits, 0, true);
 }
@@ -1850,7 +1860,7 @@ static int gemm_prepacked_impl(void* c, const void* a, const void* packed_b, con
         }
         DeviceState* dev = nullptr;
         e = device_state(st, &dev);
-        if (e) return e;
+        if (e) return packed_slab_leads_eight_blocks(m, n, k, weight_bits) ? (int)bfaintb::launch_decode_packed(p, weight_bits, st) : e;
         if (variant == BFAINTB_VARIANT_AUTO && few_rows_on_tiles(m, n, k, weight_bits, group_size != 0, true, n) && (uint64_t)256 * lda * 2u < (1ull << 31))
             return (int)launch_few_rows_on_tiles(p, weight_bits, true, st);
         std::unique_lock<std::mutex> in_order;
