@@ -1,4 +1,4 @@
-// Tiled variant, tiles of 160 to 256 rows x 256 columns, weights kept in registers: the prefill kernel, for row-major B and for B in the packed order
+// Tiled variant, tiles of 128 to 256 rows x 256 columns, weights kept in registers: the prefill kernel, for row-major B and for B in the packed order
 // (PACKED: what changes is said where the codes are fetched).
 //
 // Same job and the same reference kernel replaced as bfaintb_prefill_kernel
@@ -30,7 +30,8 @@
 // packed 107.4 / 102.6; 2048 x 28672 x 8192 4-bit g128 754 / 717, packed 734 / 708; 2560 x 4096 x 4096 4-bit g128 94.5 / 89.0.
 // Fewer blocks: rows spread evenly over the tiles (wide_tiles in bfaintb_capi.hip), so that no matrix instruction is spent on rows
 // that do not exist and the tiles make whole rounds.  us, tiles of 256 rows / as few blocks as serve: 384 x 22016 x 4096 4-bit g128 94.7 / 73.4, 8-bit
-// 82.7 / 70.8; 300 x 28672 x 4096 4-bit 89.9 / 68.9; 768 x 13824 x 5120 packed 4-bit 115 / 95.8.
+// 82.7 / 70.8; 300 x 28672 x 4096 4-bit 89.9 / 68.9, packed 81.5 / 72.0; 577 x 13824 x 5120 packed 4-bit 92.4 / 81, 8-bit 93.8 / 80.6; 768 rows
+// packed 4-bit 115 / 95.6.
 #pragma once
 #include <utility>
 #include "bfaintb_device.hpp"

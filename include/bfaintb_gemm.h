@@ -62,9 +62,9 @@ enum {
 enum {
     BFAINTB_VARIANT_AUTO = 0,   /* decode up to m = 32; beyond, whichever the library estimates faster for (m, n, k) */
     BFAINTB_VARIANT_DECODE = 1, /* split-K weight-streaming kernel (HBM-bound); m > 32 in row blocks; accepts m <= 32768 */
-    BFAINTB_VARIANT_PREFILL = 2, /* LDS-tiled MFMA kernels (MFMA-bound): 256x256 tiles, or small tiles of 128 columns and at
+    BFAINTB_VARIANT_PREFILL = 2, /* LDS-tiled MFMA kernels (MFMA-bound): tiles of 256 columns and 128 to 256 rows, or small tiles of 128 columns and at
                                   * most 128 rows while m x n holds at most 256 of those (the large tiles would leave most
-                                  * CUs idle), or tall ones of 128 columns and 160 to 256 rows in between; while even
+                                  * CUs idle), or tall ones of 128 columns and 160 to 256 rows in between, by estimated time; while even
                                   * the small tiles leave CUs idle, their kernel splits k between workgroups (same
                                   * workspace and hand-over as the decode family's split-K) */
     BFAINTB_VARIANT_PREFILL_256 = 3, /* the tiled kernel with 256x256 tiles, whatever the shape (tests, tuning) */
@@ -365,7 +365,7 @@ enum {
     BFAINTB_KERNEL_TILES_128 = 3,     /* tiles of 128 columns and 32 to 256 rows, weights in registers; up to 128 rows may split k */
     BFAINTB_KERNEL_TILES_128_LDS = 4, /* 128 x 128 tiles, both operands through LDS */
     BFAINTB_KERNEL_TILES_256X128 = 5, /* tiles of 256 rows x 128 columns, weights in registers, one chain of products an output */
-    BFAINTB_KERNEL_TILES_256 = 6,     /* 256 x 256 tiles, weights in registers */
+    BFAINTB_KERNEL_TILES_256 = 6,     /* tiles of 256 columns and 128 to 256 rows, weights in registers, one chain of products an output */
     BFAINTB_KERNEL_TILES_256_LDS = 7  /* 256 x 256 tiles, both operands through LDS */
 };
 typedef struct bfaintb_plan {
@@ -400,7 +400,8 @@ BFAINTB_API int bfaintb_gemm_variant(uint32_t m, uint32_t n, uint32_t k, int wei
  * at most 60 % of the units (640 x 11008), and that up to 128 rows always run small tiles, in as many rounds as it
  * takes (taller tiles would be half empty).  Small and tall tiles are of at most that many rows: the rows of A are spread evenly
  * over them, in steps of 32 or 64 (bfaintb_gemm_plan has the number).  The two functions answer for 8-bit codes and a k of 4096; 4-bit
- * codes with a short k keep the small tiles up to 345 of them; bfaintb_gemm_plan answers for either.  Pre-packed
+ * codes with a short k keep the small tiles up to 345 of them, and where tiles of 256 columns and fewer than 256 rows are estimated to take
+ * less time than any of these, they run; bfaintb_gemm_plan answers for all of it.  Pre-packed
  * weights run the same tiles.  (The reference arithmetic has no tall form: 256 x 256 there.) */
 BFAINTB_API uint32_t bfaintb_prefill_tile(uint32_t m, uint32_t n);
 BFAINTB_API uint32_t bfaintb_prefill_tile_cols(uint32_t m, uint32_t n);
