@@ -154,3 +154,26 @@ def test_two_threads_share_a_stream():
     torch.cuda.synchronize()
     assert all(len(o) == 40 for o in outs)
     assert all(torch.equal(c, want[j]) for o in outs for j, c in o)
+
+
+# shapes (width of the codes last) that the slab kernel, which needs neither scratch nor the device's set-up, served before the family had fewer than
+# eight column blocks a workgroup: those the family leads now, unsplit, and those it would lead if it did not split k
+NOW_FAMILY = [(5, 42576, 10752, 4), (7, 19216, 14336, 4), (13, 33872, 8320, 8), (11, 18992, 3200, 8), (6, 22144, 2048, 4)]
+STILL_SLAB = [(5, 1456, 6912, 8), (2, 10576, 1408, 4), (13, 3056, 6400, 8), (3, 13776, 2176, 4)]
+
+
+def test_calls_of_the_slab_kernel_need_no_scratch_and_no_set_up(tmp_path):
+    import awesome_fusion_amd as af
+    for m, n, k, bits in NOW_FAMILY:
+        pl = af.plan(m, n, k, bits, packed=True)
+        assert (pl.kernel, pl.splits, pl.workspace_bytes) == (af.KERNEL_DECODE_FAMILY, 1, 0), pl.as_dict()
+    for m, n, k, bits in STILL_SLAB:
+        assert af.plan(m, n, k, bits, packed=True).kernel == af.KERNEL_DECODE_SLAB
+    shapes = NOW_FAMILY + STILL_SLAB
+    slabs = [(0, 1, n // 16 * -(-m // 32)) for m, n, _, _ in shapes]
+    r = on_stand_in(tmp_path, "packed_first_capture", "\n".join("%d %d %d %d" % s for s in shapes))
+    assert r.returncode == 0
+    assert [tuple(map(int, line.split())) for line in r.stdout.split("\n") if line] == slabs
+    got = calls(tmp_path, ["%d %d %d %d 1 0" % s for s in shapes])
+    assert [x[:2] for x in got] == [(0, 1)] * len(shapes)
+    assert [x[2] for x in got[:len(NOW_FAMILY)]] == [af.plan(m, n, k, bits, packed=True).workgroups for m, n, k, bits in NOW_FAMILY]
