@@ -35,6 +35,7 @@
 #pragma once
 #include <utility>
 #include "bfaintb_device.hpp"
+#include "bfaintb_prefill_wreg_step.hpp"
 
 namespace bfaintb {
 
@@ -336,7 +337,6 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
         }
         if constexpr (GROUPED) codes[quad & 3u].s = *reinterpret_cast<const uint16_t*>(s_tile(stage_c) + (s_rd - kFarS) + blk * 512u + 32u * j);
     };
-    constexpr uint32_t kQuadReads[2] = {(PACKED ? 0u : 1u) + (GROUPED ? 1u : 0u), (PACKED || BITS == 4 ? 0u : 1u) + (GROUPED ? 1u : 0u)};  // even quads, odd ones
 
     // One vector instruction of what a quad needs before its products.  Each is held where it is written, in an order in which none
     // reads what the one before has made (the compiler would put an idle cycle between).
@@ -420,46 +420,15 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
     //   fragments of A: a group of four units waits once, for its own, and reads those of the group after the next, one in each unit;
     //   quads: read a quarter of a step before they are prepared, the first two at the end of the step before;
     //   conversion: one instruction after the other (Schedule);
-    //   memory: codes and group scales (rows: of step kt + 3, packed codes: of kt + 2) and the copies of A of step kt + 2, evenly over the step.
-    // The step's one barrier stands 24 slots before its end, where the next step's first fragments and codes are about to be read: before it
-    // the wave makes sure that its part of them has landed (requested in the step before: what may still be in flight then is this step's own)
-    // and that it has the fragments of this step.  Behind it every wave's part has landed, and nobody reads this step's stage of A,
-    // or the codes of the next one, any more: the next step's copies go there.
-    constexpr uint32_t kUnits = 2u * MT, kSlots = 8u * MT, kBarrierSlot = kSlots - 24u;
-    // Requests: codes and group scales in their order, the copies of A spread among them; packed codes, which the next step waits for at its
-    // start, ahead of them (us, among the copies / ahead: 577 x 13824 x 5120 4-bit g128 95.7 / 86.2, 8-bit 89.5 / 80.6; 300 x 28672 x 4096 79.9 / 72.0).
-    constexpr uint32_t kCodes = (GROUPED ? 1u : 0u) + (PACKED ? 4u : kCodeCopies), kRequests = kCodes + kACopies;
-    auto copies_before = [](uint32_t r) constexpr -> uint32_t { return !PACKED ? r * kACopies / kRequests : r < kCodes ? 0u : r - kCodes; };
-    auto request_slot = [](uint32_t r) constexpr -> uint32_t { return 2u + r * (kSlots - 2u) / kRequests; };
-    constexpr uint32_t kBeforeBarrier = first_at_least<kRequests>(request_slot, kBarrierSlot);
-    constexpr uint32_t kBehindCodes = [=]() constexpr {  // of a step's requests
-        uint32_t r = 0;
-        while (r - copies_before(r) < kCodes) ++r;
-        return kRequests - r;
-    }();
-    // LDS reads: of unit un's fragment (un < 8: the next step's), of a quad
-    auto frag_slot = [](uint32_t un) constexpr -> uint32_t { return un >= 8u ? 4u * (un - 8u) : kBarrierSlot + 3u * un; };
-    auto quad_slot = [](uint32_t quad) constexpr -> uint32_t {
-        return quad >= 2u ? (quad - 2u) * MT : (quad + 6u) * MT > kBarrierSlot ? (quad + 6u) * MT : kBarrierSlot + 1u;
-    };
-    auto reads_at = [=](uint32_t slot) constexpr -> uint32_t {
-        uint32_t n = 0;
-        for (uint32_t un = 0; un < kUnits; ++un) n += frag_slot(un) == slot ? 1u : 0u;
-        for (uint32_t quad = 0; quad < 8u; ++quad) n += quad_slot(quad) == slot ? kQuadReads[quad & 1u] : 0u;
-        return n;
-    };
-    // ... behind the last fragment of group g and before the group begins; and behind the step's own last one and before the barrier
-    auto in_flight = [=](uint32_t g) constexpr -> uint32_t {
-        uint32_t n = 0;
-        const uint32_t last = frag_slot(4u * g + 3u);
-        for (uint32_t slot = last + 1u; slot < 16u * g + (g < 2u ? kSlots : 0u); ++slot) n += reads_at(slot % kSlots);
-        return n;
-    };
-    auto in_flight_at_barrier = [=]() constexpr -> uint32_t {
-        uint32_t n = 0;
-        for (uint32_t slot = frag_slot(kUnits - 1u) + 1u; slot < kBarrierSlot; ++slot) n += reads_at(slot);
-        return n;
-    };
+    //   memory: codes (in rows of step kt + 3, packed of kt + 2), group scales of kt + 3 and the copies of A of kt + 2, evenly over the step.
+    // The step's one barrier stands 24 slots before its end, where the next step's first fragments and the codes after it are about to be read: before
+    // it the wave makes sure that its part of them has landed (requested in the step before: what may still be in flight then is this step's
+    // own) and that it has everything it reads of this step's A and the next one's codes and scales.  Behind it every wave's part has landed, and
+    // nobody reads this step's A or the next one's codes any more: copies requested from there on go to their places.
+    using Step = WregStep<BITS, GROUPED, PACKED, MT>;
+    static_assert(Step::quad_slot(6u) < Step::quad_slot(7u) && Step::quad_slot(7u) < Step::kBarrierSlot && Step::frag_slot(Step::kUnits - 1u) < Step::kBarrierSlot,
+                  "a step's reads of its own A and the next step's codes stand before its barrier");
+    constexpr uint32_t kUnits = Step::kUnits, kSlots = Step::kSlots, kBarrierSlot = Step::kBarrierSlot;
     bf16x8_t af[12];
     auto step = [&](auto at_c, uint32_t kt, const Ops& cur, Ops& nxt, const Raw& raw1, Raw& raw2) {
         constexpr uint32_t S = decltype(at_c)::value, kTurn = S * kUnits;
@@ -471,39 +440,39 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
         const uint32_t a_ve = last ? a_last_e : a_voff_e, a_vo = last ? a_last_o : a_voff_o;
         uint32_t a_soff = kt2 * kWrK * 2u;
         Conversion w;
-        if constexpr (PACKED) wait_vm<kBehindCodes>();  // raw1's
+        if constexpr (PACKED) wait_vm<Step::behind_codes()>();  // raw1's
         __builtin_amdgcn_sched_barrier(0);
         for_each_const<kSlots>([&](auto slot_c) {
             constexpr uint32_t slot = decltype(slot_c)::value;
             constexpr uint32_t u = slot >> 2, j = slot & 3u, blk = u / MT, mt = u % MT;
-            if constexpr (slot % 16u == 0u) wait_lds<in_flight(slot / 16u)>();
+            if constexpr (slot % 16u == 0u) wait_lds<Step::in_flight(slot / 16u)>();
             mfma16<4u * mt + j>(af[(u + kTurn) % 12u],
                                 __builtin_bit_cast(bf16x8_t, make_uint4(cur.w[blk][j][0], cur.w[blk][j][1], cur.w[blk][j][2], cur.w[blk][j][3])));
             if constexpr (slot == kBarrierSlot) {
-                wait_vm<kBeforeBarrier>();
-                wait_lds<in_flight_at_barrier()>();
+                wait_vm<Step::requests_before(kBarrierSlot)>();
+                wait_lds<0>();
                 barrier_no_fence();  // (a fenced barrier would also wait for the copies this step has just started)
             }
             for_each_const<2u>([&](auto next_c) {  // a fragment: of the unit two groups on; behind the barrier the next step's first
                 constexpr bool next = decltype(next_c)::value != 0u;
                 constexpr uint32_t un = next ? (slot - kBarrierSlot) / 3u : slot / 4u + 8u;
-                if constexpr (next ? slot >= kBarrierSlot && un < 8u && frag_slot(un) == slot : un < kUnits && frag_slot(un) == slot) {
+                if constexpr (next ? slot >= kBarrierSlot && un < 8u && Step::frag_slot(un) == slot : un < kUnits && Step::frag_slot(un) == slot) {
                     if constexpr (next) af[(un + kUnits + kTurn) % 12u] = read_frag(Next{}, 0, un);
                     else af[(un + kTurn) % 12u] = read_frag(Now{}, un / MT, un % MT);
                 }
             });
             for_each_const<8u>([&](auto quad_c) {
-                if constexpr (quad_slot(decltype(quad_c)::value) == slot) {
+                if constexpr (Step::quad_slot(decltype(quad_c)::value) == slot) {
                     if constexpr (decltype(quad_c)::value < 2u) read_quad(After{}, quad_c);
                     else read_quad(Next{}, quad_c);
                 }
             });
             constexpr uint32_t from = slot * Schedule::kOps / kSlots, to = (slot + 1u) * Schedule::kOps / kSlots;
             for_each_const<to - from>([&](auto i_c) { convert_op(nxt, w, raw1, std::integral_constant<uint32_t, from + decltype(i_c)::value>{}); });
-            constexpr uint32_t r = first_at_least<kRequests>(request_slot, slot);
-            if constexpr (r < kRequests && request_slot(r) == slot) {
-                constexpr uint32_t c = copies_before(r), q = r - c;
-                if constexpr (copies_before(r + 1u) != c) {
+            constexpr uint32_t r = Step::requests_before(slot);
+            if constexpr (Step::requests_before(slot + 1u) != r) {
+                constexpr uint32_t c = Step::copies_before(r), q = r - c;
+                if constexpr (Step::copies_before(r + 1u) != c) {
                     copy_a(After{}, std::integral_constant<uint32_t, c>{}, a_ve, a_vo, a_soff);
                     a_soff += 16u * p.lda;
                     asm("" : "+s"(a_soff));  // (or each request gets a multiplication of its own)
