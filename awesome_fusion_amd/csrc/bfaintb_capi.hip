@@ -482,8 +482,11 @@ static double family_beside_tiles_us(double us, uint32_t m, uint32_t n, int bits
 // Whether the row-blocked family, at its estimated time, is the one to run.
 static bool family_leads_tiles(double family_us, uint32_t m, uint32_t n, uint32_t k, int bits, bool packed, bool second_launch)
 {
-    // (the family is estimated at 0.8 of what it takes on the shapes that meet the tiles of 256 columns, those at what they take)
-    if (second_launch && wide_tiles(m, n, k, bits).blocks != 0u) return 1.15 * family_us < wide_tiles(m, n, k, bits).us;
+    // Never where tiles of 256 columns run.  From a k of 512 on they are estimated faster on every one of 60000 random shapes; below, the family's
+    // estimate leaves out what a workgroup's start costs, some 6 us a round of them, and it takes 1.8 to 3.9 times as long (us, family / tiles: 1952 x
+    // 28640 x 128 8-bit g32 168.6 / 49.4; 3630 x 13840 x 128 packed 4-bit 154.4 / 48.6; 350 x 33264 x 128 packed 8-bit 39.9 / 16.8; 529 x 25456 x 256
+    // packed 8-bit 50.7 / 20.7).  Nor do the tiles need the device's set-up, so such a call may be a first one under capture.
+    if (second_launch && wide_tiles(m, n, k, bits).blocks != 0u) return false;
     if (!prefill_small_tiles(m, n, k, bits)) return family_us < prefill_estimate_us(m, n, k, bits, second_launch);
     const TilePlan t = tile128_plan(m, n, k, bits, 0, second_launch);
     if (!second_launch) return family_us < t.us;  // (the estimates of the time before: see tile128_plan)

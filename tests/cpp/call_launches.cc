@@ -1,5 +1,5 @@
 // Makes the calls it reads (m n k weight_bits kind workspace_bytes, one per line; kind 0: bfaintb_gemm, 1: bfaintb_gemm_prepacked,
-// 2: bfaintb_gemm_static under capture, 3: bfaintb_gemm_reference; 0 bytes: no workspace) on a stand-in for the HIP runtime and prints what each returned,
+// 2: bfaintb_gemm_static under capture, 3: bfaintb_gemm_reference, 4: as 0 and 5: as 1, under capture; 0 bytes: no workspace) on a stand-in for the HIP runtime and prints what each returned,
 // how many kernels it launched and the workgroups of the first.
 #include "stand_in_runtime.hpp"
 
@@ -26,7 +26,8 @@ int main()
         void* const ws = bytes ? p : nullptr;
         g_launches = 0;
         g_workgroups = 0;
-        g_capturing = kind == 2;
+        g_capturing = kind == 2 || kind > 3;
+        if (kind > 3) kind -= 4;
         const int rc = kind == 3   ? bfaintb_gemm_reference(p, p, p, static_cast<float*>(p), m, n, k, k, n, n, ws, bytes, nullptr)
                        : kind == 2   ? bfaintb_gemm_static(p, p, p, p, m, n, k, k, n, n, bits, 0, nullptr)
                        : kind == 1 ? bfaintb_gemm_prepacked(p, p, p, p, nullptr, m, n, k, k, n, bits, 0, ws, bytes, nullptr)

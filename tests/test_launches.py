@@ -177,3 +177,17 @@ def test_calls_of_the_slab_kernel_need_no_scratch_and_no_set_up(tmp_path):
     got = calls(tmp_path, ["%d %d %d %d 1 0" % s for s in shapes])
     assert [x[:2] for x in got] == [(0, 1)] * len(shapes)
     assert [x[2] for x in got[:len(NOW_FAMILY)]] == [af.plan(m, n, k, bits, packed=True).workgroups for m, n, k, bits in NOW_FAMILY]
+
+
+# many rows and a short k (width of the codes last): tiles, which need neither scratch nor the device's set-up
+SHORT_K = [(1901, 12544, 128, 4), (516, 37184, 128, 8), (141, 43360, 256, 4), (2889, 28096, 128, 8), (350, 33264, 128, 8), (529, 25456, 256, 8), (2571, 45456, 128, 4)]
+
+
+def test_a_short_k_runs_tiles_and_may_be_a_first_call_under_capture(tmp_path):
+    import awesome_fusion_amd as af
+    for m, n, k, bits in SHORT_K:
+        for packed in (False, True):
+            pl = af.plan(m, n, k, bits, packed=packed)
+            assert pl.kernel >= af.KERNEL_TILES_128 and pl.splits == 1 and pl.workspace_bytes == 0, pl.as_dict()
+    got = calls(tmp_path, ["%d %d %d %d %d 0" % (*s, kind) for s in SHORT_K for kind in (4, 5, 2)])
+    assert [x[0] for x in got] == [0] * len(got) and all(x[1] >= 1 for x in got), got
