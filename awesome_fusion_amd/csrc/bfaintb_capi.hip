@@ -1665,13 +1665,21 @@ static double launch_time_us(uint32_t m, uint32_t n, uint32_t k, int bits, bool 
     if (few_rows_on_tiles(m, n, k, bits, grouped, packed, n)) return tile128_plan(m, n, k, bits, 1).us;
     if (m <= kDecodeAutoMaxM) return 6.0 + (double)n * k * bits / 8.0 / 3.3e6 * (m <= 16u ? 1.0 : 1.25);
     if (m <= kDecodeFamilyAutoMaxM) {  // (beyond 32 rows the library's own choice asks just this)
-        const double family = packed ? packed_family_time_us(m, n, k, bits, packed_family_plan(m, n, k, bits)) : decode_family_time_us(m, n, k, bits, decode_plan(m, n, k, bits, 0));
-        if (family_leads_tiles(family, m, n, k, bits, packed, true))
-            return prefill_small_tiles(m, n, k, bits) ? family_beside_tiles_us(family, m, n, bits, packed) : family;
+        const DecodePlan pl = packed ? packed_family_plan(m, n, k, bits) : decode_plan(m, n, k, bits, 0);
+        const double family = packed ? packed_family_time_us(m, n, k, bits, pl) : decode_family_time_us(m, n, k, bits, pl);
+        if (family_leads_tiles(family, m, n, k, bits, packed, true)) {
+            // (a short k: the start of a round of workgroups, 5.2 to 6.6 us at k = 128 to 640, which the estimate leaves out)
+            const double rounds = (double)((n + pl.cols - 1u) / pl.cols) * pl.splits * ((m + 16u * pl.mb - 1u) / (16u * pl.mb)) / machine_cus();
+            const double starts = k <= 1024u && rounds > 1.0 ? 6.0 * (rounds - 1.0) : 0.0;
+            return starts + (prefill_small_tiles(m, n, k, bits) ? family_beside_tiles_us(family, m, n, bits, packed) : family);
+        }
     }
     const WideTiles wide = wide_tiles(m, n, k, bits);
     if (wide.blocks != 0u) return wide.us;
-    if (prefill_small_tiles(m, n, k, bits) || prefill_tall_tiles(m, n, k, bits)) return prefill_estimate_us(m, n, k, bits);
+    // (tall tiles of one chain are estimated 4.9 us short, which the choice against the family is fitted with and which does not matter there; next to
+    // tiles of 256 columns at what they take it would send products with a short k to two launches: 50 shapes of k = 128 to 1792, 4.4 to 5.5 on nearly all)
+    if (prefill_tall_tiles(m, n, k, bits)) return prefill_estimate_us(m, n, k, bits) + (tall_tiles_in_one_chain(m, k) ? 4.9 : 0.0);
+    if (prefill_small_tiles(m, n, k, bits)) return prefill_estimate_us(m, n, k, bits);
     return square_tiles_us(m, n, k, bits);
 }
 

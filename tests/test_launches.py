@@ -191,3 +191,15 @@ def test_a_short_k_runs_tiles_and_may_be_a_first_call_under_capture(tmp_path):
             assert pl.kernel >= af.KERNEL_TILES_128 and pl.splits == 1 and pl.workspace_bytes == 0, pl.as_dict()
     got = calls(tmp_path, ["%d %d %d %d %d 0" % (*s, kind) for s in SHORT_K for kind in (4, 5, 2)])
     assert [x[0] for x in got] == [0] * len(got) and all(x[1] >= 1 for x in got), got
+
+
+# what tall tiles of one chain and the family's workgroups take to start, left out, made two launches of these (width of the codes, group size, packed)
+NOT_TWO_LAUNCHES = [(2515, 7584, 384, 4, 128, False), (1995, 10832, 256, 8, 64, True), (564, 25648, 128, 8, 64, False), (1488, 13584, 256, 8, 32, True),
+                    (2857, 12832, 128, 8, 32, True), (1130, 45424, 512, 4, 32, True), (1818, 27856, 128, 8, 64, True)]
+
+
+@pytest.mark.parametrize("m,n,k,bits,group,packed", NOT_TWO_LAUNCHES)
+def test_a_short_k_is_one_launch_where_two_take_longer(m, n, k, bits, group, packed):
+    import awesome_fusion_amd as af
+    pl = af.plan(m, n, k, bits, group, packed=packed)
+    assert (pl.kernel, pl.tile_cols, pl.launches) == (af.KERNEL_TILES_256, 256, 1), pl.as_dict()
