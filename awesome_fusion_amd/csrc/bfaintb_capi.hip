@@ -435,12 +435,12 @@ static double square_tiles_us(uint32_t m, uint32_t n, uint32_t k, int bits)
 // 4096 8-bit g128 101 / 70; 418 x 17728 x 9728 packed 8-bit g128 205 / 150; 577 x 13824 x 5120 packed 4-bit g128 93.0 / 82.8; 913 x 9296 x 3328 packed 8-bit 70.3 /
 // 55.5; 1010 x 17776 x 1024 8-bit 56.8 / 46.0.
 // (At least 96 of them: the estimates are for a machine's worth of tiles.)
-static WideTiles wide_tiles(uint32_t m, uint32_t n, uint32_t k, int bits)
+static WideTiles wide_tiles_rule(uint32_t m, uint32_t n, uint32_t k, int bits)
 {
     const WideTiles none{0u, 0u, 0.0};
     const uint64_t cus = machine_cus();
     if (prefill_small_tiles(m, n, k, bits)) {
-        if ((uint64_t)((n + 127u) / 128u) <= cus || m <= 96u || m > 128u || k < 1024u) return none;
+        if ((uint64_t)((n + 127u) / 128u) <= cus || m > 128u || k < 1024u) return none;
         const WideTiles w = wide_tiles_best(m, n, k, bits);
         return w.us < 0.95 * tile128_plan(m, n, k, bits, 0).us ? w : none;
     }
@@ -448,11 +448,31 @@ static WideTiles wide_tiles(uint32_t m, uint32_t n, uint32_t k, int bits)
     const WideTiles w = wide_tiles_best(m, n, k, bits);
     return w.rows_of_tiles * ((n + 255u) / 256u) >= 96u && w.us < square_tiles_us(m, n, k, bits) ? w : none;
 }
+// (a call asks up to five times, for its scratch, its choices and its launch: each thread keeps the last answers, one per slot of a hash of the question;
+// host time of a known call, ns, without / with: 128 x 43680 x 4096 768 / 70, 913 x 9296 x 3328 packed 731 / 68, 2048 x 28672 x 8192 4-bit 557 / 206)
+static WideTiles wide_tiles(uint32_t m, uint32_t n, uint32_t k, int bits)
+{
+    if (m <= 96u) return WideTiles{0u, 0u, 0.0};
+    struct Answer {
+        uint32_t m, n, k, bits, cus;
+        WideTiles tiles;
+    };
+    static thread_local Answer answers[256] = {};
+    const uint32_t cus = machine_cus();
+    Answer& a = answers[((m * 2654435761u) ^ (n * 2246822519u) ^ (k * 3266489917u) ^ (uint32_t)bits) >> 24];
+    if (a.m != m || a.n != n || a.k != k || a.bits != (uint32_t)bits || a.cus != cus) a = Answer{m, n, k, (uint32_t)bits, cus, wide_tiles_rule(m, n, k, bits)};
+    return a.tiles;
+}
 
+// Whether they run by the library's own choice, and nobody asks the row-blocked family.  From a k of 512 on its estimate is the higher one on every one
+// of 60000 random shapes; below, the estimate leaves out what a workgroup's start costs, some 6 us a round of them, and the family takes 1.8 to 3.9
+// times as long (us, family / tiles: 1952 x 28640 x 128 8-bit g32 168.6 / 49.4; 3630 x 13840 x 128 packed 4-bit 154.4 / 48.6; 350 x 33264 x 128 packed
+// 8-bit 39.9 / 16.8; 529 x 25456 x 256 packed 8-bit 50.7 / 20.7).  Nor do the tiles need the device's set-up, so such a call may be a first one under capture.
+static bool wide_tiles_run(uint32_t m, uint32_t n, uint32_t k, int bits, bool second_launch) { return second_launch && wide_tiles(m, n, k, bits).blocks != 0u; }
+
+// What the other tiles take.
 static double prefill_estimate_us(uint32_t m, uint32_t n, uint32_t k, int bits, bool second_launch = true)
 {
-    const WideTiles wide = wide_tiles(m, n, k, bits);
-    if (wide.blocks != 0u && second_launch) return wide.us;
     if (prefill_small_tiles(m, n, k, bits)) return tile128_plan(m, n, k, bits, 0, second_launch).us;
     const double cus = (double)machine_cus();
     if (prefill_tall_tiles(m, n, k, bits)) {
@@ -479,14 +499,9 @@ static double family_beside_tiles_us(double us, uint32_t m, uint32_t n, int bits
     return bits == 8 ? (1.035 + 0.165 * ragged) * us + 0.7 * (ragged - 1.0) + 0.0016 * m : (0.80 + 0.2 * ragged) * us + 2.3;
 }
 
-// Whether the row-blocked family, at its estimated time, is the one to run.
+// Whether the row-blocked family, at its estimated time, is the one to run; where tiles of 256 columns run it is not asked.
 static bool family_leads_tiles(double family_us, uint32_t m, uint32_t n, uint32_t k, int bits, bool packed, bool second_launch)
 {
-    // Never where tiles of 256 columns run.  From a k of 512 on they are estimated faster on every one of 60000 random shapes; below, the family's
-    // estimate leaves out what a workgroup's start costs, some 6 us a round of them, and it takes 1.8 to 3.9 times as long (us, family / tiles: 1952 x
-    // 28640 x 128 8-bit g32 168.6 / 49.4; 3630 x 13840 x 128 packed 4-bit 154.4 / 48.6; 350 x 33264 x 128 packed 8-bit 39.9 / 16.8; 529 x 25456 x 256
-    // packed 8-bit 50.7 / 20.7).  Nor do the tiles need the device's set-up, so such a call may be a first one under capture.
-    if (second_launch && wide_tiles(m, n, k, bits).blocks != 0u) return false;
     if (!prefill_small_tiles(m, n, k, bits)) return family_us < prefill_estimate_us(m, n, k, bits, second_launch);
     const TilePlan t = tile128_plan(m, n, k, bits, 0, second_launch);
     if (!second_launch) return family_us < t.us;  // (the estimates of the time before: see tile128_plan)
@@ -818,7 +833,7 @@ int resolve_variant(uint32_t m, uint32_t n, uint32_t k, int bits, int variant, b
 {
     if (variant == BFAINTB_VARIANT_AUTO) {
         if (m <= kDecodeAutoMaxM) return BFAINTB_VARIANT_DECODE;
-        if (m > kDecodeFamilyAutoMaxM) return BFAINTB_VARIANT_PREFILL;
+        if (m > kDecodeFamilyAutoMaxM || wide_tiles_run(m, n, k, bits, second_launch)) return BFAINTB_VARIANT_PREFILL;
         const DecodePlan pl = decode_plan(m, n, k, bits, 0);
         return family_leads_tiles(decode_family_time_us(m, n, k, bits, pl), m, n, k, bits, false, second_launch) ? BFAINTB_VARIANT_DECODE : BFAINTB_VARIANT_PREFILL;
     }
@@ -1527,6 +1542,7 @@ static bool packed_slab_leads_eight_blocks(uint32_t m, uint32_t n, uint32_t k, i
 }
 static bool packed_uses_slab(uint32_t m, uint32_t n, uint32_t k, int bits)
 {
+    if (m > kDecodeAutoMaxM) return false;
     const DecodePlan pl = packed_family_plan(m, n, k, bits);
     return packed_slab_leads(m, n, k, bits, pl, true) || (pl.splits > 1u && packed_slab_leads_eight_blocks(m, n, k, bits));
 }
@@ -1621,7 +1637,7 @@ static int packed_variant(uint32_t m, uint32_t n, uint32_t k, int bits, int vari
     if (is_prefill(variant)) return variant;
     if (variant != BFAINTB_VARIANT_AUTO) return BFAINTB_ERR_BAD_VARIANT;
     if (packed_uses_slab(m, n, k, bits) || m <= kDecodeAutoMaxM) return BFAINTB_VARIANT_DECODE;
-    if (m > kDecodeFamilyAutoMaxM) return BFAINTB_VARIANT_PREFILL;
+    if (m > kDecodeFamilyAutoMaxM || wide_tiles_run(m, n, k, bits, second_launch)) return BFAINTB_VARIANT_PREFILL;
     const DecodePlan pl = packed_family_plan(m, n, k, bits);
     return family_leads_tiles(packed_family_time_us(m, n, k, bits, pl), m, n, k, bits, true, second_launch) ? BFAINTB_VARIANT_DECODE : BFAINTB_VARIANT_PREFILL;
 }
@@ -1664,6 +1680,8 @@ static double launch_time_us(uint32_t m, uint32_t n, uint32_t k, int bits, bool 
 {
     if (few_rows_on_tiles(m, n, k, bits, grouped, packed, n)) return tile128_plan(m, n, k, bits, 1).us;
     if (m <= kDecodeAutoMaxM) return 6.0 + (double)n * k * bits / 8.0 / 3.3e6 * (m <= 16u ? 1.0 : 1.25);
+    const WideTiles wide = wide_tiles(m, n, k, bits);
+    if (wide.blocks != 0u) return wide.us;
     if (m <= kDecodeFamilyAutoMaxM) {  // (beyond 32 rows the library's own choice asks just this)
         const DecodePlan pl = packed ? packed_family_plan(m, n, k, bits) : decode_plan(m, n, k, bits, 0);
         const double family = packed ? packed_family_time_us(m, n, k, bits, pl) : decode_family_time_us(m, n, k, bits, pl);
@@ -1674,8 +1692,6 @@ static double launch_time_us(uint32_t m, uint32_t n, uint32_t k, int bits, bool 
             return starts + (prefill_small_tiles(m, n, k, bits) ? family_beside_tiles_us(family, m, n, bits, packed) : family);
         }
     }
-    const WideTiles wide = wide_tiles(m, n, k, bits);
-    if (wide.blocks != 0u) return wide.us;
     // (tall tiles of one chain are estimated 4.9 us short, which the choice against the family is fitted with and which does not matter there; next to
     // tiles of 256 columns at what they take it would send products with a short k to two launches: 50 shapes of k = 128 to 1792, 4.4 to 5.5 on nearly all)
     if (prefill_tall_tiles(m, n, k, bits)) return prefill_estimate_us(m, n, k, bits) + (tall_tiles_in_one_chain(m, k) ? 4.9 : 0.0);
@@ -1732,8 +1748,8 @@ static uint32_t row_split_rule(uint32_t m, uint32_t n, uint32_t k, int bits, boo
 }
 
 // (a call asks two or three times, for its scratch and for its launch, and a model asks about the same few shapes: each
-// thread keeps the last answers, one per slot of a hash of the question.  A new question costs 0.9 - 1.8 us of host time, where
-// one launch's plan takes 0.15; a known one 0.2, or 0.5 if the answer is two launches.  A prompt of a new length asks once per
+// thread keeps the last answers, one per slot of a hash of the question.  A new question costs 1.5 - 3.2 us of host time; a known one
+// 0.07 where tiles of 256 columns run, 0.2 otherwise, and 0.7 - 1 if the answer is two launches.  A prompt of a new length asks once per
 // shape of its layers, as long as no two of them share a slot)
 static uint32_t row_split_head(uint32_t m, uint32_t n, uint32_t k, int bits, bool packed, bool grouped)
 {

@@ -203,3 +203,14 @@ def test_a_short_k_is_one_launch_where_two_take_longer(m, n, k, bits, group, pac
     import awesome_fusion_amd as af
     pl = af.plan(m, n, k, bits, group, packed=packed)
     assert (pl.kernel, pl.tile_cols, pl.launches) == (af.KERNEL_TILES_256, 256, 1), pl.as_dict()
+
+
+def test_a_known_call_on_tiles_of_256_columns_takes_the_host_no_longer(tmp_path):
+    """The choice of these tiles is made once for a shape, not several times a call: against tall tiles, which are not asked about."""
+    import awesome_fusion_amd as af
+    assert af.plan(1024, 8192, 4096).kernel == af.KERNEL_TILES_128
+    shapes = ["128 43680 4096 8 0", "913 9296 3328 8 1", "384 22016 4096 4 0"]
+    r = on_stand_in(tmp_path, "host_time", "\n".join(["1024 8192 4096 8 0"] + shapes))
+    assert r.returncode == 0
+    tall, *wide = map(float, r.stdout.split())
+    assert max(wide) < 1.5 * tall, (tall, wide)
