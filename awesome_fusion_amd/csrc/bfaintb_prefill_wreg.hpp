@@ -46,8 +46,8 @@ constexpr uint32_t kWrCRowBytes = 256 * 2;     // epilogue staging row
 __device__ __forceinline__ uint32_t wr_swz(uint32_t row, uint32_t chunk) { return row * 128u + ((chunk ^ ((row >> 1) & 7u)) << 4); }
 
 // The accumulators are the accumulation registers a[0 : 16 MT - 1], by name: accumulator (mt, j) is the four from 16 mt + 4 j on.  The
-// compiler knows of them only that the kernel uses them (acc_reserve), and has no other use for them as long as it does not run out of its
-// 256 ordinary registers.  Given to it as variables, it keeps part of 256 of them in ordinary registers and shuttles them back and
+// compiler knows of them only that the kernel uses them (acc_reserve, at the start and the end of every path), and has no other use for them as
+// long as it does not run out of its 256 ordinary registers; tests/test_compiled_tiles.py looks whether it had.  Given to it as variables, it keeps part of 256 of them in ordinary registers and shuttles them back and
 // forth around every matrix instruction, or, as in-out operands of the assembly, moves some where paths through the kernel
 // meet.  What its hazard bookkeeping cannot see behind the assembly is kept safe by construction: the operands a and b are written
 // (LDS reads, conversions) long before, under waits for LDS; the accumulators are read only in the epilogue, behind explicit idle cycles
@@ -655,6 +655,7 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
             }
             if constexpr (half == 0u) __syncthreads();  // the second half overwrites the staging area
         });
+        acc_reserve<MT>();
         return;
     }
     // Residual and / or the SiLU gate: the fp32 sums are staged, as many blocks of 16 rows as the arrays hold at a time, and each thread
