@@ -464,6 +464,12 @@ static WideTiles wide_tiles(uint32_t m, uint32_t n, uint32_t k, int bits)
     return a.tiles;
 }
 
+// The same for a call that may name a split of k: one that does keeps the small tiles, which have it, wherever they would run without these.
+static WideTiles wide_tiles(uint32_t m, uint32_t n, uint32_t k, int bits, uint32_t split_k)
+{
+    return split_k != 0u && prefill_small_tiles(m, n, k, bits) ? WideTiles{0u, 0u, 0.0} : wide_tiles(m, n, k, bits);
+}
+
 // Whether they run by the library's own choice, and nobody asks the row-blocked family.  From a k of 512 on its estimate is the higher one on every one
 // of 60000 random shapes; below, the estimate leaves out what a workgroup's start costs, some 6 us a round of them, and the family takes 1.8 to 3.9
 // times as long (us, family / tiles: 1952 x 28640 x 128 8-bit g32 168.6 / 49.4; 3630 x 13840 x 128 packed 4-bit 154.4 / 48.6; 350 x 33264 x 128 packed
@@ -883,16 +889,16 @@ static hipError_t launch_few_rows_on_tiles(GemmParams p, int bits, bool packed, 
 }
 
 // whether a tiled-variant launch over row-major weights goes to the small-tile kernel that can split k
-static bool tiled_may_split(int v, uint32_t m, uint32_t n, uint32_t k, int bits)
+static bool tiled_may_split(int v, uint32_t m, uint32_t n, uint32_t k, int bits, uint32_t split_k = 0)
 {
-    return use_small_tiles(v, m, n, k, bits) && v != BFAINTB_VARIANT_PREFILL_128_LDS && !(v == BFAINTB_VARIANT_PREFILL && wide_tiles(m, n, k, bits).blocks != 0u);
+    return use_small_tiles(v, m, n, k, bits) && v != BFAINTB_VARIANT_PREFILL_128_LDS && !(v == BFAINTB_VARIANT_PREFILL && wide_tiles(m, n, k, bits, split_k).blocks != 0u);
 }
 
 size_t workspace_need(uint32_t m, uint32_t n, uint32_t k, int bits, int variant, uint32_t forced_split)
 {
     if (m == 0 || n == 0) return 0;
     if (variant == BFAINTB_VARIANT_DECODE) return split_workspace_bytes(decode_plan(m, n, k, bits, forced_split).splits, m, n);
-    if (is_prefill(variant) && tiled_may_split(variant, m, n, k, bits)) return tile_workspace_bytes(tile128_plan(m, n, k, bits, forced_split), m, n);
+    if (is_prefill(variant) && tiled_may_split(variant, m, n, k, bits, forced_split)) return tile_workspace_bytes(tile128_plan(m, n, k, bits, forced_split), m, n);
     return 0;
 }
 
@@ -1274,7 +1280,7 @@ static int gemm_impl(void* c, const void* a, const void* b, const void* scale, c
         return (int)bfaintb::launch_prefill(p, weight_bits, st, v != BFAINTB_VARIANT_PREFILL_256_LDS);
 #endif
         // row-major weights on small tiles: that form, unless the other one is asked for by name
-        small_wreg = tiled_may_split(v, m, n, k, weight_bits) && bfaintb::prefill128_wreg_serves(p);
+        small_wreg = tiled_may_split(v, m, n, k, weight_bits, split_k) && bfaintb::prefill128_wreg_serves(p);
         if (small_wreg) {
             const TilePlan tp = tile128_plan(m, n, k, weight_bits, split_k, second_launch);
             p.k_per_wg = tp.k_per_wg;
@@ -2065,7 +2071,7 @@ static int plan_whole(uint32_t m, uint32_t n, uint32_t k, int weight_bits, uint3
     }
     // the tiled kernels
     if (v == BFAINTB_VARIANT_PREFILL) {
-        const WideTiles w = wide_tiles(m, n, k, weight_bits);
+        const WideTiles w = wide_tiles(m, n, k, weight_bits, packed ? 0u : split_k);
         if (w.blocks != 0u) {
             out->variant = v;  // (no variant names these tiles)
             out->kernel = BFAINTB_KERNEL_TILES_256;

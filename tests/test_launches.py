@@ -214,3 +214,15 @@ def test_a_known_call_on_tiles_of_256_columns_takes_the_host_no_longer(tmp_path)
     assert r.returncode == 0
     tall, *wide = map(float, r.stdout.split())
     assert max(wide) < 1.5 * tall, (tall, wide)
+
+
+# 97 to 128 rows against more than a round of small tiles: tiles of 256 columns, but where the call names a split of k, which only the small ones have
+@pytest.mark.parametrize("m,n,k,bits", [(101, 38464, 3712, 4), (126, 39888, 1024, 8), (128, 43680, 4096, 8)])
+def test_a_named_split_of_k_keeps_the_tiles_that_have_it(m, n, k, bits):
+    import awesome_fusion_amd as af
+    for which in (af.AUTO, af.PREFILL):
+        assert af.plan(m, n, k, bits, which=which).tile_cols == 256
+        for split in (1, 2, 3):
+            pl = af.plan(m, n, k, bits, which=which, force_split_k=split)
+            assert (pl.kernel, pl.tile_cols, pl.splits) == (af.KERNEL_TILES_128, 128, split), pl.as_dict()
+            assert pl.workspace_bytes == af.workspace_bytes(m, n, k, bits, which=which, force_split_k=split) and (pl.workspace_bytes != 0) == (split > 1)
