@@ -91,7 +91,7 @@ __device__ __forceinline__ f32x4_t acc_read()
 }
 __device__ __forceinline__ void acc_settle() { asm volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
 
-// Waits as instructions that the compiler sees: it adds none of its own for what they cover.
+// Waits as instructions that the compiler sees: it adds none of its own for what they cover (where paths meet, only if every one of them has it covered).
 template <uint32_t IN_FLIGHT>
 __device__ __forceinline__ void wait_vm()
 {
@@ -531,19 +531,33 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
     using C3 = std::integral_constant<uint32_t, 3>;
     using C4 = std::integral_constant<uint32_t, 4>;
     using C5 = std::integral_constant<uint32_t, 5>;
-    for (uint32_t kt = 0;; kt += 6) {  // (six: stages by threes, operands by twos)
+    // Six at a time (stages by threes, operands by twos), in a loop that is left at its end only, and the last one to six behind it.  With an exit
+    // behind each step the compiler led all of them round by the loop's head, took what every step's end has in flight for what the head has, and waited
+    // there for all of a wave's copies, those of a dozen slots ago included.  us, so / now: 2684 x 3888 x 8832 4-bit g32 163.0 / 160.0, 2670 x 3104 x 4864
+    // packed 8-bit 78.4 / 75.5, 3128 x 9280 x 2304 packed 8-bit g128 124.7 / 121.1; up to a k of 768 level (the loop over whole sixes, with up to five
+    // behind it, loses up to 2 % there: its last steps' code is a workgroup's first).
+    uint32_t kt = 0;
+    for (; kt + 6 < ksteps; kt += 6) {
         step(C0{}, kt, ops0, ops1, rawa, rawb);
-        if (kt + 1 == ksteps) break;
         step(C1{}, kt + 1, ops1, ops0, rawb, rawa);
-        if (kt + 2 == ksteps) break;
         step(C2{}, kt + 2, ops0, ops1, rawa, rawb);
-        if (kt + 3 == ksteps) break;
         step(C3{}, kt + 3, ops1, ops0, rawb, rawa);
-        if (kt + 4 == ksteps) break;
         step(C4{}, kt + 4, ops0, ops1, rawa, rawb);
-        if (kt + 5 == ksteps) break;
         step(C5{}, kt + 5, ops1, ops0, rawb, rawa);
-        if (kt + 6 == ksteps) break;
+    }
+    step(C0{}, kt, ops0, ops1, rawa, rawb);
+    if (kt + 1 < ksteps) {
+        step(C1{}, kt + 1, ops1, ops0, rawb, rawa);
+        if (kt + 2 < ksteps) {
+            step(C2{}, kt + 2, ops0, ops1, rawa, rawb);
+            if (kt + 3 < ksteps) {
+                step(C3{}, kt + 3, ops1, ops0, rawb, rawa);
+                if (kt + 4 < ksteps) {
+                    step(C4{}, kt + 4, ops0, ops1, rawa, rawb);
+                    if (kt + 5 < ksteps) step(C5{}, kt + 5, ops1, ops0, rawb, rawa);
+                }
+            }
+        }
     }
 #ifdef BFAINTB_TRACE
     {   // shader cycles and 100 MHz ticks the K loop took, per wave: words 0, 1 of the wave's 8

@@ -1,6 +1,7 @@
 """What the compiler made of bfaintb_prefill_wreg_kernel, whose accumulators are accumulation registers by name (acc_reserve in
 bfaintb_prefill_wreg.hpp) and whose matrix instructions are assembly that its bookkeeping does not see into: that nothing else uses those
-registers, and that no ordinary instruction writes a matrix instruction's operands in the two wait states before it."""
+registers, that no ordinary instruction writes a matrix instruction's operands in the two wait states before it, and that a step waits for memory where
+it says so and nowhere else."""
 import os
 import re
 import shutil
@@ -57,6 +58,17 @@ def check_listing(lines):
     return count, wrong
 
 
+def memory_waits(lines, instructions):
+    """What the waits for memory among the first so many matrix instructions leave in flight."""
+    count, left = 0, []
+    for line in lines:
+        count += line.startswith("v_mfma")
+        m = re.search(r"vmcnt\((\d+)\)", line)
+        if m and 0 < count < instructions:
+            left.append(int(m[1]))
+    return left
+
+
 def test_the_checks_see_what_they_are_for():
     mfma = "v_mfma_f32_16x16x32_bf16 a[0:3], v[0:3], v[4:7], a[0:3]"
     assert check_listing(["v_accvgpr_write_b32 a0, 0", "v_mov_b32_e32 v4, v9", "s_nop 1", mfma, "v_accvgpr_read_b32 v1, a2"]) == (1, [])
@@ -86,7 +98,13 @@ def test_nothing_but_the_matrix_instructions_uses_the_accumulators(tmp_path):
         for part in listing.split("\n<")[1:]:
             name, _, body = part.partition(">:\n")
             if name in seen:
-                seen[name] = check_listing([x.split("//")[0].strip() for x in body.split("\n") if x.strip()])
+                lines = [x.split("//")[0].strip() for x in body.split("\n") if x.strip()]
+                packed, blocks = map(int, re.search(r"ILi\dELb\dELb(\d)ELi(\d+)E", name).groups())
+                # twelve steps are written out (a loop of six, up to six behind it): one wait at a step's barrier and, of packed codes, one at its
+                # start (the first step's stands before its first matrix instruction); none of them for the last copies
+                waits = memory_waits(lines, 12 * 8 * blocks)
+                seen[name] = check_listing(lines) + (len(waits) - (23 if packed else 12), min(waits))
     assert len(seen) == 40, sorted(seen)
-    for name, (count, wrong) in seen.items():
-        assert count >= 6 * 8 * 8 and not wrong, (name, count, wrong[:5])
+    for name, (count, wrong, more_waits, least) in seen.items():
+        assert count >= 12 * 8 * 8 and not wrong, (name, count, wrong[:5])
+        assert more_waits == 0 and least >= 4, (name, more_waits, least)
