@@ -282,7 +282,8 @@ __device__ __forceinline__ void apply_scales(Multipliers<CPL, HALVES>& mu, float
 }
 
 #ifdef BFAINTB_TRACE
-#define TRACE_MARK(i) do { if ((threadIdx.x & 63) == 0) p.trace[((size_t)((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 8 + (i)] = wall_clock64(); } while (0)
+#define TRACE_VALUE(i, v) do { if ((threadIdx.x & 63) == 0) p.trace[((size_t)((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 8 + (i)] = (v); } while (0)
+#define TRACE_MARK(i) TRACE_VALUE(i, wall_clock64())
 #else
 #define TRACE_MARK(i) do { } while (0)
 #endif
@@ -510,7 +511,9 @@ bfaintb_decode_kernel(const GemmParams p)
     constexpr uint32_t kLaneBytes = CPL * BITS / 8;   // bytes of one row a lane loads
     extern __shared__ __attribute__((aligned(16))) float red[];
 
-    TRACE_MARK(0);
+#ifdef BFAINTB_TRACE
+    const unsigned long long trace_start = wall_clock64();  // (stored at the second mark: a branch up here is more than the compiler can do)
+#endif
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // the same for the wave's lanes: what follows from it stays scalar
     const int nl = lane & 15;
@@ -818,6 +821,9 @@ bfaintb_decode_kernel(const GemmParams p)
             }
         }
     }
+#ifdef BFAINTB_TRACE
+    TRACE_VALUE(0, trace_start);
+#endif
     TRACE_MARK(2);
 
     // ---- add the waves' partial sums through LDS, kMBC blocks of 16 rows at a time (what fits): one barrier,
