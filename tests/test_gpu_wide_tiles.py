@@ -88,3 +88,20 @@ def test_scales_of_any_sign_and_size(units64, rows, m, n, bits, group, k):
     helpers.assert_close_at_any_scale(p, c, f"{rows} rows: {m}x{n}x{k} bits={bits} g={group}")
     if k % 128 == 0:
         helpers.assert_close_at_any_scale(p, run_packed(af, p, af.PREFILL), f"{rows} rows, packed: {m}x{n}x{k} bits={bits} g={group}")
+
+
+# 97 to 128 rows that make more small tiles than units: partial blocks of rows and columns, a partial step
+@pytest.mark.parametrize("m", [97, 100, 128])
+@pytest.mark.parametrize("bits,group,k", [(8, 0, 1024), (8, 0, 1032), (8, 64, 1088), (4, 128, 1024), (4, 0, 1280)])
+def test_few_rows_against_many_columns(units64, m, bits, group, k):
+    af, n = units64, 8208
+    p = Problem(m, n, k, bits, group, seed=m)
+    is_wide(af, 128, p)
+    c = run_gemm(p, which=af.PREFILL)
+    assert np.array_equal(c, run_gemm(p, which=af.PREFILL_256_LDS))
+    if k % 128 == 0:
+        is_wide(af, 128, p, True)
+        assert np.array_equal(run_packed(af, p, af.PREFILL), c), "packed"
+    # a call that names a split of k runs the small tiles, which have it
+    assert af.plan(m, n, k, bits, group, which=af.PREFILL, force_split_k=2).splits == 2
+    assert_close_ulp(p, run_gemm(p, which=af.PREFILL, force_split_k=2), "split")
