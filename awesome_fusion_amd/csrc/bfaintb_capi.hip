@@ -397,8 +397,11 @@ struct WideTiles {
     double us;
 };
 // What they take, in us: fitted to 24000 timings of 7269 random shapes (33 ... 4096 rows, both code widths and weight orders, weights cold), 4.3 %
-// rms.  A K-step is 128 cycles of matrix instructions a block and some 770 (8-bit) or 840 (4-bit codes, mostly with group scales) beside
-// them, at 2.39 GHz while few CUs hold few rows, and at what the board's power leaves otherwise: 0.83 of it with 14 blocks on every CU.
+// rms, of the kernel's first form.  A K-step is 128 cycles of matrix instructions a block and some 770 (8-bit) or 840 (4-bit codes, mostly with group
+// scales) beside them, at 2.39 GHz while few CUs hold few rows, and at what the board's power leaves otherwise: 0.83 of it with 14 blocks on every CU.
+// Not fitted again: the kernel takes 330 (16 blocks) to 570 (8) and 540 to 720 beside them today, packed codes alike, and the fit's other terms hold part of
+// the difference.  us, what this says / what a call takes: 384 x 22016 x 4096 8-bit 74.2 / 69.6, 577 x 13824 x 5120 packed 4-bit g128 86.1 / 83.5, packed
+// 8-bit 83.6 / 78.6, 148 x 43680 x 4096 8-bit g128 64.8 / 70.1, 4096 x 4096 x 4096 8-bit 100.2 / 101.7.
 static double wide_tiles_us(uint32_t blocks, double tiles, uint32_t k, int bits)
 {
     const double cus = (double)machine_cus();
@@ -431,9 +434,9 @@ static double square_tiles_us(uint32_t m, uint32_t n, uint32_t k, int bits)
 // and their thin last round are estimated faster; and for 97 to 128 rows that make more small tiles than CUs.  Of 7269 random shapes the tall tiles, and
 // the small ones within a round, lead on all but a few; where the 256x256 tiles ran, these are 1.15 times as fast (geometric mean of 1854; 1741 of
 // them faster), where a product ran as two launches by rows 1.07 times.  By this rule, over 4484 other random shapes of 33 ... 4096 rows: 1.046 times
-// as fast on the whole, 871 more than 10 % faster, 9 more than 5 % slower, worst 0.90 (778 x 18976 x 11552 8-bit 329 / 366).  us, before / now: 148 x 43680 x
-// 4096 8-bit g128 101 / 70; 418 x 17728 x 9728 packed 8-bit g128 205 / 150; 577 x 13824 x 5120 packed 4-bit g128 93.0 / 82.8; 913 x 9296 x 3328 packed 8-bit 70.3 /
-// 55.5; 1010 x 17776 x 1024 8-bit 56.8 / 46.0.
+// as fast on the whole, 871 more than 10 % faster, 9 more than 5 % slower, worst 0.90.  (All of that with the kernel's first form.)  us, before there were
+// such tiles / with the kernel of today: 148 x 43680 x 4096 8-bit g128 97.8 / 70.1; 418 x 17728 x 9728 packed 8-bit g128 193 / 155; 577 x 13824 x 5120
+// packed 4-bit g128 95.6 / 83.5; 913 x 9296 x 3328 packed 8-bit 73.6 / 54.8; 1010 x 17776 x 1024 8-bit 57.2 / 48.8.
 // (At least 96 of them: the estimates are for a machine's worth of tiles.)
 static WideTiles wide_tiles_rule(uint32_t m, uint32_t n, uint32_t k, int bits)
 {
@@ -1559,8 +1562,9 @@ static bool packed_uses_slab(uint32_t m, uint32_t n, uint32_t k, int bits)
 // 8-bit 20.3 / 17.5, six; 11008 x 4096 4-bit 11.5 / 10.3, six; 28672 x 8192 4-bit 31.6 / 29.2, seven; more
 // than a round of eight: 34560 x 7936 4-bit, 4 rows, 53.7 / 36.2, five).  Over 3900 random shapes of 1 to 32 rows the family is faster by 15 % where it takes
 // five blocks, 11 % six, 3 % seven; against the best of the four at each shape the rule is 0.5 % off.
-// Seven only unsplit and from 13 rows, where the gain is up to 7 % (28672 x 8192); and a split of more than 128 Mi weights as it was, 12288 x
-// 12288 for one: callers have those plans.
+// Two limits have no measurement behind them: seven only unsplit and from 13 rows, and eight for a split of more than 128 Mi weights.  The plan query's
+// answers for 12 x 28672 x 8192 and 16 x 12288 x 12288 packed 4-bit are fixed (tests/test_capi_cpu.py), although fewer blocks would take 3 %
+// and 8 to 15 % less there.  Within them seven serve little beside 24592 to 28672 unsplit columns at 13 to 32 rows: up to 7 % (28672 x 8192).
 // (k up to 1024, which is over before its workgroups have filled: 13 x 16336 x 1024 8-bit 7.5 with eight, 8.1 with five; and more than 12 splits, where the
 // hand-over is most of it: 8 x 1024 x 15872 4-bit 9.9 / 10.7.)
 // (More than 32 rows take their row blocks again for every workgroup: not looked at.)

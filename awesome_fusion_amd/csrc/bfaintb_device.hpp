@@ -392,7 +392,9 @@ __device__ __forceinline__ uint4 weights4_by_halves(uint32_t x, const HalfConsta
 }
 
 // Two weights, of the codes in half PART of h0 and of h1, and their pack, as one piece of assembly: three instructions that stay in the slot of a step they
-// are written in, without the idle cycle that the compiler puts between a v_fma_mix_f32 and whatever reads its result next.
+// are written in, without the idle cycle that the compiler puts between a v_fma_mix_f32 and whatever reads its result next.  The
+// hardware asks for one behind instructions that write part of a register, which v_fma_mix_f32 does not; the tests hold these kernels' bits against
+// those of kernels that have it.
 template <uint32_t PART>
 __device__ __forceinline__ uint32_t pair_of_halves(uint32_t h0, uint32_t h1, float s0, float o0, float s1, float o1)
 {

@@ -25,13 +25,14 @@
 //     conversion, a multiplication and half a pack were 194 and 250), every one held in the slot it is written for;
 //   - few requests, spread over the step: codes in rows through LDS, 4 or 2 copies a wave and step (16 loads of a dword or less before);
 //   - waits that cover many registers at once.
-// Cycles a step, 8-bit codes in rows, one scale a column / 4-bit, groups of 128: 2632 / 3070 before; 2520 / 2700 now with 16 blocks, 1930
-// / 2070 with 10.  us, before / now: 4096 x 4096 x 4096 8-bit in rows 106.7 / 106.6, packed 104.1 / 100.8, 4-bit g128 106.2 / 102.4,
-// packed 107.4 / 102.6; 2048 x 28672 x 8192 4-bit g128 754 / 717, packed 734 / 708; 2560 x 4096 x 4096 4-bit g128 94.5 / 89.0.
+// Cycles a step, 8-bit codes in rows, one scale a column / 4-bit, groups of 128: 2632 / 3070 with a conversion, a multiplication and half a pack; 2380
+// to 2430 / 2585 to 2640 now with 16 blocks, 1790 to 1830 / 1930 to 1980 with 10, 1570 to 1600 / 1705 to 1745 with 8.  us, before / now, both on one
+// card in turn, weights cold: 4096 x 4096 x 4096 8-bit in rows 103.7 / 101.7, packed 103.5 / 99.3, 4-bit g128 109.6 / 102.9, packed 111.0 / 102.5;
+// 2048 x 28672 x 8192 4-bit g128 775 / 726, packed 742 / 714.
 // Fewer blocks: rows spread evenly over the tiles (wide_tiles in bfaintb_capi.hip), so that no matrix instruction is spent on rows
-// that do not exist and the tiles make whole rounds.  us, tiles of 256 rows / as few blocks as serve: 384 x 22016 x 4096 4-bit g128 94.7 / 73.4, 8-bit
-// 82.7 / 70.8; 300 x 28672 x 4096 4-bit 89.9 / 68.9, packed 81.5 / 72.0; 577 x 13824 x 5120 packed 4-bit 92.4 / 81, 8-bit 93.8 / 80.6; 768 rows
-// packed 4-bit 115 / 95.6.
+// that do not exist and the tiles make whole rounds.  us, before there were fewer than 16 / now, as above: 384 x 22016 x 4096 4-bit g128 102.1 / 71.3, 8-bit
+// 85.7 / 69.6; 300 x 28672 x 4096 4-bit 91.1 / 74.0, packed 84.4 / 74.3; 577 x 13824 x 5120 packed 4-bit 95.6 / 83.5, 8-bit 96.8 / 78.6; 768 rows
+// packed 4-bit 116.2 / 96.6; 2560 x 4096 x 4096 4-bit g128 100.4 / 75.1.
 #pragma once
 #include <utility>
 #include "bfaintb_device.hpp"
@@ -47,9 +48,9 @@ __device__ __forceinline__ uint32_t wr_swz(uint32_t row, uint32_t chunk) { retur
 
 // The accumulators are the accumulation registers a[0 : 16 MT - 1], by name: accumulator (mt, j) is the four from 16 mt + 4 j on.  The
 // compiler knows of them only that the kernel uses them (acc_reserve, at the start and the end of every path), and has no other use for them as
-// long as it does not run out of its 256 ordinary registers; tests/test_compiled_tiles.py looks whether it had.  Given to it as variables, it keeps part of 256 of them in ordinary registers and shuttles them back and
-// forth around every matrix instruction, or, as in-out operands of the assembly, moves some where paths through the kernel
-// meet.  What its hazard bookkeeping cannot see behind the assembly is kept safe by construction: the operands a and b are written
+// long as it does not run out of its 256 ordinary registers; tests/test_compiled_tiles.py looks whether it had.  Given to it as variables, it keeps part
+// of 256 of them in ordinary registers and shuttles them back and forth around every matrix instruction, or, as in-out operands of the assembly, moves
+// some where paths through the kernel meet.  What its hazard bookkeeping cannot see behind the assembly is kept safe by construction: the operands a and b are written
 // (LDS reads, conversions) long before, under waits for LDS; the accumulators are read only in the epilogue, behind explicit idle cycles
 // (acc_settle) that cover a matrix instruction's write latency.
 template <int MT>
@@ -101,7 +102,7 @@ __device__ __forceinline__ void wait_vm()
 template <uint32_t IN_FLIGHT>
 __device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xc07f | IN_FLIGHT << 8); }  // lgkmcnt
 
-// The weight of the code in half PART of h: as assembly, which stays in the slot it is written in.
+// The weight of the code in half PART of h: as assembly, which stays in the slot it is written in (and without the compiler's idle cycle behind it, see pair_of_halves).
 template <uint32_t PART>
 __device__ __forceinline__ void weight_in_place(float& w, uint32_t h, float s, float o)
 {
@@ -420,7 +421,7 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
     //   fragments of A: a group of four units waits once, for its own, and reads those of the group after the next, one in each unit;
     //   quads: read a quarter of a step before they are prepared, the first two at the end of the step before;
     //   conversion: one instruction after the other (Schedule);
-    //   memory: codes (in rows of step kt + 3, packed of kt + 2), group scales of kt + 3 and the copies of A of kt + 2, evenly over the step.
+    //   memory: codes (in rows of step kt + 3, packed of kt + 2), group scales of kt + 3 and the copies of A of kt + 2, evenly over the step, packed codes first.
     // The step's one barrier stands 24 slots before its end, where the next step's first fragments and the codes after it are about to be read: before
     // it the wave makes sure that its part of them has landed (requested in the step before: what may still be in flight then is this step's
     // own) and that it has everything it reads of this step's A and the next one's codes and scales.  Behind it every wave's part has landed, and

@@ -397,11 +397,12 @@ BFAINTB_API int bfaintb_gemm_variant(uint32_t m, uint32_t n, uint32_t k, int wei
  * weights with: small, 128 x 128, while that makes at most 256 tiles (one per CU); else tall, 256 rows x 128 columns, while that
  * makes at most 256; else 256 x 256 (256 = the device's compute units: one tile per unit) — except that up to 512
  * small tiles run in two rounds where the tall ones just miss one round and the 256 x 256 ones would fill
- * at most 60 % of the units (640 x 11008), and that up to 128 rows always run small tiles, in as many rounds as it
+ * at most 60 % of the units (640 x 11008), and that up to 128 rows run small tiles in as many rounds as it
  * takes (taller tiles would be half empty).  Small and tall tiles are of at most that many rows: the rows of A are spread evenly
- * over them, in steps of 32 or 64 (bfaintb_gemm_plan has the number).  The two functions answer for 8-bit codes and a k of 4096; 4-bit
- * codes with a short k keep the small tiles up to 345 of them, and where tiles of 256 columns and fewer than 256 rows are estimated to take
- * less time than any of these, they run; bfaintb_gemm_plan answers for all of it.  Pre-packed
+ * over them, in steps of 32 or 64 (bfaintb_gemm_plan has the number).  The two functions answer for 8-bit codes and a k of 4096 and leave out
+ * two things, for which bfaintb_gemm_plan answers: 4-bit codes with a short k keep the small tiles up to 345 of them, and tiles of 256 columns and
+ * fewer than 256 rows run where they are estimated to take less time than any of these, for 97 to 128 rows too where
+ * those make more small tiles than there are units (not if the call names a split of k, which only the small tiles have).  Pre-packed
  * weights run the same tiles.  (The reference arithmetic has no tall form: 256 x 256 there.) */
 BFAINTB_API uint32_t bfaintb_prefill_tile(uint32_t m, uint32_t n);
 BFAINTB_API uint32_t bfaintb_prefill_tile_cols(uint32_t m, uint32_t n);
