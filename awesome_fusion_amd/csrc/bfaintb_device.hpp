@@ -94,6 +94,7 @@ struct GemmParams {
     uint32_t group_div_magic, group_div_shift1, group_div_shift2;
     // prefill variant: the logical 256x256 tiles one launch covers
     uint32_t tile_first, tile_count;
+    uint32_t tile_halves;  // non-zero: as two workgroups each, of 128 x 256 (tile_blocks 8)
     uint32_t cus;        // compute units the launch plan is made for (host side only)
     // split-K (decode variant only)
     uint32_t k_per_wg;   // rows of k one workgroup covers (multiple of 32 * decode_blocks_per_step * decode_waves)

@@ -612,7 +612,6 @@ __global__ void __launch_bounds__(512) bfaintb_prefill_kernel(const GemmParams p
 
 bool prefill_wreg_serves(const GemmParams& p);
 hipError_t launch_prefill_wreg(const GemmParams& p, int bits, bool packed, hipStream_t stream);
-hipError_t launch_prefill256x128_wreg(const GemmParams& p, int bits, bool packed, hipStream_t stream);
 
 template <int BITS, bool GROUPED, bool PACKED, bool REF = false>
 static hipError_t launch_prefill_t(const GemmParams& p0, hipStream_t stream, bool wreg = false)
@@ -646,10 +645,11 @@ static hipError_t launch_prefill_t(const GemmParams& p0, hipStream_t stream, boo
     if (halves) {
         p.tile_first = whole;
         p.tile_count = halves;
-        // ... as left and right halves on the kernel of 256x128 tiles that keeps the weights in registers, where that serves
+        // ... as upper and lower halves on that kernel's form of 128 rows, where it serves
         if (wreg && !REF && prefill_wreg_serves(p)) {
-            p.splits = 1;
-            return launch_prefill256x128_wreg(p, BITS, PACKED, stream);
+            p.tile_blocks = 8u;
+            p.tile_halves = 1u;
+            return launch_prefill_wreg(p, BITS, PACKED, stream);
         }
         const uint32_t grid = (2u * halves + 7u) / 8u * 8u;
         void (*half_tiles)(const GemmParams) = bfaintb_prefill_kernel<BITS, GROUPED, 2, PACKED, REF>;

@@ -33,6 +33,9 @@
 // that do not exist and the tiles make whole rounds.  us, before there were fewer than 16 / now, as above: 384 x 22016 x 4096 4-bit g128 102.1 / 71.3, 8-bit
 // 85.7 / 69.6; 300 x 28672 x 4096 4-bit 91.1 / 74.0, packed 84.4 / 74.3; 577 x 13824 x 5120 packed 4-bit 95.6 / 83.5, 8-bit 96.8 / 78.6; 768 rows
 // packed 4-bit 116.2 / 96.6; 2560 x 4096 x 4096 4-bit g128 100.4 / 75.1.
+// The thin last round of the 256x256 tiles runs as halves of 128 x 256, eight blocks, and not of 256 x 128 (bfaintb_prefill256x128_wreg_kernel): the same
+// conversions and fragment reads for the same matrix instructions, but 24 KiB copied a step instead of 36 and no weight converted twice.  us, 256 x 128 / 128 x
+// 256: 2048 x 28672 x 8192 4-bit g128 730 / 711, packed 719 / 712, 8-bit 713 / 699; 2727 x 31312 x 2816 packed 4-bit 406 / 402.
 #pragma once
 #include <utility>
 #include "bfaintb_device.hpp"
@@ -179,19 +182,23 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
 
     // ---- tile of this workgroup: ids that share an XCD (id mod 8) cover consecutive logical ids, which walk groups of
     //      4 tile-rows column by column (as in bfaintb_prefill_kernel)
-    const uint32_t tiles_m = (p.m + kRows - 1) / kRows, tiles_n = (p.n + kWrTile - 1) / kWrTile;
-    const uint32_t wgs = p.tile_count;
+    //      (eight blocks: or, with p.tile_halves, the upper and the lower halves of tiles of 256 rows, the thin last round of those)
+    const bool in_halves = MT == 8 && p.tile_halves != 0u;
+    const uint32_t tile_rows = in_halves ? 2u * kRows : kRows;
+    const uint32_t tiles_m = (p.m + tile_rows - 1) / tile_rows, tiles_n = (p.n + kWrTile - 1) / kWrTile;
+    const uint32_t wgs = in_halves ? 2u * p.tile_count : p.tile_count;
     const uint32_t per_xcd = (wgs + 7u) / 8u;
     const uint32_t local = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
     if (local >= wgs) return;
-    const uint32_t logical = p.tile_first + local;
+    const uint32_t logical = p.tile_first + (in_halves ? local >> 1 : local);
     const uint32_t group = logical / (4u * tiles_n);
     const uint32_t first_m = group * 4u;
     const uint32_t group_rows = tiles_m - first_m < 4u ? tiles_m - first_m : 4u;
     const uint32_t in_group = logical - group * 4u * tiles_n;
     const uint32_t tm = first_m + in_group % group_rows;
     const uint32_t tn = in_group / group_rows;
-    const uint32_t m0 = tm * kRows, n0 = tn * kWrTile;
+    const uint32_t m0 = tm * tile_rows + (in_halves ? (local & 1u) * kRows : 0u), n0 = tn * kWrTile;
+    if (in_halves && m0 >= p.m) return;  // the lower half of a last, flat tile
 
     const uint32_t rows_valid = p.m - m0 < kRows ? p.m - m0 : kRows;
     const uint32_t a_extent = ((rows_valid - 1u) * p.lda + p.k) * 2u;
@@ -741,11 +748,11 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
     acc_reserve<MT>();
 }
 
-// Runs `tile_count` tiles of 16 x tile_blocks (0: 16) rows from `tile_first` on (the caller splits off a last, thin round for the half-tile kernel).
+// Runs `tile_count` tiles of 16 x tile_blocks (0: 16) rows from `tile_first` on; with tile_halves (eight blocks), so many tiles of 256 rows as two of 128 each.
 template <int BITS, bool GROUPED, bool PACKED, int MT>
 static hipError_t launch_wreg_t(const GemmParams& p, hipStream_t stream)
 {
-    const uint32_t grid = (p.tile_count + 7u) / 8u * 8u;  // a whole number of workgroups per XCD; ids past the last tile exit at once
+    const uint32_t grid = ((p.tile_halves ? 2u : 1u) * p.tile_count + 7u) / 8u * 8u;  // a whole number of workgroups per XCD; ids past the last tile exit at once
     void (*kernel)(const GemmParams) = bfaintb_prefill_wreg_kernel<BITS, GROUPED, PACKED, MT>;
     return launch_kernel(kernel, dim3(grid, 1, 1), dim3(256, 1, 1), 0, stream, p);
 }

@@ -74,7 +74,7 @@ enum {
                                       * blocks of 32 k), so it agrees with the other tiled forms to rounding, not in
                                       * every bit; like every form it gives the same bits on every run */
     BFAINTB_VARIANT_PREFILL_256_LDS = 5, /* 256x256 tiles with both operands staged in LDS — the older form, which the
-                                          * reference's arithmetic and the half tiles of a thin last round still use;
+                                          * reference's arithmetic still uses;
                                           * otherwise the form that keeps the weights in registers runs (tests, tuning) */
     BFAINTB_VARIANT_PREFILL_128_LDS = 6, /* 128x128 tiles with both operands staged in LDS — the older form, kept for the
                                           * reference's arithmetic; otherwise the form that keeps the weights in

@@ -105,3 +105,27 @@ def test_few_rows_against_many_columns(units64, m, bits, group, k):
     # a call that names a split of k runs the small tiles, which have it
     assert af.plan(m, n, k, bits, group, which=af.PREFILL, force_split_k=2).splits == 2
     assert_close_ulp(p, run_gemm(p, which=af.PREFILL, force_split_k=2), "split")
+
+
+# whole rounds of 256x256 tiles and a thin last one as halves of 128 rows, or the thin round alone, planned for 8 units: a last row of tiles of one row, of 128,
+# of one more and of 256, columns a block past a tile; one step, a partial last one, six, seven
+@pytest.mark.parametrize("m,n", [(257, 1296), (384, 1296), (385, 1296), (512, 1536), (300, 272), (641, 784)])
+@pytest.mark.parametrize("bits,group,k", [(8, 0, 64), (8, 0, 200), (4, 128, 384), (8, 64, 448)])
+def test_the_thin_last_round(m, n, bits, group, k):
+    import awesome_fusion_amd as af
+    af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 8)
+    try:
+        pl = af.plan(m, n, k, bits, group, which=af.PREFILL_256)
+        tiles = -(-m // 256) * -(-n // 256)
+        rest = tiles % 8
+        assert 0 < rest <= 4 and (pl.workgroups, pl.tail_workgroups, pl.launches) == (tiles - rest, 2 * rest, (tiles > rest) + (rest > 0)), pl.as_dict()
+        p = Problem(m, n, k, bits, group, seed=m + k)
+        c = run_gemm(p, which=af.PREFILL_256)
+        assert_close_ulp(p, c, f"{m}x{n}x{k} bits={bits} g={group}")
+        assert np.array_equal(c, run_gemm(p, which=af.PREFILL_256_LDS))
+        wide = run_gemm(p, which=af.PREFILL_256, ldc=n + 24, c_fill=0x1234)
+        assert np.array_equal(wide[:, :n], c) and (wide[:, n:] == 0x1234).all()
+        if k % (64 if bits == 8 else 128) == 0:
+            assert np.array_equal(run_packed(af, p, af.PREFILL_256), c), "packed"
+    finally:
+        af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 0)
