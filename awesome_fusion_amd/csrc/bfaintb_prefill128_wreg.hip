@@ -331,7 +331,15 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (__attribute__((address_space(3))) void*)(a_tile(stage_c) + j * 1024u), 16, (j & 1u) ? vo : ve,
                                                          at_step(kt) * kTwK * 2u + j * 16u * p.lda, 0, 0);
         };
-        barrier_no_fence();  // (the first steps' copies are shared out over the computing waves: see the prologue)
+        // The first two steps' copies are shared out over the computing waves, which wait for them before they start; those of the steps behind
+        // them are this wave's, in flight meanwhile and counted by its own waits.  (Shared out as well and waited for at the start, a machine's
+        // whole pipeline had to land first.  us before / now: 32 x 22016 x 4096 4-bit g128 23.4 / 22.4, 32 x 28672 x 4096 packed 8-bit 24.5 / 23.1, 26 x
+        // 23392 x 3584 packed 4-bit 17.3 / 16.2, 54 x 22192 x 1152 packed 4-bit 10.0 / 9.3; four stages or many steps level.)
+        auto ahead = [&](auto stage_c) {
+            if constexpr (decltype(stage_c)::value < kDepth) copy_step(stage_c, clamp(decltype(stage_c)::value));
+        };
+        ahead(C2{}), ahead(C3{}), ahead(C4{}), ahead(C5{}), ahead(C6{});
+        barrier_no_fence();
         uint32_t kt = 0;
         auto turn_of = [&](auto stage_c) {  // step kt + stage
             constexpr uint32_t St = decltype(stage_c)::value;
@@ -554,11 +562,11 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
     };
     // (the first two steps' copies have to land before anything else happens: those of the last stages are issued behind that wait, a
     // microsecond's work of the memory path)
-    fetch(C0{}), fetch(C1{}), fetch(C2{});
+    fetch(C0{}), fetch(C1{});
     if constexpr (COPIER) {
-        fetch(C3{}), fetch(C4{}), fetch(C5{}), fetch(C6{});
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     } else {
+        fetch(C2{});
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kRequests) : "memory");
     }
     barrier_no_fence();
