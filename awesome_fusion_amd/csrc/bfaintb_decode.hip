@@ -441,6 +441,10 @@ __device__ __forceinline__ void reduce_splits_two_in_flight(const GemmParams& p,
     };
     u32x4_t a[NL], b[NL];
     fetch(a);
+    // (Bias and residual come with the sums; asked for last, they waited behind the emptying stores as well: 8 x 4096 x 4096 with a residual
+    // 8.40 us, 8.06 so, 1 row 7.75 / 7.50.)
+    Addends4 addends;
+    request_addends4(addends, p, first_row + rs, col);
     __builtin_amdgcn_s_sleep(kPollGap);
     fetch(b);
     uint32_t tries = 2;
@@ -482,7 +486,7 @@ __device__ __forceinline__ void reduce_splits_two_in_flight(const GemmParams& p,
             total.w += __uint_as_float(v[3]);
         }
     }
-    finish_row4(p, make_float4(total.x + sum[0].x, total.y + sum[0].y, total.z + sum[0].z, total.w + sum[0].w), first_row + rs, col);
+    finish_row4(p, make_float4(total.x + sum[0].x, total.y + sum[0].y, total.z + sum[0].z, total.w + sum[0].w), first_row + rs, col, addends);
     // The attempt that did not win may still be in flight.  Its destination registers stay this function's until it has
     // come back: with nothing holding them, the compiler handed them to the constants of the emptying stores above while
     // the loads were still due to write them (a workspace word of the second split left holding a partial sum: found
@@ -894,6 +898,12 @@ bfaintb_decode_kernel(const GemmParams p)
         if (nwaves == 8u) add_waves(std::integral_constant<uint32_t, 8>{});
         else add_waves(std::integral_constant<uint32_t, 4>{});
         const uint32_t first_row = row0 + pass_row0;  // global row of this pass's row 0
+        // (Column and row are hidden from the compiler where bias and residual are asked for early: it made their addresses above these
+        // branches, in the way of the producers' stores.)
+        auto here = [](uint32_t v) {
+            asm volatile("" : "+v"(v));
+            return v;
+        };
         if (p.splits == 1) {
 #pragma unroll
             for (uint32_t i = 0; i < kMaxR; ++i) {
@@ -925,13 +935,14 @@ bfaintb_decode_kernel(const GemmParams p)
             // flag, no read-modify-write; only this workgroup ever waits, and only on workgroups that wait for
             // nothing, so the wait ends whatever order they run in.  It is bounded all the same: a word that
             // never arrives leaves a NaN in the output instead of hanging the kernel.
+            const uint32_t out_col = here(col), out_rs = here(rs);
             // Rows a thread has in this pass: a power of two up to kMaxR; the fewer, the more splits are fetched at once.
             const uint32_t rows_per_thread = (rows_out + nrs - 1u) / nrs;
             constexpr bool kTwoAttempts = CPL <= 8;  // (see reduce_splits_two_in_flight)
-            if (kTwoAttempts && rows_per_thread <= 1u && p.splits <= 2u) reduce_splits_two_in_flight<1>(p, sum, first_row, rows_out, rs, col, col_ok);
-            else if (kTwoAttempts && rows_per_thread <= 1u && p.splits <= 3u) reduce_splits_two_in_flight<2>(p, sum, first_row, rows_out, rs, col, col_ok);
-            else if (kTwoAttempts && rows_per_thread <= 1u && p.splits <= 5u) reduce_splits_two_in_flight<4>(p, sum, first_row, rows_out, rs, col, col_ok);
-            else if (kTwoAttempts && rows_per_thread <= 1u && p.splits <= 8u) reduce_splits_two_in_flight<7>(p, sum, first_row, rows_out, rs, col, col_ok);
+            if (kTwoAttempts && rows_per_thread <= 1u && p.splits <= 2u) reduce_splits_two_in_flight<1>(p, sum, first_row, rows_out, out_rs, out_col, col_ok);
+            else if (kTwoAttempts && rows_per_thread <= 1u && p.splits <= 3u) reduce_splits_two_in_flight<2>(p, sum, first_row, rows_out, out_rs, out_col, col_ok);
+            else if (kTwoAttempts && rows_per_thread <= 1u && p.splits <= 5u) reduce_splits_two_in_flight<4>(p, sum, first_row, rows_out, out_rs, out_col, col_ok);
+            else if (kTwoAttempts && rows_per_thread <= 1u && p.splits <= 8u) reduce_splits_two_in_flight<7>(p, sum, first_row, rows_out, out_rs, out_col, col_ok);
             else if (rows_per_thread <= 1u) reduce_splits<1>(p, sum, first_row, rows_out, rs, nrs, col, col_ok);
             else if (rows_per_thread <= 2u) reduce_splits<(kMaxR < 2u ? kMaxR : 2u)>(p, sum, first_row, rows_out, rs, nrs, col, col_ok);
             else if (rows_per_thread <= 4u) reduce_splits<(kMaxR < 4u ? kMaxR : 4u)>(p, sum, first_row, rows_out, rs, nrs, col, col_ok);

@@ -189,13 +189,37 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi)
     else return pack_bf16_rne(lo, hi);
 }
 
+// What is added to four neighbouring columns of one row, as stored: requested before the sums are there (a barrier or a
+// hand-over ahead of their use), so that a launch does not end on one more trip to memory.
+// (Left as it is where there is nothing to add: nobody looks at it then.  Gated, the two outputs are one half of the eight bytes, which
+// end within the row: it has a multiple of eight outputs.)
+struct Addends4 {
+    uint2 bias, residual;
+};
+__device__ __forceinline__ void request_addends4(Addends4& a, const GemmParams& p, uint32_t row, uint32_t col)
+{
+    if (p.bias != nullptr) a.bias = *reinterpret_cast<const uint2*>(p.bias + col);
+    if (p.residual != nullptr) a.residual = *reinterpret_cast<const uint2*>(p.residual + (size_t)row * p.ldr + (p.activation == kActSiluGate ? col / 8u * 4u : col));
+}
+
+// The residual of eight neighbouring columns of a tile's row (gated: of the four outputs they make).
+__device__ __forceinline__ uint4 request_residual8(const GemmParams& p, uint32_t row, uint32_t col, bool gated)
+{
+    const uint16_t* at = p.residual + (size_t)row * p.ldr;
+    if (!gated) return *reinterpret_cast<const uint4*>(at + col);
+    const uint2 r = *reinterpret_cast<const uint2*>(at + col / 2u);
+    return make_uint4(r.x, r.y, 0u, 0u);
+}
+
 // Finishes four neighbouring columns of one row: t += bias[col .. col+3]; then either += residual[row][col .. col+3] and
 // four bf16 outputs at C[row][col ..], or (gated) the two outputs silu(t.x) * t.y and silu(t.z) * t.w, += residual[row]
 // [col/2 ..], at C[row][col/2 ..].  All additions in fp32, one rounding (a truncation with the reference's arithmetic).
-__device__ __forceinline__ void finish_row4(const GemmParams& p, float4 t, uint32_t row, uint32_t col)
+// a: what request_addends4 has brought, or not ASKED for and loaded here.
+template <bool ASKED = true>
+__device__ __forceinline__ void finish_row4(const GemmParams& p, float4 t, uint32_t row, uint32_t col, const Addends4& a)
 {
     if (p.bias != nullptr) {
-        const uint2 raw = *reinterpret_cast<const uint2*>(p.bias + col);
+        const uint2 raw = ASKED ? a.bias : *reinterpret_cast<const uint2*>(p.bias + col);
         t.x += bf16_bits_to_f32(raw.x & 0xffffu);
         t.y += bf16_bits_to_f32(raw.x >> 16);
         t.z += bf16_bits_to_f32(raw.y & 0xffffu);
@@ -204,7 +228,7 @@ __device__ __forceinline__ void finish_row4(const GemmParams& p, float4 t, uint3
     if (p.activation == kActSiluGate) {
         float o0 = silu_gate(t.x, t.y), o1 = silu_gate(t.z, t.w);
         if (p.residual != nullptr) {
-            const uint32_t raw = *reinterpret_cast<const uint32_t*>(p.residual + (size_t)row * p.ldr + col / 2u);
+            const uint32_t raw = ASKED ? ((col & 4u) ? a.residual.y : a.residual.x) : *reinterpret_cast<const uint32_t*>(p.residual + (size_t)row * p.ldr + col / 2u);
             o0 += bf16_bits_to_f32(raw & 0xffffu);
             o1 += bf16_bits_to_f32(raw >> 16);
         }
@@ -212,7 +236,7 @@ __device__ __forceinline__ void finish_row4(const GemmParams& p, float4 t, uint3
         return;
     }
     if (p.residual != nullptr) {
-        const uint2 raw = *reinterpret_cast<const uint2*>(p.residual + (size_t)row * p.ldr + col);
+        const uint2 raw = ASKED ? a.residual : *reinterpret_cast<const uint2*>(p.residual + (size_t)row * p.ldr + col);
         t.x += bf16_bits_to_f32(raw.x & 0xffffu);
         t.y += bf16_bits_to_f32(raw.x >> 16);
         t.z += bf16_bits_to_f32(raw.y & 0xffffu);
@@ -222,6 +246,11 @@ __device__ __forceinline__ void finish_row4(const GemmParams& p, float4 t, uint3
     o.x = p.reference_arith ? pack_bf16_rtz(t.x, t.y) : pack_bf16_rne(t.x, t.y);
     o.y = p.reference_arith ? pack_bf16_rtz(t.z, t.w) : pack_bf16_rne(t.z, t.w);
     *reinterpret_cast<uint2*>(p.c + (size_t)row * p.ldc + col) = o;
+}
+
+__device__ __forceinline__ void finish_row4(const GemmParams& p, float4 t, uint32_t row, uint32_t col)
+{
+    finish_row4<false>(p, t, row, col, Addends4{});
 }
 
 // Signed byte `I` of a dword as fp32: one v_cvt_f32_i32 with an SDWA sign-extending byte select.

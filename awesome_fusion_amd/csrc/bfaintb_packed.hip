@@ -381,39 +381,31 @@ __device__ __forceinline__ void decode_packed_body(const GemmParams& p)
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
         *reinterpret_cast<float4*>(&red[wave][mb][nl][4u * kg]) = make_float4(acc[mb][0], acc[mb][1], acc[mb][2], acc[mb][3]);
+    // A thread finishes at most one output: row block, A row and W column 16 nb + i; gated, where columns (2 ip, 2 ip + 1) are (gate, up) of
+    // output column 8 nb + ip, i = 2 ip.  What is added to it is on its way while the waves meet.
+    static_assert(256 * MB <= 64 * kPackedWaves, "an output per thread");
+    const bool gated = p.activation == kActSiluGate;
+    const uint32_t mb = gated ? tid >> 7 : tid >> 8, j = (gated ? tid >> 3 : tid >> 4) & 15u, i = gated ? 2u * (tid & 7u) : tid & 15u;
+    const uint32_t row = 16u * (MB * rb + mb) + j, c = gated ? 8u * nb + i / 2u : 16u * nb + i;
+    const bool mine = mb < (uint32_t)MB && row < p.m;
+    uint32_t bias[2] = {0u, 0u}, residual = 0u;
+    if (mine) {
+        if (p.bias != nullptr) bias[0] = p.bias[16u * nb + i], bias[1] = p.bias[16u * nb + (i | 1u)];
+        if (p.residual != nullptr) residual = p.residual[(size_t)row * p.ldr + c];
+    }
     __syncthreads();
-    auto wave_sum = [&](uint32_t mb, uint32_t j, uint32_t i) {
-        float sum = red[0][mb][j][i];
+    if (!mine) return;
+    auto wave_sum = [&](uint32_t at, uint32_t bias_bits) {
+        float sum = red[0][mb][j][at];
 #pragma unroll
-        for (int w = 1; w < kPackedWaves; ++w) sum += red[w][mb][j][i];
-        const uint32_t c = 16u * nb + i;
-        if (p.bias != nullptr) sum += bf16_bits_to_f32(p.bias[c]);
+        for (int w = 1; w < kPackedWaves; ++w) sum += red[w][mb][j][at];
+        if (p.bias != nullptr) sum += bf16_bits_to_f32(bias_bits);
         return sum;
     };
-    if (p.activation == kActSiluGate) {
-        // columns (2 ip, 2 ip + 1) of the block are (gate, up) of output column 8 nb + ip
-        for (uint32_t t = tid; t < 128u * MB; t += 64u * kPackedWaves) {
-            const uint32_t mb = t >> 7, j = (t >> 3) & 15u, ip = t & 7u;
-            const uint32_t row = 16u * (MB * rb + mb) + j;
-            if (row < p.m) {
-                float out = silu_gate(wave_sum(mb, j, 2u * ip), wave_sum(mb, j, 2u * ip + 1u));
-                const uint32_t c = 8u * nb + ip;
-                if (p.residual != nullptr) out += bf16_bits_to_f32(p.residual[(size_t)row * p.ldr + c]);
-                p.c[(size_t)row * p.ldc + c] = (uint16_t)(pack_bf16_rne(out, 0.f) & 0xffffu);
-            }
-        }
-        return;
-    }
-    for (uint32_t t = tid; t < 256u * MB; t += 64u * kPackedWaves) {
-        const uint32_t mb = t >> 8, j = (t >> 4) & 15u, i = t & 15u;  // row block, A row, W column
-        const uint32_t row = 16u * (MB * rb + mb) + j;
-        if (row < p.m) {
-            float sum = wave_sum(mb, j, i);
-            const uint32_t c = 16u * nb + i;
-            if (p.residual != nullptr) sum += bf16_bits_to_f32(p.residual[(size_t)row * p.ldr + c]);
-            p.c[(size_t)row * p.ldc + c] = (uint16_t)(pack_bf16_rne(sum, 0.f) & 0xffffu);
-        }
-    }
+    float out = wave_sum(i, bias[0]);
+    if (gated) out = silu_gate(out, wave_sum(i + 1u, bias[1]));
+    if (p.residual != nullptr) out += bf16_bits_to_f32(residual);
+    p.c[(size_t)row * p.ldc + c] = (uint16_t)(pack_bf16_rne(out, 0.f) & 0xffffu);
 }
 
 // (no more than four waves per SIMD asked for: told that eight are possible, the compiler delays loads to save registers)

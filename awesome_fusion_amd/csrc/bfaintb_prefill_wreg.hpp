@@ -696,7 +696,24 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
             bias8[2 * i + 1] = bf16_bits_to_f32(d[i] >> 16);
         }
     }
+    // The residual's rows of a part are requested together, a part ahead of their use: row by row, each behind the store of the row before,
+    // their trips to memory stood one behind the other with nothing else on the CU.  What bounds the part behind the loop is the residual's and
+    // the outputs' bytes (us, with the sums' rows turned in LDS as well: 4096 x 4096 x 4096 8-bit 109.9 -> 104.9, 577 x 13824 x 5120 packed 4-bit
+    // 87.9 -> 84.8; the same calls without a residual 101.5 and 82).
     constexpr uint32_t kBlocksHeld = 6u * MT / 16u, kParts = (MT + kBlocksHeld - 1u) / kBlocksHeld;
+    uint4 residual[2][2u * kBlocksHeld];
+    auto request_part = [&](auto part_c) {
+        constexpr uint32_t first = decltype(part_c)::value * kBlocksHeld, blocks = MT - first < kBlocksHeld ? MT - first : kBlocksHeld;
+        if (p.residual == nullptr) return;
+#pragma unroll
+        for (uint32_t pass = 0; pass < 2u * blocks; ++pass) {
+            const uint32_t gm = m0 + 16u * first + pass * 8u + (tid >> 5);
+            uint4& r = residual[decltype(part_c)::value & 1u][pass];
+            r = make_uint4(0u, 0u, 0u, 0u);
+            if (gm < p.m && gn < p.n) r = request_residual8(p, gm, gn, gated);
+        }
+    };
+    request_part(std::integral_constant<uint32_t, 0u>{});
     for_each_const<kParts>([&](auto part_c) {
         constexpr uint32_t first = decltype(part_c)::value * kBlocksHeld, blocks = MT - first < kBlocksHeld ? MT - first : kBlocksHeld;
         for_each_const<blocks>([&](auto mh_c) {
@@ -706,15 +723,17 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
 #pragma unroll
             for (uint32_t r = 0; r < 4; ++r)
 #pragma unroll
-                for (uint32_t j = 0; j < 4; ++j) base[r * kWrTile + wcol + 16u * j] = acc[j][r];
+                for (uint32_t j = 0; j < 4; ++j) base[r * kWrTile + ((wcol + 16u * j) ^ (kq << 4))] = acc[j][r];  // (turned by the row: the four kq write rows 4 apart)
         });
+        if constexpr (decltype(part_c)::value + 1u < kParts) request_part(std::integral_constant<uint32_t, decltype(part_c)::value + 1u>{});
         __syncthreads();
-#pragma unroll 4
+#pragma unroll
         for (uint32_t pass = 0; pass < 2u * blocks; ++pass) {
+            const uint4 r = residual[decltype(part_c)::value & 1u][pass];
             const uint32_t row = pass * 8u + (tid >> 5);  // within the part
             const uint32_t gm = m0 + 16u * first + row;
             if (gm >= p.m || gn >= p.n) continue;
-            const float* src = reinterpret_cast<const float*>(c_rows4(row >> 2, MT / 2u, kWrTile * 4u)) + (row & 3u) * kWrTile + 8u * ch;
+            const float* src = reinterpret_cast<const float*>(c_rows4(row >> 2, MT / 2u, kWrTile * 4u)) + (row & 3u) * kWrTile + ((8u * ch) ^ (((row >> 2) & 3u) << 4));
             const float4 lo = *reinterpret_cast<const float4*>(src), hi = *reinterpret_cast<const float4*>(src + 4);
             float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
 #pragma unroll
@@ -724,7 +743,6 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
 #pragma unroll
                 for (int i = 0; i < 4; ++i) o[i] = silu_gate(v[2 * i], v[2 * i + 1]);
                 if (p.residual != nullptr) {
-                    const uint2 r = *reinterpret_cast<const uint2*>(p.residual + (size_t)gm * p.ldr + gn / 2u);
                     o[0] += bf16_bits_to_f32(r.x & 0xffffu);
                     o[1] += bf16_bits_to_f32(r.x >> 16);
                     o[2] += bf16_bits_to_f32(r.y & 0xffffu);
@@ -732,7 +750,6 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
                 }
                 *reinterpret_cast<uint2*>(p.c + (size_t)gm * p.ldc + gn / 2u) = make_uint2(pack_bf16_rne(o[0], o[1]), pack_bf16_rne(o[2], o[3]));
             } else {
-                const uint4 r = *reinterpret_cast<const uint4*>(p.residual + (size_t)gm * p.ldr + gn);
                 const uint32_t d[4] = {r.x, r.y, r.z, r.w};
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
