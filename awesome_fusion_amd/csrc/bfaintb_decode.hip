@@ -504,8 +504,13 @@ template <int BITS, int CPL, int MB, bool GROUPED, bool PACKED, bool REF>
 // (packed 4-bit codes always run 4 waves: with 8 — their registers would allow it for one block of 16 rows — the 256-column
 // kernel over packed weights is slower, 28672 x 8192, m = 16: 55 against 42 us)
 __global__ void __launch_bounds__((MB <= 2 && (CPL <= 8 || MB == 1) && !(PACKED && BITS == 4 && CPL == 16)) ? 512 : 256)
-bfaintb_decode_kernel(const GemmParams p)
+bfaintb_decode_kernel(const uint8_t* b, const uint16_t* a, const uint16_t* scale, const uint32_t m, const uint32_t n, const uint32_t k, const uint32_t lda,
+                      const uint32_t ldb_bytes, const uint32_t k_per_wg, const uint32_t nwaves, const GemmParams rest)
 {
+    // What the first loads need comes in scalar registers with the launch (the Makefile asks for it): a workgroup of a launch whose arguments are
+    // new waits 0.2 to 0.4 us for the rest of them, which is read from memory.
+    GemmParams p = rest;
+    p.b = b, p.a = a, p.scale = scale, p.m = m, p.n = n, p.k = k, p.lda = lda, p.ldb_bytes = ldb_bytes, p.k_per_wg = k_per_wg;
     static_assert(CPL == 16 || CPL == 8 || (PACKED && CPL >= 5 && CPL < 8 && MB <= 2), "the forms there are");
     static_assert(!REF || (BITS == 8 && !GROUPED && !PACKED), "the reference's arithmetic: 8-bit codes, row-major, one scale per column");
     constexpr int KB = decode_blocks_per_step(BITS, CPL, PACKED, MB);  // blocks of 32 rows per pipeline step
@@ -542,8 +547,7 @@ bfaintb_decode_kernel(const GemmParams p)
     if (n_ld >= p.n) n_ld = p.n - CPL;
 
     // ---- this wave's rows of k
-    const uint32_t nwaves = blockDim.x >> 6;  // 4 or 8
-    const uint32_t k_per_wave = p.k_per_wg / nwaves;
+    const uint32_t k_per_wave = p.k_per_wg >> (nwaves == 8u ? 3 : 2);  // (4 or 8 waves)
     const uint32_t kb = ks * p.k_per_wg + (uint32_t)wave * k_per_wave;
     uint32_t ke = kb + k_per_wave;
     if (ke > p.k) ke = p.k;
@@ -688,14 +692,14 @@ bfaintb_decode_kernel(const GemmParams p)
         uint32_t steps_to_wrap = 0u;
         if constexpr (GROUPED) {
             const uint32_t kb_uniform = __builtin_amdgcn_readfirstlane(kb) + 32u * (uint32_t)KB * (uint32_t)first_step;
-            next_group_blocks = (p.group_size - kb_uniform % p.group_size) / 32u;
+            next_group_blocks = ((group_of_row(p, kb_uniform) + 1u) * p.group_size - kb_uniform) / 32u;
             steps_to_wrap = (uint32_t)(nsteps - first_step);
         }
         auto compute_stage = [&](Stage& st) {
             if constexpr (GROUPED && kRotateSteps) {
                 if (steps_to_wrap == 0u) {
                     blocks_to_group = 0u;
-                    next_group_blocks = (p.group_size - __builtin_amdgcn_readfirstlane(kb) % p.group_size) / 32u;
+                    next_group_blocks = ((group_of_row(p, __builtin_amdgcn_readfirstlane(kb)) + 1u) * p.group_size - __builtin_amdgcn_readfirstlane(kb)) / 32u;
                 }
                 --steps_to_wrap;
             }
@@ -838,7 +842,7 @@ bfaintb_decode_kernel(const GemmParams p)
     // rows per thread and pass with 4 waves (half that with 8), up to a power of two
     constexpr uint32_t kRowsAtOnce = 256u / kQuads, kMaxR = (uint32_t)next_power_of_two((16u * kMBC + kRowsAtOnce - 1u) / kRowsAtOnce);
     // thread t: 4 consecutive columns (cg = t % (kCols/4)) of rows t / (kCols/4), + threads/(kCols/4), ...
-    const uint32_t cg = threadIdx.x % kQuads, nrs = blockDim.x / kQuads;
+    const uint32_t cg = threadIdx.x % kQuads, nrs = 64u * nwaves / kQuads;
     uint32_t rs = threadIdx.x / kQuads;
     if (kQuads * kRowsAtOnce != 256u && rs >= nrs) rs = 1u << 16;  // (fewer threads than a further row has: none of the pass's rows)
     const uint32_t col = cb * kCols + 4u * cg;
@@ -969,8 +973,8 @@ static hipError_t launch_decode_t(const GemmParams& p, hipStream_t stream)
         lds += (size_t)waves * 16u * decode_table_stride(CPL) * 2u;
     }
     if (lds > 160 * 1024 - 64) return hipErrorInvalidValue;
-    void (*kernel)(const GemmParams) = bfaintb_decode_kernel<BITS, CPL, MB, GROUPED, PACKED, REF>;
-    return launch_kernel(kernel, grid, dim3(64 * waves, 1, 1), lds, stream, q);
+    auto kernel = bfaintb_decode_kernel<BITS, CPL, MB, GROUPED, PACKED, REF>;
+    return launch_kernel(kernel, grid, dim3(64 * waves, 1, 1), lds, stream, q.b, q.a, q.scale, q.m, q.n, q.k, q.lda, q.ldb_bytes, q.k_per_wg, waves, q);
 }
 
 template <int BITS, int CPL, bool PACKED>
