@@ -881,8 +881,11 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
 // ids, which walk groups of 8 tile-rows column by column).
 template <int BITS, bool GROUPED, bool PACKED, int MT, int NS, bool COPIER>
 __global__ void __launch_bounds__(COPIER ? 576 : 512) __attribute__((amdgpu_waves_per_eu(COPIER ? 3 : 2, COPIER ? 3 : 2)))
-bfaintb_prefill128_wreg_kernel(const GemmParams p)
+bfaintb_prefill128_wreg_kernel(const uint8_t* b, const uint16_t* a, const uint16_t* scale, const uint32_t m, const uint32_t n, const uint32_t k, const uint32_t lda,
+                               const uint32_t ldb_bytes, const uint32_t k_per_wg, const uint32_t splits, const uint32_t finish_launch, const GemmParams rest)
 {
+    GemmParams p = rest;  // (what the first copies need comes in scalar registers with the launch: see bfaintb_decode_kernel)
+    p.b = b, p.a = a, p.scale = scale, p.m = m, p.n = n, p.k = k, p.lda = lda, p.ldb_bytes = ldb_bytes, p.k_per_wg = k_per_wg, p.splits = splits, p.finish_launch = finish_launch;
     constexpr bool kScales = GROUPED && MT <= 12;  // (a larger tile leaves no room in LDS)
     const uint32_t tiles_m = (p.m + 16u * MT - 1u) / (16u * MT), tiles_n = (p.n + kTw - 1u) / kTw;
     const uint32_t wgs = tiles_m * tiles_n;
@@ -898,12 +901,15 @@ bfaintb_prefill128_wreg_kernel(const GemmParams p)
         ks = logical / wgs;
         logical -= ks * wgs;
     }
-    const uint32_t group = logical / (8u * tiles_n);
-    const uint32_t first_m = group * 8u;
-    const uint32_t group_rows = tiles_m - first_m < 8u ? tiles_m - first_m : 8u;
-    const uint32_t in_group = logical - group * 8u * tiles_n;
-    const uint32_t tm = first_m + in_group % group_rows;
-    const uint32_t tn = in_group / group_rows;
+    uint32_t tm = 0u, tn = logical;
+    if (tiles_m > 1u) {  // (one row of tiles: no divisions ahead of the first copies)
+        const uint32_t group = logical / (8u * tiles_n);
+        const uint32_t first_m = group * 8u;
+        const uint32_t group_rows = tiles_m - first_m < 8u ? tiles_m - first_m : 8u;
+        const uint32_t in_group = logical - group * 8u * tiles_n;
+        tm = first_m + in_group % group_rows;
+        tn = in_group / group_rows;
+    }
     tw_tile<BITS, GROUPED, PACKED, kScales, MT, NS, COPIER>(p, tm * 16u * MT, tn * kTw, ks);
 }
 
@@ -955,8 +961,9 @@ static hipError_t launch_prefill128_wreg_t(const GemmParams& p, hipStream_t stre
     const uint32_t tiles = ((p.m + 16u * MT - 1u) / (16u * MT)) * ((p.n + kTw - 1u) / kTw);
     // a whole number of workgroups per XCD; ids past the last tile exit at once
     const uint32_t grid = (p.finish_launch ? tiles * p.splits + 7u : tiles + 7u) / 8u * 8u;
-    void (*kernel)(const GemmParams) = bfaintb_prefill128_wreg_kernel<BITS, GROUPED, PACKED, MT, NS, COPIER>;
-    const hipError_t e = launch_kernel(kernel, dim3(grid, p.finish_launch ? 1u : p.splits, 1), dim3(COPIER ? 576 : 512, 1, 1), 0, stream, p);
+    auto kernel = bfaintb_prefill128_wreg_kernel<BITS, GROUPED, PACKED, MT, NS, COPIER>;
+    const hipError_t e = launch_kernel(kernel, dim3(grid, p.finish_launch ? 1u : p.splits, 1), dim3(COPIER ? 576 : 512, 1, 1), 0, stream, p.b, p.a, p.scale, p.m, p.n, p.k,
+                                       p.lda, p.ldb_bytes, p.k_per_wg, p.splits, p.finish_launch, p);
     if (e != hipSuccess || !p.finish_launch) return e;
     return launch_kernel(bfaintb_split_finish_kernel, dim3((p.m * (p.n / 4u) + 255u) / 256u, 1, 1), dim3(256, 1, 1), 0, stream, p);
 }
