@@ -504,13 +504,9 @@ template <int BITS, int CPL, int MB, bool GROUPED, bool PACKED, bool REF>
 // (packed 4-bit codes always run 4 waves: with 8 — their registers would allow it for one block of 16 rows — the 256-column
 // kernel over packed weights is slower, 28672 x 8192, m = 16: 55 against 42 us)
 __global__ void __launch_bounds__((MB <= 2 && (CPL <= 8 || MB == 1) && !(PACKED && BITS == 4 && CPL == 16)) ? 512 : 256)
-bfaintb_decode_kernel(const uint8_t* b, const uint16_t* a, const uint16_t* scale, const uint32_t m, const uint32_t n, const uint32_t k, const uint32_t lda,
-                      const uint32_t ldb_bytes, const uint32_t k_per_wg, const uint32_t nwaves, const GemmParams rest)
+bfaintb_decode_kernel(const u32x4_t addresses, const u32x4_t sizes, const u32x4_t strides, const uint32_t nwaves, const GemmParams rest)
 {
-    // What the first loads need comes in scalar registers with the launch (the Makefile asks for it): a workgroup of a launch whose arguments are
-    // new waits 0.2 to 0.4 us for the rest of them, which is read from memory.
-    GemmParams p = rest;
-    p.b = b, p.a = a, p.scale = scale, p.m = m, p.n = n, p.k = k, p.lda = lda, p.ldb_bytes = ldb_bytes, p.k_per_wg = k_per_wg;
+    const GemmParams p = with_words(rest, addresses, sizes, strides);
     static_assert(CPL == 16 || CPL == 8 || (PACKED && CPL >= 5 && CPL < 8 && MB <= 2), "the forms there are");
     static_assert(!REF || (BITS == 8 && !GROUPED && !PACKED), "the reference's arithmetic: 8-bit codes, row-major, one scale per column");
     constexpr int KB = decode_blocks_per_step(BITS, CPL, PACKED, MB);  // blocks of 32 rows per pipeline step
@@ -974,7 +970,7 @@ static hipError_t launch_decode_t(const GemmParams& p, hipStream_t stream)
     }
     if (lds > 160 * 1024 - 64) return hipErrorInvalidValue;
     auto kernel = bfaintb_decode_kernel<BITS, CPL, MB, GROUPED, PACKED, REF>;
-    return launch_kernel(kernel, grid, dim3(64 * waves, 1, 1), lds, stream, q.b, q.a, q.scale, q.m, q.n, q.k, q.lda, q.ldb_bytes, q.k_per_wg, waves, q);
+    return launch_kernel(kernel, grid, dim3(64 * waves, 1, 1), lds, stream, words_of_addresses(q), words_of_sizes(q), words_of_strides(q), waves, q);
 }
 
 template <int BITS, int CPL, bool PACKED>

@@ -115,6 +115,35 @@ struct GemmParams {
 #endif
 };
 
+// What a kernel's first loads need, ahead of its GemmParams: these words come in scalar registers with the launch (the Makefile asks for it), where a
+// workgroup of a launch whose arguments are new waits 0.2 to 0.4 us for the rest of them, which is read from memory.
+// As vectors, and addresses as numbers: the runtime takes each argument by itself and looks each pointer up.  Host time of a launch, us: the struct alone
+// 3.65, with three pointers and eight words ahead of it 3.91, with eleven numbers 3.78, with three vectors of four words and one of two 3.63.
+inline u32x4_t words_of_addresses(const GemmParams& p)
+{
+    const unsigned long long b = reinterpret_cast<unsigned long long>(p.b), a = reinterpret_cast<unsigned long long>(p.a);
+    return u32x4_t{(uint32_t)b, (uint32_t)(b >> 32), (uint32_t)a, (uint32_t)(a >> 32)};
+}
+inline u32x4_t words_of_sizes(const GemmParams& p)
+{
+    const unsigned long long scale = reinterpret_cast<unsigned long long>(p.scale);
+    return u32x4_t{(uint32_t)scale, (uint32_t)(scale >> 32), p.m, p.n};
+}
+inline u32x4_t words_of_strides(const GemmParams& p) { return u32x4_t{p.k, p.lda, p.ldb_bytes, p.k_per_wg}; }
+__device__ __forceinline__ GemmParams with_words(const GemmParams& rest, const u32x4_t addresses, const u32x4_t sizes, const u32x4_t strides)
+{
+    GemmParams p = rest;
+    // (in device memory, as the pointers of a struct argument are known to be: left open, their loads would be of the slower kind)
+    auto address = [](uint32_t lo, uint32_t hi) {
+        return (const uint8_t*)(__attribute__((address_space(1))) const uint8_t*)(((unsigned long long)hi << 32) | lo);
+    };
+    p.b = address(addresses[0], addresses[1]);
+    p.a = reinterpret_cast<const uint16_t*>(address(addresses[2], addresses[3]));
+    p.scale = reinterpret_cast<const uint16_t*>(address(sizes[0], sizes[1]));
+    p.m = sizes[2], p.n = sizes[3], p.k = strides[0], p.lda = strides[1], p.ldb_bytes = strides[2], p.k_per_wg = strides[3];
+    return p;
+}
+
 // The scale group of a row of B.  The kernels ask for it per block of 32 rows inside their inner loops, where a division
 // by the run-time group size (some 25 dependent scalar instructions) stalls the one wave of a SIMD for longer than a
 // matrix instruction runs: 128x128 tiles, groups of 128 rows, 640 x 4096 x 4096: 41.5 us with the division, 36.8 without.

@@ -881,11 +881,10 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
 // ids, which walk groups of 8 tile-rows column by column).
 template <int BITS, bool GROUPED, bool PACKED, int MT, int NS, bool COPIER>
 __global__ void __launch_bounds__(COPIER ? 576 : 512) __attribute__((amdgpu_waves_per_eu(COPIER ? 3 : 2, COPIER ? 3 : 2)))
-bfaintb_prefill128_wreg_kernel(const uint8_t* b, const uint16_t* a, const uint16_t* scale, const uint32_t m, const uint32_t n, const uint32_t k, const uint32_t lda,
-                               const uint32_t ldb_bytes, const uint32_t k_per_wg, const uint32_t splits, const uint32_t finish_launch, const GemmParams rest)
+bfaintb_prefill128_wreg_kernel(const u32x4_t addresses, const u32x4_t sizes, const u32x4_t strides, const u32x2_t in_splits, const GemmParams rest)
 {
-    GemmParams p = rest;  // (what the first copies need comes in scalar registers with the launch: see bfaintb_decode_kernel)
-    p.b = b, p.a = a, p.scale = scale, p.m = m, p.n = n, p.k = k, p.lda = lda, p.ldb_bytes = ldb_bytes, p.k_per_wg = k_per_wg, p.splits = splits, p.finish_launch = finish_launch;
+    GemmParams p = with_words(rest, addresses, sizes, strides);
+    p.splits = in_splits[0], p.finish_launch = in_splits[1];
     constexpr bool kScales = GROUPED && MT <= 12;  // (a larger tile leaves no room in LDS)
     const uint32_t tiles_m = (p.m + 16u * MT - 1u) / (16u * MT), tiles_n = (p.n + kTw - 1u) / kTw;
     const uint32_t wgs = tiles_m * tiles_n;
@@ -962,8 +961,8 @@ static hipError_t launch_prefill128_wreg_t(const GemmParams& p, hipStream_t stre
     // a whole number of workgroups per XCD; ids past the last tile exit at once
     const uint32_t grid = (p.finish_launch ? tiles * p.splits + 7u : tiles + 7u) / 8u * 8u;
     auto kernel = bfaintb_prefill128_wreg_kernel<BITS, GROUPED, PACKED, MT, NS, COPIER>;
-    const hipError_t e = launch_kernel(kernel, dim3(grid, p.finish_launch ? 1u : p.splits, 1), dim3(COPIER ? 576 : 512, 1, 1), 0, stream, p.b, p.a, p.scale, p.m, p.n, p.k,
-                                       p.lda, p.ldb_bytes, p.k_per_wg, p.splits, p.finish_launch, p);
+    const hipError_t e = launch_kernel(kernel, dim3(grid, p.finish_launch ? 1u : p.splits, 1), dim3(COPIER ? 576 : 512, 1, 1), 0, stream, words_of_addresses(p),
+                                       words_of_sizes(p), words_of_strides(p), u32x2_t{p.splits, p.finish_launch}, p);
     if (e != hipSuccess || !p.finish_launch) return e;
     return launch_kernel(bfaintb_split_finish_kernel, dim3((p.m * (p.n / 4u) + 255u) / 256u, 1, 1), dim3(256, 1, 1), 0, stream, p);
 }
