@@ -698,8 +698,9 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
     }
     // The residual's rows of a part are requested together, a part ahead of their use: row by row, each behind the store of the row before,
     // their trips to memory stood one behind the other with nothing else on the CU.  What bounds the part behind the loop is the residual's and
-    // the outputs' bytes (us, with the sums' rows turned in LDS as well: 4096 x 4096 x 4096 8-bit 109.9 -> 104.9, 577 x 13824 x 5120 packed 4-bit
-    // 87.9 -> 84.8; the same calls without a residual 101.5 and 82).
+    // the outputs' bytes (us, row by row / so: 4096 x 4096 x 4096 8-bit 111.8 / 106.6, 2048 x 22016 x 4096 8-bit 334 / 297, 577 x 13824 x 5120 packed 4-bit
+    // 91.8 / 88.2).  The staged rows are not turned against their bank conflicts: it is level or slower (768 x 28672 x 1024 packed 4-bit 60.8 turned, 60.0 so;
+    // 4-bit 1500 x 16384 x 1024 behind a gate 58.1 / 57.7).
     constexpr uint32_t kBlocksHeld = 6u * MT / 16u, kParts = (MT + kBlocksHeld - 1u) / kBlocksHeld;
     uint4 residual[2][2u * kBlocksHeld];
     auto request_part = [&](auto part_c) {
@@ -723,17 +724,15 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
 #pragma unroll
             for (uint32_t r = 0; r < 4; ++r)
 #pragma unroll
-                for (uint32_t j = 0; j < 4; ++j) base[r * kWrTile + ((wcol + 16u * j) ^ (kq << 4))] = acc[j][r];  // (turned by the row: the four kq write rows 4 apart)
+                for (uint32_t j = 0; j < 4; ++j) base[r * kWrTile + wcol + 16u * j] = acc[j][r];
         });
         if constexpr (decltype(part_c)::value + 1u < kParts) request_part(std::integral_constant<uint32_t, decltype(part_c)::value + 1u>{});
         __syncthreads();
-#pragma unroll
-        for (uint32_t pass = 0; pass < 2u * blocks; ++pass) {
-            const uint4 r = residual[decltype(part_c)::value & 1u][pass];
+        auto finish = [&](uint32_t pass, const uint4& r, auto added_c) {
             const uint32_t row = pass * 8u + (tid >> 5);  // within the part
             const uint32_t gm = m0 + 16u * first + row;
-            if (gm >= p.m || gn >= p.n) continue;
-            const float* src = reinterpret_cast<const float*>(c_rows4(row >> 2, MT / 2u, kWrTile * 4u)) + (row & 3u) * kWrTile + ((8u * ch) ^ (((row >> 2) & 3u) << 4));
+            if (gm >= p.m || gn >= p.n) return;
+            const float* src = reinterpret_cast<const float*>(c_rows4(row >> 2, MT / 2u, kWrTile * 4u)) + (row & 3u) * kWrTile + 8u * ch;
             const float4 lo = *reinterpret_cast<const float4*>(src), hi = *reinterpret_cast<const float4*>(src + 4);
             float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
 #pragma unroll
@@ -742,7 +741,8 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
                 float o[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) o[i] = silu_gate(v[2 * i], v[2 * i + 1]);
-                if (p.residual != nullptr) {
+                if constexpr (decltype(added_c)::value) {
+#pragma clang fp contract(off)  // (added to the rounded product, as by every other kernel)
                     o[0] += bf16_bits_to_f32(r.x & 0xffffu);
                     o[1] += bf16_bits_to_f32(r.x >> 16);
                     o[2] += bf16_bits_to_f32(r.y & 0xffffu);
@@ -759,6 +759,15 @@ __global__ void __launch_bounds__(256) bfaintb_prefill_wreg_kernel(const GemmPar
                 *reinterpret_cast<uint4*>(p.c + (size_t)gm * p.ldc + gn) =
                     make_uint4(pack_bf16_rne(v[0], v[1]), pack_bf16_rne(v[2], v[3]), pack_bf16_rne(v[4], v[5]), pack_bf16_rne(v[6], v[7]));
             }
+        };
+        // (Unrolled, the residual's registers have their places.  A gate alone has none and stays a loop: unrolled and turned / so, us, 1500 x 16384 x 1024 4-bit
+        // g64 58.9 / 57.7, 768 x 28672 x 1024 packed 4-bit 57.2 / 56.2, 2048 x 12288 x 1024 4-bit 61.8 / 59.3; 8-bit 60.9 / 60.0.)
+        if (p.residual != nullptr) {
+#pragma unroll
+            for (uint32_t pass = 0; pass < 2u * blocks; ++pass) finish(pass, residual[decltype(part_c)::value & 1u][pass], std::true_type{});
+        } else {
+#pragma unroll 4
+            for (uint32_t pass = 0; pass < 2u * blocks; ++pass) finish(pass, make_uint4(0u, 0u, 0u, 0u), std::false_type{});
         }
         __syncthreads();  // the next part overwrites the staging area
     });

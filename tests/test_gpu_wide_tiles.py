@@ -77,6 +77,30 @@ def test_epilogues_and_strides(units64, rows, m, n, bits, group):
     assert_close_gated(g, run_gemm(g, activation=af.ACT_SILU_GATE), "gated")
 
 
+@pytest.mark.parametrize("rows,m,n", HEIGHTS)
+@pytest.mark.parametrize("bits,group", [(8, 0), (4, 128)])
+def test_the_gate_alone_and_with_a_residual(units64, rows, m, n, bits, group):
+    """A gate alone is finished in a loop, one with a residual written out: the same sums (a residual of zeros changes no bit but a zero's sign), rows of
+    the residual longer than they need be and NaN behind, in place."""
+    from test_gpu_residual_rows import run
+    af, k = units64, 384
+    g = Problem(m, n, k, bits, group, seed=3, scale_lo=0.002, scale_hi=0.02 if bits == 8 else 0.2).with_bias()
+    is_wide(af, rows, g)
+    alone = run(af, g, False, None, None, activation=af.ACT_SILU_GATE)
+    assert_close_gated(g, alone, "gate")
+    longer = np.full((m, n // 2 + 8), 0x7FC0, np.uint16)
+    longer[:, :n // 2] = 0
+    zeros = run(af, g, False, to_dev(longer), n // 2 + 8, activation=af.ACT_SILU_GATE)
+    assert np.array_equal(zeros, np.where(alone == 0x8000, 0, alone))
+    g.with_residual()
+    g.residual_bf = np.ascontiguousarray(g.residual_bf[:, :n // 2])
+    longer[:, :n // 2] = g.residual_bf
+    c = run(af, g, False, to_dev(longer), n // 2 + 8, activation=af.ACT_SILU_GATE)
+    assert_close_gated(g, c, "gate and residual")
+    own = to_dev(g.residual_bf).clone()
+    assert np.array_equal(run(af, g, True, own, n // 2, own, activation=af.ACT_SILU_GATE), c), "in place, packed"
+
+
 # beyond 2^117 8-bit codes go a second way along k
 @pytest.mark.parametrize("rows,m,n", HEIGHTS)
 @pytest.mark.parametrize("bits,group,k", [(8, 0, 200), (8, 64, 384), (4, 0, 320), (4, 128, 384)])
