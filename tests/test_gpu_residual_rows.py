@@ -8,10 +8,73 @@ from helpers import Problem, assert_close_gated, assert_close_ulp, from_dev_u16,
 
 pytestmark = pytest.mark.gpu
 
-# decode with two fetch attempts in flight (two splits; eight), with one (rows beyond a thread's), unsplit; small tiles unsplit, split, with a second
-# launch, with the copying wave; tall tiles; 256 x 128; 256 columns (eight blocks; sixteen)
-CALLS = [(3, 4112, 2048, 8, 0), (16, 1040, 4096, 8, 0), (29, 2064, 4096, 8, 0), (5, 208, 96, 8, 0), (17, 22032, 256, 4, 128), (61, 16400, 256, 8, 0), (97, 2064, 2048, 8, 0),
-         (33, 1040, 4096, 8, 0), (300, 1040, 2048, 8, 64), (500, 12304, 320, 4, 64), (600, 12304, 2112, 8, 0), (1100, 4112, 512, 8, 0), (130, 33040, 576, 8, 0), (2100, 8208, 128, 4, 128)]
+FAMILY, SLAB, SMALL, TALL, WIDE = 1, 2, 3, 5, 6  # af.KERNEL_DECODE_FAMILY, _DECODE_SLAB, _TILES_128, _TILES_256X128, _TILES_256
+
+# m, n, k, bits, group, compute units planned for (0: all), and what runs, row-major and packed: kernel, rows and columns of a tile, waves, splits, launches,
+# workgroups of the thin last round
+CALLS = [
+    # the row-blocked family: unsplit; the sums of 2, 4, 6 and 8 splits fetched by two attempts in flight; by one (nine splits; tiles of 256 columns; two rows
+    # a thread); a packed call of one row block on the slab kernel
+    (5, 208, 96, 8, 0, 0, (FAMILY, 16, 128, 8, 1, 1, 0), None),
+    (13, 208, 320, 8, 0, 0, (FAMILY, 16, 128, 8, 2, 1, 0), (SLAB, 16, 16, 8, 1, 1, 0)),
+    (5, 208, 1024, 8, 0, 0, (FAMILY, 16, 128, 8, 4, 1, 0), (SLAB, 16, 16, 8, 1, 1, 0)),
+    (16, 1040, 4096, 8, 0, 0, (FAMILY, 16, 128, 8, 8, 1, 0), (SLAB, 16, 16, 8, 1, 1, 0)),
+    (3, 208, 2112, 8, 0, 0, (FAMILY, 16, 128, 8, 9, 1, 0), (SLAB, 16, 16, 8, 1, 1, 0)),
+    (29, 2064, 4096, 8, 0, 0, (FAMILY, 16, 128, 8, 6, 1, 0), (FAMILY, 16, 80, 8, 4, 1, 0)),
+    (13, 16400, 2048, 8, 0, 0, (FAMILY, 16, 256, 4, 3, 1, 0), (FAMILY, 16, 80, 8, 1, 1, 0)),
+    (29, 16400, 2112, 8, 64, 0, (FAMILY, 32, 256, 4, 2, 1, 0), (FAMILY, 32, 80, 8, 1, 1, 0)),
+    (33, 208, 512, 8, 0, 16, (FAMILY, 32, 128, 8, 2, 1, 0), (FAMILY, 16, 128, 8, 1, 1, 0)),
+    (61, 208, 4096, 8, 64, 32, (FAMILY, 32, 128, 8, 8, 1, 0), (FAMILY, 32, 128, 8, 8, 1, 0)),
+    (33, 1040, 96, 8, 0, 8, (FAMILY, 64, 128, 4, 1, 1, 0), None),
+    (13, 12304, 4096, 4, 128, 0, (FAMILY, 16, 256, 8, 4, 1, 0), (FAMILY, 16, 128, 8, 2, 1, 0)),
+    # tiles of 128 columns: unsplit and split in one launch, with the copying wave and without, 32 to 128 rows; with a second launch; 160 to 256 rows
+    (17, 528, 1280, 8, 0, 8, (SMALL, 32, 128, 9, 1, 1, 0), (FAMILY, 16, 80, 8, 1, 1, 0)),
+    (17, 528, 1280, 4, 128, 8, (SMALL, 32, 128, 9, 1, 1, 0), (SMALL, 32, 128, 9, 1, 1, 0)),
+    (33, 208, 96, 8, 0, 0, (SMALL, 64, 128, 8, 1, 1, 0), None),
+    (64, 6160, 256, 4, 128, 0, (SMALL, 64, 128, 8, 1, 1, 0), (SMALL, 64, 128, 9, 1, 1, 0)),
+    (33, 1072, 1280, 8, 64, 16, (SMALL, 64, 128, 8, 1, 1, 0), (SMALL, 64, 128, 9, 1, 1, 0)),
+    (33, 6160, 2048, 8, 0, 0, (SMALL, 64, 128, 8, 2, 1, 0), (FAMILY, 32, 128, 8, 2, 1, 0)),
+    (33, 8240, 2048, 8, 64, 0, (SMALL, 64, 128, 8, 2, 1, 0), (SMALL, 64, 128, 9, 2, 1, 0)),
+    (33, 4112, 4096, 8, 64, 128, (SMALL, 64, 128, 8, 3, 1, 0), (FAMILY, 16, 128, 8, 1, 1, 0)),
+    (33, 6160, 4096, 8, 0, 0, (SMALL, 64, 128, 8, 4, 1, 0), (FAMILY, 64, 128, 4, 4, 1, 0)),
+    (257, 208, 2048, 8, 64, 16, (SMALL, 96, 128, 9, 2, 1, 0), (SMALL, 96, 128, 9, 2, 1, 0)),
+    (257, 208, 2048, 8, 0, 16, (SMALL, 96, 128, 8, 2, 1, 0), (SMALL, 96, 128, 8, 2, 1, 0)),
+    (257, 528, 4096, 4, 64, 64, (SMALL, 96, 128, 9, 3, 1, 0), (FAMILY, 32, 128, 8, 1, 1, 0)),
+    (385, 208, 2048, 8, 0, 16, (SMALL, 128, 128, 8, 2, 1, 0), (SMALL, 128, 128, 8, 2, 1, 0)),
+    (300, 208, 4096, 4, 64, 32, (SMALL, 128, 128, 9, 4, 1, 0), (FAMILY, 32, 128, 8, 1, 1, 0)),
+    (300, 208, 2048, 8, 64, 16, (SMALL, 128, 128, 9, 2, 1, 0), (FAMILY, 64, 128, 4, 1, 1, 0)),
+    (97, 528, 4096, 4, 64, 16, (SMALL, 128, 128, 8, 2, 1, 0), (SMALL, 128, 128, 9, 2, 1, 0)),
+    (97, 208, 1280, 4, 128, 0, (SMALL, 128, 128, 8, 7, 2, 0), (SMALL, 128, 128, 9, 7, 2, 0)),
+    (300, 1040, 2048, 8, 64, 0, (SMALL, 128, 128, 9, 6, 2, 0), (FAMILY, 16, 128, 8, 1, 1, 0)),
+    (300, 208, 256, 8, 64, 8, (SMALL, 128, 128, 8, 1, 1, 0), (SMALL, 128, 128, 9, 1, 1, 0)),
+    (130, 528, 2112, 8, 0, 8, (SMALL, 160, 128, 8, 1, 1, 0), (SMALL, 160, 128, 8, 1, 1, 0)),
+    (161, 528, 1280, 8, 64, 8, (SMALL, 192, 128, 8, 1, 1, 0), (FAMILY, 64, 128, 4, 1, 1, 0)),
+    (200, 528, 1280, 4, 128, 8, (SMALL, 256, 128, 8, 1, 1, 0), (FAMILY, 64, 128, 4, 1, 1, 0)),
+    (200, 528, 1280, 8, 64, 8, (SMALL, 256, 128, 8, 1, 1, 0), (SMALL, 256, 128, 8, 1, 1, 0)),
+    # 256 x 128, in one chain
+    (641, 208, 256, 4, 64, 8, (TALL, 256, 128, 4, 1, 1, 0), (TALL, 256, 128, 4, 1, 1, 0)),
+    (200, 528, 256, 8, 0, 8, (TALL, 256, 128, 4, 1, 1, 0), (TALL, 256, 128, 4, 1, 1, 0)),
+    # tiles of 256 columns, 128 to 256 rows; the thin last round of the 256-row ones as halves
+    (97, 1040, 1024, 8, 64, 8, (WIDE, 128, 256, 4, 1, 1, 0), (WIDE, 128, 256, 4, 1, 1, 0)),
+    (97, 1040, 1024, 4, 64, 8, (WIDE, 128, 256, 4, 1, 1, 0), (WIDE, 128, 256, 4, 1, 1, 0)),
+    (385, 8208, 256, 8, 64, 64, (WIDE, 160, 256, 4, 1, 1, 0), (WIDE, 160, 256, 4, 1, 1, 0)),
+    (500, 8208, 256, 8, 0, 64, (WIDE, 192, 256, 4, 1, 1, 0), (WIDE, 192, 256, 4, 1, 1, 0)),
+    (385, 12304, 256, 4, 64, 8, (WIDE, 224, 256, 4, 1, 1, 0), (WIDE, 224, 256, 4, 1, 1, 0)),
+    (130, 1040, 256, 8, 64, 8, (WIDE, 256, 256, 4, 1, 1, 0), (WIDE, 256, 256, 4, 1, 1, 0)),
+    (385, 1296, 256, 8, 0, 8, (WIDE, 256, 256, 4, 1, 2, 8), (WIDE, 256, 256, 4, 1, 2, 8)),
+    (512, 1552, 384, 4, 128, 8, (WIDE, 256, 256, 4, 1, 1, 0), (WIDE, 256, 256, 4, 1, 1, 0)),
+    # larger ones
+    (3, 4112, 2048, 8, 0, 0, (FAMILY, 16, 128, 8, 4, 1, 0), (SLAB, 16, 16, 8, 1, 1, 0)),
+    (17, 22032, 256, 4, 128, 0, (FAMILY, 32, 128, 8, 1, 1, 0), (FAMILY, 16, 128, 8, 1, 1, 0)),
+    (61, 16400, 256, 8, 0, 0, (SMALL, 64, 128, 8, 1, 1, 0), (FAMILY, 64, 128, 4, 1, 1, 0)),
+    (97, 2064, 2048, 8, 0, 0, (SMALL, 128, 128, 8, 8, 2, 0), (FAMILY, 16, 128, 8, 2, 1, 0)),
+    (33, 1040, 4096, 8, 0, 0, (FAMILY, 16, 128, 8, 8, 1, 0), (FAMILY, 16, 128, 8, 8, 1, 0)),
+    (500, 12304, 320, 4, 64, 0, (TALL, 256, 128, 4, 1, 1, 0), None),
+    (600, 12304, 2112, 8, 0, 0, (SMALL, 128, 128, 8, 1, 1, 0), (SMALL, 128, 128, 8, 1, 1, 0)),
+    (1100, 4112, 512, 8, 0, 0, (TALL, 256, 128, 4, 1, 1, 0), (TALL, 256, 128, 4, 1, 1, 0)),
+    (130, 33040, 576, 8, 0, 0, (WIDE, 160, 256, 4, 1, 1, 0), (WIDE, 160, 256, 4, 1, 1, 0)),
+    (2100, 8208, 128, 4, 128, 0, (WIDE, 160, 256, 4, 1, 1, 0), (WIDE, 160, 256, 4, 1, 1, 0)),
+]
 
 
 def run(af, p, packed, residual, ldr, c=None, activation=0):
@@ -30,12 +93,26 @@ def run(af, p, packed, residual, ldr, c=None, activation=0):
     return from_dev_u16(c)
 
 
-@pytest.mark.parametrize("m,n,k,bits,group", CALLS)
-def test_residual_of_longer_rows(m, n, k, bits, group):
+def what_runs(af, m, n, k, bits, group, packed):
+    pl = af.plan(m, n, k, bits, group, packed=packed)
+    return pl.kernel, pl.tile_rows, pl.tile_cols, pl.waves, pl.splits, pl.launches, pl.tail_workgroups
+
+
+@pytest.fixture
+def planned_for():
     import awesome_fusion_amd as af
-    for packed in (False, True):
-        if packed and k % (64 if bits == 8 else 128):
+    yield lambda units: af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, units)
+    af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 0)
+
+
+@pytest.mark.parametrize("m,n,k,bits,group,units,rows_form,packed_form", CALLS)
+def test_residual_of_longer_rows(planned_for, m, n, k, bits, group, units, rows_form, packed_form):
+    import awesome_fusion_amd as af
+    planned_for(units)
+    for packed, form in ((False, rows_form), (True, packed_form)):
+        if form is None:  # (no packed order for such a k)
             continue
+        assert what_runs(af, m, n, k, bits, group, packed) == form
         p = Problem(m, n, k, bits, group, seed=m + n).with_residual()
         longer = np.full((m, n + 40), 0x7FC0, np.uint16)
         longer[:, :n] = p.residual_bf
@@ -45,9 +122,11 @@ def test_residual_of_longer_rows(m, n, k, bits, group):
         assert np.array_equal(run(af, p, packed, own, n, own), c), "in place"
         p.with_bias()
         assert_close_ulp(p, run(af, p, packed, to_dev(longer), n + 40), "bias and residual", threads=16)
-        if n % 16 == 0:
-            g = Problem(m, n, k, bits, group, seed=5, scale_lo=0.002, scale_hi=0.02 if bits == 8 else 0.2).with_bias().with_residual()
-            g.residual_bf = np.ascontiguousarray(g.residual_bf[:, :n // 2])
-            longer = np.full((m, n // 2 + 40), 0x7FC0, np.uint16)
-            longer[:, :n // 2] = g.residual_bf
-            assert_close_gated(g, run(af, g, packed, to_dev(longer), n // 2 + 40, activation=af.ACT_SILU_GATE), "gated", threads=16)
+        g = Problem(m, n, k, bits, group, seed=5, scale_lo=0.002, scale_hi=0.02 if bits == 8 else 0.2).with_bias().with_residual()
+        g.residual_bf = np.ascontiguousarray(g.residual_bf[:, :n // 2])
+        longer = np.full((m, n // 2 + 40), 0x7FC0, np.uint16)
+        longer[:, :n // 2] = g.residual_bf
+        c = run(af, g, packed, to_dev(longer), n // 2 + 40, activation=af.ACT_SILU_GATE)
+        assert_close_gated(g, c, "gated", threads=16)
+        own = to_dev(g.residual_bf).clone()
+        assert np.array_equal(run(af, g, packed, own, n // 2, own, activation=af.ACT_SILU_GATE), c), "gated, in place"

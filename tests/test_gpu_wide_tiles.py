@@ -153,3 +153,38 @@ def test_the_thin_last_round(m, n, bits, group, k):
             assert np.array_equal(run_packed(af, p, af.PREFILL_256), c), "packed"
     finally:
         af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 0)
+
+
+# the same with bias, residual (rows longer than they need be and NaN behind; in place) and the gate, by the library's own choice: last rows of tiles whose lower
+# half is empty, one row, whole, and a row of tiles of 129 rows behind two whole ones
+@pytest.mark.parametrize("m,n", [(383, 1296), (384, 1040), (385, 1296), (512, 1536), (641, 1296)])
+@pytest.mark.parametrize("bits,group,k", [(8, 0, 256), (4, 128, 384), (8, 64, 448)])
+def test_epilogues_of_the_thin_last_round(m, n, bits, group, k):
+    import awesome_fusion_amd as af
+    from test_gpu_residual_rows import run
+    af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 8)
+    try:
+        tiles = -(-m // 256) * -(-n // 256)
+        rest = tiles % 8
+        for packed in (False, True):
+            pl = af.plan(m, n, k, bits, group, packed=packed)
+            assert (pl.kernel, pl.tile_rows, pl.workgroups, pl.tail_workgroups) == (af.KERNEL_TILES_256, 256, tiles - rest, 2 * rest), pl.as_dict()
+            p = Problem(m, n, k, bits, group, seed=m + n).with_residual()
+            longer = np.full((m, n + 8), 0x7FC0, np.uint16)
+            longer[:, :n] = p.residual_bf
+            c = run(af, p, packed, to_dev(longer), n + 8)
+            assert_close_ulp(p, c, "residual", threads=16)
+            own = to_dev(p.residual_bf).clone()
+            assert np.array_equal(run(af, p, packed, own, n, own), c), "in place"
+            p.with_bias()
+            assert_close_ulp(p, run(af, p, packed, to_dev(longer), n + 8), "bias and residual", threads=16)
+            p.residual_bf = None
+            assert_close_ulp(p, run(af, p, packed, None, None), "bias", threads=16)
+            g = Problem(m, n, k, bits, group, seed=5, scale_lo=0.002, scale_hi=0.02 if bits == 8 else 0.2).with_bias()
+            assert_close_gated(g, run(af, g, packed, None, None, activation=af.ACT_SILU_GATE), "gate", threads=16)
+            g.with_residual()
+            g.residual_bf = np.ascontiguousarray(g.residual_bf[:, :n // 2])
+            own = to_dev(g.residual_bf).clone()
+            assert_close_gated(g, run(af, g, packed, own, n // 2, own, activation=af.ACT_SILU_GATE), "gate and residual, in place", threads=16)
+    finally:
+        af.debug_control(af.DEBUG_PLAN_COMPUTE_UNITS, 0)
