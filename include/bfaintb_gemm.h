@@ -155,7 +155,8 @@ BFAINTB_API int bfaintb_gemm_bias(void* c, const void* a, const void* b, const v
  * bfaintb_gemm.  The reference kernel stores the bare sums (bf16gemm_kernel_gfx90a.s:594-630);
  * these are the first epilogues of the reference's stated purpose, "gemm fusion for llm" (README.md:2): a linear layer's
  * bias and a transformer block's residual connection, without a second pass over C.  The residual may alias c when
- * ldr == ldc (every element is read by the thread that then writes it).
+ * ldr == ldc (every element that is added is read by the thread that then writes it; behind the gate a thread may read the two outputs beside its own
+ * as well, whose values it does not use).
  */
 typedef struct bfaintb_epilogue {
     const void* bias;
