@@ -414,6 +414,7 @@ __device__ __forceinline__ void reduce_splits(const GemmParams& p, const float4 
 // The selection of the winning attempt is written as copies under uniform branches: indexing the two register sets by a
 // run-time flag sent both through scratch memory (0.8 us at m = 1, 5 us at m = 16).
 constexpr int kPollGap = 8;
+constexpr int kWaitVmcnt0 = 0x0f70;  // s_waitcnt's immediate: vmcnt 0, no wait for the other counters
 template <uint32_t NL, uint32_t NSUM>
 __device__ __forceinline__ void reduce_splits_two_in_flight(const GemmParams& p, const float4 (&sum)[NSUM], uint32_t first_row, uint32_t rows,
                                                             uint32_t rs, uint32_t col, bool col_ok)
@@ -441,8 +442,8 @@ __device__ __forceinline__ void reduce_splits_two_in_flight(const GemmParams& p,
     };
     u32x4_t a[NL], b[NL];
     fetch(a);
-    // (Bias and residual come with the sums; asked for last, they waited behind the emptying stores as well: 8 x 4096 x 4096 with a residual
-    // 8.40 us, 8.06 so, 1 row 7.75 / 7.50.)
+    // (Bias and residual come with the sums; asked for last, they waited behind the emptying stores as well: a residual made a call 0.26 us longer at
+    // 1 x 4096 x 4096 8-bit, 0.25 at 40 x 2000 x 1408, and makes it none longer so.)
     Addends4 addends;
     request_addends4(addends, p, first_row + rs, col);
     __builtin_amdgcn_s_sleep(kPollGap);
@@ -472,8 +473,15 @@ __device__ __forceinline__ void reduce_splits_two_in_flight(const GemmParams& p,
     if ((threadIdx.x & 63) == 0) p.trace[((size_t)(blockIdx.y * gridDim.x + blockIdx.x) * (blockDim.x >> 6) + (threadIdx.x >> 6)) * 8 + 7] = tries;
     TRACE_MARK(1);
 #endif
+    // Everything requested has landed before the first emptying store: the compiler counts loads and stores together, and a wait that it needs for a
+    // register of the other attempt, or for an addend, further down would be one for those stores (three splits, nothing added, us with such a
+    // wait / so: 46 x 1456 x 1408 packed 8-bit 8.30 / 7.59, 40 x 2000 x 1408 8.60 / 7.96).  (The barrier, no instruction, keeps the wait one for every way
+    // out of the loop: divided among them it is not seen to hold for all.)
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_s_waitcnt(kWaitVmcnt0);
     if (!complete) __hip_atomic_store(p.ws_header, kWorkspaceGaveUp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const u32x4_t empty4 = {kEmptyWord, kEmptyWord, kEmptyWord, kEmptyWord};
+    u32x4_t empty4 = {kEmptyWord, kEmptyWord, kEmptyWord, kEmptyWord};
+    asm volatile("" : "+v"(empty4));
     float4 total = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
     for (uint32_t j = 0; j < NL; ++j) {
@@ -487,11 +495,11 @@ __device__ __forceinline__ void reduce_splits_two_in_flight(const GemmParams& p,
         }
     }
     finish_row4(p, make_float4(total.x + sum[0].x, total.y + sum[0].y, total.z + sum[0].z, total.w + sum[0].w), first_row + rs, col, addends);
-    // The attempt that did not win may still be in flight.  Its destination registers stay this function's until it has
-    // come back: with nothing holding them, the compiler handed them to the constants of the emptying stores above while
-    // the loads were still due to write them (a workspace word of the second split left holding a partial sum: found
-    // by the at-rest check of the test suite).  The wait is behind every store this thread issues, where it costs nothing.
+    // What the emptying stores send keeps its registers until they have gone: where the sums above took them over with the instruction behind a store,
+    // a word of the second split was left holding a sum (found by the at-rest check of the test suite).  The attempt that did not win keeps its own
+    // as well.  The wait is behind every store this thread issues, where it costs nothing.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("" ::"v"(empty4));
 #pragma unroll
     for (uint32_t j = 0; j < NL; ++j) asm volatile("" ::"v"(a[j]), "v"(b[j]));
 }

@@ -130,3 +130,28 @@ def test_residual_of_longer_rows(planned_for, m, n, k, bits, group, units, rows_
         assert_close_gated(g, c, "gated", threads=16)
         own = to_dev(g.residual_bf).clone()
         assert np.array_equal(run(af, g, packed, own, n // 2, own, activation=af.ACT_SILU_GATE), c), "gated, in place"
+
+
+# k in 2, 3, 4, 5 and 8 splits (the others' sums fetched by two attempts in flight), launch after launch over one workspace, with something added and without
+@pytest.mark.parametrize("k,split", [(320, 2), (768, 3), (1024, 4), (1280, 5), (2048, 8)])
+@pytest.mark.parametrize("m,n", [(16, 2064), (5, 656)])
+def test_the_workspace_is_at_rest_behind_an_epilogue(m, n, k, split):
+    import torch
+    import awesome_fusion_amd as af
+    p = Problem(m, n, k, seed=m + split).with_bias().with_residual()
+    assert what_runs(af, m, n, k, 8, 0, False) == (FAMILY, 16, 128, 8, split, 1, 0)
+    a, b, s, bias, residual = (to_dev(x) for x in (p.a_bf, p.b_bytes, p.s_bf, p.bias_bf, p.residual_bf))
+    ws = torch.empty(af.workspace_bytes(m, n, k), dtype=torch.uint8, device="cuda")
+    af.workspace_init(ws)
+    c, seen = torch.zeros((m, n), dtype=torch.int16, device="cuda"), {}
+    for launch in range(24):
+        added = launch % 3 != 2
+        af.gemm(c, a, b, s, m, n, k, workspace=ws, bias=bias if added else None, residual=residual if added else None)
+        torch.cuda.synchronize()
+        assert bool((ws[256:] == 0xFF).all()), f"split {split}, launch {launch}: not at rest"
+        got = from_dev_u16(c).copy()
+        assert np.array_equal(seen.setdefault(added, got), got), f"split {split}, launch {launch}"
+    assert_close_ulp(p, seen[True], f"split {split}, bias and residual", threads=16)
+    p.bias_bf = p.residual_bf = None
+    assert_close_ulp(p, seen[False], f"split {split}", threads=16)
+    assert af.workspace_status(ws) == 0
