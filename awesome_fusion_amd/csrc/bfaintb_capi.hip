@@ -423,8 +423,10 @@ static WideTiles wide_tiles_best(uint32_t m, uint32_t n, uint32_t k, int bits)
     }
     return best;
 }
-// The 256x256 tiles whose last round, if it is thin, runs as half tiles in a launch of its own (fitted to the same timings, 4 % rms, with halves of 256 x 128;
-// those of 128 x 256 that run now make the whole 1 to 3 % faster where they fill the machine and are level where they don't).
+// The 256x256 tiles whose last round, if it is thin, runs as half tiles in a launch of its own.  Fitted to the same timings, 4 % rms, while the halves were
+// 256 x 128, and not again: over 130 random shapes with a thin last round (257 ... 4096 rows, both code widths and weight orders) it stands 3 % higher beside
+// the estimate of the lower tiles than the times do, and the choice between them takes 0.2 % longer than the faster form on average, 4.8 % at worst; with the
+// halves at wide_tiles_us(8, 2 thin) + 2 us it would be 0.15 and 4.8.
 static double square_tiles_us(uint32_t m, uint32_t n, uint32_t k, int bits)
 {
     const uint32_t tiles = ((m + 255u) / 256u) * ((n + 255u) / 256u), thin = bfaintb::thin_round_tiles(tiles, m, machine_cus());

@@ -346,7 +346,8 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
             if constexpr (St < (uint32_t)NS) {
                 if (kt + St >= ksteps) return;
                 // the computing waves start this step behind this barrier: the copies of it and of the next have landed when at most
-                // those of the steps behind are in flight (a wait counts 63 at most)
+                // those of the steps behind are in flight (a wait counts 63 at most).  Steps 0 and 1 are not among this wave's: the computing waves'
+                // wait for all of theirs and the prologue's barrier cover them, and the count here begins with steps 2 .. kDepth - 1 in flight
                 constexpr uint32_t kAllowed = (kDepth - 2u) * kStepCopies;
                 asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAllowed < 63u ? kAllowed : 63u) : "memory");
                 barrier_no_fence();
@@ -546,7 +547,8 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
         });
     };
 
-    // ---- prologue: A tiles and codes of steps 0, 1, 2 -> stages 0, 1, 2; operands of step 0
+    // ---- prologue: A tiles and codes of the first steps -> their stages; operands of step 0.  Without the copying wave the computing waves request all of
+    // them, steps 0, 1 and 2 ahead of the first barrier.  With it they request steps 0 and 1 only, and it has requested the rest (see there).
     Ops ops0, ops1;
     if constexpr (kRing) {
 #pragma unroll
@@ -560,8 +562,8 @@ __device__ __forceinline__ void tw_tile(const GemmParams& p, const uint32_t m0, 
             dma_a(stage_c, clamp(St));
         }
     };
-    // (the first two steps' copies have to land before anything else happens: those of the last stages are issued behind that wait, a
-    // microsecond's work of the memory path)
+    // (The first two steps' copies have to land before anything else happens.  Without the copying wave those of the last stages are issued behind that
+    // wait, a microsecond's work of the memory path; with it they are under way meanwhile.)
     fetch(C0{}), fetch(C1{});
     if constexpr (COPIER) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -969,13 +971,15 @@ static hipError_t launch_prefill128_wreg_t(const GemmParams& p, hipStream_t stre
 
 // Whether a launch has the copying wave (p: the tile's blocks, the rows, the split and its share of k, the group size).  Always with two
 // blocks (see the head of the file), never with more than eight.  Otherwise, and with the fewer stages that its wait counts reach:
-// Over packed weights with grouped scales or 4-bit codes (us, without / with: 128 x 20480 x 4096 4-bit g128 35.1 / 31.7, 64 rows 28.1 / 24.9;
-// 8-bit g64 35.6 / 34.7 and 28.0 / 26.2; 4-bit, one scale per column, 33.5 / 31.6 and 23.6 / 22.9; not 8-bit, one scale per column: 34.6 /
-// 36.4 and 25.3 / 26.1, nor codes in rows: 38.7 / 39.2).
+// Over packed weights with grouped scales or 4-bit codes (us, without / with, both with the start as it is now: 128 x 20480 x 4096 4-bit g128 33.9 / 29.0,
+// 64 rows 24.4 / 22.4; 8-bit g64 35.5 / 33.3 and 26.2 / 24.8; 4-bit, one scale per column, 29.6 / 27.6 and 21.6 / 20.0; not 8-bit, one scale per column:
+// 31.5 / 32.2 and 24.5 / 23.6, nor codes in rows: 8-bit 39.1 / 38.6 and 31.1 / 30.3, 4-bit 37.9 / 38.0 and 29.3 / 29.4).
 // Codes in rows with grouped scales: where several rows of tiles split k into shares of up to 64 steps (without / with: 785 x 1440 x 4480
-// 8-bit 26.3 / 25.0, 4-bit 26.7 / 25.5; 400 x 2560 x 2560 19.9 / 18.8 and 20.3 / 19.2; 900 x 2048 x 8192 44.4 / 42.5 and 43.3 / 42.1; longer
-// shares lose what the start gains, 384 x 4096 x 11008 52.6 / 54.5 and 50.7 / 53.9, and so do unsplit ones, 640 x 4096 x 4096 8-bit 34.2 /
-// 35.9, and one row of tiles, 128 x 11008 x 4096 8-bit 26.7 / 28.5).
+// 8-bit 25.8 / 23.6, 4-bit 26.2 / 24.1; 400 x 2560 x 2560 19.4 / 17.9 and 19.4 / 18.3; 900 x 2048 x 8192 43.2 / 40.7 and 43.0 / 40.0; longer
+// shares lose what the start gains, 384 x 4096 x 11008 52.9 / 54.7 and 51.4 / 54.7, and so do most unsplit ones, 640 x 4096 x 4096 8-bit 33.8 /
+// 35.4, and one row of eight blocks, 128 x 11008 x 4096 8-bit 26.3 / 27.7).  The line was drawn before the wave had its own first copies; beyond it there
+// is now something to gain with four and six blocks of 8-bit codes in rows (64 x 8192 x 8192 26.4 / 25.0, 96 x 4096 x 11008 23.2 / 22.0, 64 x 11008 x 4096 g128 19.9 /
+// 18.9) and at 640 x 4096 x 4096 4-bit g128, 32.3 / 28.5.
 bool prefill128_wreg_copier(const GemmParams& p, int bits, bool packed)
 {
     const bool grouped = p.group_size != 0u;
